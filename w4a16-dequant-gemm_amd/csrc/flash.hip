@@ -429,7 +429,7 @@ hipError_t launch_flash(const FlashArgs& a, float* scratch, hipStream_t s) {
   hipError_t e;
   if (try_flash_mfma(a, pl, scratch, s, &e)) {
     if (e != hipSuccess) return e;
-    if (pl.nsplit == 1) return hipSuccess;  // that kernel wrote the output
+    if (pl.nsplit == 1 || flash_merges_in_place(a, pl)) return hipSuccess;  // that kernel wrote the output
     flash_phase2<<<(unsigned)(a.H * a.group), P2_THREADS, 0, s>>>(scratch, a.out, pl.nsplit, a.D);
     return hipGetLastError();
   }

@@ -21,9 +21,18 @@
 //            (D = 64 has only 8 element blocks for 16 operand rows: W4 lets lanes
 //            i and i + 8 split the elements of block i % 8 -- 4 MFMAs --, FP16 /
 //            FP8 repeat blocks 0..7 and drop the upper output rows.)
-// Whole tiles are fetched with buffer loads whose wave-uniform part lives in the
-// descriptor and the scalar offset; a ring of three raw tiles is refilled in
-// place, two tiles in flight while one is computed.
+// Tiles reach the wave in one of two ways.  Through registers: whole tiles are fetched with
+// buffer loads whose wave-uniform part lives in the descriptor and the scalar offset; a
+// ring of three raw tiles is refilled in place, two tiles in flight while one is computed.
+// Through LDS (W4 with few tiles per wave, FP8): a tile as registers need it is 21 load
+// instructions, most of them 2 or 4 bytes a lane, and a compute unit takes one such
+// instruction per 10 - 13 ns whatever it carries; at three tiles per wave eight waves had placed
+// their requests only after 3.7 - 6.3 us (time stamps, 128 slabs x 1500 positions, a call of
+// 14 us).  As global -> LDS loads of whole lines the same tile is 6 (FP8 10) instructions, read
+// back with conflict-free LDS reads.  Same registers, same arithmetic, same bytes either way.
+// Measured with the merge below and 16-byte query loads (one per MFMA instead of eight 2-byte
+// ones): 16.0 -> 14.1 us for those two, -> 12.7 us with the tiles through LDS; 32 slabs x 6007 FP8
+// 21.5 -> 19.4 -> 16.8 us.
 // Dequantisation is the bit-exact register step of dq.cuh (the k_out / v_out
 // hooks store those values); only the order of the FP32 sums differs from the
 // vector kernel.  The four waves of a workgroup interleave tiles of one split
@@ -41,6 +50,17 @@ constexpr int FM_TILE = 32;   // positions per wave tile
 constexpr int FM_WAVES = 4;
 constexpr int FM_DEPTH = 3;   // ring slots per wave: one tile computed, two in flight
 constexpr int FM_HEADS = 16;  // query heads per pass
+constexpr int FM_LDS_TILES = 12;  // W4: most tiles per wave that go through LDS (see go_kind)
+constexpr int FM_RING = 2;    // LDS slots per wave (three measured slower: 12.7 -> 13.1 us, FP8 16.8 -> 21.7)
+typedef __attribute__((address_space(3))) void* fm_lds;
+typedef __attribute__((address_space(4))) const uint32_t* fm_const_u32;  // read with scalar loads
+typedef __attribute__((address_space(4))) const int* fm_const_i32;
+// The merge by a slab's last workgroup (1.4 us from the last ticket to the output) replaces a
+// second launch of 3 - 3.5 us.  One workgroup reads all partials of a slab, so it stops paying:
+// 8 slabs x 8192 positions with 128 partials each took 11.5 us in place and 10.2 with the merge kernel.
+constexpr int FM_MERGE_SPLITS = 64;  // most splits of a slab that its last workgroup merges (one per lane)
+constexpr int FM_MERGE_MAX = 64;     // most (head, split) partials that one workgroup merges
+constexpr int FM_MERGE_SLABS = 512;  // more slabs than this are not merged in place
 
 // What one lane fetches for one tile, before expansion.
 // NC = D / 32: MFMAs per group of 16 positions = packed words (W4) per lane.
@@ -86,21 +106,36 @@ __device__ __forceinline__ h8 pack8(const h2 v[4]) {
   return h8{v[0][0], v[0][1], v[1][0], v[1][1], v[2][0], v[2][1], v[3][0], v[3][1]};
 }
 
+// Arrivals of a slab's splits, by number of splits and slab (see the end of the kernel).
+// Zero when the library is loaded and after every call.
+__device__ uint32_t flash_arrivals[(FM_MERGE_SPLITS + 1) * FM_MERGE_SLABS];
+
 // PAGED: 0 contiguous slabs, 1 pages of a multiple of 16 rows (both halves of a
 // tile lie in one page each), 2 any page size.  ALT: W4 with zero-points; FP8 with one
 // scale per slab instead of one per row.
-template <int KIND, int DH, bool HOOK, int PAGED, bool ALT>
+template <int KIND, int DH, bool HOOK, int PAGED, bool ALT, bool LDS>
 __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashArgs a,
                                                                    const int qh0,
                                                                    const int split_len,
-                                                                   float* __restrict__ part) {
+                                                                   float* __restrict__ part,
+                                                                   const int merge_here) {
   constexpr bool ASYM = KIND == KIND_W4 && ALT, SLAB_SCALE = KIND == KIND_F8 && ALT;
   constexpr int FM_D = DH;       // head dimension
   constexpr int NC = DH / 32;    // MFMAs per score group; a lane's K slice is 8 * NC elements
   constexpr int NB = DH / 8;     // 8-element blocks per row
   constexpr int WD = DH / 8;     // packed words per W4 row
   constexpr int LDW = FM_D + 4;  // floats per (wave, head) merge row: O[D], l, m
-  __shared__ float wo[FM_WAVES][FM_HEADS * LDW];
+  constexpr int ROWB = KIND == KIND_W4 ? DH / 2 : KIND == KIND_F8 ? DH : 2 * DH;  // bytes per cache row
+  constexpr bool row_scales = KIND == KIND_W4 || (KIND == KIND_F8 && !SLAB_SCALE);
+  // Tiles through LDS.  A slot: 32 K rows, 32 V rows, their scales, their
+  // zero-points; the wave's slots and later its merge rows lie in its own part of LDS.
+  constexpr int KBYTES = FM_TILE * ROWB;
+  constexpr int S_AT = 2 * KBYTES, Z_AT = S_AT + (row_scales ? 512 : 0), SLOTB = Z_AT + (ASYM ? 512 : 0);
+  constexpr int WO_BYTES = FM_HEADS * LDW * 4;
+  constexpr int WAVE_LDS = LDS && FM_RING * SLOTB > WO_BYTES ? FM_RING * SLOTB : WO_BYTES;
+  static_assert(WAVE_LDS % 16 == 0, "16-byte pieces");
+  __shared__ __attribute__((aligned(16))) uint8_t wave_lds[FM_WAVES][WAVE_LDS];
+  auto wo = [&](int w) { return (float*)wave_lds[w]; };
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c16 = lane & 15, q4 = lane >> 4;
@@ -138,7 +173,13 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
     return x;
   };
   _Float16 slab_sk = 0, slab_sv = 0;
-  if (SLAB_SCALE) slab_sk = as_half(a.s_k[slab]), slab_sv = as_half(a.s_v[slab]);
+  if (SLAB_SCALE) {  // (aligned dwords through the scalar cache: no vector request to wait for)
+    auto at = [&](const w4_half* sc) {
+      const uintptr_t p = (uintptr_t)(sc + slab);
+      return as_half((uint16_t)(*(fm_const_u32)(p & ~(uintptr_t)3) >> (8 * (p & 2))));
+    };
+    slab_sk = at(a.s_k), slab_sv = at(a.s_v);
+  }
 
   const int s0 = split * split_len;
   const int s1 = min(a.S, s0 + split_len);
@@ -146,22 +187,36 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
   const bool hook_k = HOOK && a.k_out && qh0 == 0, hook_v = HOOK && a.v_out && qh0 == 0;
 
   // Query operands: lane (head c16, k-block q4) of MFMA c holds
-  // q[head][kcol(c) + elem_of(p, hf)].
+  // q[head][kcol(c) + elem_of(p, hf)]: one 16-byte load per MFMA (at whatever alignment q
+  // has), pairs formed in registers.
   h8 qop[NC];
+  u4 qraw[NC];
   {
-    const uint16_t* qp =
-        a.q + ((long long)slab * a.group + qh0 + min(c16, nh - 1)) * FM_D;
+    const uint16_t* qp = a.q + ((long long)slab * a.group + qh0 + min(c16, nh - 1)) * FM_D;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
+      if constexpr (LDS)  // (the waits below count these requests together with the tiles')
+        asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(qraw[c]) : "v"(qp + kcol(c)) : "memory");
+      else
+        __builtin_memcpy(&qraw[c], qp + kcol(c), 16);
+    }
+  }
+  auto build_q = [&]() {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      if constexpr (LDS) asm volatile("" : "+v"(qraw[c]));
       h2 t[4];
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
-        const uint32_t lo = qp[kcol(c) + elem_of<KIND>(p, 0)], hi = qp[kcol(c) + elem_of<KIND>(p, 1)];
-        t[p] = as_h2(c16 < nh ? (lo | (hi << 16)) : 0u);
+        const int e0 = elem_of<KIND>(p, 0), e1 = elem_of<KIND>(p, 1);
+        const uint32_t sel = (e0 & 1 ? 0x0302u : 0x0100u) | ((e1 & 1 ? 0x0706u : 0x0504u) << 16);
+        const uint32_t pair = __builtin_amdgcn_perm(qraw[c][e1 >> 1], qraw[c][e0 >> 1], sel);
+        t[p] = as_h2(c16 < nh ? pair : 0u);
       }
       qop[c] = pack8(t);
     }
-  }
+  };
+  if constexpr (!LDS) build_q();
 
   // page of a position: a shift when the page size is a power of two (the scalar unit has
   // no divider: the quotient by a run-time page size is some twenty instructions, twice per tile)
@@ -179,7 +234,6 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
   // one page): buffer loads whose wave-uniform part (slab base in the
   // descriptor, tile row in the scalar offset) never touches the vector ALU.
   // A lane adds only the constant byte offsets below.
-  constexpr int ROWB = KIND == KIND_W4 ? DH / 2 : KIND == KIND_F8 ? DH : 2 * DH;  // bytes per cache row
   constexpr int VBB = ROWB / NB;                                                  // bytes per V block
   const long long slab_rows = PAGED ? a.pool_rows : a.S;
   // offsets are 32-bit: larger slabs take the general fetch for every tile
@@ -198,7 +252,6 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
   const int vq_off = 4 * q4 * ROWB + vb * VBB;      // block vb of the first of the lane's 4 V rows
   const int vs_off = 2 * (4 * q4 * G + gv);
   const int vz_off = 4 * (4 * q4 * wg + (gv >> 3));
-  constexpr bool row_scales = KIND == KIND_W4 || (KIND == KIND_F8 && !SLAB_SCALE);
 
   // Row, in the slab (in the head's pool when paged), of position t, a multiple
   // of 16 that starts a half tile.  Positions past the last whole half are
@@ -435,7 +488,7 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
       // layout -- and the two scales ride in one packed multiply.  Per element the
       // arithmetic is that of dq_w4: (1024 + n) - (1024 + z) or (64 + n) - (64 + z),
       // exact, then one rounding in the multiply by the scale.
-      h2 pe[4][NE];
+      h2 s2[4], clo[4], chi[4];
       uint32_t magic_lo = 0x64006400u, magic_hi = 0x54005400u;
       asm("" : "+v"(magic_lo));
       asm("" : "+v"(magic_hi));
@@ -443,22 +496,34 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
       const uint32_t byte0 = 2u * (uint32_t)hi8;
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) {
-        const uint32_t w0 = raw.v[2 * kk], w1 = raw.v[2 * kk + 1];
-        const h2 s2 = h2{at_use(raw.vs[2 * kk]), at_use(raw.vs[2 * kk + 1])};
+        s2[kk] = h2{at_use(raw.vs[2 * kk]), at_use(raw.vs[2 * kk + 1])};
         uint32_t zz = 0x00080008u;  // zero points of the two positions, one per half
         if (ASYM) {
           const int sh = 4 * (gv & 7);
           zz = ((raw.vz[2 * kk] >> sh) & 0xFu) | (((raw.vz[2 * kk + 1] >> sh) & 0xFu) << 16);
         }
-        const h2 clo = as_h2(0xE400E400u | zz);         // -(1024 + z), ulp 1
-        const h2 chi = as_h2(0xD400D400u | (zz << 4));  // -(64 + z), ulp 1/16
+        clo[kk] = as_h2(0xE400E400u | zz);         // -(1024 + z), ulp 1
+        chi[kk] = as_h2(0xD400D400u | (zz << 4));  // -(64 + z), ulp 1/16
+      }
+      h2 pe[4][NE];  // (two elements of every position at a time: few registers live at once)
 #pragma unroll
-        for (int b = 0; b < NE / 2; ++b) {
-          const uint32_t p = __builtin_amdgcn_perm(w1, w0, 0x0c000c00u | ((4u + b + byte0) << 16) | (b + byte0));
-          pe[kk][2 * b] = (as_h2(and_or(p, 0x000F000Fu, magic_lo)) + clo) * s2;
-          pe[kk][2 * b + 1] = (as_h2(and_or(p, 0x00F000F0u, magic_hi)) + chi) * s2;
+      for (int b = 0; b < NE / 2; ++b) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+          const uint32_t p = __builtin_amdgcn_perm(raw.v[2 * kk + 1], raw.v[2 * kk],
+                                                   0x0c000c00u | ((4u + b + byte0) << 16) | (b + byte0));
+          pe[kk][2 * b] = (as_h2(and_or(p, 0x000F000Fu, magic_lo)) + clo[kk]) * s2[kk];
+          pe[kk][2 * b + 1] = (as_h2(and_or(p, 0x00F000F0u, magic_hi)) + chi[kk]) * s2[kk];
         }
-        if constexpr (HOOK) {
+#pragma unroll
+        for (int e = 2 * b; e < 2 * b + 2; ++e) {
+          const h2 at[4] = {pe[0][e], pe[1][e], pe[2][e], pe[3][e]};
+          o[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pack8(at), pop, o[e], 0, 0, 0);
+        }
+      }
+      if constexpr (HOOK) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
           h2 n0[4], n1[4];
 #pragma unroll
           for (int i = 0; i < NE / 2; ++i) {
@@ -473,11 +538,6 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
             hook_store_v(2 * kk + 1, n1);
           }
         }
-      }
-#pragma unroll
-      for (int e = 0; e < NE; ++e) {
-        const h2 at[4] = {pe[0][e], pe[1][e], pe[2][e], pe[3][e]};
-        o[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pack8(at), pop, o[e], 0, 0, 0);
       }
     } else {
       h2 vt[8][4];
@@ -529,44 +589,216 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
       fetch(raw, tile_start(it));
     }
   };
-  // A ring slot is refilled right after the tile in it has been consumed, into
-  // the same registers: the loop carries no copies, and DEPTH - 1 tiles are in
-  // flight while one is computed.
-  // (FP8 with row scales: two slots keep two waves per SIMD resident, which pays there)
-  constexpr int DEPTH = KIND == KIND_F8 && !SLAB_SCALE ? 2 : FM_DEPTH;
-  TileRaw<KIND, NC> ring[DEPTH];
+  if constexpr (LDS) {
+    // Lane's share of the requests: unit u = lane of a load instruction is 16 bytes of LDS.
+    // K rows keep their order and swap pieces so that 16 rows x one piece (an operand read) fall
+    // on 16 bank groups; V row 4 b + a goes to place 4 a + b, so that the four rows of a read
+    // are neighbours.
+    constexpr int P = ROWB / 16, RPI = 64 / P, KI = FM_TILE / RPI;  // pieces per row, rows and loads
+    constexpr int NL = 2 * KI + (row_scales ? 2 : 0) + (ASYM ? 2 : 0);
+    auto kswz = [](int r) { return P == 8 ? (r >> 1) & 7 : P == 4 ? (r >> 2) & 3 : (r >> 3) & 1; };
+    const uint8_t* const kbase = (const uint8_t*)a.k + rows0 * ROWB;
+    const uint8_t* const vbase = (const uint8_t*)a.v + rows0 * ROWB;
+    const uint32_t lds_wave = (uint32_t)(uintptr_t)(fm_lds)wave_lds + (uint32_t)wave * WAVE_LDS;
+    const int upos = lane / P, upiece = lane % P;
+    const int odd = (int)((rows0 * G) & 1);  // one group per row: a slab may start in the middle of a dword
+    auto dma16 = [](const void* base, uint32_t off, uint32_t lds) {
+      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+    };
+    auto dma4 = [](const void* base, uint32_t off, uint32_t lds) {
+      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+    };
+    const int last16 = (s1 - 1) & ~15;  // the last half tile that has a position below s1
+    // row, in the slab, of the half tile that starts at position t (clamped to the last one)
+    auto half_row = [&](int t) -> int {
+      const int tc = min(t, last16);
+      if (PAGED == 0) return tc;
+      const int pg = page_of(tc);
+      return ((fm_const_i32)bt)[pg] * a.page + (tc - pg * a.page);
+    };
+    // Place of load instruction i of a side: half tile, row of the half and piece of this lane.
+    struct Place {
+      int j, r, piece;
+    };
+    auto place = [&](int v, int i) {
+      int r, j;
+      if constexpr (RPI == 32) j = upos >> 4, r = upos & 15;
+      else j = (i * RPI) >> 4, r = ((i * RPI) & 15) + upos;
+      if (v) r = 4 * (r & 3) + (r >> 2);
+      return Place{j, r, v ? upiece : upiece ^ kswz(r)};
+    };
+    // What the loads of a whole tile add to their scalar bases: nothing is left to compute per tile.
+    constexpr int KO = RPI == 8 ? 2 : 1;  // (eight rows a load: the two loads of a half differ)
+    uint32_t koff[KO], voff[KO];
 #pragma unroll
-  for (int d = 0; d < DEPTH; ++d) fetch_any(ring[d], d);
-  int it0 = 0;
-  // Page-table lookups run one tile ahead of the loads that need them, so the
-  // scalar load's latency is off the path to the vector loads.
-  int rb_next[2] = {slab_row(tile_start(DEPTH)), slab_row(tile_start(DEPTH) + 16)};
-  for (; it0 + 2 * DEPTH <= nwhole; it0 += DEPTH) {  // computes and fetches whole tiles only
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-      compute(ring[d], tile_start(it0 + d), std::true_type{});
-      __builtin_amdgcn_sched_barrier(0);
-      const int rb[2] = {rb_next[0], rb_next[1]};
-      const int t_after = tile_start(it0 + d + DEPTH + 1);
-      rb_next[0] = slab_row(t_after);
-      rb_next[1] = slab_row(t_after + 16);
-      fetch_whole(ring[d], rb);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < KO; ++i) {
+      const Place k = place(0, i), v = place(1, i);
+      koff[i] = k.r * ROWB + k.piece * 16;
+      voff[i] = v.r * ROWB + v.piece * 16;
     }
-  }
-  for (; it0 < nit; it0 += DEPTH) {
+    const int n16 = (16 * G + odd - 1) >> 1;  // last dword of a whole half's scales
+    const uint32_t soff = 4u * min(lane & 31, n16), zoff = 4u * (lane & 15);
+    const uint8_t* const skb = (const uint8_t*)a.s_k + (rows0 * G - odd) * 2;
+    const uint8_t* const svb = (const uint8_t*)a.s_v + (rows0 * G - odd) * 2;
+    const uint8_t* const zkb = (const uint8_t*)a.z_k + rows0 * 4;
+    const uint8_t* const zvb = (const uint8_t*)a.z_v + rows0 * 4;
+    // Requests the tile that starts at position t0, whose halves start at rows rb[0], rb[1], into
+    // slot sl.  A cut tile (its last rows lie past s1) repeats the last row of each half.
+    auto request = [&](int sl, int t0, const int rb[2]) {
+      const bool cut = t0 + FM_TILE > s1;
+      int left[2] = {16, 16};
+      if (cut) {
 #pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-      if (it0 + d < nit) compute(ring[d], tile_start(it0 + d), std::false_type{});
-      __builtin_amdgcn_sched_barrier(0);
-      fetch_any(ring[d], it0 + d + DEPTH);
-      __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < 2; ++j) left[j] = min(16, s1 - min(t0 + 16 * j, last16));
+      }
+      const uint32_t at = lds_wave + sl * SLOTB;
+#pragma unroll
+      for (int v = 0; v < 2; ++v)
+#pragma unroll
+        for (int i = 0; i < KI; ++i) {
+          uint32_t off = v ? voff[i % KO] : koff[i % KO];
+          if (cut) {
+            const Place p = place(v, i);
+            off = min(p.r, (p.j ? left[1] : left[0]) - 1) * ROWB + p.piece * 16;
+          }
+          const uint8_t* base = v ? vbase : kbase;
+          if constexpr (RPI == 32) off += (uint32_t)(lane < 32 ? rb[0] : rb[1]) * ROWB;
+          else base += (long long)rb[(i * RPI) >> 4] * ROWB;
+          dma16(base, off, at + v * KBYTES + i * 1024);
+        }
+      if constexpr (row_scales) {  // lanes 0..31: the first half's dwords, 32..63: the second's
+        uint32_t off = soff;
+        if (cut) off = 4u * min(lane & 31, ((lane < 32 ? left[0] : left[1]) * G + odd - 1) >> 1);
+        off += 2u * ((uint32_t)(lane < 32 ? rb[0] : rb[1]) * G);
+        dma4(skb, off, at + S_AT);
+        dma4(svb, off, at + S_AT + 256);
+      }
+      if constexpr (ASYM) {  // one dword per row
+        const bool hi = lane & 16;
+        uint32_t off = zoff;
+        if (cut) off = 4u * min(lane & 15, (hi ? left[1] : left[0]) - 1);
+        off += 4u * (uint32_t)(hi ? rb[1] : rb[0]);
+        dma4(zkb, off, at + Z_AT);
+        dma4(zvb, off, at + Z_AT + 256);
+      }
+    };
+    const uint8_t* const my = wave_lds[wave];
+    const int ks_at = S_AT + 2 * (c16 * G + gk + odd), vs_at = S_AT + 256 + 2 * (4 * q4 * G + gv + odd);
+    auto read_tile = [&](TileRaw<KIND, NC>& raw, int sl) {
+      const uint8_t* const slot = my + sl * SLOTB;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const uint8_t* const kr = slot + (16 * j + c16) * ROWB;
+        if constexpr (KIND == KIND_W4 && NC == 4) {
+          const u4 t4 = *(const u4*)(kr + 16 * (q4 ^ kswz(c16)));
+#pragma unroll
+          for (int c = 0; c < 4; ++c) raw.k[j][c] = t4[c];
+        } else if constexpr (KIND == KIND_W4) {
+          const u2 t2 = *(const u2*)(kr + 16 * ((q4 >> 1) ^ kswz(c16)) + 8 * (q4 & 1));
+          raw.k[j][0] = t2[0], raw.k[j][1] = t2[1];
+        } else if constexpr (KIND == KIND_F8) {
+#pragma unroll
+          for (int i = 0; i < NC / 2; ++i) {
+            const u4 t4 = *(const u4*)(kr + 16 * ((NC / 2 * q4 + i) ^ kswz(c16)));
+            raw.k[j][2 * i] = u2{t4[0], t4[1]};
+            raw.k[j][2 * i + 1] = u2{t4[2], t4[3]};
+          }
+        }
+        if constexpr (KIND != KIND_F16) {
+          if constexpr (row_scales) raw.ks[j] = *(const _Float16*)(slot + ks_at + 128 * j);
+          else raw.ks[j] = slab_sk;
+        }
+        if constexpr (ASYM) raw.kz[j] = *(const uint32_t*)(slot + Z_AT + 4 * (16 * j + c16));
+        u4 z4;
+        if constexpr (ASYM) z4 = *(const u4*)(slot + Z_AT + 256 + 4 * (16 * j + 4 * q4));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int k = 4 * j + r;
+          const uint8_t* const vr = slot + KBYTES + (16 * j + 4 * r + q4) * ROWB + vb * VBB;
+          if constexpr (KIND == KIND_W4) raw.v[k] = *(const uint32_t*)vr;
+          else if constexpr (KIND == KIND_F8) raw.v[k] = *(const u2*)vr;
+          if constexpr (KIND != KIND_F16) {
+            if constexpr (row_scales) raw.vs[k] = *(const _Float16*)(slot + vs_at + 128 * j + 2 * r * G);
+            else raw.vs[k] = slab_sv;
+          }
+          if constexpr (ASYM) raw.vz[k] = z4[r];
+        }
+      }
+    };
+#pragma unroll
+    for (int d = 0; d < FM_RING; ++d)
+      if (d < nit) {
+        const int rb[2] = {half_row(tile_start(d)), half_row(tile_start(d) + 16)};
+        request(d, tile_start(d), rb);
+      }
+    // (page lookups run one tile ahead of the request that needs them)
+    int rb_next[2] = {half_row(tile_start(FM_RING)), half_row(tile_start(FM_RING) + 16)};
+    auto wait_tile = [&](int it) {  // tile `it` has landed; the ones after it may be in flight
+      if (it + FM_RING <= nit) asm volatile("s_waitcnt vmcnt(%0)" : : "n"((FM_RING - 1) * NL) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    };
+    wait_tile(0);
+    build_q();
+    for (int it0 = 0; it0 < nit; it0 += FM_RING) {
+#pragma unroll
+      for (int d = 0; d < FM_RING; ++d) {
+        const int it = it0 + d;
+        if (it < nit) {
+          wait_tile(it);
+          TileRaw<KIND, NC> raw;
+          read_tile(raw, d);
+          if (tile_start(it) + FM_TILE <= s1) compute(raw, tile_start(it), std::true_type{});
+          else compute(raw, tile_start(it), std::false_type{});
+          asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");  // the slot has been read: refill it
+          if (it + FM_RING < nit) {
+            const int rb[2] = {rb_next[0], rb_next[1]};
+            request(d, tile_start(it + FM_RING), rb);
+            rb_next[0] = half_row(tile_start(it + FM_RING + 1));
+            rb_next[1] = half_row(tile_start(it + FM_RING + 1) + 16);
+          }
+        }
+      }
+    }
+  } else {
+    // A ring slot is refilled right after the tile in it has been consumed, into
+    // the same registers: the loop carries no copies, and DEPTH - 1 tiles are in
+    // flight while one is computed.
+    // (FP8 with row scales: two slots keep two waves per SIMD resident, which pays there)
+    constexpr int DEPTH = KIND == KIND_F8 && !SLAB_SCALE ? 2 : FM_DEPTH;
+    TileRaw<KIND, NC> ring[DEPTH];
+  #pragma unroll
+    for (int d = 0; d < DEPTH; ++d) fetch_any(ring[d], d);
+    int it0 = 0;
+    // Page-table lookups run one tile ahead of the loads that need them, so the
+    // scalar load's latency is off the path to the vector loads.
+    int rb_next[2] = {slab_row(tile_start(DEPTH)), slab_row(tile_start(DEPTH) + 16)};
+    for (; it0 + 2 * DEPTH <= nwhole; it0 += DEPTH) {  // computes and fetches whole tiles only
+  #pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+        compute(ring[d], tile_start(it0 + d), std::true_type{});
+        __builtin_amdgcn_sched_barrier(0);
+        const int rb[2] = {rb_next[0], rb_next[1]};
+        const int t_after = tile_start(it0 + d + DEPTH + 1);
+        rb_next[0] = slab_row(t_after);
+        rb_next[1] = slab_row(t_after + 16);
+        fetch_whole(ring[d], rb);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    for (; it0 < nit; it0 += DEPTH) {
+  #pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+        if (it0 + d < nit) compute(ring[d], tile_start(it0 + d), std::false_type{});
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_any(ring[d], it0 + d + DEPTH);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   }
 
   // ---- merge the four waves in wave order: lane (head c16, q4) holds
   // O[head][32 q4 + 8 r + e] in o[e][r] (output rows past D / 8 are repeats: dropped)
-  float* mine = wo[wave] + c16 * LDW;
+  float* mine = wo(wave) + c16 * LDW;
 #pragma unroll
   for (int e = 0; e < NE; ++e)
 #pragma unroll
@@ -588,53 +820,120 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
       float mw[FM_WAVES], M = -INFINITY;
 #pragma unroll
       for (int w = 0; w < FM_WAVES; ++w) {
-        mw[w] = wo[w][h * LDW + FM_D + 1];
+        mw[w] = wo(w)[h * LDW + FM_D + 1];
         M = fmaxf(M, mw[w]);
       }
       float sum = 0.0f, l = 0.0f;
 #pragma unroll
       for (int w = 0; w < FM_WAVES; ++w) {
         const float e = __expf(mw[w] - M);
-        sum += e * wo[w][h * LDW + j];
-        l += e * wo[w][h * LDW + FM_D];
+        sum += e * wo(w)[h * LDW + j];
+        l += e * wo(w)[h * LDW + FM_D];
       }
       const _Float16 hv = (_Float16)(sum * (1.0f / l));
       a.out[((long long)slab * a.group + qh0 + h) * FM_D + j] = __builtin_bit_cast(uint16_t, hv);
     }
     return;
   }
-  for (int i = threadIdx.x; i < nh * (FM_D + 1); i += FM_WAVES * 64) {
-    const int h = i / (FM_D + 1), j = i - h * (FM_D + 1);  // j < 128: O[j]; j == 128: l
+  // The split's partial: (maximum, denominator, O[D]) of every head, two floats a thread.
+  // Stores of agent scope: they are written through to where every XCD sees them, which is
+  // what the merge below needs (a fence instead would write the whole L2 of the XCD back).
+  constexpr int PAIRS = FM_D / 2 + 1;
+  auto publish = [](float* p, float lo, float hi) {
+    const uint64_t v = __builtin_bit_cast(uint32_t, lo) | ((uint64_t)__builtin_bit_cast(uint32_t, hi) << 32);
+    __hip_atomic_store((uint64_t*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  float* slab_part = part + ((long long)slab * a.group + qh0) * nsplit * (FM_D + 2);
+  for (int i = threadIdx.x; i < nh * PAIRS; i += FM_WAVES * 64) {
+    const int h = i / PAIRS, j = i - h * PAIRS;  // j == 0: maximum and denominator
     float mw[FM_WAVES], M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < FM_WAVES; ++w) {
-      mw[w] = wo[w][h * LDW + FM_D + 1];
+      mw[w] = wo(w)[h * LDW + FM_D + 1];
       M = fmaxf(M, mw[w]);
     }
-    float sum = 0.0f;
+    float sum0 = 0.0f, sum1 = 0.0f;
+    const int at = j ? 2 * j - 2 : FM_D;
 #pragma unroll
-    for (int w = 0; w < FM_WAVES; ++w) sum += __expf(mw[w] - M) * wo[w][h * LDW + j];
-    float* dst = part + (((long long)slab * a.group + qh0 + h) * nsplit + split) * (FM_D + 2);
-    if (j < FM_D) {
-      dst[2 + j] = sum;
-    } else {
-      dst[1] = sum;
-      dst[0] = M;
+    for (int w = 0; w < FM_WAVES; ++w) {
+      const float e = __expf(mw[w] - M);
+      sum0 += e * wo(w)[h * LDW + at];
+      sum1 += e * wo(w)[h * LDW + at + 1];
+    }
+    float* dst = slab_part + ((long long)h * nsplit + split) * (FM_D + 2) + 2 * j;
+    if (j) publish(dst, sum0, sum1);
+    else publish(dst, M, sum0);
+  }
+  if (!merge_here) return;
+
+  // The workgroup of a slab that finishes last merges the slab's splits.  Each one counts
+  // itself once its partial has been written (the stores have come back); the counter wraps
+  // to 0 with the last one, so the next call finds it as this one did.  There is one counter
+  // per (number of splits, slab): calls that share a counter make the same number of
+  // arrivals, so even calls that overlapped by mistake leave it at 0.
+  __shared__ uint32_t arrived;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    arrived = __builtin_amdgcn_atomic_inc32(&flash_arrivals[nsplit * FM_MERGE_SLABS + slab], (uint32_t)(nsplit - 1),
+                                            __ATOMIC_RELAXED, "agent");
+  __syncthreads();
+  if (arrived != (uint32_t)(nsplit - 1)) return;
+  // A wave takes every fourth head.  Lane t has the maximum and the denominator of split t,
+  // every lane two columns of O; all of a head's loads are in flight at once.
+  auto fetch_pair = [](const float* p) {
+    const uint64_t v = __hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return float2{__builtin_bit_cast(float, (uint32_t)v), __builtin_bit_cast(float, (uint32_t)(v >> 32))};
+  };
+  constexpr int BATCH = 16;
+  for (int h = wave; h < nh; h += FM_WAVES) {
+    const float* hp = slab_part + (long long)h * nsplit * (FM_D + 2);
+    const float* op = hp + 2 + 2 * (lane & (FM_D / 2 - 1));
+    const float2 ml = fetch_pair(hp + (long long)min(lane, nsplit - 1) * (FM_D + 2));
+    float2 col[BATCH];
+#pragma unroll
+    for (int t = 0; t < BATCH; ++t) col[t] = fetch_pair(op + (long long)min(t, nsplit - 1) * (FM_D + 2));
+    float M = lane < nsplit ? ml.x : -INFINITY;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+    const float wt = lane < nsplit ? __expf(ml.x - M) : 0.0f;
+    float den = wt * ml.y;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) den += __shfl_xor(den, off, 64);
+    float sum0 = 0.0f, sum1 = 0.0f;
+    for (int t0 = 0; t0 < nsplit; t0 += BATCH) {
+      if (t0)
+#pragma unroll
+        for (int t = 0; t < BATCH; ++t) col[t] = fetch_pair(op + (long long)min(t0 + t, nsplit - 1) * (FM_D + 2));
+#pragma unroll
+      for (int t = 0; t < BATCH; ++t) {  // (splits past the last have weight 0)
+        const float e = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wt), t0 + t));
+        sum0 += e * col[t].x;
+        sum1 += e * col[t].y;
+      }
+    }
+    const float inv = 1.0f / den;
+    const h2 hv = h2{(_Float16)(sum0 * inv), (_Float16)(sum1 * inv)};
+    w4_half* dst = a.out + ((long long)slab * a.group + qh0 + h) * FM_D + 2 * lane;
+    if (lane < FM_D / 2) {
+      dst[0] = (uint16_t)as_u32(hv);
+      dst[1] = (uint16_t)(as_u32(hv) >> 16);
     }
   }
 }
 
-template <int KIND, bool HOOK, int PAGED>
-static hipError_t go_asym(const FlashArgs& a, int qh0, const FlashPlan& pl, float* part,
-                          hipStream_t s) {
+template <int KIND, bool HOOK, int PAGED, bool LDS>
+static hipError_t go_alt(const FlashArgs& a, int qh0, const FlashPlan& pl, float* part,
+                         hipStream_t s) {
   const dim3 grid((unsigned)a.H, (unsigned)pl.nsplit);
-  const bool asym = (KIND == KIND_W4 && !a.symmetric) || (KIND == KIND_F8 && a.scale_mode == 1);
-#define W4_GO(DH, ASYM) \
-  flash_mfma_phase1<KIND, DH, HOOK, PAGED, ASYM><<<grid, FM_WAVES * 64, 0, s>>>(a, qh0, pl.split_len, part)
+  const bool alt = (KIND == KIND_W4 && !a.symmetric) || (KIND == KIND_F8 && a.scale_mode == 1);
+#define W4_GO(DH, ALT)                                                         \
+  flash_mfma_phase1<KIND, DH, HOOK, PAGED, (ALT) && KIND != KIND_F16, LDS>     \
+      <<<grid, FM_WAVES * 64, 0, s>>>(a, qh0, pl.split_len, part, flash_merges_in_place(a, pl))
   if (a.D == 128) {
-    if (asym) W4_GO(128, true); else W4_GO(128, false);
+    if (alt) W4_GO(128, true); else W4_GO(128, false);
   } else {
-    if (asym) W4_GO(64, true); else W4_GO(64, false);
+    if (alt) W4_GO(64, true); else W4_GO(64, false);
   }
 #undef W4_GO
   return hipGetLastError();
@@ -644,14 +943,31 @@ template <int KIND>
 static hipError_t go_kind(const FlashArgs& a, int qh0, const FlashPlan& pl, float* part,
                           hipStream_t s) {
   const bool hook = a.k_out || a.v_out;
-  if constexpr (KIND == KIND_W4) {
-    if (a.bt) {
-      if (a.page % 16 == 0)
-        return hook ? go_asym<KIND, true, 1>(a, qh0, pl, part, s) : go_asym<KIND, false, 1>(a, qh0, pl, part, s);
-      return hook ? go_asym<KIND, true, 2>(a, qh0, pl, part, s) : go_asym<KIND, false, 2>(a, qh0, pl, part, s);
+  if constexpr (KIND == KIND_F16) {
+    return hook ? go_alt<KIND, true, 0, false>(a, qh0, pl, part, s) : go_alt<KIND, false, 0, false>(a, qh0, pl, part, s);
+  } else {
+    // Tiles through LDS: 32-bit offsets inside a slab, scales that can be fetched as dwords, at
+    // most four groups per row.  The register path of the hooked kernels takes everything.
+    const long long slab_rows = a.bt ? a.pool_rows : a.S;
+    const bool lds_ok = slab_rows * a.D * 2 < (1ll << 31) && a.G <= 4 && (((uintptr_t)a.s_k | (uintptr_t)a.s_v) & 3) == 0;
+    if constexpr (KIND == KIND_F8) {
+      return hook || !lds_ok ? go_alt<KIND, true, 0, false>(a, qh0, pl, part, s)
+                             : go_alt<KIND, false, 0, true>(a, qh0, pl, part, s);
+    } else {
+      // W4 with more than FM_LDS_TILES tiles per wave stays in registers: once the stream runs, the
+      // read back from LDS in front of every tile costs more than the loads it saves (57.7
+      // against 60.9 us at 64 slabs x 32768 positions, 33.6 against 34.8 with 16 tiles per wave;
+      // 27.5 against 28.4 us with 12, 12.7 against 14.1 with 4).
+      const bool lds = lds_ok && pl.split_len <= FM_LDS_TILES * FM_WAVES * FM_TILE;
+      if (a.bt && a.page % 16 != 0)
+        return hook ? go_alt<KIND, true, 2, false>(a, qh0, pl, part, s) : go_alt<KIND, false, 2, false>(a, qh0, pl, part, s);
+      if (a.bt)
+        return hook ? go_alt<KIND, true, 1, false>(a, qh0, pl, part, s)
+               : lds ? go_alt<KIND, false, 1, true>(a, qh0, pl, part, s) : go_alt<KIND, false, 1, false>(a, qh0, pl, part, s);
+      return hook ? go_alt<KIND, true, 0, false>(a, qh0, pl, part, s)
+             : lds ? go_alt<KIND, false, 0, true>(a, qh0, pl, part, s) : go_alt<KIND, false, 0, false>(a, qh0, pl, part, s);
     }
   }
-  return hook ? go_asym<KIND, true, 0>(a, qh0, pl, part, s) : go_asym<KIND, false, 0>(a, qh0, pl, part, s);
 }
 
 bool flash_mfma_applies(const FlashArgs& a) {
@@ -660,6 +976,11 @@ bool flash_mfma_applies(const FlashArgs& a) {
   if (a.kind != KIND_F16 && a.gs % (a.D / 4)) return false;
   return ((((uintptr_t)a.k | (uintptr_t)a.v) & 15) == 0) &&
          ((((uintptr_t)a.k_out | (uintptr_t)a.v_out) & 15) == 0);
+}
+
+bool flash_merges_in_place(const FlashArgs& a, const FlashPlan& pl) {
+  return pl.nsplit > 1 && pl.nsplit <= FM_MERGE_SPLITS && a.H <= FM_MERGE_SLABS &&
+         min(a.group, FM_HEADS) * pl.nsplit <= FM_MERGE_MAX;
 }
 
 bool try_flash_mfma(const FlashArgs& a, const FlashPlan& pl, float* part, hipStream_t s,

@@ -108,6 +108,8 @@ struct FlashPlan {
 FlashPlan flash_plan(const FlashArgs& a);
 // flash_mfma.hip: whether the matrix-core phase 1 (D = 128) takes these arguments.
 bool flash_mfma_applies(const FlashArgs& a);
+// Whether its last workgroup of every slab merges the splits itself (no second launch).
+bool flash_merges_in_place(const FlashArgs& a, const FlashPlan& pl);
 // Launches it; false when the arguments need the general kernel (nothing is
 // launched then).
 bool try_flash_mfma(const FlashArgs& a, const FlashPlan& pl, float* part, hipStream_t s,
