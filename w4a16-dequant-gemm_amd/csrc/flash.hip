@@ -357,22 +357,58 @@ __global__ __launch_bounds__(P2_THREADS) void flash_phase2(const float* __restri
 
 // ---- host side -------------------------------------------------------------
 
+// Splits of the matrix-core kernel: t tiles of 128 positions per workgroup (one of 32 per
+// wave).  More, shorter splits start sooner and cost more to merge, and a second workgroup on a
+// compute unit shares its vector units; the terms below are measured (us, D = 128, gs = 32,
+// 4 heads per slab; x 0.7 at D = 64):
+//   t tiles take 0.5 + T t with at most one workgroup per compute unit (T = 1.0 for W4, 1.4 FP8,
+//   2.5 FP16), 1.7 + F T t with two (F = 1.25 W4, 1.8 FP8), as many times over as the grid has
+//   rounds; FP16 fits one workgroup per unit;
+//   the merge by the last workgroup 1.5 (+ 0.7 per further four heads), by a second kernel 3 + 0.03 per split, none 0.
+// Before this rule splits were multiples of 256 positions and aimed at 512 workgroups: 32 x 6007 FP8
+// 19.4 -> 15.2 us, 128 x 1500 W4 pages 12.7 -> 11.4, 32 x 3000 FP16 18.4 -> 14.0, 8 x 600 W4 6.7 -> 6.1.
+static float split_cost(const FlashArgs& a, int t, int nsplit) {
+  const float T = (a.kind == KIND_W4 ? 1.0f : a.kind == KIND_F8 ? 1.4f : 2.5f) * (a.D == 64 ? 0.7f : 1.0f);
+  const long long wgs = (long long)a.H * nsplit;
+  float c;
+  if (wgs <= 256) c = 0.5f + T * t;
+  else if (a.kind == KIND_F16) c = (float)((wgs + 255) / 256) * (1.2f + T * t);
+  else c = (float)((wgs + 511) / 512) * (1.7f + (a.kind == KIND_W4 ? 1.25f : 1.8f) * T * t);
+  if (nsplit > 1)
+    c += flash_merges_in_place(a, FlashPlan{128 * t, nsplit}) ? 1.5f + 0.7f * ((a.group - 1) / 4) : 3.0f + 0.03f * nsplit;
+  return c;
+}
+
+static FlashPlan mfma_plan(const FlashArgs& a) {
+  const int tiles = (a.S + 127) / 128;
+  // nothing is gained below one round of two workgroups per compute unit (512) or above twice that
+  const int lo = (int)(((long long)tiles * a.H + 511) / 512), hi = lo * 2 + 4;
+  FlashPlan best{128 * tiles, 1};
+  float cost = split_cost(a, tiles, 1);
+  for (int t = lo < 1 ? 1 : lo; t <= hi && t < tiles; ++t) {
+    const int n = (tiles + t - 1) / t;
+    const float c = split_cost(a, t, n);
+    if (c < cost) cost = c, best = FlashPlan{128 * t, n};
+  }
+  return best;
+}
+
 FlashPlan flash_plan(const FlashArgs& a) {
+  const auto floats = [&](const FlashPlan& p) { return (size_t)a.H * a.group * p.nsplit * (a.D + 2); };
+  const bool mfma = flash_mfma_applies(a);
+  if (mfma) {
+    const FlashPlan p = mfma_plan(a);
+    // (partials that fit the built-in scratch with the longer splits below have to fit it here)
+    if (floats(p) * sizeof(float) <= W4_NOALLOC_SCRATCH_BYTES) return p;
+  }
   // Enough workgroups to fill 256 CUs, but splits no shorter than one tile; a
   // longer split writes fewer partials.  Measured at 64 slabs x 32768 positions:
   // the matrix-core kernel is fastest with 2 workgroups per CU (512 in all; 256,
   // 768, 1024, 2048 and 4096 were slower), the vector kernel with 8.
   const int tiles = (a.S + FL_TILE - 1) / FL_TILE;
-  const int per_cu = flash_mfma_applies(a) ? 2 : 8;
-  int want = (per_cu * 256 + a.H - 1) / a.H;  // splits per slab
+  int want = ((mfma ? 2 : 8) * 256 + a.H - 1) / a.H;  // splits per slab
   if (want < 1) want = 1;
   if (want > tiles) want = tiles;
-  // Short caches: one split per slab, whose matrix-core kernel writes the output
-  // itself.  The first kernel takes 5.4 us for one tile of 256 positions per workgroup
-  // and 2 us more for every further one, the merge kernel 3.4 us (8.8 us per call for
-  // any S from 512 to 2048 with 32 heads): one more tile costs less than the merge,
-  // two cost more (S = 512: 8.8 -> 7.9 us; S = 1024 would be 9.2 -> 11.9).
-  if (flash_mfma_applies(a) && a.S <= FL_DIRECT_MAX_S) want = 1;
   const int tiles_per = (tiles + want - 1) / want;
   FlashPlan p;
   p.split_len = tiles_per * FL_TILE;
