@@ -307,3 +307,46 @@ def test_w4a4_activation_quantizer_ties_and_boundaries():
     _, q, s = _quantize_x_on_device(x16.ravel(), M, K)
     assert np.array_equal(s.cpu().numpy(), ref.scales)
     assert np.array_equal(q.cpu().numpy().view(np.uint32), ref.q)
+
+
+# One round of 128 x 32 MJ tiles for MJ = 1 .. 4, ragged in M and N; one stage of 256 k, an odd
+# number without 16-byte rows of scales, and six; scale arrays 8 bytes off a 16-byte boundary.
+@pytest.mark.parametrize("x8", [False, True])
+@pytest.mark.parametrize("K,shift", [(256, 0), (768, 0), (1536, 0), (1536, 8)])
+@pytest.mark.parametrize("M,N", [(70, 4100), (390, 4100), (610, 4100), (900, 4000)])
+def test_eight_wave_tiles(M, N, K, shift, x8):
+    c = w4amd.capi()
+    rng = np.random.default_rng(M + K)
+    B = K // 32
+    wq, ws = rng.integers(0, 256, (N, K // 2), np.uint8), rng.integers(118, 124, (N, B)).astype(np.uint8)
+    xs = rng.integers(120, 126, (M, B)).astype(np.uint8)
+
+    def codes(q):
+        return E2M1[np.stack([q & 15, q >> 4], axis=-1).reshape(len(q), -1)]
+
+    def dev(a, off):
+        t = torch.zeros(a.size + off, dtype=torch.uint8, device=DEV)
+        t[off:] = torch.from_numpy(a.ravel()).to(DEV)
+        return t, ptr(t) + off
+
+    if x8:
+        xq = rng.integers(0, 256, (M, K), np.uint8)
+        xq[(xq & 0x7F) == 0x7F] = 0  # no NaN
+        xf = torch.from_numpy(xq).view(torch.float8_e4m3fn).double().numpy()
+    else:
+        xq = rng.integers(0, 256, (M, K // 2), np.uint8)
+        xf = codes(xq)
+    scale = lambda s: np.repeat(2.0 ** (s.astype(np.float64) - 127), 32, axis=1)
+    ref = (xf * scale(xs)) @ (codes(wq) * scale(ws)).T
+    assert np.abs(ref).max() < 65000
+    (tw, pw), (tws, pws), (tx, px), (txs, pxs) = dev(wq, 0), dev(ws, shift), dev(xq, 0), dev(xs, shift)
+    out = halves(M * N, 0x7E00)
+    wview = c.packed_mx_view(N, K, B, pw, pws)
+    if x8:
+        c.gemm_mx_w4a8(wview, c.act_mx8_view(M, K, B, px, pxs), ptr(out))
+    else:
+        c.gemm_mx_w4a4(wview, c.packed_mx_view(M, K, B, px, pxs), ptr(out))
+    got = bits(out).view(np.float16).astype(np.float64).reshape(M, N)
+    # FP16 rounding of the sums is at most 2^-11 of each; FP32 sums of 1536 exact products add
+    # less than 1e-5
+    assert orc.rel_l2(got, ref) <= 5e-4

@@ -382,7 +382,7 @@ __global__ __launch_bounds__(DM_THREADS) void mxn_tile_dma_kernel(
   // 16-row group: ((block & 1) * 8 + l/8) / 2.
   typedef Dm<XF8> C;
   const int row8 = lane >> 3;
-  uint32_t wo[DM_WI], xo[C::XI];  // byte offsets (32-bit: tile_applies bounds the operands)
+  uint32_t wo[DM_WI], xo[C::XI];  // byte offsets (32-bit: tile_operands_ok bounds the operands)
 #pragma unroll
   for (int i = 0; i < DM_WI; ++i) {
     const int blk = wave + DM_WAVES * i, R = blk * 8 + row8, n = n0 + R;
@@ -797,16 +797,353 @@ __global__ __launch_bounds__(D4_THREADS) void mxn_tile4_kernel(
   }
 }
 
-// Worth it once the tile grid covers a good part of the chip; below that the
-// skinny kernel's grid.y walk is faster (measured at K = 4096: N = 4096, M = 256
-// -> 32 tiles 37 us here, 23 us there; M = 512 -> 64 tiles 31 us here; N = 14336,
-// M = 256 -> 112 tiles 34 us here, 54 us there).  x_row_bytes: K/2 or K.
-bool tile_applies(const w4_packed_mx_view& w, const void* xq, const uint8_t* xs, int M,
-                  int x_row_bytes) {
-  const long long tiles = (long long)((w.N + TL_TN - 1) / TL_TN) * ((M + TL_TM - 1) / TL_TM);
-  return M >= 128 && tiles >= 64 && w.K % 256 == 0 && (long long)w.N * w.K < (1LL << 32) &&
-         (long long)M * x_row_bytes < (1LL << 32) && ((uintptr_t)w.q & 15) == 0 &&
-         ((uintptr_t)xq & 15) == 0 && ((uintptr_t)w.scales & 7) == 0 && ((uintptr_t)xs & 7) == 0;
+// ---- the same tiles for grids of up to a few rounds ------------------------------
+// 128 rows of W x 32 MJ rows of X (MJ = 1 .. 4) with eight waves: four waves share the tile
+// (4 x 1, or 2 x 2 where MJ is even: fewer LDS bytes per product) and each half kh of a
+// 256-k stage has four of its own; the two halves' sums meet in LDS at the end.  On such
+// grids a workgroup's K / 256 stages are a chain of load latencies, so the tile is chosen for
+// how many compute units it keeps busy (plan_tile), the ring holds three to five stages (two
+// are in flight while one is multiplied; the larger tile above has one), and a wave reads the
+// operands of stage d into registers while it multiplies those of stage d - 1: one barrier per
+// stage, two waves per SIMD whose LDS reads and products overlap.  What bounds it then is LDS:
+// a stage's operands are read two to four times over, 0.3 us per stage at MJ = 1, 0.8 at MJ = 4.
+// Block scales: with K a multiple of 512 a lane fetches 16 bytes of its row (two stages) at
+// a time.  Dword by dword each row's line is touched four times as often, and those
+// instructions, 64 lines each, cost as much as the operands' own (0.1 us per stage).
+// MXFP8 x MXFP4, N = 14336, K = 4096: M = 192 31.4 -> 16.5 us (112 -> 224 workgroups), M = 64
+// 27.4 -> 9.6, M = 100 41.7 -> 11.9; N = 4096, M = 192 26.8 -> 8.7, K = 14336 75.7 -> 22.6.
+constexpr int T8_MW(int mj) { return mj % 2 == 0 ? 2 : 1; }
+constexpr int T8_WAVES = 8, T8_THREADS = 64 * T8_WAVES, T8_TN = 128;
+template <bool XF8, int MJ>
+struct T8 {
+  static constexpr int TM = 32 * MJ;
+  static constexpr int MW = T8_MW(MJ), NI = MW, JW = MJ / MW;  // waves along m; tiles of W and of X per wave
+  static constexpr int X_ROWB = XF8 ? 256 : 128;
+  static constexpr int W_BYTES = T8_TN * 128, X_BYTES = TM * X_ROWB;
+  static constexpr int TILE = W_BYTES + X_BYTES;
+  static constexpr int WI = W_BYTES / 1024 / T8_WAVES;                               // 2
+  static constexpr int XB = X_BYTES / 1024, XI = (XB + T8_WAVES - 1) / T8_WAVES;     // blocks, per wave
+  static constexpr int SLOT = (T8_TN + 128) * 16;  // scales of two stages: 128 rows of W, up to 128 of X
+  static constexpr int SLOTS = 3;
+  static constexpr int FIT = (160 * 1024 - SLOTS * SLOT - 256) / TILE, STAGES = FIT < 5 ? FIT : 5;  // 3 to 5
+  static constexpr int SC_AT = STAGES * TILE;
+  static constexpr int DUMMY_AT = SC_AT + SLOTS * SLOT;  // where waves without scales to fetch put a dword
+  static constexpr int LDS = DUMMY_AT + 256;
+  static constexpr int NB = XF8 ? 2 : 1;
+  static constexpr int C_PITCH = T8_TN * 2 + 16;
+  static_assert(LDS <= 160 * 1024 && 4 * MJ * 4096 + TM * C_PITCH <= LDS, "fits LDS");
+};
+
+template <bool XF8, int MJ, bool SC16>
+__global__ __launch_bounds__(T8_THREADS) void mxn_tile8_kernel(
+    const uint32_t* __restrict__ wq, const uint8_t* __restrict__ ws,
+    const uint32_t* __restrict__ xq, const uint8_t* __restrict__ xs, w4_half* __restrict__ c,
+    int N, int K, int B, int M, int tiles_m) {
+  typedef T8<XF8, MJ> C;
+  constexpr int S = C::STAGES;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // in an SGPR: LDS addresses go to M0
+  const int r = lane & 31, h = lane >> 5;
+  const int wn = (wave & 3) / C::MW, wm = (wave & 3) % C::MW, kh = wave >> 2;
+  constexpr int NI = C::NI, JW = C::JW;
+  // consecutive workgroup ids land on different XCDs: a contiguous run of the tile order (m
+  // fastest) per XCD, whatever the number of tiles
+  const int total = (int)gridDim.x, xcd = (int)blockIdx.x & 7;
+  const int L = xcd * (total >> 3) + min(xcd, total & 7) + ((int)blockIdx.x >> 3);
+  const int n0 = (L / tiles_m) * T8_TN, m0 = (L % tiles_m) * C::TM;
+  const int wk = K >> 3;
+
+  // What this lane fetches (byte offsets, 32 bits: tile_operands_ok bounds the operands).  Rows
+  // past N or M are clamped to the last one; their results are never stored.
+  const int row8 = lane >> 3;
+  uint32_t wo[C::WI], xo[C::XI], xdst[C::XI];
+#pragma unroll
+  for (int i = 0; i < C::WI; ++i) {
+    const int R = (wave + T8_WAVES * i) * 8 + row8, n = n0 + R;
+    wo[i] = (uint32_t)(n < N ? n : N - 1) * (uint32_t)wk * 4u + (((lane & 7) ^ ((R >> 1) & 7)) * 16);
+  }
+#pragma unroll
+  for (int i = 0; i < C::XI; ++i) {
+    const int blk = (wave + T8_WAVES * i) % C::XB;  // (surplus waves repeat a block)
+    xdst[i] = C::W_BYTES + blk * 1024;
+    if (XF8) {
+      const int R = blk * 4 + (lane >> 4), m = m0 + R;
+      xo[i] = (uint32_t)(m < M ? m : M - 1) * (uint32_t)K + (((lane & 15) ^ (R & 15)) * 16);
+    } else {
+      const int R = blk * 8 + row8, m = m0 + R;
+      xo[i] = (uint32_t)(m < M ? m : M - 1) * (uint32_t)wk * 4u + (((lane & 7) ^ ((R >> 1) & 7)) * 16);
+    }
+  }
+  // scales: SC16: waves 0, 1 W rows 64 wave + lane, waves 2, 3 X rows; else wave w: W (w < 4)
+  // or X rows 64 (w & 1) + lane, dword (w / 2) % 2 of the stage's two
+  const bool w_sc = SC16 ? wave < 2 : wave < 4;
+  const int srow = (wave & 1) * 64 + lane;
+  const int sg = w_sc ? min(n0 + srow, N - 1) : min(m0 + min(srow, C::TM - 1), M - 1);
+  const uint32_t sco = (uint32_t)sg * (uint32_t)B + (SC16 ? 0u : (uint32_t)((wave >> 1) & 1) * 4u);
+  const uint8_t* scb = w_sc ? ws : xs;
+  const char* wqb = (const char*)wq;
+  const char* xqb = (const char*)xq;
+  const int stages = K >> 8;
+  auto dma16 = [](const void* gbase, uint32_t goff, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(goff), "s"(gbase), "s"(lds_addr)
+                 : "memory", "m0");
+  };
+  auto dma4 = [](const void* gbase, uint32_t goff, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1"
+                 :
+                 : "v"(goff), "s"(gbase), "s"(lds_addr)
+                 : "memory", "m0");
+  };
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)dm_lds;
+  // par: parity of d, a constant where the loop is unrolled
+  auto request = [&](int d, uint32_t buf, int par) {
+    const uint32_t dd = (uint32_t)(d < stages ? d : stages - 1);  // past the end: valid, never used
+    const uint32_t st = lds0 + buf;
+#pragma unroll
+    for (int i = 0; i < C::WI; ++i) dma16(wqb + dd * 128u, wo[i], st + (wave + T8_WAVES * i) * 1024);
+#pragma unroll
+    for (int i = 0; i < C::XI; ++i) dma16(xqb + dd * (uint32_t)C::X_ROWB, xo[i], st + xdst[i]);
+    if (SC16) {
+      if (par == 0) {  // scales of stages d and d + 1; a constant count of loads per wave
+        const uint32_t slot = lds0 + C::SC_AT + (uint32_t)((d >> 1) % C::SLOTS) * C::SLOT;
+        if (wave < 4) dma16(scb + (dd & ~1u) * 8u, sco, slot + wave * 1024);
+        else dma4(ws, 0u, lds0 + C::DUMMY_AT);
+      }
+    } else {
+      const uint32_t slot = lds0 + C::SC_AT + (uint32_t)((d >> 1) % C::SLOTS) * C::SLOT;
+      dma4(scb + dd * 8u, sco, slot + (uint32_t)par * 2048u + ((wave >> 1) & 1) * 1024 + (w_sc ? 0 : 512) + (wave & 1) * 256);
+    }
+  };
+  auto at = [](int R, int p) { return (R >> 3) * 1024 + ((R & 7) * 8 + (p ^ ((R >> 1) & 7))) * 16; };
+  auto at8 = [](int R, int p) { return (R >> 2) * 1024 + ((R & 3) * 16 + (p ^ (R & 15))) * 16; };
+  struct Frags {  // one lane's operands of its 128-k half: [64-k step]
+    u4 a[2][NI], b[2][JW][C::NB];
+    uint32_t sa[NI], sb[JW];
+  };
+  uint32_t woff[2], xoff[2][C::NB];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    woff[s] = at(wn * (32 * NI) + r, 4 * kh + 2 * s + h);
+    if constexpr (XF8) {
+      // of the 64 k of a product an 8-bit lane group h holds k 16h.. and 32+16h..
+      xoff[s][0] = C::W_BYTES + at8(wm * (32 * JW) + r, 8 * kh + 4 * s + h);
+      xoff[s][1] = C::W_BYTES + at8(wm * (32 * JW) + r, 8 * kh + 4 * s + 2 + h);
+    } else {
+      xoff[s][0] = C::W_BYTES + at(wm * (32 * JW) + r, 4 * kh + 2 * s + h);
+    }
+  }
+  auto read_frags = [&](Frags& f, int d, uint32_t buf, int par) {
+    const uint8_t* base = dm_lds + buf;
+    const uint8_t* sc = dm_lds + C::SC_AT + ((d >> 1) % C::SLOTS) * C::SLOT;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) f.a[s][i] = *(const u4*)(base + woff[s] + i * 4096);
+#pragma unroll
+      for (int j = 0; j < JW; ++j)  // the next tile of 32 rows is 32 X_ROWB bytes further
+#pragma unroll
+        for (int b = 0; b < C::NB; ++b) f.b[s][j][b] = *(const u4*)(base + xoff[s][b] + j * 32 * C::X_ROWB);
+    }
+    if (SC16) {
+      const uint8_t* p = sc + par * 8 + kh * 4;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) f.sa[i] = *(const uint32_t*)(p + ((wn * NI + i) * 32 + r) * 16);
+#pragma unroll
+      for (int j = 0; j < JW; ++j) f.sb[j] = *(const uint32_t*)(p + (T8_TN + (wm * JW + j) * 32 + r) * 16);
+    } else {
+      const uint8_t* p = sc + par * 2048 + kh * 1024;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) f.sa[i] = *(const uint32_t*)(p + ((wn * NI + i) * 32 + r) * 4);
+#pragma unroll
+      for (int j = 0; j < JW; ++j) f.sb[j] = *(const uint32_t*)(p + 512 + ((wm * JW + j) * 32 + r) * 4);
+    }
+  };
+  f16v acc[NI][JW];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < JW; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  auto multiply = [&](const Frags& f) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int sh = 16 * s + 8 * h;
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < JW; ++j) {
+          if constexpr (XF8)
+            acc[i][j] = mfma_fp4_fp8_32(f.a[s][i], f.sa[i] >> sh, f.b[s][j][0], f.b[s][j][1], f.sb[j] >> sh, acc[i][j]);
+          else
+            acc[i][j] = mfma_fp4_32(f.a[s][i], f.sa[i] >> sh, f.b[s][j][0], f.sb[j] >> sh, acc[i][j]);
+        }
+    }
+  };
+
+  // Iteration d: stage d has landed for every wave and nobody reads stage d - 1 any more, so
+  // stage d + S - 1 is requested into the buffer of d - 1; d's operands are read while those
+  // of d - 1 are multiplied.
+  constexpr int LD = C::WI + C::XI;
+  // loads of stages d + 1 .. d + S - 2, for d of parity par
+  auto allowed = [](int par) constexpr {
+    int n = 0;
+    for (int k = 1; k <= S - 2; ++k) n += LD + (!SC16 || ((par + k) & 1) == 0 ? 1 : 0);
+    return n;
+  };
+  Frags fa, fb;
+#pragma unroll
+  for (int d = 0; d < S - 1; ++d) request(d, (uint32_t)d * C::TILE, d & 1);
+  uint32_t cur = 0, nxt = (uint32_t)(S - 1) * C::TILE;  // buffers of stage d and of stage d + S - 1
+  auto bump = [&](uint32_t& b) { b = b + C::TILE == (uint32_t)S * C::TILE ? 0u : b + C::TILE; };
+  // stage 0: nothing to multiply yet
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(allowed(0)));
+  __syncthreads();
+  request(S - 1, nxt, (S - 1) & 1);
+  read_frags(fa, 0, cur, 0);
+  bump(cur), bump(nxt);
+  int d = 1;
+#pragma unroll 1
+  for (; d + 1 < stages; d += 2) {
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(allowed(1)));
+    __syncthreads();
+    request(d + S - 1, nxt, S & 1);
+    read_frags(fb, d, cur, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(fa);
+    __builtin_amdgcn_sched_barrier(0);
+    bump(cur), bump(nxt);
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(allowed(0)));
+    __syncthreads();
+    request(d + S, nxt, (S + 1) & 1);
+    read_frags(fa, d + 1, cur, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(fb);
+    __builtin_amdgcn_sched_barrier(0);
+    bump(cur), bump(nxt);
+  }
+  if (d < stages) {  // an even number of stages: the last one
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+    __syncthreads();
+    read_frags(fb, d, cur, 1);
+    multiply(fa);
+    multiply(fb);
+  } else {
+    multiply(fa);
+  }
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // nothing may still be writing LDS below
+  __syncthreads();
+
+  // first half + second half, rounded once, through LDS to stores of whole lines.  A lane
+  // holds, of each 32 x 32 tile, n = 8 q + 4 h + e for m = tile row r.
+  float* red = (float*)dm_lds + (wave & 3) * (MJ * 16 * 64);
+  uint8_t* ct = dm_lds + 4 * MJ * 4096;
+  if (kh == 1) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < JW; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *(f4*)(red + (((i * JW + j) * 4 + q) * 64 + lane) * 4) =
+              f4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+  }
+  __syncthreads();
+  if (kh == 0) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < JW; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f4 o = *(const f4*)(red + (((i * JW + j) * 4 + q) * 64 + lane) * 4);
+          h4 out;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) out[e] = (_Float16)(acc[i][j][4 * q + e] + o[e]);
+          *(h4*)(ct + ((wm * JW + j) * 32 + r) * C::C_PITCH + (wn * NI + i) * 64 + q * 16 + h * 8) = out;
+        }
+  }
+  __syncthreads();
+  const bool lines = (N & 7) == 0 && ((uintptr_t)c & 15) == 0;  // 16-byte pieces are aligned
+  const int nn = n0 + (t & 15) * 8;
+#pragma unroll
+  for (int it = 0; it < C::TM / 32; ++it) {
+    const int row = it * 32 + (t >> 4), m = m0 + row;
+    if (m >= M || nn >= N) continue;
+    const u4 v = *(const u4*)(ct + row * C::C_PITCH + (t & 15) * 16);
+    w4_half* dst = c + (size_t)m * N + nn;
+    if (lines && nn + 8 <= N) {
+      *(u4*)dst = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (nn + e < N) dst[e] = (w4_half)(v[e >> 1] >> (16 * (e & 1)));
+    }
+  }
+}
+
+template <bool XF8, int MJ, bool SC16>
+hipError_t launch_tile8(const w4_packed_mx_view& w, const void* xq, const uint8_t* xs, int M,
+                        w4_half* c, hipStream_t s) {
+  constexpr int lds_bytes = T8<XF8, MJ>::LDS;
+  // more than 64 KB of LDS has to be granted per device, once
+  static std::atomic<bool> granted[64] = {};
+  int dev = 0;
+  if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
+  if (dev < 0 || dev >= 64 || !granted[dev]) {
+    const hipError_t e = hipFuncSetAttribute((const void*)mxn_tile8_kernel<XF8, MJ, SC16>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    if (e != hipSuccess) return e;
+    if (dev >= 0 && dev < 64) granted[dev] = true;
+  }
+  const int tiles_n = (w.N + T8_TN - 1) / T8_TN, tiles_m = (M + 32 * MJ - 1) / (32 * MJ);
+  mxn_tile8_kernel<XF8, MJ, SC16><<<dim3((unsigned)(tiles_n * tiles_m)), dim3(T8_THREADS), lds_bytes, s>>>(
+      w.q, w.scales, (const uint32_t*)xq, xs, c, w.N, w.K, w.B, M, tiles_m);
+  return hipGetLastError();
+}
+
+// ---- which kernel ----------------------------------------------------------------
+// What the tile kernels need.  x_row_bytes: K/2 or K.
+bool tile_operands_ok(const w4_packed_mx_view& w, const void* xq, const uint8_t* xs, int M, int x_row_bytes) {
+  return w.K % 256 == 0 && (long long)w.N * w.K < (1LL << 32) && (long long)M * x_row_bytes < (1LL << 32) &&
+         ((uintptr_t)w.q & 15) == 0 && ((uintptr_t)xq & 15) == 0 && ((uintptr_t)w.scales & 7) == 0 &&
+         ((uintptr_t)xs & 7) == 0;
+}
+
+// 1 .. 4: the eight-wave tile of 128 x 32 MJ; 8: the 256 x 128 tile; 0: the skinny kernel.
+// A kernel's time is its rounds over the 256 compute units times that of one workgroup, which
+// is linear in the stages (us, measured with every unit busy, K = 4096 and 14336; the scales of
+// a K that is no multiple of 512 add 0.12 per stage to the eight-wave tiles).
+// Few workgroups of the eight-wave tiles are slower than the skinny kernel, which reads W once
+// and X from L2.  Up to 64 rows it is ahead below 100 of them (N = 4096, K = 4096, M = 33: 8.1 us
+// both; N = 14336, M = 8: 11.1 -> 8.5, M = 33: 20.6 -> 9.2; K = 14336, N = 4096, M = 24: 16.7
+// against 20.9), with up to 4 rows below 160 (N = 13824, M = 1: 9.2 against 9.8; N = 28672:
+// 15.7 -> 11.3); from 65 to 128 rows up to 32 of them with 8-bit X (N = 1024, K = 4096: 6.8
+// against 7.7) and up to 64 at K <= 2048 (N = 2048, 4-bit X: 4.5 against 5.0).  Where K is no
+// multiple of 512 its guarded loads cost it 2 to 3 times as much and it keeps 32 rows (16 with
+// 4-bit X; N = 4096, K = 11008, M = 17: 20.1 against 21.9 and 24.0 -> 21.0; M = 33 26.1 -> 20.0)
+// and short K with 8-bit X (N = 1000, K = 1280, M = 64: 4.5 against 4.7).
+template <bool XF8>
+int plan_tile(const w4_packed_mx_view& w, int M) {
+  const long long tn = (w.N + T8_TN - 1) / T8_TN;
+  const float st = (float)(w.K / 256);
+  const long long wgs = tn * ((M + 31) / 32);
+  if (M <= 64 && (w.K % 512 == 0 || M <= (XF8 ? 32 : 16)) && wgs < (M <= 4 ? 160 : 100)) return 0;
+  if (M <= 128 && w.K % 512 == 0 && wgs <= (w.K <= 2048 ? 64 : XF8 ? 32 : 0)) return 0;
+  if (XF8 && M <= 128 && w.K <= 2048 && wgs <= 24) return 0;
+  static constexpr float slope[5] = {0.f, XF8 ? .33f : .29f, XF8 ? .50f : .39f, XF8 ? .75f : .55f, XF8 ? 1.0f : .65f};
+  float best = 0.f;
+  int pick = 0;
+  for (int mj = 1; mj <= 4; ++mj) {
+    const long long rounds = (tn * ((M + 32 * mj - 1) / (32 * mj)) + 255) / 256;
+    const float us = (float)rounds * (3.5f + st * (slope[mj] + (w.K % 512 ? .12f : 0.f)));
+    if (pick == 0 || us < best) best = us, pick = mj;
+  }
+  const long long big = ((w.N + TL_TN - 1) / TL_TN) * (long long)((M + TL_TM - 1) / TL_TM);
+  if (M >= 128 && (float)((big + 255) / 256) * (XF8 ? 6.9f + 1.6f * st : 5.f + 1.1f * st) < best) pick = 8;
+  return pick;
 }
 
 template <bool XF8>
@@ -842,19 +1179,39 @@ hipError_t launch_tile(const w4_packed_mx_view& w, const void* xq, const uint8_t
   return hipGetLastError();
 }
 
+template <bool XF8, int MJ>
+hipError_t launch_tile8_sc(const w4_packed_mx_view& w, const void* xq, const uint8_t* xs, int M,
+                           w4_half* c, hipStream_t s) {
+  if (w.K % 512 == 0 && (((uintptr_t)w.scales | (uintptr_t)xs) & 15) == 0)
+    return launch_tile8<XF8, MJ, true>(w, xq, xs, M, c, s);
+  return launch_tile8<XF8, MJ, false>(w, xq, xs, M, c, s);
+}
+
+// x_row_bytes: K / 2 or K
+template <bool XF8>
+hipError_t launch_mxn(const w4_packed_mx_view& w, const void* xq, const uint8_t* xs, int M,
+                      int x_row_bytes, w4_half* c, hipStream_t s) {
+  switch (tile_operands_ok(w, xq, xs, M, x_row_bytes) ? plan_tile<XF8>(w, M) : 0) {
+    case 1: return launch_tile8_sc<XF8, 1>(w, xq, xs, M, c, s);
+    case 2: return launch_tile8_sc<XF8, 2>(w, xq, xs, M, c, s);
+    case 3: return launch_tile8_sc<XF8, 3>(w, xq, xs, M, c, s);
+    case 4: return launch_tile8_sc<XF8, 4>(w, xq, xs, M, c, s);
+    case 8: return launch_tile<XF8>(w, xq, xs, M, c, s);
+    default: return launch_skinny<XF8>(w, xq, xs, M, c, s);
+  }
+}
+
 }  // namespace
 
 hipError_t launch_gemm_mx_w4a4(const w4_packed_mx_view& w, const w4_packed_mx_view& x,
                                w4_half* c, hipStream_t s) {
-  if (tile_applies(w, x.q, x.scales, x.N, w.K / 2)) return launch_tile<false>(w, x.q, x.scales, x.N, c, s);
-  return launch_skinny<false>(w, x.q, x.scales, x.N, c, s);
+  return launch_mxn<false>(w, x.q, x.scales, x.N, w.K / 2, c, s);
 }
 
 // E4M3 activations (K a multiple of 32, rows 16-byte aligned).
 hipError_t launch_gemm_mx_w4a8(const w4_packed_mx_view& w, const w4_act_mx8_view& x, w4_half* c,
                                hipStream_t s) {
-  if (tile_applies(w, x.q, x.scales, x.M, w.K)) return launch_tile<true>(w, x.q, x.scales, x.M, c, s);
-  return launch_skinny<true>(w, x.q, x.scales, x.M, c, s);
+  return launch_mxn<true>(w, x.q, x.scales, x.M, w.K, c, s);
 }
 
 }  // namespace w4k
