@@ -43,3 +43,30 @@ def test_merge_in_place(i):
     c4, q, group = cases[0]
     ref = orc.attention_f16(q, orc.dequant_cache(c4, False), orc.dequant_cache(c4, True), c4.H, group, c4.S, c4.D)
     assert orc.rel_l2(runs[0].view(np.float16), ref) <= TOL
+
+
+def test_entries_with_their_own_scratch_overlap():
+    """The entry that allocates nothing and the other one keep their partials apart, so calls of the
+    two may overlap on different streams: their arrivals have to be counted apart as well."""
+    import torch
+    c = w4amd.capi()
+    H, S, D, group = 64, 3000, 128, 4
+    c4 = orc.quantize_cache(orc.normal_weights(H * S * D, 81), orc.normal_weights(H * S * D, 82), H, S, D, 32, True)
+    dk = DevKV(c4)
+    qs = [to_dev(orc.normal_activations(H * group * D, 83 + i)) for i in range(2)]
+    want = []
+    for q in qs:
+        out = halves(H * group * D, 0x7E00)
+        c.attention_w4_flash(dk.view, ptr(q), ptr(out), group=group)
+        want.append(bits(out).copy())
+    entries = (c.attention_w4_flash, c.attention_w4_flash_noalloc)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = [[halves(H * group * D, 0x7E00) for _ in range(20)] for _ in range(2)]
+    torch.cuda.synchronize()
+    for n in range(20):
+        for i in range(2):
+            entries[i](dk.view, ptr(qs[i]), ptr(outs[i][n]), streams[i].cuda_stream, group=group)
+    torch.cuda.synchronize()
+    for i in range(2):
+        for n in range(20):
+            assert np.array_equal(bits(outs[i][n]), want[i]), (i, n)

@@ -86,17 +86,25 @@ int check_mx(const w4_packed_mx_view* p) {
 // library ever holds per device stays below twice the largest request.
 constexpr int MAX_DEVICES = 64;
 std::mutex g_scratch_mu;
-std::atomic<float*> g_scratch[MAX_DEVICES] = {};
+float* g_scratch[MAX_DEVICES][w4k::FL_SCRATCH_IDS] = {};  // every buffer made so far, by its id
+std::atomic<int> g_scratch_id[MAX_DEVICES] = {};           // the newest
 std::atomic<size_t> g_scratch_cap[MAX_DEVICES] = {};
 
-hipError_t scratch_floats(size_t n, float** out) {
+// Id of a buffer of n floats: two partials of 66 floats are the least that is merged.
+int scratch_id_of(size_t n) {
+  const int lg = 63 - __builtin_clzll((unsigned long long)n | 1);
+  return lg < 7 ? 1 : lg - 6 < w4k::FL_SCRATCH_IDS ? lg - 6 : w4k::FL_SCRATCH_IDS - 1;
+}
+
+hipError_t scratch_floats(size_t n, float** out, int* id) {
   int dev = -1;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   if (dev < 0 || dev >= MAX_DEVICES) return hipErrorInvalidDevice;
   if (n <= g_scratch_cap[dev].load(std::memory_order_acquire)) {
     // (the pointer published with this capacity, or a larger buffer published since)
-    *out = g_scratch[dev].load(std::memory_order_acquire);
+    *id = g_scratch_id[dev].load(std::memory_order_acquire);
+    *out = g_scratch[dev][*id];
     return hipSuccess;
   }
   std::lock_guard<std::mutex> lk(g_scratch_mu);
@@ -106,10 +114,12 @@ hipError_t scratch_floats(size_t n, float** out) {
     float* nb = nullptr;
     e = hipMalloc((void**)&nb, want * sizeof(float));
     if (e != hipSuccess) return e;
-    g_scratch[dev].store(nb, std::memory_order_release);
+    g_scratch[dev][scratch_id_of(want)] = nb;
+    g_scratch_id[dev].store(scratch_id_of(want), std::memory_order_release);
     g_scratch_cap[dev].store(want, std::memory_order_release);
   }
-  *out = g_scratch[dev].load(std::memory_order_relaxed);
+  *id = g_scratch_id[dev].load(std::memory_order_relaxed);
+  *out = g_scratch[dev][*id];
   return hipSuccess;
 }
 
@@ -167,7 +177,7 @@ hipError_t noalloc_scratch(float** out) {
 
 int run_flash(w4k::FlashArgs& a, w4_stream stream, const char* what) {
   float* part = nullptr;
-  hipError_t e = scratch_floats(w4k::flash_scratch_floats(a), &part);
+  hipError_t e = scratch_floats(w4k::flash_scratch_floats(a), &part, &a.scratch_id);
   if (e != hipSuccess) return runtime("flash scratch", e);
   return done(what, w4k::launch_flash(a, part, (hipStream_t)stream));
 }
@@ -344,6 +354,7 @@ int w4_attention_w4_flash_gqa_noalloc(const w4_kv_view* p, int group, const w4_h
   float* part = nullptr;
   hipError_t e = noalloc_scratch(&part);
   if (e != hipSuccess) return runtime("flash noalloc scratch", e);
+  a.scratch_id = 0;
   return done("flash_w4", w4k::launch_flash(a, part, (hipStream_t)stream));
 }
 

@@ -106,9 +106,10 @@ __device__ __forceinline__ h8 pack8(const h2 v[4]) {
   return h8{v[0][0], v[0][1], v[1][0], v[1][1], v[2][0], v[2][1], v[3][0], v[3][1]};
 }
 
-// Arrivals of a slab's splits, by number of splits and slab (see the end of the kernel).
-// Zero when the library is loaded and after every call.
-__device__ uint32_t flash_arrivals[(FM_MERGE_SPLITS + 1) * FM_MERGE_SLABS];
+// Arrivals of a slab's splits, by scratch buffer, number of splits and slab (see the end of
+// the kernel).  Zero when the library is loaded and after every call.  Calls whose partials lie
+// in different buffers may overlap, so every buffer has counters of its own.
+__device__ uint32_t flash_arrivals[FL_SCRATCH_IDS * (FM_MERGE_SPLITS + 1) * FM_MERGE_SLABS];
 
 // PAGED: 0 contiguous slabs, 1 pages of a multiple of 16 rows (both halves of a
 // tile lie in one page each), 2 any page size.  ALT: W4 with zero-points; FP8 with one
@@ -118,7 +119,7 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
                                                                    const int qh0,
                                                                    const int split_len,
                                                                    float* __restrict__ part,
-                                                                   const int merge_here) {
+                                                                   const int merge_id) {
   constexpr bool ASYM = KIND == KIND_W4 && ALT, SLAB_SCALE = KIND == KIND_F8 && ALT;
   constexpr int FM_D = DH;       // head dimension
   constexpr int NC = DH / 32;    // MFMAs per score group; a lane's K slice is 8 * NC elements
@@ -864,19 +865,20 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
     if (j) publish(dst, sum0, sum1);
     else publish(dst, M, sum0);
   }
-  if (!merge_here) return;
+  if (merge_id < 0) return;
 
   // The workgroup of a slab that finishes last merges the slab's splits.  Each one counts
   // itself once its partial has been written (the stores have come back); the counter wraps
   // to 0 with the last one, so the next call finds it as this one did.  There is one counter
-  // per (number of splits, slab): calls that share a counter make the same number of
+  // per (scratch buffer, number of splits, slab): calls that share a counter make the same number of
   // arrivals, so even calls that overlapped by mistake leave it at 0.
   __shared__ uint32_t arrived;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0)
-    arrived = __builtin_amdgcn_atomic_inc32(&flash_arrivals[nsplit * FM_MERGE_SLABS + slab], (uint32_t)(nsplit - 1),
-                                            __ATOMIC_RELAXED, "agent");
+    arrived = __builtin_amdgcn_atomic_inc32(
+        &flash_arrivals[(merge_id * (FM_MERGE_SPLITS + 1) + nsplit) * FM_MERGE_SLABS + slab], (uint32_t)(nsplit - 1),
+        __ATOMIC_RELAXED, "agent");
   __syncthreads();
   if (arrived != (uint32_t)(nsplit - 1)) return;
   // A wave takes every fourth head.  Lane t has the maximum and the denominator of split t,
@@ -929,7 +931,7 @@ static hipError_t go_alt(const FlashArgs& a, int qh0, const FlashPlan& pl, float
   const bool alt = (KIND == KIND_W4 && !a.symmetric) || (KIND == KIND_F8 && a.scale_mode == 1);
 #define W4_GO(DH, ALT)                                                         \
   flash_mfma_phase1<KIND, DH, HOOK, PAGED, (ALT) && KIND != KIND_F16, LDS>     \
-      <<<grid, FM_WAVES * 64, 0, s>>>(a, qh0, pl.split_len, part, flash_merges_in_place(a, pl))
+      <<<grid, FM_WAVES * 64, 0, s>>>(a, qh0, pl.split_len, part, flash_merges_in_place(a, pl) ? a.scratch_id : -1)
   if (a.D == 128) {
     if (alt) W4_GO(128, true); else W4_GO(128, false);
   } else {

@@ -93,11 +93,15 @@ struct FlashArgs {
   int bt_stride;   // entries per sequence table
   int page, pool_rows;
   int Hkv;         // paged: pool slabs; sequence = slab / Hkv
+  int scratch_id;  // which of the FL_SCRATCH_IDS buffers holds the partials
   const w4_half* q;
   w4_half* out;
   w4_half* k_out;
   w4_half* v_out;
 };
+// Scratch buffers that calls in flight may be using: 0 the fixed one; from 1 on the grown one and
+// those it has replaced, by the logarithm of their size (each is at least twice its predecessor).
+constexpr int FL_SCRATCH_IDS = 32;
 enum { KIND_F16 = 0, KIND_W4 = 1, KIND_F8 = 2 };  // FlashArgs::kind
 
 // Split of the sequence over workgroups (shared by both phase-1 kernels).
