@@ -506,25 +506,30 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
         clo[kk] = as_h2(0xE400E400u | zz);         // -(1024 + z), ulp 1
         chi[kk] = as_h2(0xD400D400u | (zz << 4));  // -(64 + z), ulp 1/16
       }
-      h2 pe[4][NE];  // (two elements of every position at a time: few registers live at once)
+      h2 pe[4][NE];
+      auto expand = [&](int kk, int b) {
+        const uint32_t p = __builtin_amdgcn_perm(raw.v[2 * kk + 1], raw.v[2 * kk],
+                                                 0x0c000c00u | ((4u + b + byte0) << 16) | (b + byte0));
+        pe[kk][2 * b] = (as_h2(and_or(p, 0x000F000Fu, magic_lo)) + clo[kk]) * s2[kk];
+        pe[kk][2 * b + 1] = (as_h2(and_or(p, 0x00F000F0u, magic_hi)) + chi[kk]) * s2[kk];
+      };
+      auto multiply = [&](int e) {
+        const h2 at[4] = {pe[0][e], pe[1][e], pe[2][e], pe[3][e]};
+        o[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pack8(at), pop, o[e], 0, 0, 0);
+      };
+      if constexpr (!HOOK) {  // two elements of every position at a time: few registers live at once
 #pragma unroll
-      for (int b = 0; b < NE / 2; ++b) {
+        for (int b = 0; b < NE / 2; ++b) {
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk) expand(kk, b);
+          multiply(2 * b);
+          multiply(2 * b + 1);
+        }
+      } else {  // position by position, as they are stored
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
-          const uint32_t p = __builtin_amdgcn_perm(raw.v[2 * kk + 1], raw.v[2 * kk],
-                                                   0x0c000c00u | ((4u + b + byte0) << 16) | (b + byte0));
-          pe[kk][2 * b] = (as_h2(and_or(p, 0x000F000Fu, magic_lo)) + clo[kk]) * s2[kk];
-          pe[kk][2 * b + 1] = (as_h2(and_or(p, 0x00F000F0u, magic_hi)) + chi[kk]) * s2[kk];
-        }
 #pragma unroll
-        for (int e = 2 * b; e < 2 * b + 2; ++e) {
-          const h2 at[4] = {pe[0][e], pe[1][e], pe[2][e], pe[3][e]};
-          o[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pack8(at), pop, o[e], 0, 0, 0);
-        }
-      }
-      if constexpr (HOOK) {
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
+          for (int b = 0; b < NE / 2; ++b) expand(kk, b);
           h2 n0[4], n1[4];
 #pragma unroll
           for (int i = 0; i < NE / 2; ++i) {
@@ -539,6 +544,8 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
             hook_store_v(2 * kk + 1, n1);
           }
         }
+#pragma unroll
+        for (int e = 0; e < NE; ++e) multiply(e);
       }
     } else {
       h2 vt[8][4];
