@@ -77,31 +77,26 @@ __device__ __forceinline__ uint32_t encode_e4m3(float x) {
   return sign | (uint32_t)(code > 0x7E ? 0x7E : code);
 }
 
-// encode_e4m3(v / s) for FP16-representable v and s without the division.  x = v * (1 / s)
-// is within 2^-22 (relative) of the exact quotient q.  q has 11-bit numerator and
-// denominator, so it is either exactly on a midpoint of the E4M3 grid (odd multiples
-// of half a step, at most 31) or at least 2^-16 (relative) away from every one: if x
-// is within 2^-20 of a midpoint, q is that midpoint and the tie goes to the even code;
-// otherwise x and q round alike.  (The host rounds the FP64 quotient to FP32 first,
+// Four E4M3 bytes of FP32 values (the hardware conversion rounds to nearest even, subnormals
+// included; past 448 it would give NaN, so the magnitude is capped first).  `from` gives the signs.
+__device__ __forceinline__ uint32_t pack_e4m3(const float* mag, const float* from) {
+  float x[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i] = copysignf(fminf(mag[i], 448.0f), from[i]);
+  const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(x[0], x[1], 0, false);
+  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(x[2], x[3], lo, true);
+}
+
+// |v / s| for FP16-representable v and s > 0, near enough for E4M3 without the division: x = |v| * rs
+// with rs = 1 / s to within 2^-22, then one correction by the residual |v| - x s, which is
+// exact (a multiple of ulp(x) ulp(s) that is 2^-21 of |v|: under 24 bits).  The exact quotient has
+// an 11-bit numerator and denominator: it is either on a midpoint of the E4M3 grid, which has 5
+// bits and which the correction then returns exactly, or at least 2^-16 (relative) away from
+// every midpoint, so that x rounds as it does.  (The host rounds the FP64 quotient to FP32 first,
 // which for the same reason never moves it onto or across a midpoint.)
-__device__ __forceinline__ uint32_t encode_e4m3_quotient(float v, float rs) {
-  const float x = v * rs;
-  const uint32_t sign = (__builtin_bit_cast(uint32_t, x) >> 24) & 0x80u;
-  // straight-line code (as early returns per element the compiler made 16 divergent
-  // regions per thread): saturation is the grid's own top, 448 = 14 steps of 2^5
-  const float a = fminf(fabsf(x), 448.0f);
-  int ex = (int)((__builtin_bit_cast(uint32_t, a) >> 23) & 0xFFu) - 127;
-  ex = ex < -6 ? -6 : ex;
-  const float y = a * __builtin_bit_cast(float, (uint32_t)(130 - ex) << 23);  // exact; 0 .. 16 steps
-  const float f = floorf(y);
-  const float d = fabsf((y - f) - 0.5f);  // distance from the midpoint, exact
-  float r = rintf(y);
-  r = d < y * 0x1p-20f ? f + (float)((int)f & 1) : r;
-  const int steps = (int)r;
-  int code = (ex + 7) * 8 + (steps - 8);  // with ex = -6 this is `steps` itself, subnormal or not
-  code = code > 0x7E ? 0x7E : code;
-  code = x != x ? 0x7F : code;
-  return sign | (uint32_t)code;
+__device__ __forceinline__ float quotient_magnitude(float v, float s, float rs) {
+  const float a = fabsf(v), x = a * rs;
+  return fmaf(fmaf(-x, s, a), rs, x);
 }
 
 __device__ __forceinline__ int pow2_at_least(int n) {
@@ -244,44 +239,30 @@ __global__ __launch_bounds__(QT) void quantize_rows_kernel(
   }
 }
 
-// Arithmetic type of the per-element quotient.  FP64 sources divide in FP64 as
-// the host does.  FP16 sources divide in FP32: value and scale have 11-bit
-// significands, so the exact quotient is either on a rounding boundary (k + 1/2
-// for the codes, a 25-bit midpoint for the FP32 quotient the E4M3 encoder
-// takes) or at least 2^-14 (2^-36 relative) away from it -- far more than the
-// FP32 (FP64) rounding error -- and the correctly rounded FP32 quotient gives
-// the code the host's FP64 quotient gives.
+// Arithmetic type of the elements.  FP64 sources divide in FP64 as the host does.  FP16 sources
+// work in FP32 and multiply by the reciprocal: see quotient_code and quotient_magnitude.
 template <typename T> struct Quot { typedef double type; };
 template <> struct Quot<_Float16> { typedef float type; };
 
-__device__ __forceinline__ int round_half_away_small(float v) {
-  float t = truncf(v);
-  const float frac = fabsf(v - t);
-  t = fminf(fmaxf(t, -1.0e6f), 1.0e6f);
-  int r = (int)t;
-  if (frac >= 0.5f) r += v < 0.0f ? -1 : 1;
-  return r;
+// clamp(round_half_away(v / sf) + zero, 0, 15) for FP16-representable v and sf > 0 without the
+// division.  The quotient of two 11-bit significands is on a midpoint k + 1/2 or at least 2^-12 away from
+// it, so a quotient that is made 2^-17 (relative) too large lands past the midpoint it was on,
+// away from zero, and across no other: floor(q (1 + 2^-17) + zero + 1/2) is the code.  Its error (2^-22
+// of q, 2^-20 from the sum) is below that shift from q = 1/2 on; beyond |q| = 16 every code
+// saturates.  grown = (1 / sf) (1 + 2^-17).  Four instructions an element; the two tests of the
+// remainder's sign around rint() that stood here before were fourteen.
+__device__ __forceinline__ uint32_t quotient_code(float v, float grown, float zero_half) {
+  return (uint32_t)__builtin_amdgcn_fmed3f(fmaf(v, grown, zero_half), 0.0f, 15.5f);
 }
-__device__ __forceinline__ int round_half_away_small(double v) { return (int)round_half_away(v); }
 
-// round_half_away(v / sf) for FP16-representable v and sf > 0 without the division: a
-// candidate from v * (1 / sf) (a few ulp off, so within one of the answer while
-// |v / sf| <= 64; beyond that every code saturates), then the two tests that define the
-// answer, v - (c -+ 1/2) sf against zero, each one fused multiply-add whose sign is
-// the exact sign (it rounds an exact real, and a nonzero difference of multiples of
-// 2^-25 cannot underflow).  A third fewer vector instructions than the correctly
-// rounded quotient plus its rounding, in a kernel that is bound by them.
-__device__ __forceinline__ int round_quotient_half_away(float v, float sf, float rsf) {
-  const float a = fabsf(v);  // half away from zero: round the magnitude half up, restore the sign
-  const float t = fminf(a * rsf, 64.0f);
-  const float c = rintf(t);
-  const float lo = fmaf(0.5f - c, sf, a);   // |v| - (c - 1/2) sf
-  const float hi = fmaf(-0.5f - c, sf, a);  // |v| - (c + 1/2) sf
-  int m = (int)c;
-  m -= lo < 0.0f ? 1 : 0;  // (straight-line code: as branches this was slower than the division)
-  m += hi >= 0.0f ? 1 : 0;
-  return v < 0.0f ? -m : m;
+// The value of lane ^ m, m a power of two that is the same for all lanes.
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v, int m) {
+  if (m == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);
+  if (m == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);
+  return __shfl_xor(v, m);
 }
+
+typedef uint16_t us2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ void load8(const double* p, double v[8]) {
   typedef double d2 __attribute__((ext_vector_type(2)));
@@ -302,6 +283,9 @@ __device__ __forceinline__ void load8(const _Float16* p, float v[8]) {
 // thread owns packed word `w` of the flattened (row, k) space, the gs / 8 lanes
 // of a group combine their extrema with lane exchanges and every lane derives
 // the group's scale itself -- no LDS round trip, fully coalesced 16-byte loads.
+// Bound by vector instructions, not by memory: 8 slabs x 4096 x 128 FP16 keys and values (21.5 MB)
+// took 10.1 us a call with some 220 of them a thread and take 7.3 with 97 (6.7 are the two launches
+// of a call at S = 16); E4M3 bytes 12.4 -> 8.4.
 // ZPACK: zero-point words are assembled through LDS (G and the groups per
 // workgroup both multiples of 8); otherwise nibbles are OR-ed in atomically.
 template <typename T, int MODE, bool ZPACK>
@@ -318,24 +302,57 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
   const long long w = (long long)blockIdx.x * QT + t;
   const bool live = w < nwords;
   A v[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = (A)0;
-  if (live) load8(src + w * 8, v);
-  A lo = v[0], hi = v[0];
+  A lo, hi;  // of the group; without zero-points of FP16 sources both are its largest magnitude
   bool bad = false;
+  if constexpr (sizeof(T) == 2) {
+    // extrema on pairs of halves; magnitudes as integers, which NaN and infinity end up on top of
+    u4 x = u4{0, 0, 0, 0};
+    if (live) x = *(const u4*)(src + w * 8);
+    us2 mag = __builtin_bit_cast(us2, x[0] & 0x7FFF7FFFu);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    if (sizeof(T) == 2) bad |= !(fabsf((float)v[j]) <= 65504.0f);
-    else bad |= !(fabs((double)v[j]) <= DBL_MAX);
-    lo = v[j] < lo ? v[j] : lo;
-    hi = v[j] > hi ? v[j] : hi;
+    for (int i = 1; i < 4; ++i)
+      mag = __builtin_elementwise_max(mag, __builtin_bit_cast(us2, x[i] & 0x7FFF7FFFu));
+    uint32_t top = mag[0] > mag[1] ? mag[0] : mag[1];
+    bad = top >= 0x7C00u;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (A)__builtin_bit_cast(_Float16, (uint16_t)(x[j >> 1] >> (16 * (j & 1))));
+    if constexpr (MODE == QM_ASYM) {
+      // (minimum, -maximum) in one register
+      h2 mn = as_h2(x[0]), mx = mn;
+#pragma unroll
+      for (int i = 1; i < 4; ++i) {
+        mn = __builtin_elementwise_min(mn, as_h2(x[i]));
+        mx = __builtin_elementwise_max(mx, as_h2(x[i]));
+      }
+      h2 ext = __builtin_elementwise_min(h2{mn[0], (_Float16)-mx[0]}, h2{mn[1], (_Float16)-mx[1]});
+      for (int m = 1; m < wpg; m <<= 1) ext = __builtin_elementwise_min(ext, as_h2(lane_xor(as_u32(ext), m)));
+      lo = (A)ext[0];
+      hi = -(A)ext[1];
+    } else {
+      for (int m = 1; m < wpg; m <<= 1) {
+        const uint32_t o = lane_xor(top, m);
+        top = o > top ? o : top;
+      }
+      lo = hi = (A)__builtin_bit_cast(_Float16, (uint16_t)top);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (A)0;
+    if (live) load8(src + w * 8, v);
+    lo = hi = v[0];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      bad |= !(fabs((double)v[j]) <= DBL_MAX);
+      lo = v[j] < lo ? v[j] : lo;
+      hi = v[j] > hi ? v[j] : hi;
+    }
+    for (int m = 1; m < wpg; m <<= 1) {
+      const A olo = __shfl_xor(lo, m), ohi = __shfl_xor(hi, m);
+      lo = olo < lo ? olo : lo;
+      hi = ohi > hi ? ohi : hi;
+    }
   }
   if (bad) atomicOr(status, 1);
-  for (int m = 1; m < wpg; m <<= 1) {
-    const A olo = __shfl_xor(lo, m), ohi = __shfl_xor(hi, m);
-    lo = olo < lo ? olo : lo;
-    hi = ohi > hi ? ohi : hi;
-  }
   // Scale of the group, in every lane.  The step goes FP64 -> FP32 -> FP16 on the
   // host.  For FP16 sources without zero-points the FP32 step is amax / 7 (/ 448)
   // of an 11-bit amax: its binary expansion is periodic with period 3, so it is
@@ -350,7 +367,7 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
     step_f = (float)(dhi > dlo ? (dhi - dlo) / 15.0 : 1.0);
     has_signal = dhi != dlo;
   } else if (sizeof(T) == 2) {
-    const float amax = fmaxf(fabsf((float)lo), fabsf((float)hi));
+    const float amax = (float)hi;
     step_f = amax > 0.0f ? amax / (MODE == QM_F8 ? 448.0f : 7.0f) : 1.0f;
     has_signal = amax > 0.0f;
   } else {
@@ -389,25 +406,33 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
   if (!live) return;
   const A sfa = (A)sf;
   if (MODE == QM_F8) {
-    uint32_t b[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if constexpr (sizeof(T) == 2) b[j] = encode_e4m3_quotient((float)v[j], __builtin_amdgcn_rcpf(sf));
-      else b[j] = encode_e4m3((float)(v[j] / sfa));
-    }
     u2 out;
-    out[0] = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
-    out[1] = b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24);
+    if constexpr (sizeof(T) == 2) {
+      const float rsf = __builtin_amdgcn_rcpf(sf);
+      float mag[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) mag[j] = quotient_magnitude(v[j], sf, rsf);
+      out[0] = pack_e4m3(mag, v);
+      out[1] = pack_e4m3(mag + 4, v + 4);
+    } else {
+      uint32_t b[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) b[j] = encode_e4m3((float)(v[j] / sfa));
+      out[0] = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
+      out[1] = b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24);
+    }
     *(u2*)(q8 + w * 8) = out;
   } else {
     uint32_t word = 0;
-    const float rsf = __builtin_amdgcn_rcpf(sf);
+    const float grown = __builtin_amdgcn_rcpf(sf) * (1.0f + 0x1p-17f), zero_half = (float)zero + 0.5f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      int c;
-      if constexpr (sizeof(T) == 2) c = round_quotient_half_away((float)v[j], sf, rsf) + zero;
-      else c = round_half_away_small(v[j] / sfa) + zero;
-      word |= (uint32_t)(c < 0 ? 0 : (c > 15 ? 15 : c)) << (4 * j);
+      if constexpr (sizeof(T) == 2) {
+        word |= quotient_code(v[j], grown, zero_half) << (4 * j);
+      } else {
+        const int c = (int)round_half_away(v[j] / sfa) + zero;
+        word |= (uint32_t)(c < 0 ? 0 : (c > 15 ? 15 : c)) << (4 * j);
+      }
     }
     q32[w] = word;
   }
@@ -517,18 +542,16 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
   }
   if (F8) {
     uint8_t* dst = q8 + row * (long long)K + k0;
-    uint32_t c[8];
+    float val[8], mag[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) c[j] = encode_e4m3((float)u[j]);
+    for (int j = 0; j < 8; ++j) val[j] = (float)u[j], mag[j] = fabsf(val[j]);
+    const u2 out = u2{pack_e4m3(mag, val), pack_e4m3(mag + 4, val + 4)};
     if (n == 8 && ((uintptr_t)dst & 7) == 0) {
-      u2 out;
-      out[0] = c[0] | (c[1] << 8) | (c[2] << 16) | (c[3] << 24);
-      out[1] = c[4] | (c[5] << 8) | (c[6] << 16) | (c[7] << 24);
       *(u2*)dst = out;
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        if (j < n) dst[j] = (uint8_t)c[j];
+        if (j < n) dst[j] = (uint8_t)(out[j >> 2] >> (8 * (j & 3)));
     }
   } else {
     uint32_t word = 0;
