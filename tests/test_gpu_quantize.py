@@ -424,3 +424,26 @@ def test_quantize_cache_status_word():
     assert int(_host(st)[0]) == 2
     with pytest.raises(ValueError, match="FP16 range"):
         orc.quantize_cache_f8(k, v, H, S, D, gs)
+
+
+# Cache rows with zero-points whose words are put together by one workgroup: one to four groups a
+# row, the shortest row, rows that do not fill the last workgroup, and sixteen groups (two words)
+@pytest.mark.parametrize("f16", [False, True], ids=["f64src", "f16src"])
+@pytest.mark.parametrize("D,gs", [(8, 8), (16, 8), (64, 64), (64, 16), (128, 32), (128, 8), (512, 128)])
+def test_zero_point_words_of_short_rows(D, gs, f16):
+    H, S = 3, 37
+    c = w4amd.capi()
+    k, v, kd, vd = _sources(H, S, D, 0x2E20 + D + gs, f16)
+    ref = orc.quantize_cache(k, v, H, S, D, gs, False)
+    rows, G = H * S, ref.G
+    dev = {n: torch.full((rows * per,), 0x5A5A5A5A, dtype=torch.int32, device=DEV)
+           for n, per in (("q_k", orc.words(D)), ("q_v", orc.words(D)), ("z_k", orc.words(G)), ("z_v", orc.words(G)))}
+    s = {n: torch.full((rows * G,), 0x7E00, dtype=torch.int16, device=DEV) for n in ("s_k", "s_v")}
+    st = _status()
+    view = c.kv_view(H, S, D, gs, G, False, ptr(dev["q_k"]), ptr(s["s_k"]), ptr(dev["z_k"]),
+                     ptr(dev["q_v"]), ptr(s["s_v"]), ptr(dev["z_v"]))
+    c.quantize_cache(view, ptr(kd), ptr(vd), ptr(st), src_f16=f16)
+    assert int(_host(st)[0]) == 0
+    for name, t in (dev | s).items():
+        want = getattr(ref, name)
+        assert np.array_equal(_host(t).view(want.dtype), want), name

@@ -286,8 +286,10 @@ __device__ __forceinline__ void load8(const _Float16* p, float v[8]) {
 // Bound by vector instructions, not by memory: 8 slabs x 4096 x 128 FP16 keys and values (21.5 MB)
 // took 10.1 us a call with some 220 of them a thread and take 7.3 with 97 (6.7 are the two launches
 // of a call at S = 16); E4M3 bytes 12.4 -> 8.4.
-// ZPACK: zero-point words are assembled through LDS (G and the groups per
-// workgroup both multiples of 8); otherwise nibbles are OR-ed in atomically.
+// ZPACK: zero-point words are assembled through LDS (G and the groups per workgroup both
+// multiples of 8, or whole rows per workgroup: cache rows); otherwise nibbles are OR-ed in
+// atomically, into words that a launch per side has cleared before (8 x 4096 x 128 with gs = 32:
+// 13.6 us a call with those launches and FP64 divisions for step and zero-point, 9.2 without).
 template <typename T, int MODE, bool ZPACK>
 __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
     const Sides<T> sd, long long nwords, int wpg, int wpg_shift, int G, int* __restrict__ status) {
@@ -364,7 +366,17 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
   if (MODE == QM_ASYM) {
     dlo = fmin(dlo, 0.0);
     dhi = fmax(dhi, 0.0);
-    step_f = (float)(dhi > dlo ? (dhi - dlo) / 15.0 : 1.0);
+    const double range = dhi - dlo;
+    double step;
+    if constexpr (sizeof(T) == 2) {
+      // range / 15, correctly rounded: a quotient by the rounded reciprocal, corrected once by its
+      // residual (the range is between 2^-24 and 2^17, so nothing under- or overflows)
+      const double q = range * (1.0 / 15.0);
+      step = fma(fma(-q, 15.0, range), 1.0 / 15.0, q);
+    } else {
+      step = range / 15.0;
+    }
+    step_f = (float)(range > 0.0 ? step : 1.0);
     has_signal = dhi != dlo;
   } else if (sizeof(T) == 2) {
     const float amax = (float)hi;
@@ -379,7 +391,11 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
   const _Float16 sh = (_Float16)step_f;
   const float sf = (float)sh;
   int zero = 8;
-  if (MODE == QM_ASYM) zero = clamp_code(round_half_away(-dlo / (double)sf));
+  const float grown = __builtin_amdgcn_rcpf(sf) * (1.0f + 0x1p-17f);
+  if constexpr (MODE == QM_ASYM) {
+    if constexpr (sizeof(T) == 2) zero = (int)quotient_code(-(float)dlo, grown, 0.5f);
+    else zero = clamp_code(round_half_away(-dlo / (double)sf));
+  }
   const bool leader = live && (t & (wpg - 1)) == 0;
   const long long gid = w >> wpg_shift;
   if (leader) {
@@ -395,12 +411,22 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
     if ((t & (wpg - 1)) == 0) s_zero[t >> wpg_shift] = zero;
     __syncthreads();
     const int gpb = QT >> wpg_shift;
-    const long long zw = ((long long)blockIdx.x * gpb >> 3) + t;
-    if (t < (gpb >> 3) && zw * 8 * wpg < nwords) {
-      uint32_t word = 0;
+    if ((G & 7) == 0) {
+      const long long zw = ((long long)blockIdx.x * gpb >> 3) + t;
+      if (t < (gpb >> 3) && zw * 8 * wpg < nwords) {
+        uint32_t word = 0;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) word |= (uint32_t)s_zero[t * 8 + j] << (4 * j);
-      zeros[zw] = word;
+        for (int j = 0; j < 8; ++j) word |= (uint32_t)s_zero[t * 8 + j] << (4 * j);
+        zeros[zw] = word;
+      }
+    } else {  // whole rows per workgroup: thread t makes word t of them
+      const int wpr = (G + 7) >> 3, r = t / wpr, i = t - r * wpr;
+      const long long row = (long long)blockIdx.x * (gpb / G) + r;
+      if (r < gpb / G && row * G * wpg < nwords) {
+        uint32_t word = 0;
+        for (int g = 8 * i; g < min(8 * i + 8, G); ++g) word |= (uint32_t)s_zero[r * G + g] << (4 * (g & 7));
+        zeros[row * wpr + i] = word;
+      }
     }
   }
   if (!live) return;
@@ -424,7 +450,7 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
     *(u2*)(q8 + w * 8) = out;
   } else {
     uint32_t word = 0;
-    const float grown = __builtin_amdgcn_rcpf(sf) * (1.0f + 0x1p-17f), zero_half = (float)zero + 0.5f;
+    const float zero_half = (float)zero + 0.5f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       if constexpr (sizeof(T) == 2) {
@@ -578,7 +604,8 @@ hipError_t launch_rows_t(const Sides<T>& sd, int nsides, long long rows, int K, 
     aligned = aligned && ((uintptr_t)sd.src[i] & 15) == 0 &&
               (MODE != QM_F8 || ((uintptr_t)sd.q8[i] & 7) == 0);
   const bool fast = pow2 && wpg <= 64 && K % gs == 0 && aligned;
-  const bool zpack = fast && MODE == QM_ASYM && G % 8 == 0 && (QT / wpg) % 8 == 0;
+  // (a workgroup covers 2048 elements; with whole rows a row has at most one word per thread)
+  const bool zpack = fast && MODE == QM_ASYM && ((G % 8 == 0 && (QT / wpg) % 8 == 0) || (QT * 8) % K == 0);
   if (MODE == QM_ASYM && !zpack) {
     // zero-points are OR-ed in nibble by nibble
     const long long nz = rows * words(G);
