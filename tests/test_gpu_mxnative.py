@@ -350,3 +350,36 @@ def test_eight_wave_tiles(M, N, K, shift, x8):
     # FP16 rounding of the sums is at most 2^-11 of each; FP32 sums of 1536 exact products add
     # less than 1e-5
     assert orc.rel_l2(got, ref) <= 5e-4
+
+
+@pytest.mark.parametrize("fmt", ["mx4", "mx8"])
+def test_activation_quantizers_every_half(fmt):
+    """FP16 activations whose blocks hold every magnitude down to 2^-9 of the block's maximum, for
+    maxima on and beside the two formats' powers of two, as whole rows and as one ragged row: the
+    codes and scales of the host, ties and signed zeros included."""
+    c = w4amd.capi()
+    mags = np.arange(0x7C00, dtype=np.uint16).view(np.float16)
+    rows = []
+    for top in (6.0, 7.0, 448.0, 1.0, 2.0 ** -14, 6.0 * 2.0 ** -12, 65504.0, 3e-6):
+        for m in (np.float16(top), np.nextafter(np.float16(top), np.float16(0))):
+            v = mags[(mags <= m) & (mags >= np.float32(m) / 512)]
+            v = np.concatenate([v, np.zeros(-len(v) % 31, np.float16)]).reshape(-1, 31)
+            sign = np.where(np.arange(v.size).reshape(v.shape) % 3 == 0, np.float16(-1), np.float16(1))
+            rows.append(np.concatenate([np.full((len(v), 1), m, np.float16), v * sign], axis=1))
+    x = np.concatenate(rows)
+    for M, K in (x.shape, (1, x.size - 3)):
+        flat = np.ascontiguousarray(x.ravel()[:M * K])
+        ref = (orc.quantize_mx if fmt == "mx4" else orc.quantize_mx8)(flat.astype(np.float64), M, K)
+        if fmt == "mx4":
+            _, q, s = _quantize_x_on_device(flat, M, K)
+            q = q.cpu().numpy().view(np.uint32)
+        else:
+            q8, s = (torch.full((n,), 0x5A, dtype=torch.uint8, device=DEV) for n in (M * K, M * ((K + 31) // 32)))
+            st = torch.full((1,), -1, dtype=torch.int32, device=DEV)
+            xd = to_dev(flat)
+            c.quantize_mx8_f16(c.act_mx8_view(M, K, (K + 31) // 32, ptr(q8), ptr(s)), ptr(xd), ptr(st))
+            torch.cuda.synchronize()
+            assert int(st.item()) == 0
+            q = q8.cpu().numpy()
+        assert np.array_equal(s.cpu().numpy(), ref.scales)
+        assert np.array_equal(q, ref.q)

@@ -482,17 +482,22 @@ __device__ __forceinline__ int mx_exponent(double amax, bool* out_of_range) {
   return e;
 }
 
+// The same from the FP32 value of a nonzero FP16 maximum: TOP is 1.5 * 2^2 or 1.75 * 2^8, so e is
+// p - 2 (p - 8), and one more where the significand is past TOP's.  (e is -32 .. 14: in range.)
+template <int TOP>
+__device__ __forceinline__ int mx_exponent_f16(float amax) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, amax);
+  return amax > 0.0f ? (int)((b + (TOP == 6 ? 0x3FFFFFu : 0x1FFFFFu)) >> 23) - (TOP == 6 ? 129 : 135) : 0;
+}
+
 // mx.hpp:103-108: index of the nearest E2M1 magnitude, the lower one on ties.
-// (In FP32 for FP16 sources: the scaled value has 11 significant bits, so every
-// difference below is exact and a tie is a tie.)
-template <typename A>
-__device__ __forceinline__ int nearest_e2m1(A a) {
-  const A mags[8] = {(A)0.0, (A)0.5, (A)1.0, (A)1.5, (A)2.0, (A)3.0, (A)4.0, (A)6.0};
+__device__ __forceinline__ int nearest_e2m1(double a) {
+  const double mags[8] = {0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0};
   int best = 0;
-  A dbest = a;
+  double dbest = a;
 #pragma unroll
   for (int i = 1; i < 8; ++i) {
-    const A d = __builtin_elementwise_abs(mags[i] - a);
+    const double d = __builtin_elementwise_abs(mags[i] - a);
     if (d < dbest) {
       best = i;
       dbest = d;
@@ -501,9 +506,24 @@ __device__ __forceinline__ int nearest_e2m1(A a) {
   return best;
 }
 
+// The packed word of eight scaled FP16 values, at most 6 in magnitude.  The hardware conversion
+// rounds to nearest even; values made 2^-14 (relative) smaller leave a tie towards zero, and
+// pass no other: with 11 significant bits a value is on a tie or 2^-11 (relative) past it.
+__device__ __forceinline__ uint32_t pack_e2m1(const float* u) {
+  constexpr float SHRINK = 1.0f - 0x1p-14f;
+  uint32_t w = 0;
+  w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, u[0] * SHRINK, u[1] * SHRINK, 1.0f, 0);
+  w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, u[2] * SHRINK, u[3] * SHRINK, 1.0f, 1);
+  w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, u[4] * SHRINK, u[5] * SHRINK, 1.0f, 2);
+  return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, u[6] * SHRINK, u[7] * SHRINK, 1.0f, 3);
+}
+
 // Four threads per 32-element block, eight elements each: one packed word of
 // E2M1 codes, or (F8: the MXFP8 activation format, no host counterpart in the
-// reference; same block rule with 448 in place of 6) eight E4M3 bytes.
+// reference; same block rule with 448 in place of 6) eight E4M3 bytes.  FP16 sources
+// were bound by vector instructions (seven compares and selects a code, the exponent in FP64):
+// 2048 x 4096 took 12.7 us a call into MXFP4 and 12.0 into MXFP8, and takes 6.4 and 7.0 with the
+// hardware conversions and the exponent from integer arithmetic (the two launches alone: 5.7).
 template <typename T, bool FULL, bool F8>
 __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ src,
                                                          long long rows, int K, int B,
@@ -528,8 +548,6 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
   // everything the encoders do with an 11-bit significand
   typedef typename Quot<T>::type A;
   A v[8];
-  A amax = (A)0;
-  bool bad = false;
   if constexpr (FULL) {  // K a multiple of 8 and 16-byte aligned rows: four 16-byte loads
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = (A)0;
@@ -538,22 +556,39 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = j < n ? (A)base[j] : (A)0;
   }
+  int e;
+  if constexpr (sizeof(T) == 2) {
+    // the largest magnitude as an integer, which NaN and infinity end up on top of
+    uint32_t top = 0;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const A av = v[j] < (A)0 ? -v[j] : v[j];
-    bad |= !(av <= (A)(sizeof(T) == 2 ? 65504.0 : DBL_MAX));
-    amax = av > amax ? av : amax;
-  }
-  if (bad) atomicOr(status, 1);
-  {
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t mag = __builtin_bit_cast(uint32_t, v[j]) & 0x7FFFFFFFu;
+      top = mag > top ? mag : top;
+    }
+    if (top >= 0x7F800000u) atomicOr(status, 1);
+    const uint32_t o1 = lane_xor(top, 1);
+    top = o1 > top ? o1 : top;
+    const uint32_t o2 = lane_xor(top, 2);
+    top = o2 > top ? o2 : top;
+    e = mx_exponent_f16<F8 ? 448 : 6>(__builtin_bit_cast(float, top));
+  } else {
+    A amax = (A)0;
+    bool bad = false;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const A av = v[j] < (A)0 ? -v[j] : v[j];
+      bad |= !(av <= (A)DBL_MAX);
+      amax = av > amax ? av : amax;
+    }
+    if (bad) atomicOr(status, 1);
     const A o1 = __shfl_xor(amax, 1);
     amax = o1 > amax ? o1 : amax;
     const A o2 = __shfl_xor(amax, 2);
     amax = o2 > amax ? o2 : amax;
+    bool range = false;
+    e = mx_exponent<F8 ? 448 : 6>((double)amax, &range);
+    if (range && j4 == 0) atomicOr(status, 2);
   }
-  bool range = false;
-  const int e = mx_exponent<F8 ? 448 : 6>((double)amax, &range);
-  if (range && j4 == 0) atomicOr(status, 2);
   if (n == 0) return;
   A u[8];  // v / 2^e
   if constexpr (sizeof(T) == 2) {
@@ -581,13 +616,17 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
     }
   } else {
     uint32_t word = 0;
+    if constexpr (sizeof(T) == 2) {
+      word = pack_e2m1(u);  // (elements past the row are +0: code 0)
+    } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (j < n) {
-        const uint32_t code = (__builtin_signbit(u[j]) ? 8u : 0u) |
-                              (uint32_t)nearest_e2m1<A>(u[j] < (A)0 ? -u[j] : u[j]);
-        word |= code << (4 * j);
-      }
+      for (int j = 0; j < 8; ++j)
+        if (j < n) {
+          const uint32_t code = (__builtin_signbit(u[j]) ? 8u : 0u) |
+                                (uint32_t)nearest_e2m1(u[j] < (A)0 ? -u[j] : u[j]);
+          word |= code << (4 * j);
+        }
+    }
     q[row * (long long)words(K) + b * 4 + j4] = word;
   }
   if (j4 == 0) scales[blk] = (uint8_t)(e + 127);
