@@ -332,3 +332,29 @@ def test_unhooked_kernels_with_one_signed_and_offset_activations(shape):
             ch, _ = _run(c.gemm, dp.view, x_d, M, N, K)
             cu, _ = _run(c.gemm, dp.view, x_d, M, N, K, hook=False)
             cross_gate(ch, cu, ref, name)
+
+
+@pytest.mark.parametrize("fmt", ["w4", "w4z", "mx"])
+@pytest.mark.parametrize("K", [14336, 10368, 8192, 5120, 3072])
+def test_long_k_rows_that_do_not_fill_the_last_tile(K, fmt):
+    """Long K, 33 to 64 activation rows: three row tiles, and four with half of the last one's rows
+    fetched.  A row's bytes do not depend on how many others there are; nothing is stored past
+    the last one."""
+    c = w4amd.capi()
+    N = 48
+    w = orc.normal_weights(N * K, 0x10E0 + K)
+    p = orc.quantize_mx(w, N, K) if fmt == "mx" else orc.quantize(w, N, K, 64, fmt == "w4")
+    dp, call = (DevPackedMx(p), c.gemm_mma_mx) if fmt == "mx" else (DevPacked(p), c.gemm_mma)
+    w_ref = orc.dequant_all_mx(p) if fmt == "mx" else orc.dequant_all(p)
+    x = orc.normal_activations(64 * K, 0x10E1 + K)
+    x_d = to_dev(x)
+    full = halves(64 * N, 0x7E00)
+    call(dp.view, ptr(x_d), ptr(full), 64)
+    full = bits(full).reshape(64, N)
+    assert orc.rel_l2(full.view(np.float16), orc.gemm_oracle(x, 64, K, w_ref, N).reshape(64, N)) <= TOL
+    for M in (33, 40, 47, 48, 49, 52, 55, 56, 57):
+        out = halves(65 * N, 0x7E00)
+        call(dp.view, ptr(to_dev(x[:M * K])), ptr(out), M)
+        got = bits(out).reshape(65, N)
+        assert np.array_equal(got[:M], full[:M]), M
+        assert (got[M:] == 0x7E00).all(), M

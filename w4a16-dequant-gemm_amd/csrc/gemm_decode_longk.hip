@@ -58,6 +58,9 @@ constexpr int LK_MAX_M = 64;
 constexpr int lk_nbuf(int MT, int NQ) {
   return MT > 1 ? 4 : 8 / NQ < 2 ? 2 : 8 / NQ < 4 ? 8 / NQ : 4;
 }
+// Quads of rows fetched of row tile mt: all of a tile that another follows, NQ of the last.
+constexpr int lk_quads(int MT, int NQ, int mt) { return mt < MT - 1 ? 4 : NQ; }
+constexpr int lk_slot(int MT, int NQ) { return MT > 1 ? 4 : NQ; }  // KB of a ring slot
 constexpr int lk_lau(int MT, int NQ) { return lk_nbuf(MT, NQ) / MT / 2 > 2 ? lk_nbuf(MT, NQ) / MT / 2 : 2; }
 constexpr int lk_waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
 extern __shared__ __attribute__((aligned(16))) uint8_t lk_lds[];
@@ -96,7 +99,7 @@ constexpr LkSched<CH * MT> lk_schedule() {
     if (2 * u + 1 < CH) clast[2 * u + 1] = seq - 1;
   };
   for (int u = 0; u < NBUF && u < UN; ++u) {
-    seq += NQ, xlast[u] = seq - 1;
+    seq += lk_quads(MT, NQ, u % MT), xlast[u] = seq - 1;
     if ((u + 1) % (2 * MT) == 0 && cu < LAU) codes(cu++);
   }
   while (cu < LAU) codes(cu++);
@@ -108,7 +111,7 @@ constexpr LkSched<CH * MT> lk_schedule() {
     if (need > done) done = need;
     s.allowed[u] = seq - 1 - done;
     if (seq - 1 - done > s.peak) s.peak = seq - 1 - done;
-    if (u + NBUF < UN) seq += NQ, xlast[u + NBUF] = seq - 1;
+    if (u + NBUF < UN) seq += lk_quads(MT, NQ, (u + NBUF) % MT), xlast[u + NBUF] = seq - 1;
     if (u % MT == MT - 1 && (u / MT) % 2 == 0) codes(u / MT / 2 + LAU);
   }
   return s;
@@ -119,10 +122,14 @@ constexpr LkSched<CH * MT> lk_schedule() {
 // are fetched from a clamped address and meet zero activations).  gs_shift: log2(gs) if
 // gs is a power of two, else -1.  MT tiles of 16 activation rows (grid.y walks M in
 // steps of 16 MT).  G: groups (W4) or blocks (MXFP4) per row.
-// NQ: quads of activation rows fetched per row tile (with one row tile, M <= 4 NQ: the
-// quads past M would repeat row M - 1 and feed columns of the product that are never
-// stored; they are left out and those columns are computed from whatever the buffer
-// holds).  Arguments are scalars and pointers so that they arrive preloaded in SGPRs.
+// NQ: quads of activation rows fetched of the last row tile (the quads past M would repeat
+// row M - 1 and feed columns of the product that are never stored; they are left out and
+// those columns are computed from whatever the buffer holds).  Every workgroup fetches all
+// of x out of L2, so rows that do not exist cost time: with three row tiles for 33 to 48 rows
+// and half of the fourth for 49 to 56, N = 4096, K = 14336, MXFP4: M = 33 26.3 -> 22.8 us, 48 26.7 -> 24.8,
+// 50 26.9 -> 26.0; N = 5120, K = 13824: M = 33 45.6 -> 38.8; W4 the same to a few per cent.  Two further
+// forms of the last tile are not compiled: a step of four rows is worth 2 %.
+// Arguments are scalars and pointers so that they arrive preloaded in SGPRs.
 template <int FMT, int CH, int MT, int NQ>
 __global__ __launch_bounds__(LK_THREADS) void mfma_decode_longk_kernel(
     const uint32_t* __restrict__ q, const void* __restrict__ scales,
@@ -133,8 +140,7 @@ __global__ __launch_bounds__(LK_THREADS) void mfma_decode_longk_kernel(
   constexpr LkSched<UN> SCH = lk_schedule<CH, MT, NQ, NSC>();
   static_assert(SCH.peak < 64, "vmcnt is a 6-bit counter");
   static_assert(SCH.allowed[UN - 1] == 0, "the last unit waits for every request");
-  static_assert(MT == 1 || NQ == 4, "several row tiles: whole tiles of 16 rows");
-  constexpr int XBYTES = NBUF * NQ * 1024;  // the wave's ring: NBUF units of NQ KB
+  constexpr int SLOT = lk_slot(MT, NQ), XBYTES = NBUF * SLOT * 1024;  // the wave's ring: NBUF slots
   const int WPR = K >> 3, nchunks = K >> 7;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -154,11 +160,11 @@ __global__ __launch_bounds__(LK_THREADS) void mfma_decode_longk_kernel(
   auto request_x = [&](int u) {
     const int cidx = chunk_of(u / MT), mt = u % MT;
 #pragma unroll
-    for (int rq = 0; rq < NQ; ++rq) {
+    for (int rq = 0; rq < lk_quads(MT, NQ, mt); ++rq) {
       const int r16 = 4 * rq + (lane >> 4), row = m0 + 16 * mt + r16;
       const uint32_t off = (uint32_t)min(row, M - 1) * (uint32_t)(K * 2) + (uint32_t)cidx * 256u +
                            (uint32_t)(((lane & 15) ^ r16) * 16);
-      const uint32_t dst = region + (uint32_t)((u % NBUF) * NQ + rq) * 1024u;
+      const uint32_t dst = region + (uint32_t)((u % NBUF) * SLOT + rq) * 1024u;
       asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
                    :
                    : "v"(off), "s"(xb), "s"(dst)
@@ -265,7 +271,7 @@ __global__ __launch_bounds__(LK_THREADS) void mfma_decode_longk_kernel(
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       // (lanes of rows past the fetched quads read the last fetched one)
-      xv[mt][j] = *(const u4*)(mine + ((u % NBUF) * NQ + min(r >> 2, NQ - 1)) * 1024 +
+      xv[mt][j] = *(const u4*)(mine + ((u % NBUF) * SLOT + min(r >> 2, lk_quads(MT, NQ, mt) - 1)) * 1024 +
                                ((r & 3) * 16 + ((4 * b + j) ^ r)) * 16);
     }
     if (wave * CH + i >= nchunks) {  // a chunk past the end of the row: zero activations
@@ -357,7 +363,7 @@ int lk_cus() {
 
 template <int FMT, int CH, int MT, int NQ>
 hipError_t longk_go(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s) {
-  constexpr int lds_bytes = LK_WAVES * lk_nbuf(MT, NQ) * NQ * 1024;
+  constexpr int lds_bytes = LK_WAVES * lk_nbuf(MT, NQ) * lk_slot(MT, NQ) * 1024;
   static std::atomic<bool> granted[64] = {};  // more than 64 KB of LDS has to be granted per device, once
   int dev = 0;
   if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
@@ -382,7 +388,9 @@ hipError_t longk_m(const WView& v, const w4_half* x, w4_half* c, int M, hipStrea
   if (M <= 12) return longk_go<FMT, CH, 1, 3>(v, x, c, M, s);
   if (M <= 16) return longk_go<FMT, CH, 1, 4>(v, x, c, M, s);
   if (M <= 32) return longk_go<FMT, CH, 2, 4>(v, x, c, M, s);
-  return longk_go<FMT, CH, 4, 4>(v, x, c, M, s);  // grid.y walks 64 rows at a time
+  if (M <= 48) return longk_go<FMT, CH, 3, 4>(v, x, c, M, s);
+  if (M <= 56) return longk_go<FMT, CH, 4, 2>(v, x, c, M, s);
+  return longk_go<FMT, CH, 4, 4>(v, x, c, M, s);  // (M <= 64)
 }
 
 template <int FMT>
