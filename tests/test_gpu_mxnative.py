@@ -383,3 +383,54 @@ def test_activation_quantizers_every_half(fmt):
             q = q8.cpu().numpy()
         assert np.array_equal(s.cpu().numpy(), ref.scales)
         assert np.array_equal(q, ref.q)
+
+
+@pytest.mark.parametrize("K", [96, 100])
+@pytest.mark.parametrize("fmt", ["mx4", "mx8"])
+def test_activation_quantizers_nan_and_infinity(fmt, K):
+    """A NaN activation is no maximum: its block's exponent and other codes are those with a zero in its
+    place.  MXFP8 holds it (0x7F, which the scaled matrix cores read as NaN), E2M1 cannot (0).  A block with
+    an infinity is out of range (bit 1 of the status): exponent 127, as from FP64 sources."""
+    c = w4amd.capi()
+    M, B = 12, (K + 31) // 32
+    rng = np.random.default_rng(K)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    hole = np.zeros(x.shape, bool)
+    for r in range(M - 1):
+        hole[r, [0, 7, 8, 31, 33, 64, 95, K - 1][r % 8]] = True
+    hole[M - 1, :32] = True  # a block of nothing else
+    clean = np.where(hole, np.float16(0), x)
+    ref = (orc.quantize_mx if fmt == "mx4" else orc.quantize_mx8)(clean.astype(np.float64).ravel(), M, K)
+
+    def run(values):
+        st = torch.full((1,), -1, dtype=torch.int32, device=DEV)
+        xd, s = to_dev(np.ascontiguousarray(values).ravel()), torch.full((M * B,), 0x5A, dtype=torch.uint8, device=DEV)
+        if fmt == "mx4":
+            q = torch.full((M * orc.words(K),), 0x5A5A5A5A, dtype=torch.int32, device=DEV)
+            c.quantize_mx_f16(c.packed_mx_view(M, K, B, ptr(q), ptr(s)), ptr(xd), ptr(st))
+            w = q.cpu().numpy().view(np.uint32).reshape(M, -1, 1)
+            codes = (w >> (4 * np.arange(8, dtype=np.uint32)) & 15).reshape(M, -1)[:, :K]
+        else:
+            q = torch.full((M * K,), 0x5A, dtype=torch.uint8, device=DEV)
+            c.quantize_mx8_f16(c.act_mx8_view(M, K, B, ptr(q), ptr(s)), ptr(xd), ptr(st))
+            codes = q.cpu().numpy().reshape(M, K)
+        return codes, s.cpu().numpy().reshape(M, B), int(st.item())
+
+    base, base_s, st = run(clean)
+    assert st == 0 and np.array_equal(base_s.ravel(), ref.scales)
+    got, s, st = run(np.where(hole, np.float16(np.nan), x))
+    assert st == 1
+    assert np.array_equal(s, base_s)
+    assert np.array_equal(got[~hole], base[~hole])
+    assert ((got[hole] & (7 if fmt == "mx4" else 0x7F)) == (0 if fmt == "mx4" else 0x7F)).all()
+    inf = clean.copy()
+    inf[3, 40], inf[5, K - 1] = np.inf, -np.inf
+    got, s, st = run(inf)
+    assert st == 3
+    hit = np.zeros((M, B), bool)
+    hit[3, 1], hit[5, (K - 1) // 32] = True, True
+    assert (s[hit] == 254).all() and np.array_equal(s[~hit], base_s[~hit])
+    cols = np.repeat(hit, 32, axis=1)[:, :K]
+    assert np.array_equal(got[~cols], base[~cols])
+    if fmt == "mx8":
+        assert (got[3, 40] & 0x7F) == 0x7E and (got[5, K - 1] & 0x7F) == 0x7E

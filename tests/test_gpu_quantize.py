@@ -447,3 +447,79 @@ def test_zero_point_words_of_short_rows(D, gs, f16):
     for name, t in (dev | s).items():
         want = getattr(ref, name)
         assert np.array_equal(_host(t).view(want.dtype), want), name
+
+
+# ---- non-finite FP16 sources ---------------------------------------------------
+# The status word says so, and outputs are unspecified then; a caller that does not wait for the
+# status still has to meet the NaN where the format can hold one, and nothing else may change.
+NAN_AT = (0, 3, 17, 31, 64, 65, 127)
+
+
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("fmt", ["f8", "w4", "w4z"])
+def test_quantize_cache_nan_keeps_its_byte_and_its_neighbours(fmt, gs):
+    """A NaN is coded 0x7F (E4M3) and is no extremum: the scales, zero-points and codes of all other
+    elements are those of the row with a zero in its place, which no extremum notices either."""
+    c = w4amd.capi()
+    H, S, D = 2, 9, 128
+    rng = np.random.default_rng(gs)
+    k = rng.standard_normal((H * S, D)).astype(np.float16)
+    hole = np.zeros(k.shape, bool)
+    for r in range(H * S - 1):
+        hole[r, NAN_AT[r % len(NAN_AT)]] = True
+        hole[r, rng.integers(D, size=r % 3)] = True
+    hole[-1] = True  # a row of nothing else
+    clean, dirty = np.where(hole, np.float16(0), k), np.where(hole, np.float16(np.nan), k)
+    rows, G, st = H * S, D // gs, _status()
+    src = to_dev(dirty.ravel())
+    sk, sv = (torch.full((rows * G,), 0x7E00, dtype=torch.int16, device=DEV) for _ in range(2))
+    flat = clean.ravel().astype(np.float64)
+    if fmt == "f8":
+        ref = orc.quantize_cache_f8(flat, flat, H, S, D, gs)
+        qk, qv = (torch.full((rows * D,), 0x5A, dtype=torch.uint8, device=DEV) for _ in range(2))
+        c.quantize_cache_f8(c.kv_f8_view(H, S, D, gs, G, ptr(qk), ptr(sk), ptr(qv), ptr(sv)), ptr(src), ptr(src),
+                            ptr(st), src_f16=True)
+        got, want = _host(qk).reshape(rows, D), ref.q_k.reshape(rows, D)
+        assert ((got & 0x7F)[hole] == 0x7F).all()
+        assert np.array_equal(_host(qk), _host(qv))
+    else:
+        ref = orc.quantize_cache(flat, flat, H, S, D, gs, fmt == "w4")
+        qk, qv = (torch.full((rows * D // 8,), 0x5A5A5A5A, dtype=torch.int32, device=DEV) for _ in range(2))
+        zk, zv = (None if fmt == "w4" else torch.full((rows,), 0x5A5A5A5A, dtype=torch.int32, device=DEV) for _ in range(2))
+        c.quantize_cache(c.kv_view(H, S, D, gs, G, fmt == "w4", ptr(qk), ptr(sk), ptr(zk), ptr(qv), ptr(sv), ptr(zv)),
+                         ptr(src), ptr(src), ptr(st), src_f16=True)
+        nibbles = lambda q: (q.view(np.uint32).reshape(rows, -1, 1) >> (4 * np.arange(8, dtype=np.uint32)) & 15).reshape(rows, D)
+        got, want = nibbles(_host(qk)), nibbles(ref.q_k)
+        if fmt == "w4z":
+            assert np.array_equal(_host(zk).view(np.uint32)[:-1], ref.z_k[:-1])
+    assert int(_host(st)[0]) == 1
+    keep = ~hole
+    assert np.array_equal(_host(sk).view(np.uint16)[:-G], ref.s_k[:-G])
+    assert np.array_equal(got[keep], want[keep])
+
+
+def test_quantize_cache_f8_infinity_f16_source():
+    """A group with an infinity has an infinite scale: 0 for its finite elements, NaN for the infinity
+    (infinity over infinity), and every one of them is a NaN again when it is expanded."""
+    c = w4amd.capi()
+    H, S, D, gs = 1, 4, 64, 32
+    k = np.random.default_rng(3).standard_normal((S, D)).astype(np.float16)
+    k[1, 5], k[2, 40] = np.inf, -np.inf
+    q = [torch.full((S * D,), 0x5A, dtype=torch.uint8, device=DEV) for _ in range(2)]
+    s = [torch.full((S * 2,), 0x7E00, dtype=torch.int16, device=DEV) for _ in range(2)]
+    st, src = _status(), to_dev(k.ravel())
+    c.quantize_cache_f8(c.kv_f8_view(H, S, D, gs, 2, ptr(q[0]), ptr(s[0]), ptr(q[1]), ptr(s[1])), ptr(src), ptr(src),
+                        ptr(st), src_f16=True)
+    assert int(_host(st)[0]) == 3
+    got, scales = _host(q[0]).reshape(S, D) & 0x7F, _host(s[0]).view(np.uint16).reshape(S, 2)
+    clean = np.where(np.isinf(k), 0, k).astype(np.float64).ravel()
+    fine = orc.quantize_cache_f8(clean, clean, H, S, D, gs)
+    for r in range(S):
+        for g in range(2):
+            cols = slice(32 * g, 32 * g + 32)
+            if np.isinf(k[r, cols]).any():
+                assert scales[r, g] == 0x7C00
+                assert np.array_equal(got[r, cols], np.where(np.isinf(k[r, cols]), 0x7F, 0))
+            else:
+                assert scales[r, g] == fine.s_k.reshape(S, 2)[r, g]
+                assert np.array_equal(got[r, cols], fine.q_k.reshape(S, D)[r, cols] & 0x7F)

@@ -78,11 +78,12 @@ __device__ __forceinline__ uint32_t encode_e4m3(float x) {
 }
 
 // Four E4M3 bytes of FP32 values (the hardware conversion rounds to nearest even, subnormals
-// included; past 448 it would give NaN, so the magnitude is capped first).  `from` gives the signs.
+// included; past 448 it would give NaN, so the magnitude is capped first, by a minimum that hands a
+// NaN on: its byte is 0x7F, as from encode_e4m3).  `from` gives the signs.
 __device__ __forceinline__ uint32_t pack_e4m3(const float* mag, const float* from) {
   float x[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) x[i] = copysignf(fminf(mag[i], 448.0f), from[i]);
+  for (int i = 0; i < 4; ++i) x[i] = copysignf(__builtin_elementwise_minimum(mag[i], 448.0f), from[i]);
   const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(x[0], x[1], 0, false);
   return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(x[2], x[3], lo, true);
 }
@@ -305,9 +306,9 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
   const bool live = w < nwords;
   A v[8];
   A lo, hi;  // of the group; without zero-points of FP16 sources both are its largest magnitude
-  bool bad = false;
   if constexpr (sizeof(T) == 2) {
-    // extrema on pairs of halves; magnitudes as integers, which NaN and infinity end up on top of
+    // extrema on pairs of halves (whose minimum and maximum ignore a NaN); magnitudes as integers,
+    // which NaN and infinity end up on top of
     u4 x = u4{0, 0, 0, 0};
     if (live) x = *(const u4*)(src + w * 8);
     us2 mag = __builtin_bit_cast(us2, x[0] & 0x7FFF7FFFu);
@@ -315,7 +316,16 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
     for (int i = 1; i < 4; ++i)
       mag = __builtin_elementwise_max(mag, __builtin_bit_cast(us2, x[i] & 0x7FFF7FFFu));
     uint32_t top = mag[0] > mag[1] ? mag[0] : mag[1];
-    bad = top >= 0x7C00u;
+    // (a branch of the whole wave: as one of single lanes it cost 2 % of the kernel)
+    if (__builtin_amdgcn_ballot_w64(top >= 0x7C00u) != 0) {
+      if (top >= 0x7C00u) atomicOr(status, 1);
+      top = 0;  // a NaN is no extremum: the scale is that of the group's other elements
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t m = (x[i >> 1] >> (16 * (i & 1))) & 0x7FFFu;
+        top = m > top && m <= 0x7C00u ? m : top;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = (A)__builtin_bit_cast(_Float16, (uint16_t)(x[j >> 1] >> (16 * (j & 1))));
     if constexpr (MODE == QM_ASYM) {
@@ -342,19 +352,20 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
     for (int j = 0; j < 8; ++j) v[j] = (A)0;
     if (live) load8(src + w * 8, v);
     lo = hi = v[0];
+    bool bad = false;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       bad |= !(fabs((double)v[j]) <= DBL_MAX);
       lo = v[j] < lo ? v[j] : lo;
       hi = v[j] > hi ? v[j] : hi;
     }
+    if (bad) atomicOr(status, 1);
     for (int m = 1; m < wpg; m <<= 1) {
       const A olo = __shfl_xor(lo, m), ohi = __shfl_xor(hi, m);
       lo = olo < lo ? olo : lo;
       hi = ohi > hi ? ohi : hi;
     }
   }
-  if (bad) atomicOr(status, 1);
   // Scale of the group, in every lane.  The step goes FP64 -> FP32 -> FP16 on the
   // host.  For FP16 sources without zero-points the FP32 step is amax / 7 (/ 448)
   // of an 11-bit amax: its binary expansion is periodic with period 3, so it is
@@ -438,6 +449,10 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
       float mag[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) mag[j] = quotient_magnitude(v[j], sf, rsf);
+      if (!(sf <= 65504.0f)) {  // a group with an infinity: 0 for its other elements
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mag[j] = fabsf(v[j]) < INFINITY ? 0.0f : (float)NAN;
+      }
       out[0] = pack_e4m3(mag, v);
       out[1] = pack_e4m3(mag + 4, v + 4);
     } else {
@@ -482,7 +497,7 @@ __device__ __forceinline__ int mx_exponent(double amax, bool* out_of_range) {
   return e;
 }
 
-// The same from the FP32 value of a nonzero FP16 maximum: TOP is 1.5 * 2^2 or 1.75 * 2^8, so e is
+// The same from the FP32 value of a finite FP16 maximum: TOP is 1.5 * 2^2 or 1.75 * 2^8, so e is
 // p - 2 (p - 8), and one more where the significand is past TOP's.  (e is -32 .. 14: in range.)
 template <int TOP>
 __device__ __forceinline__ int mx_exponent_f16(float amax) {
@@ -557,6 +572,7 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
     for (int j = 0; j < 8; ++j) v[j] = j < n ? (A)base[j] : (A)0;
   }
   int e;
+  bool bad = false;
   if constexpr (sizeof(T) == 2) {
     // the largest magnitude as an integer, which NaN and infinity end up on top of
     uint32_t top = 0;
@@ -565,15 +581,27 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
       const uint32_t mag = __builtin_bit_cast(uint32_t, v[j]) & 0x7FFFFFFFu;
       top = mag > top ? mag : top;
     }
-    if (top >= 0x7F800000u) atomicOr(status, 1);
+    bad = top >= 0x7F800000u;
+    if (bad) {  // a NaN is no maximum: the exponent is that of the block's other elements
+      atomicOr(status, 1);
+      top = 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t mag = __builtin_bit_cast(uint32_t, v[j]) & 0x7FFFFFFFu;
+        top = mag > top && mag <= 0x7F800000u ? mag : top;
+      }
+    }
     const uint32_t o1 = lane_xor(top, 1);
     top = o1 > top ? o1 : top;
     const uint32_t o2 = lane_xor(top, 2);
     top = o2 > top ? o2 : top;
     e = mx_exponent_f16<F8 ? 448 : 6>(__builtin_bit_cast(float, top));
+    if (top == 0x7F800000u) {
+      e = 127;
+      if (j4 == 0) atomicOr(status, 2);
+    }
   } else {
     A amax = (A)0;
-    bool bad = false;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const A av = v[j] < (A)0 ? -v[j] : v[j];
@@ -617,6 +645,10 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
   } else {
     uint32_t word = 0;
     if constexpr (sizeof(T) == 2) {
+      if (bad) {  // E2M1 has no code for them: zeros, as from FP64 sources
+#pragma unroll
+        for (int j = 0; j < 8; ++j) u[j] = fabsf(u[j]) < INFINITY ? u[j] : copysignf(0.0f, u[j]);
+      }
       word = pack_e2m1(u);  // (elements past the row are +0: code 0)
     } else {
 #pragma unroll
