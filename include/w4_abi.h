@@ -175,14 +175,24 @@ int w4_attention_w4_flash_paged_batched(const w4_kv_view* p, const int* bt,
                                         const w4_half* q, w4_half* out,
                                         w4_stream stream);
 
+/* How a flash-decode call without hooks would run (plain arithmetic, no GPU needed; no counterpart
+ * in the reference): kind 0 FP16, 1 W4, 2 FP8 with a scale per row; H slabs in all; gs ignored for FP16;
+ * page 0 for a contiguous cache; cache and scale arrays aligned to 16 bytes.
+ * plan[0]: splits per slab -- with 1 the call uses no memory but its arguments', so it may overlap with
+ *          others on other streams (every cache of up to 512 positions with D = 64 or 128 and, when
+ *          quantized, gs a multiple of D / 4);
+ * plan[1]: positions per split;  plan[2]: 1 if there is no second launch that merges them;
+ * plan[3]: 0 vector kernel, 1 matrix cores with tiles through registers, 2 through LDS. */
+int w4_flash_plan_for(int kind, int H, int group, int S, int D, int gs, int page, int* plan);
+
 /* No counterpart in the reference: w4_attention_w4_flash_gqa for callers that
  * cannot allocate device memory (HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same arguments, kernels and output bytes;
  * the split-S partials live in a W4_NOALLOC_SCRATCH_BYTES array built into the
  * library (one copy per GPU, held until the process ends) instead of the
  * library's grow-only buffer, and the call makes no hipMalloc / hipFree.  Calls
- * whose partials (slabs * group * splits * (D + 2) floats, splits chosen so that
- * about 512 workgroups run) do not fit are rejected with W4_EINVAL.  Every call
+ * whose partials (slabs * group * splits * (D + 2) floats, splits as
+ * w4_flash_plan_for gives them) do not fit are rejected with W4_EINVAL.  Every call
  * on one GPU shares that GPU's array: calls that overlap on one GPU race. */
 #define W4_NOALLOC_SCRATCH_BYTES (4u << 20)
 int w4_attention_w4_flash_gqa_noalloc(const w4_kv_view* p, int group,

@@ -56,6 +56,23 @@ def test_validation_runs_without_a_device():
     assert lib.w4_dispatch_mma_min_m_for_mx(4096, 4096) == lib.w4_dispatch_mma_min_m()
 
 
+def test_flash_plan_of_short_caches_shares_nothing():
+    """Caches of up to 512 positions on the matrix cores: one split per slab, so neither scratch nor
+    arrival counters are touched and calls on several streams may overlap."""
+    capi = w4amd.capi()
+    for kind in (0, 1, 2):
+        for D, gs in ((64, 32), (128, 32), (128, 128)):
+            for H in (1, 8, 64, 300, 5000):
+                for group in (1, 4, 16, 64):
+                    for S in (1, 127, 128, 300, 384, 511, 512):
+                        splits, length, direct, route = capi.flash_plan_for(kind, H, group, S, D, gs)
+                        assert (splits, direct) == (1, 1) and length >= S and route >= 1, (kind, H, group, S, D)
+    for bad in [(3, 8, 1, 100, 128, 32), (1, 8, 65, 100, 128, 32), (1, 8, 1, 100, 128, 12), (1, 0, 1, 100, 128, 32),
+                (0, 8, 1, 100, 128, 32, 16)]:
+        with pytest.raises(ValueError):
+            capi.flash_plan_for(*bad)
+
+
 def test_quantize_contracts():
     """Malformed calls are rejected before the device is touched (pack.hpp:64-72,
     mx.hpp:71-76, kvcache.hpp:60-68, kvfp8.hpp:70-79)."""

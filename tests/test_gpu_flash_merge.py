@@ -70,3 +70,29 @@ def test_entries_with_their_own_scratch_overlap():
     for i in range(2):
         for n in range(20):
             assert np.array_equal(bits(outs[i][n]), want[i]), (i, n)
+
+
+def test_short_caches_overlap_on_two_streams():
+    """One split per slab: no scratch, so calls of one entry may be in flight on several streams."""
+    import torch
+    c = w4amd.capi()
+    H, S, D, group = 16, 512, 128, 4
+    c4 = orc.quantize_cache(orc.normal_weights(H * S * D, 91), orc.normal_weights(H * S * D, 92), H, S, D, 32, True)
+    dk = DevKV(c4)
+    assert c.flash_plan_for(1, H, group, S, D, 32)[0] == 1
+    qs = [to_dev(orc.normal_activations(H * group * D, 93 + i)) for i in range(2)]
+    want = []
+    for q in qs:
+        out = halves(H * group * D, 0x7E00)
+        c.attention_w4_flash(dk.view, ptr(q), ptr(out), group=group)
+        want.append(bits(out).copy())
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = [[halves(H * group * D, 0x7E00) for _ in range(20)] for _ in range(2)]
+    torch.cuda.synchronize()
+    for n in range(20):
+        for i in range(2):
+            c.attention_w4_flash(dk.view, ptr(qs[i]), ptr(outs[i][n]), streams[i].cuda_stream, group=group)
+    torch.cuda.synchronize()
+    for i in range(2):
+        for n in range(20):
+            assert np.array_equal(bits(outs[i][n]), want[i]), (i, n)

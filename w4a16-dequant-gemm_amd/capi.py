@@ -58,6 +58,7 @@ SIGNATURES = {
     "w4_attention_fp16_flash": ([vp, vp, vp, vp, C.c_int, C.c_int, C.c_int, vp], C.c_int),
     "w4_attention_f8_flash": ([C.POINTER(KVF8View), vp, vp, vp, vp, vp], C.c_int),
     "w4_attention_w4_flash_paged": ([C.POINTER(KVView), vp, C.c_int, C.c_int, vp, vp, vp, vp, vp], C.c_int),
+    "w4_flash_plan_for": ([C.c_int] * 7 + [C.POINTER(C.c_int)], C.c_int),
     "w4_dequant_f8": ([vp, vp, vp, C.c_int, C.c_int, C.c_int, vp], C.c_int),
     "w4_attention_w4_flash_gqa": ([C.POINTER(KVView), C.c_int, vp, vp, vp, vp, vp], C.c_int),
     "w4_attention_w4_flash_gqa_noalloc": ([C.POINTER(KVView), C.c_int, vp, vp, vp, vp, vp], C.c_int),
@@ -189,6 +190,13 @@ def attention_w4_flash_paged_batched(view, bt, nseq, bt_stride, page, npages, gr
                                      stream=0):
     check(load().w4_attention_w4_flash_paged_batched(C.byref(view), _n(bt), nseq, bt_stride, page,
                                                      npages, group, _n(q), _n(out), _n(stream)))
+
+
+def flash_plan_for(kind, H, group, S, D, gs, page=0):
+    """(splits per slab, positions per split, merged without a second launch, 0 vector / 1 register / 2 LDS)"""
+    plan = (C.c_int * 4)()
+    check(load().w4_flash_plan_for(kind, H, group, S, D, gs, page, plan))
+    return tuple(plan)
 
 
 def dequant_f8(q, s, w, S, D, gs, stream=0):

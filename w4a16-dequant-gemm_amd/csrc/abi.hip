@@ -175,6 +175,7 @@ hipError_t noalloc_scratch(float** out) {
   return hipSuccess;
 }
 
+// (a split that is alone in its slab leaves no partials: such a call reads and writes no scratch)
 int run_flash(w4k::FlashArgs& a, w4_stream stream, const char* what) {
   float* part = nullptr;
   hipError_t e = scratch_floats(w4k::flash_scratch_floats(a), &part, &a.scratch_id);
@@ -452,6 +453,27 @@ int w4_attention_w4_flash_paged_batched(const w4_kv_view* p, const int* bt, int 
   a.bt = bt; a.bt_stride = bt_stride; a.page = page; a.pool_rows = npages * page;
   a.q = q; a.out = out;
   return run_flash(a, stream, "flash_w4_paged");
+}
+
+int w4_flash_plan_for(int kind, int H, int group, int S, int D, int gs, int page, int* plan) {
+  REQUIRE(kind >= 0 && kind <= 2 && plan, "flash plan: bad kind");
+  if (int rc = check_kv_common(H, S, D, gs, (D + gs - 1) / (gs > 0 ? gs : 1), "flash plan")) return rc;
+  REQUIRE(group >= 1 && group <= 64 && page >= 0 && (page == 0 || kind == 1), "flash plan: bad group or page");
+  w4k::FlashArgs a{};
+  static const int any_table = 0;
+  a.kind = kind;
+  a.H = H; a.S = S; a.D = D; a.gs = gs; a.G = kind == 0 ? 1 : (D + gs - 1) / gs;
+  a.symmetric = 1;
+  a.group = group;
+  a.Hkv = H;
+  if (page) a.bt = &any_table, a.page = page, a.pool_rows = (S + page - 1) / page * page;
+  const w4k::FlashPlan p = w4k::flash_plan(a);
+  const bool mfma = w4k::flash_mfma_applies(a);
+  plan[0] = p.nsplit;
+  plan[1] = p.split_len;
+  plan[2] = mfma && (p.nsplit == 1 || w4k::flash_merges_in_place(a, p));
+  plan[3] = !mfma ? 0 : w4k::flash_tiles_in_lds(a, p) ? 2 : 1;
+  return W4_OK;
 }
 
 int w4_dequant_f8(const uint8_t* q, const w4_half* s, w4_half* w, int S, int D, int gs,

@@ -50,7 +50,7 @@ constexpr int FM_TILE = 32;   // positions per wave tile
 constexpr int FM_WAVES = 4;
 constexpr int FM_DEPTH = 3;   // ring slots per wave: one tile computed, two in flight
 constexpr int FM_HEADS = 16;  // query heads per pass
-constexpr int FM_LDS_TILES = 12;  // W4: most tiles per wave that go through LDS (see go_kind)
+constexpr int FM_LDS_TILES = 12;  // W4: most tiles per wave that go through LDS (see flash_tiles_in_lds)
 constexpr int FM_RING = 2;    // LDS slots per wave (three measured slower: 12.7 -> 13.1 us, FP8 16.8 -> 21.7)
 typedef __attribute__((address_space(3))) void* fm_lds;
 typedef __attribute__((address_space(4))) const uint32_t* fm_const_u32;  // read with scalar loads
@@ -955,19 +955,10 @@ static hipError_t go_kind(const FlashArgs& a, int qh0, const FlashPlan& pl, floa
   if constexpr (KIND == KIND_F16) {
     return hook ? go_alt<KIND, true, 0, false>(a, qh0, pl, part, s) : go_alt<KIND, false, 0, false>(a, qh0, pl, part, s);
   } else {
-    // Tiles through LDS: 32-bit offsets inside a slab, scales that can be fetched as dwords, at
-    // most four groups per row.  The register path of the hooked kernels takes everything.
-    const long long slab_rows = a.bt ? a.pool_rows : a.S;
-    const bool lds_ok = slab_rows * a.D * 2 < (1ll << 31) && a.G <= 4 && (((uintptr_t)a.s_k | (uintptr_t)a.s_v) & 3) == 0;
+    const bool lds = flash_tiles_in_lds(a, pl);  // (the register path of the hooked kernels takes everything)
     if constexpr (KIND == KIND_F8) {
-      return hook || !lds_ok ? go_alt<KIND, true, 0, false>(a, qh0, pl, part, s)
-                             : go_alt<KIND, false, 0, true>(a, qh0, pl, part, s);
+      return lds ? go_alt<KIND, false, 0, true>(a, qh0, pl, part, s) : go_alt<KIND, true, 0, false>(a, qh0, pl, part, s);
     } else {
-      // W4 with more than FM_LDS_TILES tiles per wave stays in registers: once the stream runs, the
-      // read back from LDS in front of every tile costs more than the loads it saves (57.7
-      // against 60.9 us at 64 slabs x 32768 positions, 33.6 against 34.8 with 16 tiles per wave;
-      // 27.5 against 28.4 us with 12, 12.7 against 14.1 with 4).
-      const bool lds = lds_ok && pl.split_len <= FM_LDS_TILES * FM_WAVES * FM_TILE;
       if (a.bt && a.page % 16 != 0)
         return hook ? go_alt<KIND, true, 2, false>(a, qh0, pl, part, s) : go_alt<KIND, false, 2, false>(a, qh0, pl, part, s);
       if (a.bt)
@@ -985,6 +976,19 @@ bool flash_mfma_applies(const FlashArgs& a) {
   if (a.kind != KIND_F16 && a.gs % (a.D / 4)) return false;
   return ((((uintptr_t)a.k | (uintptr_t)a.v) & 15) == 0) &&
          ((((uintptr_t)a.k_out | (uintptr_t)a.v_out) & 15) == 0);
+}
+
+// Tiles through LDS: 32-bit offsets inside a slab, scales that can be fetched as dwords, at most
+// four groups per row, pages of whole half tiles.
+// W4 with more than FM_LDS_TILES tiles per wave stays in registers: once the stream runs, the
+// read back from LDS in front of every tile costs more than the loads it saves (57.7
+// against 60.9 us at 64 slabs x 32768 positions, 33.6 against 34.8 with 16 tiles per wave;
+// 27.5 against 28.4 us with 12, 12.7 against 14.1 with 4).
+bool flash_tiles_in_lds(const FlashArgs& a, const FlashPlan& pl) {
+  if (a.kind == KIND_F16 || a.k_out || a.v_out || (a.bt && a.page % 16)) return false;
+  const long long slab_rows = a.bt ? a.pool_rows : a.S;
+  if (slab_rows * a.D * 2 >= (1ll << 31) || a.G > 4 || (((uintptr_t)a.s_k | (uintptr_t)a.s_v) & 3)) return false;
+  return a.kind == KIND_F8 || pl.split_len <= FM_LDS_TILES * FM_WAVES * FM_TILE;
 }
 
 bool flash_merges_in_place(const FlashArgs& a, const FlashPlan& pl) {

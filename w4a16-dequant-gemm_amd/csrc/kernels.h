@@ -105,6 +105,7 @@ constexpr int FL_SCRATCH_IDS = 32;
 enum { KIND_F16 = 0, KIND_W4 = 1, KIND_F8 = 2 };  // FlashArgs::kind
 
 // Split of the sequence over workgroups (shared by both phase-1 kernels).
+constexpr int FL_DIRECT_MAX_S = 512;  // longest cache that always has one split per slab (matrix-core kernel)
 struct FlashPlan {
   int split_len, nsplit;
 };
@@ -113,6 +114,8 @@ FlashPlan flash_plan(const FlashArgs& a);
 bool flash_mfma_applies(const FlashArgs& a);
 // Whether its last workgroup of every slab merges the splits itself (no second launch).
 bool flash_merges_in_place(const FlashArgs& a, const FlashPlan& pl);
+// Whether its tiles go through LDS (else through registers).
+bool flash_tiles_in_lds(const FlashArgs& a, const FlashPlan& pl);
 // Launches it; false when the arguments need the general kernel (nothing is
 // launched then).
 bool try_flash_mfma(const FlashArgs& a, const FlashPlan& pl, float* part, hipStream_t s,
