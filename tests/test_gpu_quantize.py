@@ -523,3 +523,60 @@ def test_quantize_cache_f8_infinity_f16_source():
             else:
                 assert scales[r, g] == fine.s_k.reshape(S, 2)[r, g]
                 assert np.array_equal(got[r, cols], fine.q_k.reshape(S, D)[r, cols] & 0x7F)
+
+
+@pytest.mark.parametrize("what", ["tiny", "infinite"])
+@pytest.mark.parametrize("fmt", ["f8", "w4", "w4z"])
+def test_quantize_cache_f16_steps_that_are_no_number(fmt, what):
+    """Groups whose step rounds to 0 or is infinite: codes are those of the quotients v / step, an element over
+    a step of 0 being infinite (E4M3: 448, so that it expands to 0 and not to a NaN) and 0 / 0 and infinity over
+    infinity saturating (E4M3: a NaN).  Groups beside them are untouched."""
+    c = w4amd.capi()
+    H, S, D, gs = 2, 10, 128, 32
+    rows, G = H * S, D // gs
+    k = np.random.default_rng(7).standard_normal((rows, D)).astype(np.float16)
+    if what == "tiny":  # multiples of 2^-24 whose extremum over 7 (15, 448) is at most 2^-25
+        top = {"f8": 224, "w4": 3, "w4z": 3}[fmt]
+        odd = (np.arange(gs) * 37 % (2 * top + 1) - top).astype(np.float64) * 2.0 ** -24
+    else:
+        odd = np.linspace(-3, 3, gs)
+        odd[3], odd[11] = np.inf, -np.inf
+    hit = np.zeros((rows, G), bool)
+    hit[1, 2] = hit[7, 0] = hit[rows - 1, 3] = True
+    cols = np.repeat(hit, gs, axis=1)
+    clean = np.where(cols, 0, k.astype(np.float64))
+    k[cols] = np.tile(odd, 3).astype(np.float16)
+    flat, st, src = clean.ravel(), _status(), to_dev(k.ravel())
+    s = [torch.full((rows * G,), 0x5A5A, dtype=torch.int16, device=DEV) for _ in range(2)]
+    zero = 0
+    if fmt == "f8":
+        ref = orc.quantize_cache_f8(flat, flat, H, S, D, gs)
+        q = [torch.full((rows * D,), 0x5A, dtype=torch.uint8, device=DEV) for _ in range(2)]
+        c.quantize_cache_f8(c.kv_f8_view(H, S, D, gs, G, ptr(q[0]), ptr(s[0]), ptr(q[1]), ptr(s[1])), ptr(src),
+                            ptr(src), ptr(st), src_f16=True)
+        got, want = _host(q[0]).reshape(rows, D), ref.q_k.reshape(rows, D)
+        sign = np.where(np.signbit(odd), 0x80, 0)
+        codes = np.where(odd != 0, sign | 0x7E, 0x7F) if what == "tiny" else np.where(np.isinf(odd), 0x7F, sign)
+        free = 0x80 * ((codes & 0x7F) == 0x7F)  # the sign of a NaN
+    else:
+        ref = orc.quantize_cache(flat, flat, H, S, D, gs, fmt == "w4")
+        q = [torch.full((rows * D // 8,), 0x5A5A5A5A, dtype=torch.int32, device=DEV) for _ in range(2)]
+        z = [torch.full((rows,), 0x5A5A5A5A, dtype=torch.int32, device=DEV) for _ in range(2)]
+        zp = [0, 0] if fmt == "w4" else [ptr(t) for t in z]
+        c.quantize_cache(c.kv_view(H, S, D, gs, G, fmt == "w4", ptr(q[0]), ptr(s[0]), zp[0], ptr(q[1]), ptr(s[1]), zp[1]),
+                         ptr(src), ptr(src), ptr(st), src_f16=True)
+        nibbles = lambda a, n: (a.view(np.uint32).reshape(rows, -1, 1) >> (4 * np.arange(8, dtype=np.uint32)) & 15).reshape(rows, -1)[:, :n]
+        got, want = nibbles(_host(q[0]), D), nibbles(ref.q_k, D)
+        zero = 8 if fmt == "w4" else 15 if what == "tiny" else 0
+        if fmt == "w4z":
+            zeros = nibbles(_host(z[0]), G)
+            assert np.array_equal(zeros[~hit], nibbles(ref.z_k, G)[~hit]) and (zeros[hit] == zero).all()
+        codes = np.where(odd < 0, 0, 15) if what == "tiny" else np.where(np.isinf(odd), np.where(odd < 0, 0, 15), zero)
+        free = np.zeros(gs, int)
+    assert int(_host(st)[0]) == (2 if what == "tiny" else 3)
+    scales = _host(s[0]).view(np.uint16).reshape(rows, G)
+    assert (scales[hit] == (0 if what == "tiny" else 0x7C00)).all()
+    assert np.array_equal(scales[~hit], ref.s_k.reshape(rows, G)[~hit])
+    assert np.array_equal(got[~cols], want[~cols])
+    assert np.array_equal(got[cols].reshape(3, gs) | free, np.tile(codes | free, (3, 1)))
+    assert np.array_equal(_host(q[0]), _host(q[1]))

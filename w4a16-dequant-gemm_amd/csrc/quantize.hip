@@ -77,13 +77,13 @@ __device__ __forceinline__ uint32_t encode_e4m3(float x) {
   return sign | (uint32_t)(code > 0x7E ? 0x7E : code);
 }
 
-// Four E4M3 bytes of FP32 values (the hardware conversion rounds to nearest even, subnormals
-// included; past 448 it would give NaN, so the magnitude is capped first, by a minimum that hands a
-// NaN on: its byte is 0x7F, as from encode_e4m3).  `from` gives the signs.
+// Four E4M3 bytes of FP32 values that are not NaN (the hardware conversion rounds to nearest even,
+// subnormals included; past 448 it would give NaN, so the magnitude is capped first).  `from`
+// gives the signs.
 __device__ __forceinline__ uint32_t pack_e4m3(const float* mag, const float* from) {
   float x[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) x[i] = copysignf(__builtin_elementwise_minimum(mag[i], 448.0f), from[i]);
+  for (int i = 0; i < 4; ++i) x[i] = copysignf(fminf(mag[i], 448.0f), from[i]);
   const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(x[0], x[1], 0, false);
   return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(x[2], x[3], lo, true);
 }
@@ -256,6 +256,18 @@ __device__ __forceinline__ uint32_t quotient_code(float v, float grown, float ze
   return (uint32_t)__builtin_amdgcn_fmed3f(fmaf(v, grown, zero_half), 0.0f, 15.5f);
 }
 
+// Codes where the above does not hold: elements or steps that are not finite, a step of 0 (the group's
+// extremum is below half of the smallest FP16 value times 7, 15 or 448).  rsf = 1 / sf.  A quotient
+// of 64 or more or a NaN saturates, upwards unless v < 0.
+__device__ __forceinline__ uint32_t quotient_code_any(float v, float sf, float rsf, int zero) {
+  const float a = fabsf(v), t = fminf(a * rsf, 64.0f), c = rintf(t);
+  int m = (int)c;  // round half up by the sign of |v| - (c -+ 1/2) sf
+  if (fmaf(0.5f - c, sf, a) < 0.0f) --m;
+  if (fmaf(-0.5f - c, sf, a) >= 0.0f) ++m;
+  m = zero + (v < 0.0f ? -m : m);
+  return (uint32_t)(m < 0 ? 0 : m > 15 ? 15 : m);
+}
+
 // The value of lane ^ m, m a power of two that is the same for all lanes.
 __device__ __forceinline__ uint32_t lane_xor(uint32_t v, int m) {
   if (m == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);
@@ -306,6 +318,7 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
   const bool live = w < nwords;
   A v[8];
   A lo, hi;  // of the group; without zero-points of FP16 sources both are its largest magnitude
+  bool special = false;  // FP16 sources: whether the wave has an element that is not finite
   if constexpr (sizeof(T) == 2) {
     // extrema on pairs of halves (whose minimum and maximum ignore a NaN); magnitudes as integers,
     // which NaN and infinity end up on top of
@@ -317,7 +330,8 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
       mag = __builtin_elementwise_max(mag, __builtin_bit_cast(us2, x[i] & 0x7FFF7FFFu));
     uint32_t top = mag[0] > mag[1] ? mag[0] : mag[1];
     // (a branch of the whole wave: as one of single lanes it cost 2 % of the kernel)
-    if (__builtin_amdgcn_ballot_w64(top >= 0x7C00u) != 0) {
+    special = __builtin_amdgcn_ballot_w64(top >= 0x7C00u) != 0;
+    if (special) {
       if (top >= 0x7C00u) atomicOr(status, 1);
       top = 0;  // a NaN is no extremum: the scale is that of the group's other elements
 #pragma unroll
@@ -381,9 +395,10 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
     double step;
     if constexpr (sizeof(T) == 2) {
       // range / 15, correctly rounded: a quotient by the rounded reciprocal, corrected once by its
-      // residual (the range is between 2^-24 and 2^17, so nothing under- or overflows)
+      // residual (a finite range is between 2^-24 and 2^17, so nothing under- or overflows; an
+      // infinite one leaves NaN, and the minimum turns that into a step past FP16's range)
       const double q = range * (1.0 / 15.0);
-      step = fma(fma(-q, 15.0, range), 1.0 / 15.0, q);
+      step = fmin(fma(fma(-q, 15.0, range), 1.0 / 15.0, q), DBL_MAX);
     } else {
       step = range / 15.0;
     }
@@ -440,6 +455,29 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
       }
     }
   }
+  if constexpr (sizeof(T) == 2) {
+    // (elements are read again: kept for this path, their registers cost the other one 3 %)
+    const bool plain = __builtin_amdgcn_classf(sf, 0x100);  // positive and finite
+    if (special || __builtin_amdgcn_ballot_w64(!plain) != 0) {
+      if (!live) return;
+      const float rsf = __builtin_amdgcn_rcpf(sf);
+      float u[8];
+      load8(src + w * 8, u);
+      u2 out = u2{0, 0};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if (MODE == QM_F8) {  // NaN is 0x7F; a step of 0 or infinity leaves no residual to correct by
+          const float x = u[j] * rsf;
+          out[j >> 2] |= encode_e4m3(plain ? copysignf(quotient_magnitude(u[j], sf, rsf), x) : x) << (8 * (j & 3));
+        } else {
+          out[0] |= quotient_code_any(u[j], sf, rsf, zero) << (4 * j);
+        }
+      }
+      if (MODE == QM_F8) *(u2*)(q8 + w * 8) = out;
+      else q32[w] = out[0];
+      return;
+    }
+  }
   if (!live) return;
   const A sfa = (A)sf;
   if (MODE == QM_F8) {
@@ -449,10 +487,6 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
       float mag[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) mag[j] = quotient_magnitude(v[j], sf, rsf);
-      if (!(sf <= 65504.0f)) {  // a group with an infinity: 0 for its other elements
-#pragma unroll
-        for (int j = 0; j < 8; ++j) mag[j] = fabsf(v[j]) < INFINITY ? 0.0f : (float)NAN;
-      }
       out[0] = pack_e4m3(mag, v);
       out[1] = pack_e4m3(mag + 4, v + 4);
     } else {
@@ -634,7 +668,12 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
     float val[8], mag[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) val[j] = (float)u[j], mag[j] = fabsf(val[j]);
-    const u2 out = u2{pack_e4m3(mag, val), pack_e4m3(mag + 4, val + 4)};
+    u2 out = u2{pack_e4m3(mag, val), pack_e4m3(mag + 4, val + 4)};
+    if (bad) {  // NaN is 0x7F
+      out = u2{0, 0};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) out[j >> 2] |= encode_e4m3(val[j]) << (8 * (j & 3));
+    }
     if (n == 8 && ((uintptr_t)dst & 7) == 0) {
       *(u2*)dst = out;
     } else {
