@@ -58,6 +58,18 @@ def test_asm_loaded_registers_are_never_parked(kernels):
     assert not bad, "\n".join(_demangle([k[".name"] for k in bad]))
 
 
+def test_flash_kernels_without_hooks_for_every_route(kernels):
+    """Calls without hooks run kernels without them: through registers for every cache kind (FP16,
+    W4, FP8), head dimension and scale / zero-point form, through LDS for the quantized kinds."""
+    names = [k[".name"] for k in kernels if "flash_mfma_phase1" in k[".name"]]
+    for kind in (0, 1, 2):
+        for D in (64, 128):
+            for alt in ((0,) if kind == 0 else (0, 1)):
+                for lds in ((0,) if kind == 0 else (0, 1)):
+                    tag = "flash_mfma_phase1ILi%dELi%dELb0ELi0ELb%dELb%dEE" % (kind, D, alt, lds)
+                    assert any(tag in n for n in names), tag
+
+
 def test_wave64_and_workgroup_sizes(kernels):
     for k in kernels:
         assert k[".wavefront_size"] == 64

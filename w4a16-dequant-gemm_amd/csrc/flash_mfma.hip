@@ -955,9 +955,10 @@ static hipError_t go_kind(const FlashArgs& a, int qh0, const FlashPlan& pl, floa
   if constexpr (KIND == KIND_F16) {
     return hook ? go_alt<KIND, true, 0, false>(a, qh0, pl, part, s) : go_alt<KIND, false, 0, false>(a, qh0, pl, part, s);
   } else {
-    const bool lds = flash_tiles_in_lds(a, pl);  // (the register path of the hooked kernels takes everything)
+    const bool lds = flash_tiles_in_lds(a, pl);
     if constexpr (KIND == KIND_F8) {
-      return lds ? go_alt<KIND, false, 0, true>(a, qh0, pl, part, s) : go_alt<KIND, true, 0, false>(a, qh0, pl, part, s);
+      return hook ? go_alt<KIND, true, 0, false>(a, qh0, pl, part, s)
+             : lds ? go_alt<KIND, false, 0, true>(a, qh0, pl, part, s) : go_alt<KIND, false, 0, false>(a, qh0, pl, part, s);
     } else {
       if (a.bt && a.page % 16 != 0)
         return hook ? go_alt<KIND, true, 2, false>(a, qh0, pl, part, s) : go_alt<KIND, false, 2, false>(a, qh0, pl, part, s);
