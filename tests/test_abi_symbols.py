@@ -73,6 +73,19 @@ def test_flash_plan_of_short_caches_shares_nothing():
             capi.flash_plan_for(*bad)
 
 
+def test_flash_scale_dwords_end_with_their_array():
+    """Tiles through LDS fetch row scales as dwords: caches whose scale arrays hold an odd number of
+    halves (one group per row, odd slabs times odd positions) take the register kernels."""
+    capi = w4amd.capi()
+    for kind in (1, 2):
+        for D in (64, 128):
+            for H in (1, 2, 3, 5, 8):
+                for S in (1, 77, 600, 601, 1500, 1501):
+                    for gs in (D, D // 2, D // 4):
+                        route = capi.flash_plan_for(kind, H, 1, S, D, gs)[3]
+                        assert route == (1 if gs == D and H * S % 2 else 2), (kind, H, S, D, gs, route)
+
+
 def test_quantize_contracts():
     """Malformed calls are rejected before the device is touched (pack.hpp:64-72,
     mx.hpp:71-76, kvcache.hpp:60-68, kvfp8.hpp:70-79)."""

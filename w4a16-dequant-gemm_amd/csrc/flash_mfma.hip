@@ -53,8 +53,7 @@ constexpr int FM_HEADS = 16;  // query heads per pass
 constexpr int FM_LDS_TILES = 12;  // W4: most tiles per wave that go through LDS (see flash_tiles_in_lds)
 constexpr int FM_RING = 2;    // LDS slots per wave (three measured slower: 12.7 -> 13.1 us, FP8 16.8 -> 21.7)
 typedef __attribute__((address_space(3))) void* fm_lds;
-typedef __attribute__((address_space(4))) const uint32_t* fm_const_u32;  // read with scalar loads
-typedef __attribute__((address_space(4))) const int* fm_const_i32;
+typedef __attribute__((address_space(4))) const int* fm_const_i32;  // read with scalar loads
 // The merge by a slab's last workgroup (1.4 us from the last ticket to the output) replaces a
 // second launch of 3 - 3.5 us.  One workgroup reads all partials of a slab, so it stops paying:
 // 8 slabs x 8192 positions with 128 partials each took 11.5 us in place and 10.2 with the merge kernel.
@@ -173,13 +172,15 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
     asm("" : "+v"(x));
     return x;
   };
+  // One scale per slab.  (Through LDS: two more requests that the waits below count together with
+  // the query's, so nothing waits for them alone.)
   _Float16 slab_sk = 0, slab_sv = 0;
-  if (SLAB_SCALE) {  // (aligned dwords through the scalar cache: no vector request to wait for)
-    auto at = [&](const w4_half* sc) {
-      const uintptr_t p = (uintptr_t)(sc + slab);
-      return as_half((uint16_t)(*(fm_const_u32)(p & ~(uintptr_t)3) >> (8 * (p & 2))));
-    };
-    slab_sk = at(a.s_k), slab_sv = at(a.s_v);
+  uint32_t slab_raw[2];
+  if constexpr (SLAB_SCALE && LDS) {
+    asm volatile("global_load_ushort %0, %1, off" : "=v"(slab_raw[0]) : "v"(a.s_k + slab) : "memory");
+    asm volatile("global_load_ushort %0, %1, off" : "=v"(slab_raw[1]) : "v"(a.s_v + slab) : "memory");
+  } else if constexpr (SLAB_SCALE) {
+    slab_sk = as_half(a.s_k[slab]), slab_sv = as_half(a.s_v[slab]);
   }
 
   const int s0 = split * split_len;
@@ -747,6 +748,10 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
     };
     wait_tile(0);
     build_q();
+    if constexpr (SLAB_SCALE) {
+      asm volatile("" : "+v"(slab_raw[0]), "+v"(slab_raw[1]));
+      slab_sk = as_half((uint16_t)slab_raw[0]), slab_sv = as_half((uint16_t)slab_raw[1]);
+    }
     for (int it0 = 0; it0 < nit; it0 += FM_RING) {
 #pragma unroll
       for (int d = 0; d < FM_RING; ++d) {
@@ -979,8 +984,10 @@ bool flash_mfma_applies(const FlashArgs& a) {
          ((((uintptr_t)a.k_out | (uintptr_t)a.v_out) & 15) == 0);
 }
 
-// Tiles through LDS: 32-bit offsets inside a slab, scales that can be fetched as dwords, at most
-// four groups per row, pages of whole half tiles.
+// Tiles through LDS: 32-bit offsets inside a slab, at most four groups per row, pages of whole half
+// tiles, and row scales that can be fetched as dwords: arrays that begin on one and hold a whole
+// number of them (with one group per row and an odd number of rows in all, the last dword would end two
+// bytes behind the array).
 // W4 with more than FM_LDS_TILES tiles per wave stays in registers: once the stream runs, the
 // read back from LDS in front of every tile costs more than the loads it saves (57.7
 // against 60.9 us at 64 slabs x 32768 positions, 33.6 against 34.8 with 16 tiles per wave;
@@ -989,6 +996,8 @@ bool flash_tiles_in_lds(const FlashArgs& a, const FlashPlan& pl) {
   if (a.kind == KIND_F16 || a.k_out || a.v_out || (a.bt && a.page % 16)) return false;
   const long long slab_rows = a.bt ? a.pool_rows : a.S;
   if (slab_rows * a.D * 2 >= (1ll << 31) || a.G > 4 || (((uintptr_t)a.s_k | (uintptr_t)a.s_v) & 3)) return false;
+  const bool row_scales = a.kind == KIND_W4 || a.scale_mode != 1;
+  if (row_scales && (a.bt ? a.Hkv : a.H) * slab_rows * a.G % 2) return false;
   return a.kind == KIND_F8 || pl.split_len <= FM_LDS_TILES * FM_WAVES * FM_TILE;
 }
 
