@@ -1,47 +1,92 @@
 """Split-S flash decode whose last workgroup of every slab merges the slab's splits
 (csrc/flash_mfma.hip): numbers of splits and heads at the edges of the rule that chooses it
-(2 and 64 splits, 64 (head, split) partials in one workgroup, just past both, several passes of 16
-heads), called again and in between calls with other numbers of splits: the arrival counters have
-to be back at zero after each.  kvflash.cuh:350-363 is the reference's entry for these shapes."""
+(64 splits and more, 64 (head, split) partials in one workgroup and more, several passes of 16
+heads) for every kind of cache, called again and in between calls with other numbers of splits: the
+arrival counters have to be back at zero after each.  The plan query pins the number of splits and
+where they are merged.  kvflash.cuh:350-363 is the reference's entry for these shapes."""
 import numpy as np
 import pytest
 
 import orc
 import w4amd
-from devutil import DevKV, bits, halves, ptr, to_dev
+from devutil import DevKV, DevKVF8, bits, halves, ptr, to_dev
+from test_gpu_attention import _paged_pool
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-3  # rel L2 against the FP64 oracle, as in test_gpu_attention.py
+F16, W4, F8 = 0, 1, 2
 
-# (slabs, positions, head dim, query heads per slab, symmetric)
-SHAPES = [(1, 16384, 128, 1, True),    # 64 splits, one per lane of the merging wave
-          (1, 17000, 128, 1, False),   # more splits than that: the merge kernel
-          (4, 4000, 128, 4, True),     # 64 partials per slab
-          (4, 4000, 128, 5, False),    # more
-          (8, 600, 64, 7, True),       # few splits, heads that do not divide over the waves
-          (2, 1000, 128, 19, True),    # two passes over the heads, one merged in place, one not
-          (130, 700, 128, 2, False)]   # a slab count past one per compute unit and XCD round
+# (cache, slabs, positions, head dim, query heads per slab, symmetric, page; splits, merged in place)
+SHAPES = [(W4, 1, 16384, 128, 1, True, 0, 64, True),    # 64 splits, one per lane of the merging wave
+          (W4, 8, 16384, 128, 1, True, 0, 64, True),    # the same for several slabs
+          (W4, 1, 16793, 128, 4, False, 0, 66, False),  # more splits than that
+          (W4, 1, 24000, 128, 1, False, 16, 63, True),
+          (W4, 4, 4000, 128, 4, True, 0, 16, True),     # 64 partials per slab
+          (W4, 4, 4000, 128, 5, False, 0, 32, False),   # more
+          (W4, 4, 4000, 128, 4, True, 16, 16, True),
+          (W4, 8, 600, 64, 7, True, 0, 5, True),        # few splits, heads that do not divide over the waves
+          (W4, 71, 1000, 128, 17, True, 0, 3, True),    # two passes over the heads, one after the other
+          (W4, 60, 1000, 128, 19, True, 0, 4, True),
+          (W4, 130, 700, 128, 2, False, 48, 3, True),   # a slab count past one per compute unit and XCD round
+          (F8, 1, 16384, 64, 1, True, 0, 64, True),
+          (F8, 4, 4000, 128, 4, True, 0, 16, True),
+          (F8, 4, 4000, 128, 5, True, 0, 32, False),
+          (F8, 71, 1000, 128, 17, True, 0, 3, True),
+          (F16, 1, 16384, 128, 1, True, 0, 64, True),
+          (F16, 4, 4000, 128, 4, True, 0, 32, False),
+          (F16, 8, 600, 64, 7, True, 0, 5, True),
+          (F16, 71, 1000, 64, 17, True, 0, 3, True)]
+
+
+class _Case:
+    def __init__(self, i):
+        self.c = c = w4amd.capi()
+        self.kind, self.H, self.S, self.D, self.group, sym, self.page, splits, merged = SHAPES[i]
+        H, S, D = self.H, self.S, self.D
+        plan = c.flash_plan_for(self.kind, H, self.group, S, D, 32, self.page)
+        assert (plan[0], plan[2]) == (splits, merged), plan
+        k, v = orc.normal_weights(H * S * D, 71 + i), orc.normal_weights(H * S * D, 171 + i)
+        if self.kind == F8:
+            cache = orc.quantize_cache_f8(k, v, H, S, D, 32)
+            self.kd, self.vd = orc.dequant_cache_f8(cache, False), orc.dequant_cache_f8(cache, True)
+            self.dk = DevKVF8(cache)
+        else:
+            cache = orc.quantize_cache(k, v, H, S, D, 32, sym)
+            self.kd, self.vd = orc.dequant_cache(cache, False), orc.dequant_cache(cache, True)
+            if self.kind == F16:
+                self.k16, self.v16 = to_dev(self.kd), to_dev(self.vd)
+            elif self.page:
+                self.npages = (S + self.page - 1) // self.page
+                bt = np.random.default_rng(i).permutation(self.npages).astype(np.int32)
+                self.keep, self.view = _paged_pool(cache, self.page, bt)
+                self.bt = to_dev(bt)
+            else:
+                self.dk = DevKV(cache)
+        self.q = orc.normal_activations(H * self.group * D, 271 + i)
+        self.q_d = to_dev(self.q)
+
+    def run(self):
+        c, H, S, D, group = self.c, self.H, self.S, self.D, self.group
+        out = halves(H * group * D, 0x7E00)
+        if self.kind == F16:
+            c.attention_fp16_flash(ptr(self.q_d), ptr(self.k16), ptr(self.v16), ptr(out), H, S, D, group=group)
+        elif self.kind == F8:
+            c.attention_f8_flash(self.dk.view, ptr(self.q_d), ptr(out), group=group)
+        elif self.page:
+            c.attention_w4_flash_paged_batched(self.view, ptr(self.bt), 1, self.npages, self.page, self.npages,
+                                               group, ptr(self.q_d), ptr(out))
+        else:
+            c.attention_w4_flash(self.dk.view, ptr(self.q_d), ptr(out), group=group)
+        return bits(out).copy()
 
 
 @pytest.mark.parametrize("i", range(len(SHAPES)))
 def test_merge_in_place(i):
-    c = w4amd.capi()
-    cases = []
-    for j in (i, (i + 1) % len(SHAPES)):
-        H, S, D, group, sym = SHAPES[j]
-        c4 = orc.quantize_cache(orc.normal_weights(H * S * D, 71 + j), orc.normal_weights(H * S * D, 171 + j),
-                                H, S, D, 32, sym)
-        cases.append((c4, orc.normal_activations(H * group * D, 271 + j), group))
-    runs = []
-    for c4, q, group in cases * 3:  # three times each, in turn
-        out = halves(c4.H * group * c4.D, 0x7E00)
-        dk, q_d = DevKV(c4), to_dev(q)
-        c.attention_w4_flash(dk.view, ptr(q_d), ptr(out), group=group)
-        runs.append(bits(out).copy())
+    a, b = _Case(i), _Case((i + 1) % len(SHAPES))
+    runs = [x.run() for x in (a, b) * 3]  # three times each, in turn
     for r in (2, 4):
         assert np.array_equal(runs[r], runs[0]) and np.array_equal(runs[r + 1], runs[1])
-    c4, q, group = cases[0]
-    ref = orc.attention_f16(q, orc.dequant_cache(c4, False), orc.dequant_cache(c4, True), c4.H, group, c4.S, c4.D)
+    ref = orc.attention_f16(a.q, a.kd, a.vd, a.H, a.group, a.S, a.D)
     assert orc.rel_l2(runs[0].view(np.float16), ref) <= TOL
 
 

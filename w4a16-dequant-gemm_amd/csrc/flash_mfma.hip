@@ -56,7 +56,8 @@ typedef __attribute__((address_space(3))) void* fm_lds;
 typedef __attribute__((address_space(4))) const int* fm_const_i32;  // read with scalar loads
 // The merge by a slab's last workgroup (1.4 us from the last ticket to the output) replaces a
 // second launch of 3 - 3.5 us.  One workgroup reads all partials of a slab, so it stops paying:
-// 8 slabs x 8192 positions with 128 partials each took 11.5 us in place and 10.2 with the merge kernel.
+// 8 slabs x 8192 positions with 128 partials each took 11.5 us in place and 10.2 with the merge kernel
+// (before the arrivals were counted on lines of their own).
 constexpr int FM_MERGE_SPLITS = 64;  // most splits of a slab that its last workgroup merges (one per lane)
 constexpr int FM_MERGE_MAX = 64;     // most (head, split) partials that one workgroup merges
 constexpr int FM_MERGE_SLABS = 512;  // more slabs than this are not merged in place
@@ -107,7 +108,11 @@ __device__ __forceinline__ h8 pack8(const h2 v[4]) {
 
 // Arrivals of a slab's splits, by scratch buffer, number of splits and slab (see the end of
 // the kernel).  Zero when the library is loaded and after every call.  Calls whose partials lie
-// in different buffers may overlap, so every buffer has counters of its own.
+// in different buffers may overlap, so every buffer has counters of its own.  The slabs of a call
+// spread over the FM_MERGE_SLABS counters of their number of splits: atomics on one 128-byte line
+// wait for each other, and with neighbouring counters the 512 arrivals of 8 slabs in 64 splits each were on
+// one line (8 x 16384, W4, one head: 14.3 -> 11.2 us, with the merge
+// kernel 12.2; 4 x 8192 of D = 64: 9.4 -> 7.5, 8.1).
 __device__ uint32_t flash_arrivals[FL_SCRATCH_IDS * (FM_MERGE_SPLITS + 1) * FM_MERGE_SLABS];
 
 // PAGED: 0 contiguous slabs, 1 pages of a multiple of 16 rows (both halves of a
@@ -118,7 +123,7 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
                                                                    const int qh0,
                                                                    const int split_len,
                                                                    float* __restrict__ part,
-                                                                   const int merge_id) {
+                                                                   const int merge_at) {
   constexpr bool ASYM = KIND == KIND_W4 && ALT, SLAB_SCALE = KIND == KIND_F8 && ALT;
   constexpr int FM_D = DH;       // head dimension
   constexpr int NC = DH / 32;    // MFMAs per score group; a lane's K slice is 8 * NC elements
@@ -877,20 +882,19 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
     if (j) publish(dst, sum0, sum1);
     else publish(dst, M, sum0);
   }
-  if (merge_id < 0) return;
+  if (merge_at < 0) return;
 
   // The workgroup of a slab that finishes last merges the slab's splits.  Each one counts
   // itself once its partial has been written (the stores have come back); the counter wraps
-  // to 0 with the last one, so the next call finds it as this one did.  There is one counter
-  // per (scratch buffer, number of splits, slab): calls that share a counter make the same number of
-  // arrivals, so even calls that overlapped by mistake leave it at 0.
+  // to 0 with the last one, so the next call finds it as this one did.  There is one counter per
+  // (scratch buffer, number of splits, place of the slab): calls that share a counter make the same
+  // number of arrivals, so even calls that overlapped by mistake leave it at 0.
   __shared__ uint32_t arrived;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0)
     arrived = __builtin_amdgcn_atomic_inc32(
-        &flash_arrivals[(merge_id * (FM_MERGE_SPLITS + 1) + nsplit) * FM_MERGE_SLABS + slab], (uint32_t)(nsplit - 1),
-        __ATOMIC_RELAXED, "agent");
+        &flash_arrivals[(merge_at >> 4) + (slab << (merge_at & 15))], (uint32_t)(nsplit - 1), __ATOMIC_RELAXED, "agent");
   __syncthreads();
   if (arrived != (uint32_t)(nsplit - 1)) return;
   // A wave takes every fourth head.  Lane t has the maximum and the denominator of split t,
@@ -936,6 +940,15 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
   }
 }
 
+// Where a call's arrivals are counted: 16 times the first counter plus the logarithm of the distance
+// between two slabs' (a.H << distance <= FM_MERGE_SLABS); -1 where another kernel merges.
+static int merge_place(const FlashArgs& a, const FlashPlan& pl) {
+  if (!flash_merges_in_place(a, pl)) return -1;
+  int shift = 0;
+  while (a.H << (shift + 1) <= FM_MERGE_SLABS) ++shift;
+  return (a.scratch_id * (FM_MERGE_SPLITS + 1) + pl.nsplit) * FM_MERGE_SLABS * 16 + shift;
+}
+
 template <int KIND, bool HOOK, int PAGED, bool LDS>
 static hipError_t go_alt(const FlashArgs& a, int qh0, const FlashPlan& pl, float* part,
                          hipStream_t s) {
@@ -943,7 +956,7 @@ static hipError_t go_alt(const FlashArgs& a, int qh0, const FlashPlan& pl, float
   const bool alt = (KIND == KIND_W4 && !a.symmetric) || (KIND == KIND_F8 && a.scale_mode == 1);
 #define W4_GO(DH, ALT)                                                         \
   flash_mfma_phase1<KIND, DH, HOOK, PAGED, (ALT) && KIND != KIND_F16, LDS>     \
-      <<<grid, FM_WAVES * 64, 0, s>>>(a, qh0, pl.split_len, part, flash_merges_in_place(a, pl) ? a.scratch_id : -1)
+      <<<grid, FM_WAVES * 64, 0, s>>>(a, qh0, pl.split_len, part, merge_place(a, pl))
   if (a.D == 128) {
     if (alt) W4_GO(128, true); else W4_GO(128, false);
   } else {
