@@ -73,6 +73,18 @@ def test_flash_plan_of_short_caches_shares_nothing():
             capi.flash_plan_for(*bad)
 
 
+def test_flash_plan_of_many_heads():
+    """More than 12 query heads per slab: from four splits on a kernel of its own merges them."""
+    capi = w4amd.capi()
+    for kind in (0, 1, 2):
+        for S in (900, 1000, 1024, 2000, 5000, 16384):
+            for H in (8, 37, 64, 71, 128, 200):
+                for group in (4, 12, 13, 16, 19):
+                    splits, _, one_launch, _ = capi.flash_plan_for(kind, H, group, S, 128, 32)
+                    heads = min(group, 16)
+                    assert one_launch == (splits == 1 or heads * splits <= (48 if heads > 12 else 64))
+
+
 def test_flash_scale_dwords_end_with_their_array():
     """Tiles through LDS fetch row scales as dwords: caches whose scale arrays hold an odd number of
     halves (one group per row, odd slabs times odd positions) take the register kernels."""

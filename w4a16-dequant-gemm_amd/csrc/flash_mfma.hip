@@ -61,6 +61,9 @@ typedef __attribute__((address_space(4))) const int* fm_const_i32;  // read with
 constexpr int FM_MERGE_SPLITS = 64;  // most splits of a slab that its last workgroup merges (one per lane)
 constexpr int FM_MERGE_MAX = 64;     // most (head, split) partials that one workgroup merges
 constexpr int FM_MERGE_SLABS = 512;  // more slabs than this are not merged in place
+// With more than 12 heads every wave merges four, one after the other, and from four splits on the
+// second launch is ahead (16 heads: by 0.5 us, median of 123 calls; three splits: behind by 1.2).
+constexpr int FM_MERGE_MAX_4 = 48;
 
 // What one lane fetches for one tile, before expansion.
 // NC = D / 32: MFMAs per group of 16 positions = packed words (W4) per lane.
@@ -1015,8 +1018,9 @@ bool flash_tiles_in_lds(const FlashArgs& a, const FlashPlan& pl) {
 }
 
 bool flash_merges_in_place(const FlashArgs& a, const FlashPlan& pl) {
+  const int heads = min(a.group, FM_HEADS);
   return pl.nsplit > 1 && pl.nsplit <= FM_MERGE_SPLITS && a.H <= FM_MERGE_SLABS &&
-         min(a.group, FM_HEADS) * pl.nsplit <= FM_MERGE_MAX;
+         heads * pl.nsplit <= (heads > 12 ? FM_MERGE_MAX_4 : FM_MERGE_MAX);
 }
 
 bool try_flash_mfma(const FlashArgs& a, const FlashPlan& pl, float* part, hipStream_t s,
