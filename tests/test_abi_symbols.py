@@ -73,6 +73,23 @@ def test_flash_plan_of_short_caches_shares_nothing():
             capi.flash_plan_for(*bad)
 
 
+def test_flash_long_splits_keep_tiles_in_registers():
+    """Many tiles per wave go through registers: W4 and FP8 with D = 64 from 13 on, FP8 with D = 128 from 16
+    on where no compute unit has two workgroups."""
+    capi = w4amd.capi()
+    seen = set()
+    for kind, gs in ((1, 32), (2, 32), (2, 64)):
+        for D in (64, 128):
+            for H in (1, 16, 100, 256, 300, 512, 700):
+                for S in (700, 1500, 1700, 1900, 2100, 4096, 8192, 20000, 32768):
+                    splits, length, _, route = capi.flash_plan_for(kind, H, 4, S, D, gs)
+                    tiles = length // 128
+                    lds = tiles <= 12 if kind == 1 or D == 64 else tiles <= 15 or H * splits > 256
+                    assert route == (2 if lds else 1), (kind, D, H, S, splits, length, route)
+                    seen.add((kind, D, lds))
+    assert len(seen) == 8
+
+
 def test_flash_plan_of_many_heads():
     """More than 12 query heads per slab: from four splits on a kernel of its own merges them."""
     capi = w4amd.capi()

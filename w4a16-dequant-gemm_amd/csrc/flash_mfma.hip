@@ -24,7 +24,7 @@
 // Tiles reach the wave in one of two ways.  Through registers: whole tiles are fetched with
 // buffer loads whose wave-uniform part lives in the descriptor and the scalar offset; a
 // ring of three raw tiles is refilled in place, two tiles in flight while one is computed.
-// Through LDS (W4 with few tiles per wave, FP8): a tile as registers need it is 21 load
+// Through LDS (few tiles per wave; FP8 with D = 128 and two workgroups per compute unit always): a tile as registers need it is 21 load
 // instructions, most of them 2 or 4 bytes a lane, and a compute unit takes one such
 // instruction per 10 - 13 ns whatever it carries; at three tiles per wave eight waves had placed
 // their requests only after 3.7 - 6.3 us (time stamps, 128 slabs x 1500 positions, a call of
@@ -50,7 +50,8 @@ constexpr int FM_TILE = 32;   // positions per wave tile
 constexpr int FM_WAVES = 4;
 constexpr int FM_DEPTH = 3;   // ring slots per wave: one tile computed, two in flight
 constexpr int FM_HEADS = 16;  // query heads per pass
-constexpr int FM_LDS_TILES = 12;  // W4: most tiles per wave that go through LDS (see flash_tiles_in_lds)
+constexpr int FM_LDS_TILES = 12;  // W4, FP8 with D = 64: most tiles per wave that go through LDS (see flash_tiles_in_lds)
+constexpr int FM_LDS_TILES_ALONE = 15;  // FP8, D = 128, one workgroup per compute unit
 constexpr int FM_RING = 2;    // LDS slots per wave (three measured slower: 12.7 -> 13.1 us, FP8 16.8 -> 21.7)
 typedef __attribute__((address_space(3))) void* fm_lds;
 typedef __attribute__((address_space(4))) const int* fm_const_i32;  // read with scalar loads
@@ -1007,14 +1008,19 @@ bool flash_mfma_applies(const FlashArgs& a) {
 // W4 with more than FM_LDS_TILES tiles per wave stays in registers: once the stream runs, the
 // read back from LDS in front of every tile costs more than the loads it saves (57.7
 // against 60.9 us at 64 slabs x 32768 positions, 33.6 against 34.8 with 16 tiles per wave;
-// 27.5 against 28.4 us with 12, 12.7 against 14.1 with 4).
+// 27.5 against 28.4 us with 12, 12.7 against 14.1 with 4).  FP8 likewise with D = 64 (time through
+// registers over that through LDS, medians of 3 - 80 calls: 8 tiles 0.98 - 1.07, 12 0.99 - 1.02, 16 0.92 -
+// 0.99, 32 0.87 - 0.94) and with D = 128 where every workgroup has a compute unit to itself (12 1.09, 16 0.99,
+// 32 0.92); with two of them on a unit LDS stays ahead (16 1.03, 32 1.02 - 1.04).
 bool flash_tiles_in_lds(const FlashArgs& a, const FlashPlan& pl) {
   if (a.kind == KIND_F16 || a.k_out || a.v_out || (a.bt && a.page % 16)) return false;
   const long long slab_rows = a.bt ? a.pool_rows : a.S;
   if (slab_rows * a.D * 2 >= (1ll << 31) || a.G > 4 || (((uintptr_t)a.s_k | (uintptr_t)a.s_v) & 3)) return false;
   const bool row_scales = a.kind == KIND_W4 || a.scale_mode != 1;
   if (row_scales && (a.bt ? a.Hkv : a.H) * slab_rows * a.G % 2) return false;
-  return a.kind == KIND_F8 || pl.split_len <= FM_LDS_TILES * FM_WAVES * FM_TILE;
+  const int tiles = pl.split_len / (FM_WAVES * FM_TILE);
+  if (a.kind == KIND_W4 || a.D == 64) return tiles <= FM_LDS_TILES;
+  return tiles <= FM_LDS_TILES_ALONE || (long long)a.H * pl.nsplit > 256;
 }
 
 bool flash_merges_in_place(const FlashArgs& a, const FlashPlan& pl) {
