@@ -362,8 +362,10 @@ __global__ __launch_bounds__(P2_THREADS) void flash_phase2(const float* __restri
 // compute unit shares its vector units; the terms below are measured (us, D = 128, gs = 32,
 // 4 heads per slab; x 0.7 at D = 64):
 //   t tiles take 0.5 + T t with at most one workgroup per compute unit (T = 1.0 for W4, 1.4 FP8,
-//   2.5 FP16), 1.7 + F T t with two (F = 1.25 W4, 1.8 FP8), as many times over as the grid has
-//   rounds; FP16 fits one workgroup per unit;
+//   2.5 FP16), 1.7 + F T t with two (F = 1.25 W4, 1.8 FP8, 1.5 FP8 with D = 64); past two on each the
+//   rounds overlap: x rounds' worth of workgroups take x + 0.3 times F T t, and 1.7 for each begun
+//   (counted whole, a grid of 1.2 rounds seemed as long as two, and 260 - 400 slabs were never split: 300 x 4096
+//   FP8 with D = 64, one split 62 us, two 50 - 54); FP16 fits one workgroup per unit;
 //   the merge by the last workgroup 1.5 (+ 0.7 per further four heads), by a second kernel 3 + 0.03 per split, none 0.
 // Before this rule splits were multiples of 256 positions and aimed at 512 workgroups: 32 x 6007 FP8
 // 19.4 -> 15.2 us, 128 x 1500 W4 pages 12.7 -> 11.4, 32 x 3000 FP16 18.4 -> 14.0, 8 x 600 W4 6.7 -> 6.1.
@@ -373,7 +375,10 @@ static float split_cost(const FlashArgs& a, int t, int nsplit) {
   float c;
   if (wgs <= 256) c = 0.5f + T * t;
   else if (a.kind == KIND_F16) c = (float)((wgs + 255) / 256) * (1.2f + T * t);
-  else c = (float)((wgs + 511) / 512) * (1.7f + (a.kind == KIND_W4 ? 1.25f : 1.8f) * T * t);
+  else {
+    const float x = (float)wgs / 512, F = a.kind == KIND_W4 ? 1.25f : a.D == 64 ? 1.5f : 1.8f;
+    c = 1.7f * (float)((wgs + 511) / 512) + F * T * t * (x <= 1.0f ? 1.0f : x + 0.3f);
+  }
   if (nsplit > 1)
     c += flash_merges_in_place(a, FlashPlan{128 * t, nsplit}) ? 1.5f + 0.7f * ((a.group - 1) / 4) : 3.0f + 0.03f * nsplit;
   return c;
@@ -381,8 +386,8 @@ static float split_cost(const FlashArgs& a, int t, int nsplit) {
 
 static FlashPlan mfma_plan(const FlashArgs& a) {
   const int tiles = (a.S + 127) / 128;
-  // nothing is gained below one round of two workgroups per compute unit (512) or above twice that
-  const int lo = (int)(((long long)tiles * a.H + 511) / 512), hi = lo * 2 + 4;
+  // nothing is gained by more than two rounds of two workgroups per compute unit (512) or less than half a round
+  const int one = (int)(((long long)tiles * a.H + 511) / 512), lo = (one + 1) / 2, hi = one * 2 + 4;
   FlashPlan best{128 * tiles, 1};
   float cost = split_cost(a, tiles, 1);
   for (int t = lo < 1 ? 1 : lo; t <= hi && t < tiles; ++t) {
