@@ -364,7 +364,7 @@ __global__ __launch_bounds__(P2_THREADS) void flash_phase2(const float* __restri
 //   t tiles take 0.5 + T t with at most one workgroup per compute unit (T = 1.0 for W4, 1.4 FP8,
 //   2.5 FP16), 1.7 + F T t with two (F = 1.25 W4, 1.8 FP8, 1.5 FP8 with D = 64); past two on each the
 //   rounds overlap: x rounds' worth of workgroups take x + 0.3 times F T t, and 1.7 for each begun
-//   (counted whole, a grid of 1.2 rounds seemed as long as two, and 260 - 400 slabs were never split: 300 x 4096
+//   (counted whole, a grid of 1.2 rounds seemed as long as two, and 260 - 325 slabs were never split: 300 x 4096
 //   FP8 with D = 64, one split 62 us, two 50 - 54); FP16 fits one workgroup per unit;
 //   the merge by the last workgroup 1.5 (+ 0.7 per further four heads), by a second kernel 3 + 0.03 per split, none 0.
 // Before this rule splits were multiples of 256 positions and aimed at 512 workgroups: 32 x 6007 FP8
