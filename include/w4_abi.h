@@ -243,6 +243,10 @@ int w4_quantize_mx8_f16(const w4_act_mx8_view* out, const w4_half* x, int* statu
                         w4_stream stream);
 int w4_gemm_mx_w4a8(const w4_packed_mx_view* w, const w4_act_mx8_view* x,
                     w4_half* c, w4_stream stream);
+/* Which kernel those two run (plain arithmetic, no GPU needed; no counterpart in the reference): x8
+ * nonzero for MXFP8 activations; arrays aligned to 16 bytes.  *plan: 0 no tiles; 1 - 4 eight-wave tiles
+ * of 128 columns x 32 times as many activation rows; 8 tiles of 256 x 128. */
+int w4_gemm_mx_plan_for(int x8, int M, int N, int K, int* plan);
 
 #ifdef __cplusplus
 }

@@ -572,6 +572,12 @@ int w4_gemm_mx_w4a8(const w4_packed_mx_view* w, const w4_act_mx8_view* x, w4_hal
   return done("gemm_mx_w4a8", w4k::launch_gemm_mx_w4a8(*w, *x, c, (hipStream_t)stream));
 }
 
+int w4_gemm_mx_plan_for(int x8, int M, int N, int K, int* plan) {
+  REQUIRE(plan && M >= 1 && N >= 1 && K >= 1, "mx plan: bad dims");
+  *plan = w4k::mx_plan(x8 != 0, M, N, K);
+  return W4_OK;
+}
+
 int w4_quantize_cache(const w4_kv_view* out, const void* k, const void* v, int src_f16,
                       int* status, w4_stream stream) {
   REQUIRE(out != nullptr, "quantize_cache: null view");

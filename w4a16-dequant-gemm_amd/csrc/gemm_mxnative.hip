@@ -1117,22 +1117,40 @@ bool tile_operands_ok(const w4_packed_mx_view& w, const void* xq, const uint8_t*
 // is linear in the stages (us, measured with every unit busy, K = 4096 and 14336; the scales of
 // a K that is no multiple of 512 add 0.12 per stage to the eight-wave tiles).
 // Few workgroups of the eight-wave tiles are slower than the skinny kernel, which reads W once
-// and X from L2.  Up to 64 rows it is ahead below 100 of them (N = 4096, K = 4096, M = 33: 8.1 us
-// both; N = 14336, M = 8: 11.1 -> 8.5, M = 33: 20.6 -> 9.2; K = 14336, N = 4096, M = 24: 16.7
-// against 20.9), with up to 4 rows below 160 (N = 13824, M = 1: 9.2 against 9.8; N = 28672:
-// 15.7 -> 11.3); from 65 to 128 rows up to 32 of them with 8-bit X (N = 1024, K = 4096: 6.8
-// against 7.7) and up to 64 at K <= 2048 (N = 2048, 4-bit X: 4.5 against 5.0).  Where K is no
-// multiple of 512 its guarded loads cost it 2 to 3 times as much and it keeps 32 rows (16 with
-// 4-bit X; N = 4096, K = 11008, M = 17: 20.1 against 21.9 and 24.0 -> 21.0; M = 33 26.1 -> 20.0)
+// and X from L2; how many are too few depends on the rows, and on where W comes from.  With W in
+// the last-level cache (a few matrices of one size, 130 MB in all) the tiles are ahead much sooner than with W in
+// memory (700 MB), where a large model's matrices are.  The lines below lie where the mean of the logarithms of tile /
+// skinny over both changes its sign (9000 random calls; cache and memory):
+//   4-bit X, 101 - 120 workgroups: M = 5 - 8 0.92 and 1.28 (K = 4096), 1.03 and 1.48 (5120); M = 9 - 12 0.87 and 1.21,
+//   1.00 and 1.39; M = 13 - 16 0.84 and 1.11, 0.94 and 1.33; M = 17 - 24 0.70 and 0.94, 0.81 and 1.13;
+//   171 - 200: M <= 2 0.95 and 1.13, M = 3, 4 0.91 and 1.06, M = 5 - 8 0.84 and 0.99;
+//   N = K = 8192 (128): M = 33 - 48 0.91 and 1.25, M = 49 - 64 0.79 and 1.13;
+//   8-bit X, 101 - 120: M = 5 - 8 0.85 and 1.10 (K = 4096), 0.89 and 1.26 (5120); M = 9 - 12 0.81 and 1.13 (5120).
+//   N = 13824, K = 5120, M = 5, 4-bit X, memory: 10.7 us, with tiles 15.9.
+// More than 64 rows of narrow matrices (up to 16 tiles of columns): 4-bit X up to 48 workgroups 1.02 - 1.3 both, with
+// M = 97 - 128 up to 64; 8-bit X up to 32 1.1 - 1.3; 4-bit X at N = 4096, K = 14336 0.83 - 0.86 and 1.25 - 1.27 (K = 4096
+// 0.83 - 0.87 and 1.11 - 1.15, which stays with the tiles).  At K <= 2048 up to 64 with either (N = 2048, 4-bit X: 4.5
+// against 5.0).
+// Where K is no multiple of 512 the skinny kernel's guarded loads cost it 2 to 3 times as much and it keeps 32 rows
+// (16 with 4-bit X; N = 4096, K = 11008, M = 17: 20.1 against 21.9 and 24.0 -> 21.0; M = 33 26.1 -> 20.0)
 // and short K with 8-bit X (N = 1000, K = 1280, M = 64: 4.5 against 4.7).
+template <bool XF8>
+int fewest_tile_workgroups(int M, int K) {
+  if (K % 512) return M > (XF8 ? 32 : 16) ? 0 : M <= 4 ? 160 : 100;
+  if (XF8) return M <= 4 ? 160 : M <= 8 && K > 4096 ? 121 : 100;
+  if (M <= 12) return M <= 2 ? 200 : M <= 4 ? 171 : M <= 8 ? 140 : 121;
+  return M <= 16 && K > 4096 ? 121 : M > 32 && M <= 48 && K > 6144 ? 140 : 100;
+}
+
 template <bool XF8>
 int plan_tile(const w4_packed_mx_view& w, int M) {
   const long long tn = (w.N + T8_TN - 1) / T8_TN;
   const float st = (float)(w.K / 256);
   const long long wgs = tn * ((M + 31) / 32);
-  if (M <= 64 && (w.K % 512 == 0 || M <= (XF8 ? 32 : 16)) && wgs < (M <= 4 ? 160 : 100)) return 0;
-  if (M <= 128 && w.K % 512 == 0 && wgs <= (w.K <= 2048 ? 64 : XF8 ? 32 : 0)) return 0;
-  if (XF8 && M <= 128 && w.K <= 2048 && wgs <= 24) return 0;
+  if (M <= 64 && wgs < fewest_tile_workgroups<XF8>(M, w.K)) return 0;
+  if (M <= 128 && w.K <= 2048 && wgs <= (w.K % 512 ? XF8 ? 24 : 0 : 64)) return 0;
+  if (M <= 512 && w.K % 512 == 0 && wgs <= (XF8 ? 32 : M > 96 && M <= 128 ? 64 : 48)) return 0;
+  if (!XF8 && M > 64 && M <= 128 && w.K % 512 == 0 && w.K > 8192 && tn <= 33) return 0;
   static constexpr float slope[5] = {0.f, XF8 ? .33f : .29f, XF8 ? .50f : .39f, XF8 ? .75f : .55f, XF8 ? 1.0f : .65f};
   float best = 0.f;
   int pick = 0;
@@ -1202,6 +1220,13 @@ hipError_t launch_mxn(const w4_packed_mx_view& w, const void* xq, const uint8_t*
 }
 
 }  // namespace
+
+int mx_plan(bool x8, int M, int N, int K) {
+  w4_packed_mx_view w{};
+  w.N = N, w.K = K, w.B = (K + 31) / 32;
+  if (!tile_operands_ok(w, nullptr, nullptr, M, x8 ? K : K / 2)) return 0;
+  return x8 ? plan_tile<true>(w, M) : plan_tile<false>(w, M);
+}
 
 hipError_t launch_gemm_mx_w4a4(const w4_packed_mx_view& w, const w4_packed_mx_view& x,
                                w4_half* c, hipStream_t s) {

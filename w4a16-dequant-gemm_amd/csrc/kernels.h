@@ -146,6 +146,8 @@ hipError_t launch_gemm_mx_w4a4(const w4_packed_mx_view& w, const w4_packed_mx_vi
                                w4_half* c, hipStream_t s);
 hipError_t launch_gemm_mx_w4a8(const w4_packed_mx_view& w, const w4_act_mx8_view& x, w4_half* c,
                                hipStream_t s);
+// Which kernel they take with arrays aligned to 16 bytes (x8: E4M3 activations): see w4_gemm_mx_plan_for.
+int mx_plan(bool x8, int M, int N, int K);
 hipError_t launch_quantize_mx8(const void* src, int src_f16, long long rows, int K, uint8_t* q,
                                uint8_t* scales, int* status, hipStream_t s);
 hipError_t launch_fill_words(uint32_t* p, long long n, uint32_t value, hipStream_t s);
