@@ -5,10 +5,11 @@ No kernel may use scratch memory: an instantiation that spills registers runs se
 times slower than the next smaller one that fits (a scale pick that the compiler put in
 scratch cost 1.8 us of a 10.5 us call once), so the launchers cap what they ask for at
 what fits and do not compile the rest -- this test is what keeps the two in step.  The
-vector GEMM kernel that writes registers with hand-placed loads and waits must not have
+kernels that write registers with hand-placed loads and waits must not have
 any of them parked in the AGPR half of the register file either: the compiler does not
 know when such a register lands, and a copy made before the wait copies stale bits."""
 import os
+import re
 import subprocess
 import sys
 
@@ -52,9 +53,13 @@ def test_no_kernel_uses_scratch_memory(kernels):
 
 
 def test_asm_loaded_registers_are_never_parked(kernels):
+    """(also flash decode with tiles through LDS: query rows and slab scales are loaded ahead of the wait
+    that covers them)"""
     rows4 = [k for k in kernels if "simt_rows4_kernel" in k[".name"]]
+    flash = [k for k in kernels if re.search(r"flash_mfma_phase1ILi\dELi\d+ELb\dELi\dELb\dELb1EE", k[".name"])]
     assert rows4, "the four-rows vector kernel is missing from the library"
-    bad = [k for k in rows4 if k.get(".agpr_count", 0)]
+    assert len(flash) == 12, "W4 contiguous and paged, FP8; two head dimensions; two scale / zero-point forms"
+    bad = [k for k in rows4 + flash if k.get(".agpr_count", 0) or k.get(".vgpr_spill_count", 0)]
     assert not bad, "\n".join(_demangle([k[".name"] for k in bad]))
 
 

@@ -28,8 +28,10 @@ ATT = [(1, 1, 64, 32), (2, 7, 64, 8), (4, 128, 128, 128), (2, 300, 96, 32), (3, 
        # output itself and touches no scratch)
        (2, 512, 128, 32), (2, 513, 128, 32), (1, 512, 64, 16), (2, 400, 128, 64)]
 BIG = [(2, 5000, 64, 32), (1, 9000, 128, 64)]
-# more slabs than workgroups wanted: one split per slab, 9 to 11 tiles per wave
-LONG_SPLITS = [(520, 1300, 128, 32), (600, 1100, 64, 32)]
+# more slabs than workgroups wanted: one split per slab; 9 to 11 tiles per wave (through LDS), 13 and 14 (through
+# registers: W4 at both head dimensions, FP8 with D = 64), each with a cut tile at the end
+LONG_SPLITS = [(520, 1300, 128, 32), (600, 1100, 64, 32), (520, 1715, 128, 32), (520, 1605, 64, 32)]
+LONG_ROUTES = [2, 2, 1, 1]
 
 
 def _w4_case(H, S, D, gs, sym, seed, group=1):
@@ -123,9 +125,12 @@ def test_f8_flash(i):
     _check_f8(H, S, D, gs, k, v, q)
 
 
-def test_f8_flash_long_splits():
-    """Splits of 6 and more tiles per wave: the loop that only sees whole tiles."""
-    H, S, D, gs = LONG_SPLITS[0]
+@pytest.mark.parametrize("i", [0, 3])
+def test_f8_flash_long_splits(i):
+    """Splits of 6 and more tiles per wave: the loops over whole tiles, through LDS and (in registers) the one
+    that sees no others."""
+    H, S, D, gs = LONG_SPLITS[i]
+    assert w4amd.capi().flash_plan_for(2, H, 1, S, D, gs)[3] == LONG_ROUTES[i]
     rng = np.random.default_rng(0xF81B)
     k, v = rng.standard_normal(H * S * D), rng.standard_normal(H * S * D)
     _check_f8(H, S, D, gs, k, v, orc.normal_activations(H * D, 0xF81C))
@@ -286,18 +291,21 @@ def test_paged_equals_contiguous(i, sym):
 @pytest.mark.parametrize("sym", [True, False], ids=["sym", "asym"])
 @pytest.mark.parametrize("i", range(len(LONG_SPLITS)))
 def test_w4_flash_long_splits(i, sym):
-    """So many slabs that each gets one or two splits: a wave walks 6 and more tiles,
-    which takes the loop that only sees whole tiles (its look-ahead of the page
-    table included), then the loop for the cut tiles at the end."""
+    """So many slabs that each gets one split: a wave walks 9 to 14 tiles, through LDS
+    or through registers.  The latter takes the loop that only sees whole tiles (its look-ahead of
+    the page table included), then the loop for the cut tiles at the end; pages of 48 rows are no
+    power of two, pages of 24 no multiple of a half tile either (registers always)."""
     c = w4amd.capi()
     H, S, D, gs = LONG_SPLITS[i]
+    assert c.flash_plan_for(1, H, 1, S, D, gs)[0::3] == (1, LONG_ROUTES[i])
     seed = 0x10E6 ^ (i * 977 + (0 if sym else 1))
     rng = np.random.default_rng(seed)
     k, v = rng.standard_normal(H * S * D), rng.standard_normal(H * S * D)
     c4 = orc.quantize_cache(k, v, H, S, D, gs, sym)
     q = orc.normal_activations(H * D, seed + 2)
     o_w4, dk, q_d, kd, vd, ref = _check_w4(c4, q)
-    for page in (16, 48):
+    for page in (16, 48, 24):
+        assert c.flash_plan_for(1, H, 1, S, D, gs, page)[3] == (1 if page == 24 else LONG_ROUTES[i])
         npages = (S + page - 1) // page
         bt = np.random.default_rng(seed ^ page).permutation(npages).astype(np.int32)
         keep, view = _paged_pool(c4, page, bt)

@@ -23,10 +23,9 @@ SHAPES = [(1, 64, 512), (16, 256, 4096), (5, 100, 1000), (3, 48, 100), (33, 80, 
           (1, 16, 8), (200, 200, 200),
           # a few hundred rows on the skinny kernel's grid.y walk
           (128, 256, 512), (96, 64, 128), (200, 300, 1024), (300, 520, 384), (129, 257, 256),
-          # many rows of X on the skinny kernel's grid.y walk (too few tiles for the tiled kernel)
-          (384, 256, 512), (500, 300, 1024), (385, 520, 256),
-          # K % 256 == 0 and at least 64 tiles of 256 x 128: the LDS-tiled kernel, ragged on both
-          # sides, 2 to 5 stages of 256 k
+          # many rows of X on the skinny kernel's grid.y walk (too few tiles, or no whole stages of 256 k)
+          (384, 256, 512), (500, 300, 1024), (385, 520, 256), (500, 300, 992), (385, 520, 320),
+          # several rounds' worth of eight-wave tiles, ragged on both sides, 2 to 5 stages of 256 k
           (900, 2100, 512), (1030, 2050, 768), (1024, 2048, 1280)]
 
 
@@ -163,7 +162,8 @@ def test_w4a4_prefill_shape_sampled_rows():
 # ---- W4A8: MXFP4 weights against MXFP8 (E4M3, block-scaled) activations ---------------
 W4A8_SHAPES = [(1, 64, 512), (16, 256, 4096), (5, 100, 992), (33, 80, 640), (64, 128, 1024),
                (100, 64, 512), (2, 33, 32), (48, 16, 96), (300, 520, 384),
-               # at least 64 tiles and K % 256 == 0: the LDS-tiled kernel with 8-bit X
+               (500, 300, 992), (385, 520, 320),
+               # eight-wave tiles, ragged on both sides
                (900, 2100, 512), (1030, 2050, 768), (1024, 2048, 1280)]
 
 
@@ -315,6 +315,20 @@ def test_w4a4_activation_quantizer_ties_and_boundaries():
 @pytest.mark.parametrize("K,shift", [(256, 0), (768, 0), (1536, 0), (1536, 8)])
 @pytest.mark.parametrize("M,N", [(70, 4100), (390, 4100), (610, 4100), (900, 4000)])
 def test_eight_wave_tiles(M, N, K, shift, x8):
+    assert w4amd.capi().gemm_mx_plan_for(x8, M, N, K) in (1, 2, 3, 4)
+    _product_of_random_codes(M, N, K, shift, x8)
+
+
+# The 256 x 128 tiles, ragged in M and N: one stage of 256 k, odd and even numbers of them.
+@pytest.mark.parametrize("x8", [False, True])
+@pytest.mark.parametrize("M,N,K,shift", [(2030, 4090, 256, 0), (2030, 4090, 512, 0), (2030, 4090, 768, 8),
+                                         (2041, 4089, 1280, 0), (4000, 4090, 512, 8)])
+def test_large_tiles(M, N, K, shift, x8):
+    assert w4amd.capi().gemm_mx_plan_for(x8, M, N, K) == 8
+    _product_of_random_codes(M, N, K, shift, x8)
+
+
+def _product_of_random_codes(M, N, K, shift, x8):
     c = w4amd.capi()
     rng = np.random.default_rng(M + K)
     B = K // 32
