@@ -102,6 +102,16 @@ def test_flash_long_splits_keep_tiles_in_registers():
     assert len(seen) == 8
 
 
+def test_flash_partials_stay_inside_the_fixed_scratch():
+    """Calls whose partials fit the array of the entry that allocates nothing with fewer splits are not
+    split beyond it (260 slabs x 16 heads: one split of 4096 positions)."""
+    capi = w4amd.capi()
+    for H, group, S, D in [(260, 16, 4096, 128), (88, 48, 1300, 64), (91, 64, 2048, 64), (300, 11, 4096, 128),
+                           (200, 24, 1500, 128)]:
+        splits = capi.flash_plan_for(1, H, group, S, D, 32)[0]
+        assert H * group * splits * (D + 2) * 4 <= 4 << 20, (H, group, S, D, splits)
+
+
 def test_flash_plan_of_many_heads():
     """More than 12 query heads per slab: from four splits on a kernel of its own merges them."""
     capi = w4amd.capi()

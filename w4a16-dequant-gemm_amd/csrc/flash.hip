@@ -369,7 +369,7 @@ __global__ __launch_bounds__(P2_THREADS) void flash_phase2(const float* __restri
 //   the merge by the last workgroup 1.5 (+ 0.7 per further four heads), by a second kernel 3 + 0.03 per split, none 0.
 // Before this rule splits were multiples of 256 positions and aimed at 512 workgroups: 32 x 6007 FP8
 // 19.4 -> 15.2 us, 128 x 1500 W4 pages 12.7 -> 11.4, 32 x 3000 FP16 18.4 -> 14.0, 8 x 600 W4 6.7 -> 6.1.
-static float split_cost(const FlashArgs& a, int t, int nsplit) {
+static float split_cost(const FlashArgs& a, int t, int nsplit, bool coarse) {
   const float T = (a.kind == KIND_W4 ? 1.0f : a.kind == KIND_F8 ? 1.4f : 2.5f) * (a.D == 64 ? 0.7f : 1.0f);
   const long long wgs = (long long)a.H * nsplit;
   float c;
@@ -377,22 +377,28 @@ static float split_cost(const FlashArgs& a, int t, int nsplit) {
   else if (a.kind == KIND_F16) c = (float)((wgs + 255) / 256) * (1.2f + T * t);
   else {
     const float x = (float)wgs / 512, F = a.kind == KIND_W4 ? 1.25f : a.D == 64 ? 1.5f : 1.8f;
-    c = 1.7f * (float)((wgs + 511) / 512) + F * T * t * (x <= 1.0f ? 1.0f : x + 0.3f);
+    const float rounds = (float)((wgs + 511) / 512);
+    c = 1.7f * rounds + F * T * t * (coarse || x <= 1.0f ? rounds : x + 0.3f);
   }
+  const bool in_place = flash_merges_in_place(a, FlashPlan{128 * t, nsplit}) ||
+                        (coarse && a.H <= 512 && a.group > 12 && nsplit <= 4 && min(a.group, 16) * nsplit <= 64);
   if (nsplit > 1)
-    c += flash_merges_in_place(a, FlashPlan{128 * t, nsplit}) ? 1.5f + 0.7f * ((a.group - 1) / 4) : 3.0f + 0.03f * nsplit;
+    c += in_place ? 1.5f + 0.7f * ((a.group - 1) / 4) : 3.0f + 0.03f * nsplit;
   return c;
 }
 
-static FlashPlan mfma_plan(const FlashArgs& a) {
+// coarse: the estimate with whole rounds only, which splits less: begun ones count as whole, merging 16 heads of
+// four splits costs what it does in place, and nothing is split past one round.
+static FlashPlan mfma_plan(const FlashArgs& a, bool coarse) {
   const int tiles = (a.S + 127) / 128;
   // nothing is gained by more than two rounds of two workgroups per compute unit (512) or less than half a round
-  const int one = (int)(((long long)tiles * a.H + 511) / 512), lo = (one + 1) / 2, hi = one * 2 + 4;
+  const int one = (int)(((long long)tiles * a.H + 511) / 512), lo = coarse ? one : (one + 1) / 2,
+            hi = one * 2 + 4;
   FlashPlan best{128 * tiles, 1};
-  float cost = split_cost(a, tiles, 1);
+  float cost = split_cost(a, tiles, 1, coarse);
   for (int t = lo < 1 ? 1 : lo; t <= hi && t < tiles; ++t) {
     const int n = (tiles + t - 1) / t;
-    const float c = split_cost(a, t, n);
+    const float c = split_cost(a, t, n, coarse);
     if (c < cost) cost = c, best = FlashPlan{128 * t, n};
   }
   return best;
@@ -405,9 +411,10 @@ FlashPlan flash_plan(const FlashArgs& a) {
   // arrival counters: such calls may overlap on different streams, and they keep that.  (Three or four
   // splits of 8 - 64 slabs would be ahead: 8 slabs x 384 - 512 positions, W4, by about 0.5 us of 6.)
   if (mfma && a.S <= FL_DIRECT_MAX_S) return FlashPlan{(a.S + 127) / 128 * 128, 1};
-  if (mfma) {
-    const FlashPlan p = mfma_plan(a);
-    // (partials that fit the built-in scratch with the longer splits below have to fit it here)
+  // (partials that fit the built-in scratch with fewer or longer splits have to fit it here)
+  for (const bool coarse : {false, true}) {
+    if (!mfma) break;
+    const FlashPlan p = mfma_plan(a, coarse);
     if (floats(p) * sizeof(float) <= W4_NOALLOC_SCRATCH_BYTES) return p;
   }
   // Enough workgroups to fill 256 CUs, but splits no shorter than one tile; a
