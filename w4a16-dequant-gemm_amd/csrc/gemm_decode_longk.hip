@@ -127,8 +127,10 @@ constexpr LkSched<CH * MT> lk_schedule() {
 // those columns are computed from whatever the buffer holds).  Every workgroup fetches all
 // of x out of L2, so rows that do not exist cost time: with three row tiles for 33 to 48 rows
 // and half of the fourth for 49 to 56, N = 4096, K = 14336, MXFP4: M = 33 26.3 -> 22.8 us, 48 26.7 -> 24.8,
-// 50 26.9 -> 26.0; N = 5120, K = 13824: M = 33 45.6 -> 38.8; W4 the same to a few per cent.  Two further
-// forms of the last tile are not compiled: a step of four rows is worth 2 %.
+// 50 26.9 -> 26.0; N = 5120, K = 13824: M = 33 45.6 -> 38.8; W4 the same to a few per cent.
+// Steps of four rows in the last tile are worth 2 % and are not compiled.  Nor is its half for 17 to 24 and 33 to 40
+// rows: 3.5 % and 2 - 4 % at N = 4096 (K = 14336, W4: 19.8 -> 19.1 and 24.4 -> 23.8 us), nothing at N = K = 8192,
+// for 1.5 MB more of library.
 // Arguments are scalars and pointers so that they arrive preloaded in SGPRs.
 template <int FMT, int CH, int MT, int NQ>
 __global__ __launch_bounds__(LK_THREADS) void mfma_decode_longk_kernel(
