@@ -25,17 +25,17 @@ SHAPES = [(W4, 1, 16384, 128, 1, True, 0, 64, True),    # 64 splits, one per lan
           (W4, 4, 4000, 128, 5, False, 0, 32, False),   # more
           (W4, 4, 4000, 128, 4, True, 16, 16, True),
           (W4, 8, 600, 64, 7, True, 0, 5, True),        # few splits, heads that do not divide over the waves
-          (W4, 130, 1280, 128, 17, True, 0, 3, True),    # two passes over the heads, one after the other
+          (W4, 80, 650, 128, 17, True, 0, 3, True),    # two passes over the heads, one after the other
           (W4, 60, 1000, 128, 19, True, 0, 4, False),   # more than 12 heads in a pass: up to three splits
           (W4, 130, 700, 128, 2, False, 48, 3, True),   # a slab count past one per compute unit and XCD round
           (F8, 1, 16384, 64, 1, True, 0, 64, True),
           (F8, 4, 4000, 128, 4, True, 0, 16, True),
           (F8, 4, 4000, 128, 5, True, 0, 32, False),
-          (F8, 130, 1280, 128, 17, True, 0, 3, True),
+          (F8, 100, 600, 128, 17, True, 0, 3, True),
           (F16, 1, 16384, 128, 1, True, 0, 64, True),
           (F16, 4, 4000, 128, 4, True, 0, 32, False),
           (F16, 8, 600, 64, 7, True, 0, 5, True),
-          (F16, 130, 1280, 128, 17, True, 0, 3, True)]
+          (F16, 100, 600, 128, 17, True, 0, 3, True)]
 
 
 class _Case:
