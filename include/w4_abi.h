@@ -179,8 +179,8 @@ int w4_attention_w4_flash_paged_batched(const w4_kv_view* p, const int* bt,
  * in the reference): kind 0 FP16, 1 W4, 2 FP8 with a scale per row; H slabs in all; gs ignored for FP16;
  * page 0 for a contiguous cache; cache and scale arrays aligned to 16 bytes.
  * plan[0]: splits per slab -- with 1 the call uses no memory but its arguments', so it may overlap with
- *          others on other streams (every cache of up to 512 positions with D = 64 or 128 and, when
- *          quantized, gs a multiple of D / 4);
+ *          others on other streams (with D = 64 or 128 and, when quantized, gs a multiple of D / 4:
+ *          every cache of up to 512 positions, and every call of 512 slabs and more);
  * plan[1]: positions per split;  plan[2]: 1 if there is no second launch that merges them;
  * plan[3]: 0 vector kernel, 1 matrix cores with tiles through registers, 2 through LDS. */
 int w4_flash_plan_for(int kind, int H, int group, int S, int D, int gs, int page, int* plan);

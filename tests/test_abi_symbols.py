@@ -57,8 +57,8 @@ def test_validation_runs_without_a_device():
 
 
 def test_flash_plan_of_short_caches_shares_nothing():
-    """Caches of up to 512 positions on the matrix cores: one split per slab, so neither scratch nor
-    arrival counters are touched and calls on several streams may overlap."""
+    """Caches of up to 512 positions, and 512 slabs and more, on the matrix cores: one split per slab, so
+    neither scratch nor arrival counters are touched and calls on several streams may overlap."""
     capi = w4amd.capi()
     for kind in (0, 1, 2):
         for D, gs in ((64, 32), (128, 32), (128, 128)):
@@ -67,6 +67,9 @@ def test_flash_plan_of_short_caches_shares_nothing():
                     for S in (1, 127, 128, 300, 384, 511, 512):
                         splits, length, direct, route = capi.flash_plan_for(kind, H, group, S, D, gs)
                         assert (splits, direct) == (1, 1) and length >= S and route >= 1, (kind, H, group, S, D)
+            for H in (512, 520, 560, 608, 700, 1030):
+                for S in (513, 1500, 4096, 6000, 32768):
+                    assert capi.flash_plan_for(kind, H, 4, S, D, gs)[0] == 1, (kind, H, S, D, gs)
     for bad in [(3, 8, 1, 100, 128, 32), (1, 8, 65, 100, 128, 32), (1, 8, 1, 100, 128, 12), (1, 0, 1, 100, 128, 32),
                 (0, 8, 1, 100, 128, 32, 16)]:
         with pytest.raises(ValueError):

@@ -407,10 +407,10 @@ static FlashPlan mfma_plan(const FlashArgs& a, bool coarse) {
 FlashPlan flash_plan(const FlashArgs& a) {
   const auto floats = [&](const FlashPlan& p) { return (size_t)a.H * a.group * p.nsplit * (a.D + 2); };
   const bool mfma = flash_mfma_applies(a);
-  // Up to 512 positions one split per slab, which touches neither the shared scratch nor the
-  // arrival counters: such calls may overlap on different streams, and they keep that.  (Three or four
+  // Up to 512 positions, and from 512 slabs on, one split per slab, which touches neither the shared scratch nor
+  // the arrival counters: such calls may overlap on different streams, and they keep that.  (Three or four
   // splits of 8 - 64 slabs would be ahead: 8 slabs x 384 - 512 positions, W4, by about 0.5 us of 6.)
-  if (mfma && a.S <= FL_DIRECT_MAX_S) return FlashPlan{(a.S + 127) / 128 * 128, 1};
+  if (mfma && (a.S <= FL_DIRECT_MAX_S || a.H >= FL_DIRECT_MIN_H)) return FlashPlan{(a.S + 127) / 128 * 128, 1};
   // (partials that fit the built-in scratch with fewer or longer splits have to fit it here)
   for (const bool coarse : {false, true}) {
     if (!mfma) break;

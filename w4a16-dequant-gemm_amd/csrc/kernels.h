@@ -106,6 +106,7 @@ enum { KIND_F16 = 0, KIND_W4 = 1, KIND_F8 = 2 };  // FlashArgs::kind
 
 // Split of the sequence over workgroups (shared by both phase-1 kernels).
 constexpr int FL_DIRECT_MAX_S = 512;  // longest cache that always has one split per slab (matrix-core kernel)
+constexpr int FL_DIRECT_MIN_H = 512;  // number of slabs from which on every cache has
 struct FlashPlan {
   int split_len, nsplit;
 };
