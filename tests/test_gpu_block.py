@@ -1,0 +1,98 @@
+"""The block kernel of middle M (9 to a few hundred rows, at long K from 3 on; mma.cuh:234-260 is the reference's
+dispatch for these shapes): every block shape at the edges where it can go wrong -- rows of x and of
+W that end inside a block or a tile, K that ends inside a unit of 256 or a chunk of 128, waves
+without a unit, group sizes from 32 to a whole row.
+
+A hooked call takes the same kernel, so its output is compared byte for byte with the unhooked one;
+its weights are the oracle's bytes; the output is within 1e-3 of the FP64 oracle (the reference's
+gate, tests/test_gpu.cu:184-193)."""
+import numpy as np
+import pytest
+import torch
+
+import orc
+import w4amd
+from devutil import DevPacked, DevPackedMx, bits, halves, ptr, to_dev
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-3
+
+
+def _check(fn, view, w_ref, x, M, N, K, seed):
+    x_d, w_ref_d = to_dev(x), to_dev(w_ref)
+    # a guard row past the result and past the weights: nothing is written behind them
+    c_h, c_u, w_d = halves(M * N + N, 0x7E00), halves(M * N + N, 0x7E00), halves(N * K + 64, 0x7E00)
+    fn(view, ptr(x_d), ptr(c_h), M, 0, ptr(w_d))
+    fn(view, ptr(x_d), ptr(c_u), M, 0, 0)
+    assert torch.equal(w_d[: N * K], w_ref_d), "w_out bitwise"
+    assert bool((w_d[N * K:] == 0x7E00).all()) and bool((c_u[M * N:] == 0x7E00).all())
+    assert torch.equal(c_h, c_u), "hooked and unhooked calls are one kernel"
+    rng = np.random.default_rng(seed)
+    ms = np.unique(np.concatenate([[0, min(15, M - 1), min(16, M - 1), M - 1], rng.choice(M, size=min(M, 24), replace=False)]))
+    ns = np.unique(np.concatenate([[0, 15, N - 1], rng.choice(N, size=min(N, 160), replace=False)]))
+    ref = orc.gemm_oracle(np.ascontiguousarray(x.reshape(M, K)[ms]), len(ms), K,
+                          np.ascontiguousarray(w_ref.reshape(N, K)[ns]), len(ns))
+    got = np.ascontiguousarray(bits(c_u)[: M * N].reshape(M, N)[ms][:, ns]).view(np.float16)
+    assert orc.rel_l2(got, ref) <= TOL
+
+
+# (M, N, K): which block the planner picks on 256 compute units
+SHAPES = [
+    (3, 528, 4352),     # one tile of W a workgroup, half a unit at the end of some waves
+    (16, 4096, 2304),   # the same, whole tiles of x; the last wave has one unit
+    (9, 8208, 4384),    # 64 x 16 blocks at the resident kernel's widths, ragged N and K
+    (17, 272, 256),     # one unit: seven waves have none; N ends inside a block
+    (33, 528, 4096),    # two tiles of x, the third row of tiles one row high
+    (48, 2064, 2336),   # K ends inside a chunk, in a unit of its own
+    (100, 4096, 1152),  # 32 x 64 blocks; half a unit at the end
+    (128, 6144, 512),   # 48 x 64 blocks
+    (96, 8208, 1024),   # 64 x 32 and larger blocks, ragged N
+    (190, 4112, 2304),  # 64 x 64
+    (150, 11008, 2048), # 64 x 80
+    (333, 4080, 2176),  # 64 x 96, rows end inside a block
+]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("gs,sym", [(128, True), (64, False), (32, True), (32, False), (0, False)])
+def test_w4_block(M, N, K, gs, sym):
+    if gs == 0:
+        gs = K  # one group per row
+    c = w4amd.capi()
+    seed = M + N + K + gs + sym
+    w = orc.normal_weights(N * K, seed) * 0.02
+    if not sym:
+        w = w + 0.01  # off-centre groups: zero-points away from 8
+    p = orc.quantize(w, N, K, gs, sym)
+    w_ref = orc.dequant_all(p)
+    x = orc.normal_activations(M * K, seed + 1)
+    dp = DevPacked(p)
+    _check(c.gemm, dp.view, w_ref, x, M, N, K, seed)
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_mxfp4_block(M, N, K):
+    c = w4amd.capi()
+    seed = M + N + K
+    p = orc.quantize_mx(orc.outlier_weights(N, K, seed), N, K)
+    w_ref = orc.dequant_all_mx(p)
+    x = orc.normal_activations(M * K, seed + 1)
+    dp = DevPackedMx(p)
+    _check(c.gemm_mx, dp.view, w_ref, x, M, N, K, seed)
+
+
+def test_block_shapes_add_in_one_order():
+    """Rows at which the planner goes through blocks of 16 x 16 up to 64 x 96: K is split over the waves
+    in the same way in all of them, so a row of the product has the same bytes in every call."""
+    c = w4amd.capi()
+    K, N = 4096, 2048
+    p = orc.quantize(orc.normal_weights(N * K, 9) * 0.02, N, K, 128, True)
+    x = orc.normal_activations(600 * K, 10)
+    dp, x_d = DevPacked(p), to_dev(x)
+    full = None
+    for M in (600, 448, 320, 200, 128, 100, 64, 32, 17, 9):
+        out = halves(M * N, 0x7E00)
+        c.gemm(dp.view, ptr(x_d), ptr(out), M, 0, 0)
+        got = bits(out).reshape(M, N)
+        full = got if full is None else full
+        assert np.array_equal(got, full[:M]), M

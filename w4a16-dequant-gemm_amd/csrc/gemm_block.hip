@@ -1,0 +1,497 @@
+// W4A16 / MXFP4 GEMM for middle M (9 to a few hundred rows, at long K from 3 on): a workgroup owns a block of
+// 16 NT rows of W x 16 MT activation rows, its eight waves split K.  mma.cuh:63-230 is the
+// reference's kernel for this path.
+//
+// What bounds these shapes is the path from L2 into a compute unit: it takes 1 KB per 7 - 10 ns
+// whatever lies in it, as long as the 4 (better 8) neighbouring lanes of a load instruction lie in
+// one line; a load in MFMA operand layout (neighbouring lanes in different rows) takes 28 ns.  So
+//   * the block is as square as the operands' sizes ask for: per k a workgroup moves 8 NT bytes of codes
+//     and 32 MT bytes of activations, N = 4096, M = 64: 64 B with 64 x 16 blocks against 136 with one
+//     16-row tile of W per workgroup and all of x;
+//   * both operands come as whole lines by global_load_lds_dwordx4 into LDS that belongs to one
+//     wave, are read back into registers in operand layout (XOR-swizzled, conflict-free) and their
+//     place is requested again at once, so that the whole LDS is on its way while the wave expands
+//     and multiplies.  Waves meet only at the two ends: group parameters of the block's rows are
+//     copied into LDS first, and the waves' sums are added in wave order last.
+// Workgroups that share rows of W are neighbours on one XCD, whose L2 then gets them once.
+#include <atomic>
+#include <type_traits>
+#include <utility>
+
+#include "dq.cuh"
+#include "kernels.h"
+
+namespace w4k {
+namespace {
+
+// (the compiler takes lambdas this large out of line, with their registers in scratch memory)
+#define BK_INLINE __attribute__((always_inline))
+
+typedef __attribute__((address_space(3))) void* lds_ptr;
+constexpr int BK_WAVES = 8, BK_THREADS = 64 * BK_WAVES;
+constexpr int BK_UNIT = 256;  // k of a unit: one 128-byte line of a row of codes, two of a row of x
+constexpr int BK_XS = 2;      // pieces in a wave's ring of x
+constexpr int bk_wave_bytes(int NT, int XS) { return NT * 2048 + XS * 4096; }
+constexpr int bk_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
+extern __shared__ __attribute__((aligned(16))) uint8_t bk_lds[];
+
+__device__ __forceinline__ h8 bk_expand(uint32_t w, h2 cneg, h2 s2, uint32_t mask, uint32_t magic) {
+  u4 out;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t p = __builtin_amdgcn_perm(0u, w, 0x0c000c00u | (uint32_t)(i << 16) | (uint32_t)i);
+    const uint32_t v = (p & mask) | magic;
+    out[i] = as_u32((as_h2(v) + cneg) * s2);
+  }
+  return __builtin_bit_cast(h8, out);
+}
+
+// f(integral_constant<int, 0>), f(integral_constant<int, 1>), ...: a loop whose index is
+// a constant expression inside the body (wait counts are instruction immediates)
+template <class F, int... I>
+__device__ __forceinline__ void bk_for(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+__device__ __forceinline__ void bk_dma(uint32_t off, const void* base, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(dst) : "memory", "m0");
+}
+
+// FMT: 0 W4 symmetric, 1 W4 with zero-points, 2 MXFP4.  G: groups (W4) or blocks (MXFP4) per row.
+// gs_shift: log2(gs) if gs is a power of two, else -1.  mgroups: blocks along M.  XS: pieces of x (16 rows x 128 k, 4 KB) in a
+// wave's ring; three measured no better than two.
+template <int FMT, int NT, int MT, int XS, bool AHEAD>
+__global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
+    const uint32_t* __restrict__ q, const void* __restrict__ scales, const uint32_t* __restrict__ zeros,
+    const w4_half* __restrict__ x, w4_half* __restrict__ c, const int N, const int K, const int M,
+    const int gs_shift, const int G, const int gs, const int mgroups, w4_half* __restrict__ w_out) {
+  constexpr bool MX = FMT == 2;
+  constexpr int WB = bk_wave_bytes(NT, XS), ROWS = 16 * NT, NP = 2 * MT;
+  // Step of a unit at which its codes have been read back and the next unit's are requested: with
+  // many row tiles one chunk's codes are read at a time (registers).
+  constexpr int PC = !AHEAD && MT >= 3 ? MT : 0;
+  static_assert(XS >= 2 && XS <= (PC ? MT : NP), "a unit's first piece is requested after its codes");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, b = lane >> 4;
+  const int local = (int)(blockIdx.x >> 3);
+  const int n0 = ((int)(blockIdx.x & 7) + 8 * (local / mgroups)) * ROWS, m0 = (local % mgroups) * (16 * MT);
+  if (n0 >= N) return;
+  const int units = (K + BK_UNIT - 1) / BK_UNIT;
+  const uint32_t wrow = (uint32_t)(K >> 1), xrow = (uint32_t)(K * 2);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)bk_lds;
+  const uint32_t region = lds0 + (uint32_t)wave * WB;
+  uint8_t* const mine = bk_lds + wave * WB;
+  uint8_t* const params = bk_lds + BK_WAVES * WB;
+
+  // ---- group parameters of the block's rows: one contiguous run each, 1 KB a load ----
+  const int live = min(ROWS, N - n0);
+  const int pb = live * G * (MX ? 1 : 2), wg = words(G), zb = live * wg * 4;
+  const int zoff = (ROWS * G * (MX ? 1 : 2) + 1023) & ~1023;
+  {
+    const char* ps = (const char*)scales + (size_t)n0 * G * (MX ? 1 : 2);
+    for (int o = wave * 1024; o < pb; o += BK_WAVES * 1024)
+      bk_dma((uint32_t)min(o + lane * 16, pb - 16), ps, lds0 + BK_WAVES * WB + o);
+    if (FMT == 1) {
+      const char* pz = (const char*)zeros + (size_t)n0 * wg * 4;
+      for (int o = wave * 1024; o < zb; o += BK_WAVES * 1024)
+        bk_dma((uint32_t)min(o + lane * 16, zb - 16), pz, lds0 + BK_WAVES * WB + zoff + o);
+    }
+  }
+
+  // ---- requests ----
+  // codes of a unit: 2 NT loads of 8 rows x 128 bytes; lane l: row l / 8, piece (l % 8) ^ key, key = (row of the
+  // tile / 2) % 8, so that the 16 rows a piece is read back from lie in 16 distinct groups of banks.  A tile past
+  // N (whole ones: N is a multiple of 16) repeats the block's first.
+  // (In both requests the pieces past the end of a row, which only the last unit has, are a branch of
+  // their own: as selects they were a third of the loop's vector instructions.)
+  uint32_t cpiece[2], coff[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int row = 8 * h + (lane >> 3);
+    cpiece[h] = (uint32_t)(((lane & 7) ^ (row >> 1)) & 7) * 16;
+    coff[h] = (uint32_t)row * wrow + cpiece[h];
+  }
+  const char* const qb = (const char*)q + (size_t)n0 * wrow;
+  auto request_codes = [&](int U) BK_INLINE {
+    const bool tail = (U + 1) * BK_UNIT > K;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const char* base = qb + (16 * t < live ? (size_t)(16 * t) * wrow : 0) + (size_t)U * 128;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        uint32_t o = coff[h];
+        if (tail) {  // the unit's first piece instead
+          if ((uint32_t)U * 128 + cpiece[h] >= wrow) o -= cpiece[h];
+          asm volatile("" : "+v"(o) : : "memory");
+        }
+        bk_dma(o, base, region + (2 * t + h) * 1024u);
+      }
+    }
+  };
+  // piece p = (chunk p / MT of the unit, row tile p % MT): 4 loads of 4 rows x 256 bytes, piece (l % 16) ^ (row % 16)
+  const char* const xb = (const char*)x + (size_t)m0 * xrow;
+  const int mlast = M - 1 - m0;
+  constexpr int XO = MT <= 4 ? MT : 0;  // offsets worked out once, where registers allow
+  uint32_t xoff[XO ? XO : 1][4];
+#pragma unroll
+  for (int mt = 0; mt < XO; ++mt)
+#pragma unroll
+    for (int rq = 0; rq < 4; ++rq) {
+      const int r16 = 4 * rq + (lane >> 4);
+      xoff[mt][rq] = (uint32_t)min(16 * mt + r16, mlast) * xrow + (uint32_t)(((lane & 15) ^ r16) * 16);
+    }
+  auto request_x = [&](int U, int p, int slot) BK_INLINE {
+    const int ch = p / MT, mt = p % MT;
+    const uint32_t k2 = (uint32_t)(U * 2 + ch) * 256u;  // byte of the row
+    const uint32_t dst = region + NT * 2048u + (uint32_t)slot * 4096u;
+    auto offset = [&](int rq) BK_INLINE {
+      const int r16 = 4 * rq + (lane >> 4);
+      return XO ? xoff[XO ? mt : 0][rq]
+                : (uint32_t)min(16 * mt + r16, mlast) * xrow + (uint32_t)(((lane & 15) ^ r16) * 16);
+    };
+    if (k2 + 256 > xrow) {
+      asm volatile("" ::: "memory");
+      const bool past = k2 >= xrow;  // all of the chunk: the chunk before instead
+      const char* base = xb + (past ? k2 - 256 : k2);
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq) {
+        const uint32_t piece = (uint32_t)(((lane & 15) ^ (4 * rq + (lane >> 4))) * 16);
+        bk_dma(offset(rq) - (past || k2 + piece >= xrow ? piece : 0u), base, dst + rq * 1024u);
+      }
+    } else {
+      const char* base = xb + k2;
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq) bk_dma(offset(rq), base, dst + rq * 1024u);
+    }
+  };
+
+  const int nu = (units - wave + BK_WAVES - 1) / BK_WAVES;  // wave w takes units w, w + 8, ...
+  if (nu > 0) {
+    request_codes(wave);
+#pragma unroll
+    for (int p = 0; p < XS; ++p) request_x(wave, p, p);
+    __builtin_amdgcn_s_waitcnt(bk_vm(2 * NT + 4 * XS));
+  } else {
+    __builtin_amdgcn_s_waitcnt(bk_vm(0));
+  }
+  asm volatile("s_barrier" ::: "memory");  // the parameters are there
+
+  uint32_t mask = 0x00F0000Fu, magic = 0x54006400u;
+  asm volatile("" : "+s"(mask));   // opaque: as literals they cost two instructions
+  asm volatile("" : "+v"(magic));  // instead of one and-or
+  f4 acc[NT][MT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f4{0.f, 0.f, 0.f, 0.f};
+  u4 cw[PC ? 1 : 2][NT];
+  h8 A[NT][4];
+  uint32_t sc[NT], zw[NT];  // group parameters of a lane's 32 k of a chunk, and their group
+  int g = 0, slot = 0;      // slot: of the piece that is multiplied
+  const bool hook = w_out && m0 == 0;
+
+  auto read_codes = [&](int h, u4* w) BK_INLINE {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      w[t] = *(const u4*)(mine + t * 2048 + r * 128 + (((4 * h + b) ^ (r >> 1)) & 7) * 16);
+  };
+  auto read_x = [&](int at, h8* v) BK_INLINE {  // B operands: MFMA j contracts k = 128 chunk + 32 b + 8 j .. + 7 = piece 4 b + j
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      v[j] = *(const h8*)(mine + NT * 2048 + at * 4096 + (r >> 2) * 1024 + ((r & 3) * 16 + ((4 * b + j) ^ r)) * 16);
+  };
+  auto read_params = [&](int chunk) BK_INLINE {
+    const int kc = min(chunk * 128 + 32 * b, K - 32);
+    g = MX ? (kc >> 5) : gs_shift >= 0 ? (kc >> gs_shift) : kc / gs;
+    const uint8_t* ps = params + (r * G + g) * (MX ? 1 : 2);
+    const uint8_t* pz = params + zoff + (r * wg + (g >> 3)) * 4;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (MX) sc[t] = ps[t * 16 * G];
+      else sc[t] = *(const uint16_t*)(ps + t * 32 * G);
+      if (FMT == 1) zw[t] = *(const uint32_t*)(pz + t * 64 * wg);
+    }
+  };
+  auto request_next = [&](auto pc, int U, bool more) BK_INLINE {  // into the places that are free at step p of unit U
+    constexpr int p = decltype(pc)::value;
+    if (p == PC && more) request_codes(U + BK_WAVES);
+    if (p + XS < NP) request_x(U, p + XS, slot);
+    else if (more) request_x(U + BK_WAVES, p + XS - NP, slot);
+    slot = slot + 1 < XS ? slot + 1 : 0;
+  };
+  // the codes in w, with the parameters given, become the weights of a chunk; k: the lane's first
+  auto expand = [&](const u4* w, const uint32_t* scale, const uint32_t* zword, int group, int k) BK_INLINE {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      h2 cneg, s2;
+      float sf = 0.f;
+      if (MX) {
+        sf = mx_scale(scale[t]);
+      } else {
+        const uint32_t z = FMT == 1 ? ((zword[t] >> (4 * (group & 7))) & 0xFu) : 8u;
+        cneg = as_h2(0xD400E400u | (z << 20) | z);
+        s2 = splat_bits(scale[t]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (MX) {
+          h2 n4[4];
+          dq_mx(w[t][j], sf, n4);
+          A[t][j] = __builtin_bit_cast(h8, u4{as_u32(n4[0]), as_u32(n4[1]), as_u32(n4[2]), as_u32(n4[3])});
+        } else {
+          A[t][j] = bk_expand(w[t][j], cneg, s2, mask, magic);
+        }
+      }
+    }
+    if (hook) {  // these registers are the weights
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        if (16 * t < live && k < K) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            *(h8*)(w_out + (size_t)(n0 + 16 * t + r) * K + k + 8 * j) = A[t][j];
+        }
+    }
+  };
+  auto multiply = [&](int mt, int chunk, h8* v) BK_INLINE {
+    if (chunk * 128 + 128 > K) {  // the row ends inside this chunk: activations past it are zero
+      if (chunk * 128 + 32 * b >= K) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = __builtin_bit_cast(h8, u4{0u, 0u, 0u, 0u});
+      }
+      asm volatile("" ::: "memory");
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[t][j], v[j], acc[t][mt], 0, 0, 0);
+  };
+  auto landed = [&]() BK_INLINE {  // after a wait: what was waited for is read from here on
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  if constexpr (AHEAD) {
+    // A piece is read back while the one before it is multiplied (few row tiles: N = 4096, K = 14336, M = 64
+    // 19.7 -> 17.9 us; with larger blocks the second set of registers costs more than it gives).
+    h8 xv[2][4];
+    if (nu > 0) {
+      __builtin_amdgcn_s_waitcnt(bk_vm(4 * (XS - 1)));
+      landed();
+      read_codes(0, cw[0]), read_codes(1, cw[1]);
+      read_x(0, xv[0]);
+      read_params(2 * wave);
+    }
+    for (int U = wave; U < units; U += BK_WAVES) {
+      const bool more = U + BK_WAVES < units;
+      bk_for([&](auto pc) BK_INLINE {
+        constexpr int p = decltype(pc)::value, ch = p / MT, mt = p % MT;
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this piece is in registers and its place free
+        landed();
+        request_next(pc, U, more);
+        uint32_t scale[NT], zword[NT];
+        const int group = g;
+        if (mt == 0) {
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            scale[t] = sc[t];
+            if (FMT == 1) zword[t] = zw[t];
+          }
+        }
+        // requests younger than the next piece: the ring's others and, early in a unit, the next unit's codes
+        if (p + 1 < NP || more) {
+          constexpr int left = NP - 2 - p < 0 ? 0 : NP - 2 - p < XS - 1 ? NP - 2 - p : XS - 1;
+          if (more) __builtin_amdgcn_s_waitcnt(bk_vm(4 * (XS - 1) + (p < XS - 1 ? 2 * NT : 0)));
+          else __builtin_amdgcn_s_waitcnt(bk_vm(4 * left));
+          landed();
+          if (MT > 1 && p == NP - 1) read_codes(0, cw[0]), read_codes(1, cw[1]);
+          read_x(slot, xv[(p + 1) & 1]);
+          if (p == MT - 1) read_params(2 * U + 1);
+          if (p == NP - 1) read_params(2 * (U + BK_WAVES));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (mt == 0) expand(cw[ch], scale, zword, group, U * BK_UNIT + ch * 128 + 32 * b);
+        multiply(mt, 2 * U + ch, xv[p & 1]);
+        if (MT == 1 && p == NP - 1 && more) read_codes(0, cw[0]), read_codes(1, cw[1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }, std::make_integer_sequence<int, NP>{});
+    }
+  } else {
+    for (int U = wave; U < units; U += BK_WAVES) {
+      const bool more = U + BK_WAVES < units;
+      bk_for([&](auto pc) BK_INLINE {
+        constexpr int p = decltype(pc)::value, ch = p / MT, mt = p % MT;
+        // requests younger than the ones needed: the ring's other pieces, and next unit's codes
+        constexpr int R = XS - 1, left = NP - 1 - p < R ? NP - 1 - p : R;
+        if (more) __builtin_amdgcn_s_waitcnt(bk_vm(4 * R + (p > PC && p < PC + XS ? 2 * NT : 0)));
+        else __builtin_amdgcn_s_waitcnt(bk_vm(4 * left));
+        landed();
+        if (PC && mt == 0) read_codes(ch, cw[0]);
+        if (!PC && p == 0) read_codes(0, cw[0]), read_codes(1, cw[PC ? 0 : 1]);
+        h8 xv[4];
+        read_x(slot, xv);
+        if (mt == 0) read_params(2 * U + ch);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the places are free
+        landed();
+        request_next(pc, U, more);
+        __builtin_amdgcn_sched_barrier(0);
+        if (mt == 0) expand(cw[PC ? 0 : ch], sc, zw, g, U * BK_UNIT + ch * 128 + 32 * b);
+        multiply(mt, 2 * U + ch, xv);
+        __builtin_amdgcn_sched_barrier(0);
+      }, std::make_integer_sequence<int, NP>{});
+    }
+  }
+
+  // ---- the waves' sums, added in wave order; PH row tiles at a time, as LDS holds ----
+  constexpr int PH = (BK_WAVES * WB) / (BK_WAVES * NT * 1024) < MT ? (BK_WAVES * WB) / (BK_WAVES * NT * 1024) : MT;
+  f4* const red = (f4*)bk_lds;  // [wave][t][PH][64]
+#pragma unroll
+  for (int mb = 0; mb < MT; mb += PH) {
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < PH; ++i)
+        if (mb + i < MT) red[((wave * NT + t) * PH + i) * 64 + lane] = acc[t][mb + i];
+    __syncthreads();
+    // a thread makes 8 consecutive outputs of one activation row: 2 NT of them are the row's 16 NT
+    for (int e = (int)threadIdx.x; e < PH * 16 * 2 * NT; e += BK_THREADS) {
+      const int seg = e % (2 * NT), row = e / (2 * NT), i = row >> 4, rr = row & 15, t = seg >> 1;
+      const int m = m0 + 16 * (mb + i) + rr, n = n0 + 8 * seg;
+      if (mb + i >= MT || m >= M || n >= N) continue;
+      const int at = (t * PH + i) * 64 + 32 * (seg & 1) + rr;
+      f4 s0 = red[at], s1 = red[at + 16];
+#pragma unroll
+      for (int w = 1; w < BK_WAVES; ++w) {
+        s0 += red[w * NT * PH * 64 + at];
+        s1 += red[w * NT * PH * 64 + at + 16];
+      }
+      const h8 hv = h8{(_Float16)s0[0], (_Float16)s0[1], (_Float16)s0[2], (_Float16)s0[3],
+                       (_Float16)s1[0], (_Float16)s1[1], (_Float16)s1[2], (_Float16)s1[3]};
+      *(h8*)(c + (size_t)m * N + n) = hv;
+    }
+  }
+}
+
+// Bytes of LDS of a workgroup with NT tiles of W.
+int bk_lds_bytes(const WView& v, int NT) {
+  const int G = v.mx ? v.B : v.G;
+  const long long p = 16LL * NT * G * (v.mx ? 1 : 2), z = v.mx || v.symmetric ? 0 : 64LL * NT * words(G);
+  const long long bytes = BK_WAVES * bk_wave_bytes(NT, BK_XS) + ((p + 1023) & ~1023LL) + ((z + 1023) & ~1023LL);
+  return bytes > (1 << 20) ? 1 << 20 : (int)bytes;
+}
+constexpr int BK_MAX_LDS = 160 * 1024;
+
+template <int FMT, int NT, int MT>
+hipError_t block_go(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out) {
+  constexpr int XS = BK_XS;
+  constexpr bool AHEAD = NT <= 2;
+  const int lds_bytes = bk_lds_bytes(v, NT);
+  static std::atomic<bool> granted[64] = {};  // more than 64 KB of LDS has to be granted per device, once
+  int dev = 0;
+  if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
+  if (dev < 0 || dev >= 64 || !granted[dev]) {
+    const hipError_t e = hipFuncSetAttribute((const void*)mfma_block_kernel<FMT, NT, MT, XS, AHEAD>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, BK_MAX_LDS);
+    if (e != hipSuccess) return e;
+    if (dev >= 0 && dev < 64) granted[dev] = true;
+  }
+  const bool pow2 = !v.mx && (v.gs & (v.gs - 1)) == 0;
+  const int mg = (M + 16 * MT - 1) / (16 * MT), ng = (v.N + 16 * NT - 1) / (16 * NT);
+  mfma_block_kernel<FMT, NT, MT, XS, AHEAD><<<dim3((unsigned)(8 * ((ng + 7) / 8) * mg)), BK_THREADS, lds_bytes, s>>>(
+      v.q, v.scales, v.zeros, x, c, v.N, v.K, M, pow2 ? __builtin_ctz((unsigned)v.gs) : -1,
+      v.mx ? v.B : v.G, v.gs, mg, w_out);
+  return hipGetLastError();
+}
+
+// Blocks and what a wave needs for 128 k of one, in units of 10 ns, W4 and MXFP4 (N = 4096, K = 14336 with
+// as many rows as make one round of workgroups, and N = 5120, K = 13824; a call takes 3.5 us more).
+struct BkShape {
+  int nt, mt, cost_w4, cost_mx;
+};
+constexpr BkShape BK_SHAPES[] = {{1, 1, 50, 45},   {2, 1, 83, 56},   {2, 2, 106, 89},  {4, 1, 136, 80},  {2, 4, 171, 155},
+                                 {4, 2, 175, 125}, {3, 4, 195, 173}, {4, 4, 260, 215}, {4, 5, 290, 250}, {4, 6, 330, 290}};
+
+// Compute units of the current device (per-device cache); 0 on error.
+int bk_cus() {
+  static std::atomic<int> cached[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  if (dev >= 0 && dev < 64 && cached[dev]) return cached[dev];
+  int n = 0;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+  if (dev >= 0 && dev < 64) cached[dev] = n;
+  return n;
+}
+
+// The block that covers the call in the least time (rounds of workgroups x cost of one), as an index into
+// BK_SHAPES; -1: none, or another kernel is ahead.
+int block_plan(const WView& v, int M) {
+  if (M < 3 || M > 8192 || (M < 9 && v.K <= 4096) || (M < 17 && v.K <= 2048)) return -1;
+  if (v.K % 32 || v.N % 16 || (!v.mx && v.gs % 32)) return -1;
+  const int cus = bk_cus();
+  if (cus < 8) return -1;
+  // Few rows: one 16-row tile of W a workgroup from M = 9 on (N = K = 4096, M = 8 / 12 / 16: 5.2 / 5.3 / 5.4 against
+  // 5.0 / 5.5 / 5.8 us; K = 2048, M = 16 4.2 against 3.9), wider matrices at long K only (N = 11008, K = 4096,
+  // M = 16 9.4 against 7.7 us).  (Ruled out first: calls this short see host time.)
+  if (M < 17 && v.K <= 4096 && v.N > 16 * cus) return -1;
+  // Several rounds only pay against the register-staged tile and stream kernels, which take what the
+  // direct-to-LDS tile kernel leaves (K = 9760, N = 3072, M = 448: 105 -> 69 us in two rounds; at K = 8192, N = 8192,
+  // M = 256, which is that kernel's, two rounds take 50 us against 48).
+  const bool dma = v.K % 128 == 0 && (v.mx || v.gs == 32 || v.gs == 64 || v.gs % 128 == 0);
+  int best = -1;
+  long long least = 0;
+  for (int i = 0; i < (int)(sizeof BK_SHAPES / sizeof BK_SHAPES[0]); ++i) {
+    const BkShape& s = BK_SHAPES[i];
+    if (bk_lds_bytes(v, s.nt) > BK_MAX_LDS) continue;
+    const long long ng = (v.N + 16 * s.nt - 1) / (16 * s.nt), mg = (M + 16 * s.mt - 1) / (16 * s.mt);
+    const long long per_xcd = (ng + 7) / 8 * mg, rounds = (per_xcd + cus / 8 - 1) / (cus / 8);
+    if (rounds > (dma || M < 17 ? 1 : 8)) continue;
+    const long long cost = rounds * (v.mx ? s.cost_mx : s.cost_w4);
+    if (best < 0 || cost < least) best = i, least = cost;
+  }
+  if (best < 0) return -1;
+  if (!dma) return best;
+  // One round at K of one or two units a wave and many rows: N = 4096, K = 1024, M = 192 7.8 against 6.9 us,
+  // K = 2048, M = 333 12.1 against 10.9.
+  if ((v.K < 2048 && M > 128) || (v.K < 4096 && M > 256)) return -1;
+  // Up to 32 rows of wide matrices at the resident kernel's own K: N = 11008, M = 32 12.4 against 10.4 us; W4 at the
+  // shorter of the two always: N = 2048, M = 32 5.1 against 4.9.
+  if (M <= 32 && (v.K == 2048 || v.K == 4096) && BK_SHAPES[best].nt == 4) return -1;
+  if (M <= 32 && v.K == 2048 && !v.mx) return -1;
+  return best;
+}
+
+template <int FMT>
+hipError_t block_fmt(int shape, const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out) {
+  switch (shape) {
+    case 0: return block_go<FMT, 1, 1>(v, x, c, M, s, w_out);
+    case 1: return block_go<FMT, 2, 1>(v, x, c, M, s, w_out);
+    case 2: return block_go<FMT, 2, 2>(v, x, c, M, s, w_out);
+    case 3: return block_go<FMT, 4, 1>(v, x, c, M, s, w_out);
+    case 4: return block_go<FMT, 2, 4>(v, x, c, M, s, w_out);
+    case 5: return block_go<FMT, 4, 2>(v, x, c, M, s, w_out);
+    case 6: return block_go<FMT, 3, 4>(v, x, c, M, s, w_out);
+    case 7: return block_go<FMT, 4, 4>(v, x, c, M, s, w_out);
+    case 8: return block_go<FMT, 4, 5>(v, x, c, M, s, w_out);
+    default: return block_go<FMT, 4, 6>(v, x, c, M, s, w_out);
+  }
+}
+
+}  // namespace
+
+bool try_block(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out, hipError_t* err) {
+  if (((uintptr_t)v.q | (uintptr_t)v.scales | (uintptr_t)v.zeros | (uintptr_t)x | (uintptr_t)c | (uintptr_t)w_out) & 15)
+    return false;
+  const int shape = block_plan(v, M);
+  if (shape < 0) return false;
+  if (v.mx) *err = block_fmt<2>(shape, v, x, c, M, s, w_out);
+  else if (v.symmetric) *err = block_fmt<0>(shape, v, x, c, M, s, w_out);
+  else *err = block_fmt<1>(shape, v, x, c, M, s, w_out);
+  return true;
+}
+
+}  // namespace w4k

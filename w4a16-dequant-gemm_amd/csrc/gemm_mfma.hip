@@ -902,6 +902,7 @@ template <int MX>
 static hipError_t launch_fmt(const WView& v, const w4_half* x, w4_half* c, int M,
                              hipStream_t s, w4_half* w_out) {
   hipError_t terr = hipSuccess;
+  if (try_block(v, x, c, M, s, w_out, &terr)) return terr;
   // Shapes of the kernel that fetches the activations once per workgroup (M <= 256):
   // hooked calls take the K-split kernel, which adds in the same order.
   const bool wvec = (v.K % 32 == 0) && (((uintptr_t)v.q) & 15) == 0;

@@ -50,6 +50,11 @@ bool try_tile_dma(const WView& v, const w4_half* x, w4_half* c, int M, hipStream
 bool try_tile256(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, int cus,
                  hipError_t* err);
 
+// gemm_block.hip: middle M (17 to a few hundred rows), blocks of W and x as square as one round of
+// workgroups allows, hooked calls included; false (nothing launched) when another kernel is ahead.
+bool try_block(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out,
+               hipError_t* err);
+
 // gemm_decode_resident.hip: M <= 64 with the activations fetched once per workgroup
 // (several 16-row tiles each).  Same order of additions as the K-split decode
 // kernels of gemm_mfma.hip, which serve the hooked calls of these shapes.
