@@ -492,14 +492,9 @@ int w4_dequant_f8(const uint8_t* q, const w4_half* s, w4_half* w, int S, int D, 
 // kvcache.hpp:60-68, kvfp8.hpp:70-79); what they find in the data (non-finite
 // input, scale out of range) lands in *status instead of a throw.
 
-static int start_status(int* status, w4_stream stream, const char* what) {
-  return done(what, w4k::launch_fill_words((uint32_t*)status, 1, 0u, (hipStream_t)stream));
-}
-
 int w4_quantize(const w4_packed_view* out, const double* w, int* status, w4_stream stream) {
   if (int rc = check_packed(out, "quantize")) return rc;
   REQUIRE(w && status, "quantize: null pointer");
-  if (int rc = start_status(status, stream, "quantize")) return rc;
   const w4k::QuantSide side{w, (uint32_t*)out->q, nullptr, (w4_half*)out->scales,
                             (uint32_t*)out->zeros};
   return done("quantize", w4k::launch_quantize_rows(out->symmetric ? 0 : 1, &side, 1, 0, out->N,
@@ -512,7 +507,6 @@ int w4_quantize_mx(const w4_packed_mx_view* out, const double* w, int* status,
   REQUIRE(out->N >= 1 && out->K >= 1, "quantize_mx: bad dims");
   REQUIRE(out->B == (out->K + 31) / 32, "quantize_mx: B inconsistent with K");
   REQUIRE(out->q && out->scales && w && status, "quantize_mx: null pointer");
-  if (int rc = start_status(status, stream, "quantize_mx")) return rc;
   return done("quantize_mx",
               w4k::launch_quantize_mx(w, 0, out->N, out->K, (uint32_t*)out->q,
                                       (uint8_t*)out->scales, status, (hipStream_t)stream));
@@ -524,7 +518,6 @@ int w4_quantize_mx_f16(const w4_packed_mx_view* out, const w4_half* x, int* stat
   REQUIRE(out->N >= 1 && out->K >= 1, "quantize_mx: bad dims");
   REQUIRE(out->B == (out->K + 31) / 32, "quantize_mx: B inconsistent with K");
   REQUIRE(out->q && out->scales && x && status, "quantize_mx: null pointer");
-  if (int rc = start_status(status, stream, "quantize_mx")) return rc;
   return done("quantize_mx",
               w4k::launch_quantize_mx(x, 1, out->N, out->K, (uint32_t*)out->q,
                                       (uint8_t*)out->scales, status, (hipStream_t)stream));
@@ -554,7 +547,6 @@ int w4_quantize_mx8_f16(const w4_act_mx8_view* out, const w4_half* x, int* statu
                         w4_stream stream) {
   if (int rc = check_mx8(out)) return rc;
   REQUIRE(x && status, "quantize_mx8: null pointer");
-  if (int rc = start_status(status, stream, "quantize_mx8")) return rc;
   return done("quantize_mx8",
               w4k::launch_quantize_mx8(x, 1, out->M, out->K, (uint8_t*)out->q,
                                        (uint8_t*)out->scales, status, (hipStream_t)stream));
@@ -589,7 +581,6 @@ int w4_quantize_cache(const w4_kv_view* out, const void* k, const void* v, int s
   REQUIRE(out->symmetric || (out->z_k && out->z_v), "quantize_cache: asymmetric without zeros");
   REQUIRE(!out->symmetric || (!out->z_k && !out->z_v),
           "quantize_cache: symmetric carries no zeros");
-  if (int rc = start_status(status, stream, "quantize_cache")) return rc;
   const w4k::QuantSide sides[2] = {
       {k, (uint32_t*)out->q_k, nullptr, (w4_half*)out->s_k, (uint32_t*)out->z_k},
       {v, (uint32_t*)out->q_v, nullptr, (w4_half*)out->s_v, (uint32_t*)out->z_v}};
@@ -608,7 +599,6 @@ int w4_quantize_cache_f8(const w4_kv_f8_view* out, const void* k, const void* v,
           "quantize_cache_f8: G inconsistent with D, gs");
   REQUIRE(out->q_k && out->s_k && out->q_v && out->s_v && k && v && status,
           "quantize_cache_f8: null pointer");
-  if (int rc = start_status(status, stream, "quantize_cache_f8")) return rc;
   const w4k::QuantSide sides[2] = {{k, nullptr, (uint8_t*)out->q_k, (w4_half*)out->s_k, nullptr},
                                    {v, nullptr, (uint8_t*)out->q_v, (w4_half*)out->s_v, nullptr}};
   return done("quantize_cache_f8",

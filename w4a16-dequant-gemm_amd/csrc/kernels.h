@@ -133,8 +133,8 @@ hipError_t launch_flash(const FlashArgs& a, float* scratch, hipStream_t s);
 
 // quantize.hip -- the host quantizers as kernels.  mode: 0 W4 symmetric, 1 W4 with
 // zero-points, 2 E4M3 bytes; src is FP64 or (src_f16) FP16; `rows` rows of K
-// elements, groups of gs along K.  status: bit 0 non-finite input, bit 1 scale
-// out of range (OR-ed in by the kernels).
+// elements, groups of gs along K.  status: cleared by the call, then bit 0
+// non-finite input, bit 1 scale out of range.
 struct QuantSide {  // one source and its outputs (q32: W4 words, q8: E4M3 bytes)
   const void* src;
   uint32_t* q32;
@@ -156,6 +156,5 @@ hipError_t launch_gemm_mx_w4a8(const w4_packed_mx_view& w, const w4_act_mx8_view
 int mx_plan(bool x8, int M, int N, int K);
 hipError_t launch_quantize_mx8(const void* src, int src_f16, long long rows, int K, uint8_t* q,
                                uint8_t* scales, int* status, hipStream_t s);
-hipError_t launch_fill_words(uint32_t* p, long long n, uint32_t value, hipStream_t s);
 
 }  // namespace w4k

@@ -21,6 +21,8 @@
 // bit 1 scale out of range.  Outputs are unspecified when it ends non-zero.
 #include <float.h>
 
+#include <atomic>
+
 #include "dq.cuh"
 #include "kernels.h"
 
@@ -28,6 +30,40 @@ namespace w4k {
 namespace {
 
 constexpr int QT = 256;  // threads per workgroup
+
+// The caller's status word, which a call first clears and then ORs what it found into.  A launch of
+// its own for the clearing was 2.5 us of a call of 7 (8 x 4096 x 128 keys and values) and of 6 (one row);
+// so the first workgroup clears, says so in a slot that only this call's ticket names, and a lane
+// that has something to report -- which is rare -- waits for that.  The first workgroup is placed
+// first and waits for nobody before it has said so; a wait that has lasted some 10 ms reports all the
+// same (two calls in flight on the device whose tickets share a slot: QZ_SLOTS calls apart).
+// Stores and loads at agent scope and a wait for the store in between are the order that is needed, as in
+// the flash kernels' merge; a release fence would write a whole L2 back.
+// ticket 0: an earlier launch has cleared the word (calls that a graph captures: a replay would
+// find its ticket from the replay before).
+constexpr int QZ_SLOTS = 4096;
+__device__ uint32_t qz_cleared[QZ_SLOTS];
+struct Status {
+  int* word;
+  uint32_t ticket;
+};
+
+__device__ __forceinline__ void begin_status(const Status& st) {
+  if (st.ticket && (blockIdx.x | blockIdx.y | threadIdx.x) == 0) {
+    __hip_atomic_store(st.word, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __hip_atomic_store(&qz_cleared[st.ticket % QZ_SLOTS], st.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+__device__ __forceinline__ void report(const Status& st, int bits) {
+  for (int n = 0; st.ticket && n < 65536; ++n) {
+    if (__hip_atomic_load(&qz_cleared[st.ticket % QZ_SLOTS], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == st.ticket)
+      break;
+    __builtin_amdgcn_s_sleep(4);
+  }
+  atomicOr(st.word, bits);
+}
 
 __global__ void fill_words_kernel(uint32_t* p, long long n, uint32_t value) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -111,7 +147,8 @@ __device__ __forceinline__ int pow2_at_least(int n) {
 // source element type (double or _Float16).
 template <typename T, int MODE>
 __global__ __launch_bounds__(QT) void quantize_rows_kernel(
-    const Sides<T> sd, long long rows, int K, int gs, int G, int* __restrict__ status) {
+    const Sides<T> sd, long long rows, int K, int gs, int G, const Status status) {
+  begin_status(status);
   const T* __restrict__ src = sd.src[blockIdx.y];
   uint32_t* __restrict__ q32 = sd.q32[blockIdx.y];
   uint8_t* __restrict__ q8 = sd.q8[blockIdx.y];
@@ -158,7 +195,7 @@ __global__ __launch_bounds__(QT) void quantize_rows_kernel(
       }
     }
   }
-  if (bad) atomicOr(status, 1);
+  if (bad) report(status, 1);
 
   s_lo[t] = lo;
   s_hi[t] = hi;
@@ -192,7 +229,7 @@ __global__ __launch_bounds__(QT) void quantize_rows_kernel(
     asm volatile("" : "+v"(step_f));
     const _Float16 sh = (_Float16)step_f;
     const float sf = (float)sh;
-    if (!(fabsf(sf) <= FLT_MAX) || (sf == 0.0f && has_signal)) atomicOr(status, 2);
+    if (!(fabsf(sf) <= FLT_MAX) || (sf == 0.0f && has_signal)) report(status, 2);
     int zero = 8;
     if (MODE == QM_ASYM) {
       zero = clamp_code(round_half_away(-lo / (double)sf));
@@ -305,7 +342,8 @@ __device__ __forceinline__ void load8(const _Float16* p, float v[8]) {
 // 13.6 us a call with those launches and FP64 divisions for step and zero-point, 9.2 without).
 template <typename T, int MODE, bool ZPACK>
 __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
-    const Sides<T> sd, long long nwords, int wpg, int wpg_shift, int G, int* __restrict__ status) {
+    const Sides<T> sd, long long nwords, int wpg, int wpg_shift, int G, const Status status) {
+  begin_status(status);
   const T* __restrict__ src = sd.src[blockIdx.y];
   uint32_t* __restrict__ q32 = sd.q32[blockIdx.y];
   uint8_t* __restrict__ q8 = sd.q8[blockIdx.y];
@@ -332,7 +370,7 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
     // (a branch of the whole wave: as one of single lanes it cost 2 % of the kernel)
     special = __builtin_amdgcn_ballot_w64(top >= 0x7C00u) != 0;
     if (special) {
-      if (top >= 0x7C00u) atomicOr(status, 1);
+      if (top >= 0x7C00u) report(status, 1);
       top = 0;  // a NaN is no extremum: the scale is that of the group's other elements
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -373,7 +411,7 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
       lo = v[j] < lo ? v[j] : lo;
       hi = v[j] > hi ? v[j] : hi;
     }
-    if (bad) atomicOr(status, 1);
+    if (bad) report(status, 1);
     for (int m = 1; m < wpg; m <<= 1) {
       const A olo = __shfl_xor(lo, m), ohi = __shfl_xor(hi, m);
       lo = olo < lo ? olo : lo;
@@ -425,7 +463,7 @@ __global__ __launch_bounds__(QT) void quantize_rows_fast_kernel(
   const bool leader = live && (t & (wpg - 1)) == 0;
   const long long gid = w >> wpg_shift;
   if (leader) {
-    if (!(fabsf(sf) <= FLT_MAX) || (sf == 0.0f && has_signal)) atomicOr(status, 2);
+    if (!(fabsf(sf) <= FLT_MAX) || (sf == 0.0f && has_signal)) report(status, 2);
     scales[gid] = __builtin_bit_cast(uint16_t, sh);
     if (MODE == QM_ASYM && !ZPACK) {
       const long long row = gid / G;
@@ -579,7 +617,8 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
                                                          uint32_t* __restrict__ q,
                                                          uint8_t* __restrict__ q8,
                                                          uint8_t* __restrict__ scales,
-                                                         int* __restrict__ status) {
+                                                         const Status status) {
+  begin_status(status);
   const long long id = (long long)blockIdx.x * QT + threadIdx.x;
   const long long blk = id >> 2;
   const int j4 = (int)(id & 3);
@@ -617,7 +656,7 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
     }
     bad = top >= 0x7F800000u;
     if (bad) {  // a NaN is no maximum: the exponent is that of the block's other elements
-      atomicOr(status, 1);
+      report(status, 1);
       top = 0;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -632,7 +671,7 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
     e = mx_exponent_f16<F8 ? 448 : 6>(__builtin_bit_cast(float, top));
     if (top == 0x7F800000u) {
       e = 127;
-      if (j4 == 0) atomicOr(status, 2);
+      if (j4 == 0) report(status, 2);
     }
   } else {
     A amax = (A)0;
@@ -642,14 +681,14 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
       bad |= !(av <= (A)DBL_MAX);
       amax = av > amax ? av : amax;
     }
-    if (bad) atomicOr(status, 1);
+    if (bad) report(status, 1);
     const A o1 = __shfl_xor(amax, 1);
     amax = o1 > amax ? o1 : amax;
     const A o2 = __shfl_xor(amax, 2);
     amax = o2 > amax ? o2 : amax;
     bool range = false;
     e = mx_exponent<F8 ? 448 : 6>((double)amax, &range);
-    if (range && j4 == 0) atomicOr(status, 2);
+    if (range && j4 == 0) report(status, 2);
   }
   if (n == 0) return;
   A u[8];  // v / 2^e
@@ -705,7 +744,7 @@ __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ s
 
 template <typename T, int MODE>
 hipError_t launch_rows_t(const Sides<T>& sd, int nsides, long long rows, int K, int gs,
-                         int* status, hipStream_t s) {
+                         const Status& status, hipStream_t s) {
   const int G = (K + gs - 1) / gs;
   const int wpg = gs >> 3, tpg = wpg < QT ? wpg : QT, gpb = QT / tpg;
   const bool pow2 = (wpg & (wpg - 1)) == 0;
@@ -745,7 +784,7 @@ hipError_t launch_rows_t(const Sides<T>& sd, int nsides, long long rows, int K, 
 
 template <typename T>
 hipError_t launch_rows(int mode, const QuantSide* sides, int nsides, long long rows, int K, int gs,
-                       int* status, hipStream_t s) {
+                       const Status& status, hipStream_t s) {
   Sides<T> sd{};
   for (int i = 0; i < nsides; ++i) {
     sd.src[i] = (const T*)sides[i].src;
@@ -761,22 +800,40 @@ hipError_t launch_rows(int mode, const QuantSide* sides, int nsides, long long r
 
 }  // namespace
 
-hipError_t launch_fill_words(uint32_t* p, long long n, uint32_t value, hipStream_t s) {
-  fill_words_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(p, n, value);
+// Ticket of a call whose kernel clears the status word itself; 0, and a launch that does it, where the stream
+// is being captured (the legacy stream cannot be).
+static hipError_t start_status(int* word, hipStream_t s, Status* st) {
+  *st = Status{word, 0};
+  bool own = s == nullptr;
+  if (!own) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+    else own = cap == hipStreamCaptureStatusNone;
+  }
+  if (own) {
+    static std::atomic<uint32_t> tickets{0};
+    while (st->ticket == 0) st->ticket = tickets.fetch_add(1, std::memory_order_relaxed) + 1;  // (not 0 when it wraps)
+    return hipSuccess;
+  }
+  fill_words_kernel<<<dim3(1), dim3(64), 0, s>>>((uint32_t*)word, 1, 0u);
   return hipGetLastError();
 }
 
 hipError_t launch_quantize_rows(int mode, const QuantSide* sides, int nsides, int src_f16,
-                                long long rows, int K, int gs, int* status, hipStream_t s) {
+                                long long rows, int K, int gs, int* word, hipStream_t s) {
+  Status status;
+  if (hipError_t e = start_status(word, s, &status); e != hipSuccess) return e;
   return src_f16 ? launch_rows<_Float16>(mode, sides, nsides, rows, K, gs, status, s)
                  : launch_rows<double>(mode, sides, nsides, rows, K, gs, status, s);
 }
 
 hipError_t launch_quantize_mx(const void* src, int src_f16, long long rows, int K, uint32_t* q,
-                              uint8_t* scales, int* status, hipStream_t s) {
+                              uint8_t* scales, int* word, hipStream_t s) {
   const int B = (K + 31) / 32;
   const long long blocks = (rows * B * 4 + QT - 1) / QT;
   if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
+  Status status;
+  if (hipError_t e = start_status(word, s, &status); e != hipSuccess) return e;
   const dim3 grid((unsigned)blocks), block(QT);
   const bool vec = K % 8 == 0 && ((uintptr_t)src & 15) == 0;
   if (src_f16 && vec)
@@ -795,10 +852,12 @@ hipError_t launch_quantize_mx(const void* src, int src_f16, long long rows, int 
 }
 
 hipError_t launch_quantize_mx8(const void* src, int src_f16, long long rows, int K, uint8_t* q,
-                               uint8_t* scales, int* status, hipStream_t s) {
+                               uint8_t* scales, int* word, hipStream_t s) {
   const int B = (K + 31) / 32;
   const long long blocks = (rows * B * 4 + QT - 1) / QT;
   if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
+  Status status;
+  if (hipError_t e = start_status(word, s, &status); e != hipSuccess) return e;
   const dim3 grid((unsigned)blocks), block(QT);
   if (src_f16 && K % 8 == 0 && ((uintptr_t)src & 15) == 0)
     quantize_mx_kernel<_Float16, true, true><<<grid, block, 0, s>>>((const _Float16*)src, rows, K,
