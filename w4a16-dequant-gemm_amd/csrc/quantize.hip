@@ -33,30 +33,38 @@ constexpr int QT = 256;  // threads per workgroup
 
 // The caller's status word, which a call first clears and then ORs what it found into.  A launch of
 // its own for the clearing was 2.5 us of a call of 7 (8 x 4096 x 128 keys and values) and of 6 (one row);
-// so the first workgroup clears, says so in a slot that only this call's ticket names, and a lane
-// that has something to report -- which is rare -- waits for that.  The first workgroup is placed
-// first and waits for nobody before it has said so; a wait that has lasted some 10 ms reports all the
-// same (two calls in flight on the device whose tickets share a slot: QZ_SLOTS calls apart).
+// so the word is cleared once by whoever comes first, the first workgroup or a lane that has something to
+// report (which is rare): the first to leave the call's ticket in a slot of qz_claimed clears and then says so in
+// qz_cleared, and a reporting lane waits for that before it ORs.  It waits for a wave that is running and a few
+// instructions from the end of the wait, never for a workgroup that has yet to be placed: the XCD of the
+// first workgroup may be full of another stream's work for any time.  The wait is bounded for calls in flight
+// at once whose tickets share a slot (QZ_SLOTS calls apart).
 // Stores and loads at agent scope and a wait for the store in between are the order that is needed, as in
 // the flash kernels' merge; a release fence would write a whole L2 back.
 // ticket 0: an earlier launch has cleared the word (calls that a graph captures: a replay would
 // find its ticket from the replay before).
 constexpr int QZ_SLOTS = 4096;
-__device__ uint32_t qz_cleared[QZ_SLOTS];
+__device__ uint32_t qz_claimed[QZ_SLOTS], qz_cleared[QZ_SLOTS];
 struct Status {
   int* word;
   uint32_t ticket;
 };
 
-__device__ __forceinline__ void begin_status(const Status& st) {
-  if (st.ticket && (blockIdx.x | blockIdx.y | threadIdx.x) == 0) {
+__device__ __forceinline__ void clear_once(const Status& st) {
+  const uint32_t slot = st.ticket % QZ_SLOTS;
+  if (__hip_atomic_exchange(&qz_claimed[slot], st.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != st.ticket) {
     __hip_atomic_store(st.word, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __hip_atomic_store(&qz_cleared[st.ticket % QZ_SLOTS], st.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&qz_cleared[slot], st.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
+__device__ __forceinline__ void begin_status(const Status& st) {
+  if (st.ticket && (blockIdx.x | blockIdx.y | threadIdx.x) == 0) clear_once(st);
+}
+
 __device__ __forceinline__ void report(const Status& st, int bits) {
+  if (st.ticket) clear_once(st);
   for (int n = 0; st.ticket && n < 65536; ++n) {
     if (__hip_atomic_load(&qz_cleared[st.ticket % QZ_SLOTS], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == st.ticket)
       break;
