@@ -96,3 +96,38 @@ def test_block_shapes_add_in_one_order():
         got = bits(out).reshape(M, N)
         full = got if full is None else full
         assert np.array_equal(got, full[:M]), M
+
+
+@pytest.mark.parametrize("M,N,K", [(100, 4096, 384), (33, 528, 2176), (16, 4096, 2400), (200, 4096, 4224)])
+@pytest.mark.parametrize("kind", ["mx", 32, 64, 128])
+def test_last_group_near_the_largest_half(M, N, K, kind):
+    """K ends inside a unit and the row's last group is the only one with weights near 65504: codes of
+    other groups would overflow with its scale, and nothing of the kind may reach the product."""
+    c = w4amd.capi()
+    rng = np.random.default_rng(M + K)
+    gs = 32 if kind == "mx" else kind
+    first = (K - 1) // gs * gs  # of the last group
+    codes = rng.integers(0, 16, (N, K))
+    if kind == "mx":
+        codes[:, :first] |= 7                                    # +-6
+        codes[:, first:] = rng.choice([0, 1, 2, 3, 4, 5, 9, 13], (N, K - first))  # up to +-3: 49152
+    else:
+        codes[:, first:] = rng.choice([7, 8, 9], (N, K - first))  # -1, 0, 1 times 60000
+    words = (codes.reshape(N, K // 8, 8).astype(np.uint64) << (4 * np.arange(8, dtype=np.uint64))).sum(-1)
+    x = orc.normal_activations(M * K, 3).view(np.float16).reshape(M, K).copy()
+    x[:, first:] *= np.float16(2.0 ** -12)
+    x = x.view(np.uint16).ravel()
+    G = (K + gs - 1) // gs
+    if kind == "mx":
+        p = orc.quantize_mx(np.ones(N * K), N, K)
+        s = np.full((N, G), 127 - 6, np.uint8)
+        s[:, -1] = 127 + 14
+        p.q[:], p.scales[:] = words.astype(np.uint32).ravel(), s.ravel()
+        dp, fn, w_ref = DevPackedMx(p), c.gemm_mx, orc.dequant_all_mx(p)
+    else:
+        p = orc.quantize(np.ones(N * K), N, K, gs, True)
+        s = np.full((N, G), 0.01, np.float16)
+        s[:, -1] = 60000
+        p.q[:], p.scales[:] = words.astype(np.uint32).ravel(), s.view(np.uint16).ravel()
+        dp, fn, w_ref = DevPacked(p), c.gemm, orc.dequant_all(p)
+    _check(fn, dp.view, w_ref, x, M, N, K, K)

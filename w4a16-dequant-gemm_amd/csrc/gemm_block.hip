@@ -212,6 +212,15 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
       else sc[t] = *(const uint16_t*)(ps + t * 32 * G);
       if (FMT == 1) zw[t] = *(const uint32_t*)(pz + t * 64 * wg);
     }
+    // Lanes past the end of the row hold codes of another group than g's: with its scale they can overflow FP16,
+    // and infinity times the zeroed activations is NaN.  A scale of 0 (MXFP4: 2^-127) makes them zeros.
+    if (chunk * 128 + 128 > K) {
+      if (chunk * 128 + 32 * b >= K) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) sc[t] = 0;
+      }
+      asm volatile("" ::: "memory");
+    }
   };
   auto request_next = [&](auto pc, int U, bool more) BK_INLINE {  // into the places that are free at step p of unit U
     constexpr int p = decltype(pc)::value;
