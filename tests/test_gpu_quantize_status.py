@@ -2,6 +2,8 @@
 condition that the host reports by throwing (pack.hpp:64-72, mx.hpp:71-76, kvcache.hpp:60-68) found in it
 wherever the element lies -- with one workgroup and with thousands, on several streams at once, and on
 every replay of a captured call."""
+import ctypes
+
 import pytest
 import torch
 
@@ -129,3 +131,72 @@ def test_replays_of_a_captured_call(kind):
         graph.replay()
         torch.cuda.synchronize()
         assert st.item() == (BAD if i % 2 else 0), (kind, i)
+
+
+def _ms(fn):
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    a.record()
+    fn()
+    b.record()
+    b.synchronize()
+    return a.elapsed_time(b)
+
+
+def test_no_other_call_clears_the_word_again():
+    """A call that finds something at its start and something else at its end, and one 4096 calls later
+    that runs in the middle of it on another stream: both bits of the first call are reported."""
+    c = w4amd.capi()
+    N, K, gs = 65536, 4800, 48  # (no power of two: the general kernel, some milliseconds)
+    w = torch.ones(N, K, dtype=torch.float64, device=DEV)
+    w[0, 0], w[-1, -1] = float("nan"), 1e300
+    q, sc = torch.empty(N, K // 8, dtype=torch.int32, device=DEV), torch.empty(N, K // gs, dtype=torch.float16, device=DEV)
+    long_view = c.packed_view(N, K, gs, K // gs, True, ptr(q), ptr(sc))
+    call, keep = _kv("w4", 1, 1, 64, 32)
+    k, v = _inputs(1, 1, 64)
+    st = torch.zeros(3, dtype=torch.int32, device=DEV)
+    c.quantize(long_view, ptr(w), ptr(st))
+    long_ms = _ms(lambda: c.quantize(long_view, ptr(w), ptr(st)))
+    torch.cuda._sleep(1000)
+    per_ms = 1e6 / _ms(lambda: torch.cuda._sleep(1000000))  # cycles of a millisecond
+    for _ in range(5):
+        gate, s1, s2, s3 = [torch.cuda.Stream() for _ in range(4)]  # (some may share a hardware queue)
+        st.fill_(0x55)
+        torch.cuda.synchronize()
+        start = torch.cuda.Event()
+        with torch.cuda.stream(gate):
+            torch.cuda._sleep(int(60 * per_ms))  # until everything below is enqueued
+            start.record()
+        s1.wait_event(start)
+        s2.wait_event(start)
+        c.quantize(long_view, ptr(w), ptr(st), stream=s1.cuda_stream)
+        for _ in range(4095):
+            call(k, v, ptr(st) + 4, s3.cuda_stream)
+        with torch.cuda.stream(s2):
+            torch.cuda._sleep(int(long_ms / 2 * per_ms))
+        call(k, v, ptr(st) + 8, s2.cuda_stream)
+        torch.cuda.synchronize()
+        assert st.tolist() == [BAD | RANGE, 0, 0]
+
+
+def test_more_streams_than_slots():
+    """Streams past the ones that have a slot clear the word by a launch of its own."""
+    hip = ctypes.CDLL(w4amd.capi().LIB_PATH)  # (the runtime that the library is linked to)
+    streams = []
+    for _ in range(80):
+        s = ctypes.c_void_p()
+        assert hip.hipStreamCreate(ctypes.byref(s)) == 0
+        streams.append(s.value)
+    call, keep = _kv("w4z", 2, 33, 128, 32)
+    k, v = _inputs(2, 33, 128)
+    bad = k.clone()
+    bad[0, 7, 3] = INF
+    st = torch.full((80,), 0x66, dtype=torch.int32, device=DEV)
+    torch.cuda.synchronize()
+    for _ in range(2):
+        for i, s in enumerate(streams):
+            call(bad if i % 3 else k, v, ptr(st) + 4 * i, s)
+        torch.cuda.synchronize()
+        assert [bool(x & BAD) for x in st.tolist()] == [bool(i % 3) for i in range(80)]
+        assert all(x == 0 for x in st.tolist()[::3])
+    for s in streams:
+        assert hip.hipStreamDestroy(ctypes.c_void_p(s)) == 0

@@ -21,7 +21,7 @@
 // bit 1 scale out of range.  Outputs are unspecified when it ends non-zero.
 #include <float.h>
 
-#include <atomic>
+#include <mutex>
 
 #include "dq.cuh"
 #include "kernels.h"
@@ -34,28 +34,32 @@ constexpr int QT = 256;  // threads per workgroup
 // The caller's status word, which a call first clears and then ORs what it found into.  A launch of
 // its own for the clearing was 2.5 us of a call of 7 (8 x 4096 x 128 keys and values) and of 6 (one row);
 // so the word is cleared once by whoever comes first, the first workgroup or a lane that has something to
-// report (which is rare): the first to leave the call's ticket in a slot of qz_claimed clears and then says so in
+// report (which is rare): the first to leave the call's ticket in qz_claimed clears and then says so in
 // qz_cleared, and a reporting lane waits for that before it ORs.  It waits for a wave that is running and a few
 // instructions from the end of the wait, never for a workgroup that has yet to be placed: the XCD of the
-// first workgroup may be full of another stream's work for any time.  The wait is bounded for calls in flight
-// at once whose tickets share a slot (QZ_SLOTS calls apart).
+// first workgroup may be full of another stream's work for any time.
+// A slot belongs to one stream, whose calls run one after the other with ascending tickets (StatusCall): no
+// other call can take the slot over between two arrivals of a call, which would clear the word again.
+// Tickets only ever replace lower ones, so that what may be left of a stream destroyed with work in
+// flight takes nothing from a stream that has its address.
 // Stores and loads at agent scope and a wait for the store in between are the order that is needed, as in
 // the flash kernels' merge; a release fence would write a whole L2 back.
-// ticket 0: an earlier launch has cleared the word (calls that a graph captures: a replay would
-// find its ticket from the replay before).
-constexpr int QZ_SLOTS = 4096;
-__device__ uint32_t qz_claimed[QZ_SLOTS], qz_cleared[QZ_SLOTS];
+// ticket: the call's number in its slot x QZ_SLOTS + the slot; 0: an earlier launch has cleared the word.
+// (One word, so that all arguments of a kernel arrive in registers.)
+constexpr int QZ_SLOTS = 64;
+typedef unsigned long long qz_ticket;
+__device__ qz_ticket qz_claimed[QZ_SLOTS], qz_cleared[QZ_SLOTS];
 struct Status {
   int* word;
-  uint32_t ticket;
+  qz_ticket ticket;
 };
 
 __device__ __forceinline__ void clear_once(const Status& st) {
-  const uint32_t slot = st.ticket % QZ_SLOTS;
-  if (__hip_atomic_exchange(&qz_claimed[slot], st.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != st.ticket) {
+  const uint32_t slot = (uint32_t)st.ticket % QZ_SLOTS;
+  if (__hip_atomic_fetch_max(&qz_claimed[slot], st.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < st.ticket) {
     __hip_atomic_store(st.word, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __hip_atomic_store(&qz_cleared[slot], st.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_fetch_max(&qz_cleared[slot], st.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -66,7 +70,7 @@ __device__ __forceinline__ void begin_status(const Status& st) {
 __device__ __forceinline__ void report(const Status& st, int bits) {
   if (st.ticket) clear_once(st);
   for (int n = 0; st.ticket && n < 65536; ++n) {
-    if (__hip_atomic_load(&qz_cleared[st.ticket % QZ_SLOTS], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == st.ticket)
+    if (__hip_atomic_load(&qz_cleared[(uint32_t)st.ticket % QZ_SLOTS], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= st.ticket)
       break;
     __builtin_amdgcn_s_sleep(4);
   }
@@ -806,31 +810,68 @@ hipError_t launch_rows(int mode, const QuantSide* sides, int nsides, long long r
   return launch_rows_t<T, QM_F8>(sd, nsides, rows, K, gs, status, s);
 }
 
-}  // namespace
+// The status word of one call, from its ticket to the launch.
+//
+// Calls get a slot by the stream they are on, so that only calls that run one after the other share
+// one; the slot's lock is held until the kernel is enqueued, so that threads that use one stream enqueue
+// in the order of their tickets.  A slot stays its stream's (a stream created later at the same
+// address goes on with its tickets).  A launch of its own clears the word, and the ticket is 0, where
+// that cannot be had: in a stream that is being captured (a replay would find its ticket from the replay
+// before; the legacy stream cannot be captured), for the handles that stand for the legacy and the
+// calling thread's stream, and for streams past the first QZ_SLOTS.
+class StatusCall {
+ public:
+  hipError_t begin(int* word, hipStream_t s) {
+    st_ = Status{word, 0};
+    if (Slot* const slot = slot_of(s)) {
+      held_ = std::unique_lock<std::mutex>(slot->lock);
+      st_.ticket = ++slot->calls * QZ_SLOTS + (qz_ticket)(slot - slots);
+      return hipSuccess;
+    }
+    fill_words_kernel<<<dim3(1), dim3(64), 0, s>>>((uint32_t*)word, 1, 0u);
+    return hipGetLastError();
+  }
+  const Status& status() const { return st_; }
 
-// Ticket of a call whose kernel clears the status word itself; 0, and a launch that does it, where the stream
-// is being captured (the legacy stream cannot be).
-static hipError_t start_status(int* word, hipStream_t s, Status* st) {
-  *st = Status{word, 0};
-  bool own = s == nullptr;
-  if (!own) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
-    else own = cap == hipStreamCaptureStatusNone;
+ private:
+  struct Slot {
+    std::mutex lock;  // of calls
+    qz_ticket calls = 0;
+    int dev = -1;
+    hipStream_t stream = nullptr;
+  };
+  static Slot slots[QZ_SLOTS];
+
+  static Slot* slot_of(hipStream_t s) {
+    int dev = 0;
+    if (s == hipStreamLegacy || s == hipStreamPerThread || hipGetDevice(&dev) != hipSuccess) return nullptr;
+    if (s != nullptr) {
+      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(s, &cap) != hipSuccess) return (void)hipGetLastError(), nullptr;
+      if (cap != hipStreamCaptureStatusNone) return nullptr;
+    }
+    static std::mutex table;  // of dev and stream of all slots
+    static int used = 0;
+    const std::lock_guard<std::mutex> guard(table);
+    for (int i = 0; i < used; ++i)
+      if (slots[i].stream == s && slots[i].dev == dev) return &slots[i];
+    if (used == QZ_SLOTS) return nullptr;
+    slots[used].dev = dev, slots[used].stream = s;
+    return &slots[used++];
   }
-  if (own) {
-    static std::atomic<uint32_t> tickets{0};
-    while (st->ticket == 0) st->ticket = tickets.fetch_add(1, std::memory_order_relaxed) + 1;  // (not 0 when it wraps)
-    return hipSuccess;
-  }
-  fill_words_kernel<<<dim3(1), dim3(64), 0, s>>>((uint32_t*)word, 1, 0u);
-  return hipGetLastError();
-}
+
+  Status st_{};
+  std::unique_lock<std::mutex> held_;
+};
+StatusCall::Slot StatusCall::slots[QZ_SLOTS];
+
+}  // namespace
 
 hipError_t launch_quantize_rows(int mode, const QuantSide* sides, int nsides, int src_f16,
                                 long long rows, int K, int gs, int* word, hipStream_t s) {
-  Status status;
-  if (hipError_t e = start_status(word, s, &status); e != hipSuccess) return e;
+  StatusCall call;
+  if (hipError_t e = call.begin(word, s); e != hipSuccess) return e;
+  const Status& status = call.status();
   return src_f16 ? launch_rows<_Float16>(mode, sides, nsides, rows, K, gs, status, s)
                  : launch_rows<double>(mode, sides, nsides, rows, K, gs, status, s);
 }
@@ -840,8 +881,9 @@ hipError_t launch_quantize_mx(const void* src, int src_f16, long long rows, int 
   const int B = (K + 31) / 32;
   const long long blocks = (rows * B * 4 + QT - 1) / QT;
   if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
-  Status status;
-  if (hipError_t e = start_status(word, s, &status); e != hipSuccess) return e;
+  StatusCall call;
+  if (hipError_t e = call.begin(word, s); e != hipSuccess) return e;
+  const Status& status = call.status();
   const dim3 grid((unsigned)blocks), block(QT);
   const bool vec = K % 8 == 0 && ((uintptr_t)src & 15) == 0;
   if (src_f16 && vec)
@@ -864,8 +906,9 @@ hipError_t launch_quantize_mx8(const void* src, int src_f16, long long rows, int
   const int B = (K + 31) / 32;
   const long long blocks = (rows * B * 4 + QT - 1) / QT;
   if (blocks > 0x7FFFFFFFLL) return hipErrorInvalidConfiguration;
-  Status status;
-  if (hipError_t e = start_status(word, s, &status); e != hipSuccess) return e;
+  StatusCall call;
+  if (hipError_t e = call.begin(word, s); e != hipSuccess) return e;
+  const Status& status = call.status();
   const dim3 grid((unsigned)blocks), block(QT);
   if (src_f16 && K % 8 == 0 && ((uintptr_t)src & 15) == 0)
     quantize_mx_kernel<_Float16, true, true><<<grid, block, 0, s>>>((const _Float16*)src, rows, K,
