@@ -131,3 +131,28 @@ def test_last_group_near_the_largest_half(M, N, K, kind):
         p.q[:], p.scales[:] = words.astype(np.uint32).ravel(), s.view(np.uint16).ravel()
         dp, fn, w_ref = DevPacked(p), c.gemm, orc.dequant_all(p)
     _check(fn, dp.view, w_ref, x, M, N, K, K)
+
+
+@pytest.mark.parametrize("M,N,K,gs,sym", [(9, 4096, 4096, 128, True), (32, 4096, 4096, 128, False), (17, 8192, 8192, 256, True),
+                                          (32, 8192, 8192, 128, False), (24, 528, 4352, 4352, True), (200, 4096, 4224, 128, True),
+                                          (333, 4080, 4096, 128, False)])
+def test_whole_chunk_groups_keep_their_scales_out_of_fp16(M, N, K, gs, sym):
+    """Groups of whole 128-k chunks: (q - z) s is not rounded to FP16 before the sum, so an output is the
+    product in FP64 rounded once, but where FP32 sums (some 1e-6 of the norm) end on the other side of a
+    rounding boundary (ulp 5e-4 to 1e-3 of the value): one or two per cent of them.  Weights rounded first
+    (1.7e-4 of the norm) move more than a quarter of the outputs."""
+    rng = np.random.default_rng(M)
+    w = orc.normal_weights(N * K, M + N) * 0.02 + (0.0 if sym else 0.01)
+    p = orc.quantize(w, N, K, gs, sym)
+    x = orc.normal_activations(M * K, 3)
+    dp, x_d, out = DevPacked(p), to_dev(x), halves(M * N)
+    w4amd.capi().gemm(dp.view, ptr(x_d), ptr(out), M, 0, 0)
+    ns = np.unique(rng.choice(N, size=200))
+    sh = 4 * np.arange(8, dtype=np.uint32)
+    q = ((p.q.reshape(N, -1)[ns][:, :, None] >> sh) & 15).reshape(len(ns), -1)[:, :K].astype(np.float64)
+    z = 8.0 if sym else ((p.zeros.reshape(N, -1)[ns][:, :, None] >> sh) & 15).reshape(len(ns), -1)[:, np.arange(K) // gs].astype(np.float64)
+    s = p.scales.reshape(N, -1)[ns].view(np.float16).astype(np.float64)[:, np.arange(K) // gs]
+    exact = x.view(np.float16).reshape(M, K).astype(np.float64) @ ((q - z) * s).T
+    got = np.ascontiguousarray(bits(out).reshape(M, N)[:, ns])
+    moved = np.mean(got != exact.astype(np.float16).view(np.uint16))
+    assert moved <= 0.04, moved

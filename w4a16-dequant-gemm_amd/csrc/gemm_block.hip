@@ -35,13 +35,16 @@ constexpr int bk_wave_bytes(int NT, int XS) { return NT * 2048 + XS * 4096; }
 constexpr int bk_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
 extern __shared__ __attribute__((aligned(16))) uint8_t bk_lds[];
 
+// SCALED: times the group's scale (s2), else the codes minus the zero-point.
+template <bool SCALED>
 __device__ __forceinline__ h8 bk_expand(uint32_t w, h2 cneg, h2 s2, uint32_t mask, uint32_t magic) {
   u4 out;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint32_t p = __builtin_amdgcn_perm(0u, w, 0x0c000c00u | (uint32_t)(i << 16) | (uint32_t)i);
     const uint32_t v = (p & mask) | magic;
-    out[i] = as_u32((as_h2(v) + cneg) * s2);
+    const h2 d = as_h2(v) + cneg;
+    out[i] = as_u32(SCALED ? d * s2 : d);
   }
   return __builtin_bit_cast(h8, out);
 }
@@ -59,13 +62,17 @@ __device__ __forceinline__ void bk_dma(uint32_t off, const void* base, uint32_t 
 
 // FMT: 0 W4 symmetric, 1 W4 with zero-points, 2 MXFP4.  G: groups (W4) or blocks (MXFP4) per row.
 // gs_shift: log2(gs) if gs is a power of two, else -1.  mgroups: blocks along M.  XS: pieces of x (16 rows x 128 k, 4 KB) in a
-// wave's ring; three measured no better than two.
-template <int FMT, int NT, int MT, int XS, bool AHEAD>
+// wave's ring; three measured no better than two.  LATE (W4, gs a multiple of 128: a chunk of 128 k is in one
+// group): the operands are the codes minus the zero-point, exact in FP16, and the scale is applied to a
+// chunk's FP32 sums, as the resident kernel does in the shapes that this one took over from it
+// (rounding q s to FP16 first: 2.7e-4 from the product in FP64 instead of 2.1e-4, K = 4096, M = 16).
+template <int FMT, int NT, int MT, int XS, bool AHEAD, bool LATE>
 __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
     const uint32_t* __restrict__ q, const void* __restrict__ scales, const uint32_t* __restrict__ zeros,
     const w4_half* __restrict__ x, w4_half* __restrict__ c, const int N, const int K, const int M,
     const int gs_shift, const int G, const int gs, const int mgroups, w4_half* __restrict__ w_out) {
   constexpr bool MX = FMT == 2;
+  static_assert(!(MX && LATE), "an MXFP4 chunk has four scales");
   constexpr int WB = bk_wave_bytes(NT, XS), ROWS = 16 * NT, NP = 2 * MT;
   // Step of a unit at which its codes have been read back and the next unit's are requested: with
   // many row tiles one chunk's codes are read at a time (registers).
@@ -132,35 +139,36 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
   // piece p = (chunk p / MT of the unit, row tile p % MT): 4 loads of 4 rows x 256 bytes, piece (l % 16) ^ (row % 16)
   const char* const xb = (const char*)x + (size_t)m0 * xrow;
   const int mlast = M - 1 - m0;
-  constexpr int XO = MT <= 4 ? MT : 0;  // offsets worked out once, where registers allow
-  uint32_t xoff[XO ? XO : 1][4];
+  // Offsets are worked out once: for every tile and load where registers allow; larger blocks have those of a whole
+  // tile of rows, from its first row, and of the tile that M ends in, which stands in for the tiles
+  // behind it as well.
+  constexpr bool XALL = MT <= 4;
+  const int mend = mlast >> 4;
+  uint32_t xoff[XALL ? MT : 2][4];
 #pragma unroll
-  for (int mt = 0; mt < XO; ++mt)
+  for (int i = 0; i < (XALL ? MT : 2); ++i)
 #pragma unroll
     for (int rq = 0; rq < 4; ++rq) {
-      const int r16 = 4 * rq + (lane >> 4);
-      xoff[mt][rq] = (uint32_t)min(16 * mt + r16, mlast) * xrow + (uint32_t)(((lane & 15) ^ r16) * 16);
+      const int r16 = 4 * rq + (lane >> 4), row = XALL ? min(16 * i + r16, mlast) : i ? min(16 * mend + r16, mlast) : r16;
+      xoff[i][rq] = (uint32_t)row * xrow + (uint32_t)(((lane & 15) ^ r16) * 16);
     }
   auto request_x = [&](int U, int p, int slot) BK_INLINE {
     const int ch = p / MT, mt = p % MT;
     const uint32_t k2 = (uint32_t)(U * 2 + ch) * 256u;  // byte of the row
     const uint32_t dst = region + NT * 2048u + (uint32_t)slot * 4096u;
-    auto offset = [&](int rq) BK_INLINE {
-      const int r16 = 4 * rq + (lane >> 4);
-      return XO ? xoff[XO ? mt : 0][rq]
-                : (uint32_t)min(16 * mt + r16, mlast) * xrow + (uint32_t)(((lane & 15) ^ r16) * 16);
-    };
+    const char* const tile = xb + (!XALL && mt < mend ? (size_t)(16 * mt) * xrow : 0);
+    auto offset = [&](int rq) BK_INLINE { return XALL ? xoff[mt][rq] : mt < mend ? xoff[0][rq] : xoff[1][rq]; };
     if (k2 + 256 > xrow) {
       asm volatile("" ::: "memory");
       const bool past = k2 >= xrow;  // all of the chunk: the chunk before instead
-      const char* base = xb + (past ? k2 - 256 : k2);
+      const char* base = tile + (past ? k2 - 256 : k2);
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq) {
         const uint32_t piece = (uint32_t)(((lane & 15) ^ (4 * rq + (lane >> 4))) * 16);
         bk_dma(offset(rq) - (past || k2 + piece >= xrow ? piece : 0u), base, dst + rq * 1024u);
       }
     } else {
-      const char* base = xb + k2;
+      const char* base = tile + k2;
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq) bk_dma(offset(rq), base, dst + rq * 1024u);
     }
@@ -187,8 +195,12 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
     for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f4{0.f, 0.f, 0.f, 0.f};
   u4 cw[PC ? 1 : 2][NT];
   h8 A[NT][4];
-  uint32_t sc[NT], zw[NT];  // group parameters of a lane's 32 k of a chunk, and their group
-  int g = 0, slot = 0;      // slot: of the piece that is multiplied
+  // group parameters of a lane's 32 k of a chunk, and their group; LATE: scales of the rows of its four sums
+  typedef std::conditional_t<LATE, h4, uint32_t> scale_t;
+  scale_t sc[NT];
+  uint32_t zw[NT];
+  [[maybe_unused]] h4 late[NT];  // the scales of the chunk that is multiplied
+  int g = 0, slot = 0;  // slot: of the piece that is multiplied
   const bool hook = w_out && m0 == 0;
 
   auto read_codes = [&](int h, u4* w) BK_INLINE {
@@ -202,22 +214,27 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
       v[j] = *(const h8*)(mine + NT * 2048 + at * 4096 + (r >> 2) * 1024 + ((r & 3) * 16 + ((4 * b + j) ^ r)) * 16);
   };
   auto read_params = [&](int chunk) BK_INLINE {
-    const int kc = min(chunk * 128 + 32 * b, K - 32);
+    const int kc = min(chunk * 128 + (LATE ? 0 : 32 * b), K - 32);
     g = MX ? (kc >> 5) : gs_shift >= 0 ? (kc >> gs_shift) : kc / gs;
-    const uint8_t* ps = params + (r * G + g) * (MX ? 1 : 2);
+    const uint8_t* ps = params + ((LATE ? 4 * b : r) * G + g) * (MX ? 1 : 2);
     const uint8_t* pz = params + zoff + (r * wg + (g >> 3)) * 4;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      if (MX) sc[t] = ps[t * 16 * G];
-      else sc[t] = *(const uint16_t*)(ps + t * 32 * G);
+      if constexpr (LATE) {
+        const _Float16* p = (const _Float16*)ps + t * 16 * G;
+        sc[t] = h4{p[0], p[G], p[2 * G], p[3 * G]};
+      } else {
+        sc[t] = MX ? ps[t * 16 * G] : *(const uint16_t*)(ps + t * 32 * G);
+      }
       if (FMT == 1) zw[t] = *(const uint32_t*)(pz + t * 64 * wg);
     }
     // Lanes past the end of the row hold codes of another group than g's: with its scale they can overflow FP16,
     // and infinity times the zeroed activations is NaN.  A scale of 0 (MXFP4: 2^-127) makes them zeros.
+    // (LATE: the codes are finite, the scale of a chunk that is past the end as a whole may not be.)
     if (chunk * 128 + 128 > K) {
-      if (chunk * 128 + 32 * b >= K) {
+      if (chunk * 128 + (LATE ? 0 : 32 * b) >= K) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t) sc[t] = 0;
+        for (int t = 0; t < NT; ++t) sc[t] = scale_t{};
       }
       asm volatile("" ::: "memory");
     }
@@ -230,17 +247,18 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
     slot = slot + 1 < XS ? slot + 1 : 0;
   };
   // the codes in w, with the parameters given, become the weights of a chunk; k: the lane's first
-  auto expand = [&](const u4* w, const uint32_t* scale, const uint32_t* zword, int group, int k) BK_INLINE {
+  auto expand = [&](const u4* w, const scale_t* scale, const uint32_t* zword, int group, int k) BK_INLINE {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      h2 cneg, s2;
+      h2 cneg, s2 = h2{0, 0};
       float sf = 0.f;
-      if (MX) {
+      if constexpr (MX) {
         sf = mx_scale(scale[t]);
       } else {
         const uint32_t z = FMT == 1 ? ((zword[t] >> (4 * (group & 7))) & 0xFu) : 8u;
         cneg = as_h2(0xD400E400u | (z << 20) | z);
-        s2 = splat_bits(scale[t]);
+        if constexpr (LATE) late[t] = scale[t];
+        else s2 = splat_bits(scale[t]);
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -249,22 +267,37 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
           dq_mx(w[t][j], sf, n4);
           A[t][j] = __builtin_bit_cast(h8, u4{as_u32(n4[0]), as_u32(n4[1]), as_u32(n4[2]), as_u32(n4[3])});
         } else {
-          A[t][j] = bk_expand(w[t][j], cneg, s2, mask, magic);
+          A[t][j] = bk_expand<!LATE>(w[t][j], cneg, s2, mask, magic);
         }
       }
     }
-    if (hook) {  // these registers are the weights
-      asm volatile("" ::: "memory");
+    if (hook) {  // these registers are the weights (LATE: times the scale of the lane's row)
+      int row = r;
+      asm volatile("" : "+v"(row) : : "memory");  // (addresses ahead of the loop would take registers in every call)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         if (16 * t < live && k < K) {
+          const _Float16 own = LATE ? *(const _Float16*)(params + ((t * 16 + row) * G + group) * 2) : (_Float16)1.f;
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            *(h8*)(w_out + (size_t)(n0 + 16 * t + r) * K + k + 8 * j) = A[t][j];
+            *(h8*)(w_out + (size_t)(n0 + 16 * t + row) * K + k + 8 * j) = LATE ? A[t][j] * own : A[t][j];
         }
     }
   };
-  auto multiply = [&](int mt, int chunk, h8* v) BK_INLINE {
+  // LATE: a chunk's sums of two tiles of W, which are scaled while the next two multiply
+  constexpr int ST = 2, LAST = (NT - 1) / ST * ST;
+  [[maybe_unused]] f4 held[ST];
+  auto add_scaled = [&](int t0, int mt) BK_INLINE {
+#pragma unroll
+    for (int t = t0; t < t0 + ST && t < NT; ++t) {
+      asm volatile("" : "+v"(late[t]));  // (stays in halves: v_fma_mix_f32 takes them)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[t][mt][i] = fmaf(held[t - t0][i], (float)late[t][i], acc[t][mt][i]);
+      // (here and not at the end of the unit, where the compiler would put it with all chunk sums alive)
+      asm volatile("" : "+v"(acc[t][mt]));
+    }
+  };
+  auto multiply = [&](auto mtc, int chunk, h8* v) BK_INLINE {
     if (chunk * 128 + 128 > K) {  // the row ends inside this chunk: activations past it are zero
       if (chunk * 128 + 32 * b >= K) {
 #pragma unroll
@@ -272,11 +305,29 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
       }
       asm volatile("" ::: "memory");
     }
+    if constexpr (LATE) {
+      constexpr int mt = decltype(mtc)::value;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+      for (int t0 = 0; t0 < NT; t0 += ST) {
+        f4 part[ST];
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-        acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[t][j], v[j], acc[t][mt], 0, 0, 0);
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int t = t0; t < t0 + ST && t < NT; ++t)
+            part[t - t0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[t][j], v[j], j ? part[t - t0] : f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        if (t0 > 0) add_scaled(t0 - ST, mt);
+        else if (mt > 0) add_scaled(LAST, mt - 1);
+#pragma unroll
+        for (int i = 0; i < ST && t0 + i < NT; ++i) held[i] = part[i];
+      }
+      if (mt == MT - 1) add_scaled(LAST, mt);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          acc[t][mtc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[t][j], v[j], acc[t][mtc], 0, 0, 0);
+    }
   };
   auto landed = [&]() BK_INLINE {  // after a wait: what was waited for is read from here on
     asm volatile("" ::: "memory");
@@ -301,7 +352,8 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this piece is in registers and its place free
         landed();
         request_next(pc, U, more);
-        uint32_t scale[NT], zword[NT];
+        scale_t scale[NT];
+        uint32_t zword[NT];
         const int group = g;
         if (mt == 0) {
 #pragma unroll
@@ -323,7 +375,7 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
         }
         __builtin_amdgcn_sched_barrier(0);
         if (mt == 0) expand(cw[ch], scale, zword, group, U * BK_UNIT + ch * 128 + 32 * b);
-        multiply(mt, 2 * U + ch, xv[p & 1]);
+        multiply(std::integral_constant<int, mt>{}, 2 * U + ch, xv[p & 1]);
         if (MT == 1 && p == NP - 1 && more) read_codes(0, cw[0]), read_codes(1, cw[1]);
         __builtin_amdgcn_sched_barrier(0);
       }, std::make_integer_sequence<int, NP>{});
@@ -348,7 +400,7 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
         request_next(pc, U, more);
         __builtin_amdgcn_sched_barrier(0);
         if (mt == 0) expand(cw[PC ? 0 : ch], sc, zw, g, U * BK_UNIT + ch * 128 + 32 * b);
-        multiply(mt, 2 * U + ch, xv);
+        multiply(std::integral_constant<int, mt>{}, 2 * U + ch, xv);
         __builtin_amdgcn_sched_barrier(0);
       }, std::make_integer_sequence<int, NP>{});
     }
@@ -394,8 +446,8 @@ int bk_lds_bytes(const WView& v, int NT) {
 }
 constexpr int BK_MAX_LDS = 160 * 1024;
 
-template <int FMT, int NT, int MT>
-hipError_t block_go(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out) {
+template <int FMT, int NT, int MT, bool LATE>
+hipError_t block_go_as(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out) {
   constexpr int XS = BK_XS;
   constexpr bool AHEAD = NT <= 2;
   const int lds_bytes = bk_lds_bytes(v, NT);
@@ -403,17 +455,25 @@ hipError_t block_go(const WView& v, const w4_half* x, w4_half* c, int M, hipStre
   int dev = 0;
   if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
   if (dev < 0 || dev >= 64 || !granted[dev]) {
-    const hipError_t e = hipFuncSetAttribute((const void*)mfma_block_kernel<FMT, NT, MT, XS, AHEAD>,
+    const hipError_t e = hipFuncSetAttribute((const void*)mfma_block_kernel<FMT, NT, MT, XS, AHEAD, LATE>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, BK_MAX_LDS);
     if (e != hipSuccess) return e;
     if (dev >= 0 && dev < 64) granted[dev] = true;
   }
   const bool pow2 = !v.mx && (v.gs & (v.gs - 1)) == 0;
   const int mg = (M + 16 * MT - 1) / (16 * MT), ng = (v.N + 16 * NT - 1) / (16 * NT);
-  mfma_block_kernel<FMT, NT, MT, XS, AHEAD><<<dim3((unsigned)(8 * ((ng + 7) / 8) * mg)), BK_THREADS, lds_bytes, s>>>(
+  mfma_block_kernel<FMT, NT, MT, XS, AHEAD, LATE><<<dim3((unsigned)(8 * ((ng + 7) / 8) * mg)), BK_THREADS, lds_bytes, s>>>(
       v.q, v.scales, v.zeros, x, c, v.N, v.K, M, pow2 ? __builtin_ctz((unsigned)v.gs) : -1,
       v.mx ? v.B : v.G, v.gs, mg, w_out);
   return hipGetLastError();
+}
+
+template <int FMT, int NT, int MT>
+hipError_t block_go(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out) {
+  if constexpr (FMT != 2) {
+    if (v.gs % 128 == 0) return block_go_as<FMT, NT, MT, true>(v, x, c, M, s, w_out);
+  }
+  return block_go_as<FMT, NT, MT, false>(v, x, c, M, s, w_out);
 }
 
 // Blocks and what a wave needs for 128 k of one, in units of 10 ns, W4 and MXFP4 (N = 4096, K = 14336 with
