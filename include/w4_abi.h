@@ -225,6 +225,13 @@ int w4_quantize_cache(const w4_kv_view* out, const void* k, const void* v,
 int w4_quantize_cache_f8(const w4_kv_f8_view* out, const void* k, const void* v,
                          int src_f16, int* status, w4_stream stream);
 
+/* Which kernel the matrix-core GEMM runs on the current GPU (no counterpart in the reference): fmt 0 W4
+ * symmetric, 1 W4 with zero-points, 2 MXFP4 (gs ignored); no hook, arrays aligned to 16 bytes.  *plan: 10 x the
+ * 16-row tiles of W + the row tiles of x of a block (11 .. 46); 1 the long-K decode kernel, 2 the one that keeps
+ * the activations, 3 the one for odd group sizes and ragged K; 0 tiles, stream and the others.  Without a
+ * GPU no kernel is told apart (0, or 3). */
+int w4_gemm_plan_for(int fmt, int M, int N, int K, int gs, int* plan);
+
 /* ---- W4A4 on the scaled matrix cores (no counterpart in the reference, whose
  * MXFP4 kernels keep FP16 activations: include/w4/mxfused.cuh:166-198,291-307).
  * c[M,N] = X[M,K] * W[N,K]^T with both operands packed MXFP4 (x->N = M rows,

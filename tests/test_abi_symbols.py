@@ -156,6 +156,15 @@ def test_mx_plan():
             plan(*bad)
 
 
+def test_gemm_plan_contracts():
+    """Bad sizes and formats are refused; without a GPU no kernel that depends on its compute units is named."""
+    plan = w4amd.capi().gemm_plan_for
+    for bad in [(0, 0, 8, 64), (0, 8, 0, 64), (1, 8, 8, 0), (3, 8, 8, 64), (-1, 8, 8, 64), (0, 8, 8, 64, 12), (1, 8, 8, 64, 0)]:
+        with pytest.raises(ValueError):
+            plan(*bad)
+    assert plan(0, 1, 64, 64, 32) in (0, 3) and plan(2, 1, 64, 64) == 0
+
+
 def test_quantize_contracts():
     """Malformed calls are rejected before the device is touched (pack.hpp:64-72,
     mx.hpp:71-76, kvcache.hpp:60-68, kvfp8.hpp:70-79)."""

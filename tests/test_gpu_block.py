@@ -36,20 +36,21 @@ def _check(fn, view, w_ref, x, M, N, K, seed):
     assert orc.rel_l2(got, ref) <= TOL
 
 
-# (M, N, K): which block the planner picks on 256 compute units
+# (M, N, K): rows of x and of W that end inside a block or a tile, short and long K.  (test_every_block names the
+# block; those marked * are another kernel's for most group sizes, and hooked and unhooked calls agree there too.)
 SHAPES = [
-    (3, 528, 4352),     # one tile of W a workgroup, half a unit at the end of some waves
-    (16, 4096, 2304),   # the same, whole tiles of x; the last wave has one unit
+    (3, 528, 4352),     # * long-K kernel
+    (16, 4096, 2304),   # * long-K kernel
     (9, 8208, 4384),    # 64 x 16 blocks at the resident kernel's widths, ragged N and K
     (17, 272, 256),     # one unit: seven waves have none; N ends inside a block
-    (33, 528, 4096),    # two tiles of x, the third row of tiles one row high
+    (33, 528, 4096),    # one tile of W a workgroup, two tiles of x, the third row of tiles one row high
     (48, 2064, 2336),   # K ends inside a chunk, in a unit of its own
     (100, 4096, 1152),  # 32 x 64 blocks; half a unit at the end
-    (128, 6144, 512),   # 48 x 64 blocks
-    (96, 8208, 1024),   # 64 x 32 and larger blocks, ragged N
-    (190, 4112, 2304),  # 64 x 64
-    (150, 11008, 2048), # 64 x 80
-    (333, 4080, 2176),  # 64 x 96, rows end inside a block
+    (128, 6144, 512),   # * direct-to-LDS tiles; gs = 32 with zero-points: 48 x 64 blocks
+    (96, 8208, 1024),   # * the same; 64 x 96 blocks
+    (190, 4112, 2304),  # * the same; 64 x 64
+    (150, 11008, 2048), # * direct-to-LDS tiles (two rounds of blocks)
+    (333, 4080, 2176),  # * direct-to-LDS tiles
 ]
 
 
@@ -98,7 +99,7 @@ def test_block_shapes_add_in_one_order():
         assert np.array_equal(got, full[:M]), M
 
 
-@pytest.mark.parametrize("M,N,K", [(100, 4096, 384), (33, 528, 2176), (16, 4096, 2400), (200, 4096, 4224)])
+@pytest.mark.parametrize("M,N,K", [(60, 2064, 384), (33, 528, 2176), (16, 4096, 2400), (200, 4096, 4224)])
 @pytest.mark.parametrize("kind", ["mx", 32, 64, 128])
 def test_last_group_near_the_largest_half(M, N, K, kind):
     """K ends inside a unit and the row's last group is the only one with weights near 65504: codes of
@@ -156,3 +157,54 @@ def test_whole_chunk_groups_keep_their_scales_out_of_fp16(M, N, K, gs, sym):
     got = np.ascontiguousarray(bits(out).reshape(M, N)[:, ns])
     moved = np.mean(got != exact.astype(np.float16).view(np.uint16))
     assert moved <= 0.04, moved
+
+
+# every block of every format: M ends inside a block and inside a row tile, N inside a block, K inside a unit
+# (1152, 2176: after its first chunk; 2336, 2400: inside a chunk)
+BLOCKS = [
+    (11, 89, 256, 1152), (21, 227, 272, 2176), (22, 401, 272, 2336), (22, 276, 528, 2336), (24, 373, 528, 2336), (24, 377, 1040, 2336),
+    (34, 409, 1040, 2400), (41, 75, 2720, 1152), (41, 345, 272, 2336), (42, 91, 4192, 1152), (42, 406, 528, 2336),
+    (44, 412, 1568, 2336), (45, 391, 2160, 2336), (46, 403, 2608, 2336)]
+
+
+@pytest.mark.parametrize("fmt,gs", [(0, 32), (0, 64), (0, 128), (1, 32), (1, 64), (1, 128), (2, 32)])
+@pytest.mark.parametrize("block,M,N,K", BLOCKS)
+def test_every_block(block, M, N, K, fmt, gs):
+    c = w4amd.capi()
+    got = c.gemm_plan_for(fmt, M, N, K, gs)
+    if got != block:  # four of the blocks need other sizes with MXFP4, whose costs differ
+        assert (fmt == 2 or block in (22, 24, 41, 42)) and got > 10, (got, block)
+        return
+    seed = M + N + K + gs + fmt
+    x = orc.normal_activations(M * K, seed + 1)
+    if fmt == 2:
+        p = orc.quantize_mx(orc.outlier_weights(N, K, seed), N, K)
+        dp = DevPackedMx(p)
+        return _check(c.gemm_mx, dp.view, orc.dequant_all_mx(p), x, M, N, K, seed)
+    p = orc.quantize(orc.normal_weights(N * K, seed) * 0.02 + 0.01 * fmt, N, K, gs, fmt == 0)
+    dp = DevPacked(p)
+    _check(c.gemm, dp.view, orc.dequant_all(p), x, M, N, K, seed)
+
+
+def test_every_block_is_listed():
+    """Each block of each format, with groups inside a chunk and with whole chunks, is one that the test above runs."""
+    plan = w4amd.capi().gemm_plan_for
+    for fmt, gs in [(0, 32), (0, 64), (0, 128), (1, 32), (1, 64), (1, 128), (2, 32)]:
+        seen = {block for block, M, N, K in BLOCKS if plan(fmt, M, N, K, gs) == block}
+        assert seen == {11, 21, 22, 24, 34, 41, 42, 44, 45, 46}, (fmt, gs, seen)
+
+
+def test_plan_lines():
+    """Where blocks measured slower than the kernel before them that kernel has the call, and the other way
+    round: (format, M, N, K, gs) on both sides of the lines."""
+    plan = w4amd.capi().gemm_plan_for
+    other = [(0, 3, 128, 5120, 128), (0, 3, 4096, 6144, 64), (0, 7, 1024, 4224, 128), (0, 11, 128, 2304, 64),
+             (0, 14, 1024, 4096, 128), (2, 3, 128, 4224, 32), (0, 4, 11008, 13824, 64), (0, 3, 11008, 6144, 32),
+             (0, 17, 3952, 1920, 128), (0, 42, 2800, 1152, 64), (0, 72, 8192, 1152, 128), (2, 146, 6144, 2304, 32),
+             (2, 2857, 288, 11904, 32), (2, 1256, 544, 4608, 32), (0, 984, 8192, 1088, 64), (0, 895, 8192, 5120, 96),
+             (0, 28, 8736, 512, 128), (0, 236, 28672, 1088, 128), (2, 503, 16384, 1088, 32)]
+    assert [a for a in other if plan(*a) > 9] == []
+    blocks = [(2, 50, 4096, 14336, 32), (1, 333, 4096, 4096, 64), (0, 16, 4096, 14336, 128), (0, 128, 4096, 4096, 128),
+              (0, 64, 5120, 13824, 128), (0, 448, 3072, 9760, 128), (0, 7, 4096, 13824, 64), (2, 12, 8192, 8192, 32),
+              (0, 667, 13824, 5120, 96), (1, 1140, 5120, 13824, 96), (0, 89, 4096, 1152, 128), (1, 82, 6560, 1664, 32)]
+    assert [a for a in blocks if plan(*a) < 10] == []

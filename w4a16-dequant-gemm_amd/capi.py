@@ -72,6 +72,7 @@ SIGNATURES = {
     "w4_gemm_mx_w4a4": ([C.POINTER(PackedMxView), C.POINTER(PackedMxView), vp, vp], C.c_int),
     "w4_quantize_mx8_f16": ([C.POINTER(ActMx8View), vp, vp, vp], C.c_int),
     "w4_gemm_mx_w4a8": ([C.POINTER(PackedMxView), C.POINTER(ActMx8View), vp, vp], C.c_int),
+    "w4_gemm_plan_for": ([C.c_int] * 5 + [C.POINTER(C.c_int)], C.c_int),
     "w4_gemm_mx_plan_for": ([C.c_int] * 4 + [C.POINTER(C.c_int)], C.c_int),
     "w4_quantize_cache": ([C.POINTER(KVView), vp, vp, C.c_int, vp, vp], C.c_int),
     "w4_quantize_cache_f8": ([C.POINTER(KVF8View), vp, vp, C.c_int, vp, vp], C.c_int),
@@ -244,6 +245,13 @@ def quantize_mx8_f16(view, x, status, stream=0):
 def gemm_mx_w4a8(w_view, x_view, c, stream=0):
     """MXFP4 weights against MXFP8 activations (x_view.M rows); scaled matrix cores."""
     check(load().w4_gemm_mx_w4a8(C.byref(w_view), C.byref(x_view), _n(c), _n(stream)))
+
+
+def gemm_plan_for(fmt, M, N, K, gs=32):
+    """10 x tiles of W + row tiles of a block / 1 long-K / 2 resident / 3 general decode kernel / 0 others"""
+    plan = C.c_int()
+    check(load().w4_gemm_plan_for(fmt, M, N, K, gs, C.byref(plan)))
+    return plan.value
 
 
 def gemm_mx_plan_for(x8, M, N, K):

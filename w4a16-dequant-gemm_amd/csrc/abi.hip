@@ -564,6 +564,17 @@ int w4_gemm_mx_w4a8(const w4_packed_mx_view* w, const w4_act_mx8_view* x, w4_hal
   return done("gemm_mx_w4a8", w4k::launch_gemm_mx_w4a8(*w, *x, c, (hipStream_t)stream));
 }
 
+int w4_gemm_plan_for(int fmt, int M, int N, int K, int gs, int* plan) {
+  REQUIRE(plan && M >= 1 && N >= 1 && K >= 1, "gemm plan: bad dims");
+  REQUIRE(fmt >= 0 && fmt <= 2 && (fmt == 2 || (gs >= 8 && gs % 8 == 0)), "gemm plan: bad format");
+  w4k::WView v{};
+  v.mx = fmt == 2, v.N = N, v.K = K, v.symmetric = fmt != 1;
+  v.gs = fmt == 2 ? 32 : gs;
+  v.G = v.B = (K + v.gs - 1) / v.gs;
+  *plan = w4k::gemm_plan(v, M);
+  return W4_OK;
+}
+
 int w4_gemm_mx_plan_for(int x8, int M, int N, int K, int* plan) {
   REQUIRE(plan && M >= 1 && N >= 1 && K >= 1, "mx plan: bad dims");
   *plan = w4k::mx_plan(x8 != 0, M, N, K);

@@ -1,4 +1,4 @@
-// W4A16 / MXFP4 GEMM for middle M (9 to a few hundred rows, at long K from 3 on): a workgroup owns a block of
+// W4A16 / MXFP4 GEMM for middle M (9 to some hundred rows, at long K from 3 on): a workgroup owns a block of
 // 16 NT rows of W x 16 MT activation rows, its eight waves split K.  mma.cuh:63-230 is the
 // reference's kernel for this path.
 //
@@ -496,23 +496,84 @@ int bk_cus() {
   return n;
 }
 
+// Few rows (M < 17) and at most one tile of W a compute unit, K in whole chunks: the longest K that stays with the long-K
+// kernel, which fetches only the quads of x that exist and has no parameters to wait for.  [symmetric W4, with
+// zero-points, MXFP4][M up to 4, 8, 12, 16][tiles for half of the compute units, or more].  M = 3: N = 128, K = 5120 5.5 us
+// against 4.5, N = 4096, K = 6144 7.3 against 6.4; M = 7: N = 1024, K = 4224 6.0 against 5.2; M = 11: N = 128, K = 4352 5.0
+// against 4.7.  At K = 14336 blocks are 1.05 (M = 4) to 1.3 times (M = 16) as fast.
+constexpr int BK_LONGEST[3][4][2] = {{{1 << 30, 10240}, {8192, 6144}, {6144, 0}, {5120, 0}},
+                                     {{6144, 5120}, {6143, 5120}, {4608, 0}, {4096, 0}},
+                                     {{9216, 7168}, {6144, 5120}, {5120, 0}, {4096, 0}}};
+
+// Whether blocks of shape s in `rounds` rounds of workgroups are ahead of the kernel that has the call otherwise.
+// That kernel is told apart by the same arithmetic as in the dispatcher and the kernels' own rules. The lines come
+// from 10800 shapes of 3 to 3000 rows, both kernels timed in turn.  Few tiles or a short K leave a block its start
+// and the sum of eight waves.
+bool block_ahead(const WView& v, int M, const BkShape& s, long long rounds, bool dma, int cus) {
+  const int tiles = v.N / 16, area = s.nt * s.mt, units = (v.K + BK_UNIT - 1) / BK_UNIT, K = v.K;
+  const bool whole = K % 128 == 0, sym = !v.mx && v.symmetric;
+  if (M < 17) {
+    // up to 8 rows in blocks of 64: N = 11008, K = 13824, M = 4 37.6 us against 32.5 (M = 13 36.3 against 49.6)
+    if (s.mt > 1 && M < 9) return false;
+    // MXFP4 in no whole chunks: behind on a few tiles of a short row only (N = 128, K = 4128, M = 5 4.7 us against 4.3)
+    if (!whole) return !v.mx || 8 * tiles >= cus || K >= (M < 9 ? 6144 : 3072);
+    // four tiles of symmetric W4, whose expansion bounds them, for 3 or 4 rows, where the other kernel has up to three
+    // rounds: N = 11008, K = 6144 15.5 against 14.1 (N = 13824, K = 5120 14.5 against 17.0)
+    if (tiles > cus) return s.nt < 4 || M > 4 || !sym || tiles > 3 * cus;
+    if (K < 4096) return false;  // M = 11: N = 128, K = 2304 4.4 against 4.0; M = 14: N = 1024, K = 3072 5.1 against 4.6
+    return K > BK_LONGEST[v.mx ? 2 : sym ? 0 : 1][(M - 1) / 4][2 * tiles >= cus];
+  }
+  if (whole && M <= 64 && tiles <= cus && K > 1024 && K != 2048 && K != 4096) {
+    // the long-K kernel again: N = 2576, K = 1664, gs = 96, M = 43 7.9 us in two rounds against 5.7; more than one tile
+    // a block where it has one a compute unit: N = 3952, K = 1920, M = 17 5.7 against 4.9, K = 2688 6.4 against 5.7
+    if (rounds > 1) return false;
+    return 2 * tiles <= cus || area < 2 || K >= (area == 2 && !v.mx ? 3072 : 2048);
+  }
+  if (M >= 65 && dma && (long long)((v.N + 255) / 256) * ((M + 127) / 128) >= 8) {
+    // Direct-to-LDS tiles.  A block's size is bounded by the units of K it has to work through: K = 1152, N = 8192, M = 72
+    // 10.5 us against 8.5 (64 x 64), N = 4096, M = 89 7.4 against 8.7 (32 x 64); nine units are two for one wave and
+    // one for the others: K = 2304, N = 6144, M = 146 12.4 against 9.9.
+    // N = 288, K = 11904, M = 2857 84.6 against 57.4; N = 544, K = 4608 (18 units), M = 1256 21.1 against 18.5
+    if (M > 1536 || (M > 1024 && v.N >= 256 && 32 * ((units + 7) / 8) > 5 * units)) return false;
+    // gs = 32 with zero-points has tiles of 256 rows of W only there: N = 6560, K = 1664, M = 82 10.7 against 18.3
+    if (!v.mx && !sym && v.gs == 32) return units > 1 || area <= 2;
+    constexpr int largest[14] = {0, 2, 2, 4, 8, 8, 12, 12, 24, 12, 20, 20, 20, 20};
+    return units > 13 || area <= largest[units];
+  }
+  // What those tiles do not take; several rounds pay there as well (K = 9760, N = 3072, M = 448: 105 -> 69 us in two).
+  if (M >= 96 && K % 64 == 0) {
+    // Register-staged tiles of 256 x 128, which are ahead where they fill their own rounds.  In rounds of 64 x 96 blocks:
+    // N = 8192, K = 1088, M = 984 69 us in four against 38; K = 5120, gs = 96, M = 895 121 in five against 104 (256
+    // tiles), N = 13824, M = 667 132 in six against 182 (324); N = 5120, K = 13824, M = 1140 211 in four against 270.
+    const long long others = (long long)((M + 255) / 256) * ((v.N + 127) / 128), other_rounds = (others + cus - 1) / cus;
+    if (8 * others < cus) return true;
+    const long long load = rounds * (v.mx ? s.cost_mx : s.cost_w4), r = (load + 329) / 330;
+    constexpr int shortest[5] = {0, 0, 512, 1024, 2304};
+    return K >= (r < 5 ? shortest[r] : 3072) && (r < 4 || load < (K < 6144 ? 1320 : 1980) * other_rounds);
+  }
+  // The stream kernel.  N = 8736, K = 512, M = 28 6.0 us in 64 x 32 blocks against 4.6; N = 1120, K = 256, M = 45 in
+  // 64 x 16 4.5 against 4.7; N = 592, K = 9248, M = 2834 144 in three rounds against 119
+  if (rounds == 1) return area <= (K <= 512 ? 4 : K < 768 ? 12 : 24);
+  return K >= (rounds == 2 ? 768 : 1024) && (M <= 1536 || rounds == 2);
+}
+
 // The block that covers the call in the least time (rounds of workgroups x cost of one), as an index into
 // BK_SHAPES; -1: none, or another kernel is ahead.
 int block_plan(const WView& v, int M) {
   if (M < 3 || M > 8192 || (M < 9 && v.K <= 4096) || (M < 17 && v.K <= 2048)) return -1;
   if (v.K % 32 || v.N % 16 || (!v.mx && v.gs % 32)) return -1;
+  if (v.K >= 1 << 24) return -1;  // offsets inside a block have 32 bits
   const int cus = bk_cus();
   if (cus < 8) return -1;
-  // Few rows: one 16-row tile of W a workgroup from M = 9 on (N = K = 4096, M = 8 / 12 / 16: 5.2 / 5.3 / 5.4 against
+  // Few rows: one 16-row tile of W a workgroup (N = K = 4096, M = 8 / 12 / 16: 5.2 / 5.3 / 5.4 against
   // 5.0 / 5.5 / 5.8 us; K = 2048, M = 16 4.2 against 3.9), wider matrices at long K only (N = 11008, K = 4096,
   // M = 16 9.4 against 7.7 us).  (Ruled out first: calls this short see host time.)
   if (M < 17 && v.K <= 4096 && v.N > 16 * cus) return -1;
-  // Several rounds only pay against the register-staged tile and stream kernels, which take what the
-  // direct-to-LDS tile kernel leaves (K = 9760, N = 3072, M = 448: 105 -> 69 us in two rounds; at K = 8192, N = 8192,
-  // M = 256, which is that kernel's, two rounds take 50 us against 48).
+  // The direct-to-LDS tile kernel's operands: one round of workgroups only (K = 8192, N = 8192, M = 256: two take 50 us
+  // against its 48).
   const bool dma = v.K % 128 == 0 && (v.mx || v.gs == 32 || v.gs == 64 || v.gs % 128 == 0);
   int best = -1;
-  long long least = 0;
+  long long least = 0, best_rounds = 0;
   for (int i = 0; i < (int)(sizeof BK_SHAPES / sizeof BK_SHAPES[0]); ++i) {
     const BkShape& s = BK_SHAPES[i];
     if (bk_lds_bytes(v, s.nt) > BK_MAX_LDS) continue;
@@ -520,9 +581,9 @@ int block_plan(const WView& v, int M) {
     const long long per_xcd = (ng + 7) / 8 * mg, rounds = (per_xcd + cus / 8 - 1) / (cus / 8);
     if (rounds > (dma || M < 17 ? 1 : 8)) continue;
     const long long cost = rounds * (v.mx ? s.cost_mx : s.cost_w4);
-    if (best < 0 || cost < least) best = i, least = cost;
+    if (best < 0 || cost < least) best = i, least = cost, best_rounds = rounds;
   }
-  if (best < 0) return -1;
+  if (best < 0 || !block_ahead(v, M, BK_SHAPES[best], best_rounds, dma, cus)) return -1;
   if (!dma) return best;
   // One round at K of one or two units a wave and many rows: N = 4096, K = 1024, M = 192 7.8 against 6.9 us,
   // K = 2048, M = 333 12.1 against 10.9.
@@ -551,6 +612,11 @@ hipError_t block_fmt(int shape, const WView& v, const w4_half* x, w4_half* c, in
 }
 
 }  // namespace
+
+int block_shape(const WView& v, int M) {
+  const int i = block_plan(v, M);
+  return i < 0 ? 0 : 10 * BK_SHAPES[i].nt + BK_SHAPES[i].mt;
+}
 
 bool try_block(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out, hipError_t* err) {
   if (((uintptr_t)v.q | (uintptr_t)v.scales | (uintptr_t)v.zeros | (uintptr_t)x | (uintptr_t)c | (uintptr_t)w_out) & 15)

@@ -943,6 +943,14 @@ static hipError_t launch_fmt(const WView& v, const w4_half* x, w4_half* c, int M
   return launch_tiles<MX, 4>(v, x, c, M, s, w_out);
 }
 
+int gemm_plan(const WView& v, int M) {
+  if (const int shape = block_shape(v, M)) return shape;
+  if (v.K % 32 == 0 && decode_longk_applies(v, nullptr, nullptr, M)) return 1;
+  if (v.K % 32 == 0 && decode_resident_applies(v, nullptr, nullptr, M)) return 2;
+  if (!v.mx && decode_general_applies(v, nullptr, nullptr, M)) return 3;
+  return 0;
+}
+
 hipError_t launch_gemm_mfma(const WView& v, const w4_half* x, w4_half* c, int M,
                             hipStream_t s, w4_half* w_out) {
   return v.mx ? launch_fmt<1>(v, x, c, M, s, w_out) : launch_fmt<0>(v, x, c, M, s, w_out);

@@ -38,6 +38,8 @@ hipError_t launch_gemm_simt(const WView& v, const w4_half* x, w4_half* c, int M,
 // gemm_mfma.hip
 hipError_t launch_gemm_mfma(const WView& v, const w4_half* x, w4_half* c, int M,
                             hipStream_t s, w4_half* w_out);
+// Which kernel it takes, without a hook, for operands aligned to 16 bytes: see w4_gemm_plan_for.
+int gemm_plan(const WView& v, int M);
 
 // gemm_tile_dma.hip: large-M W4 kernel with direct-to-LDS operand loads; false
 // (nothing launched) when the arguments are not its shape.
@@ -50,10 +52,12 @@ bool try_tile_dma(const WView& v, const w4_half* x, w4_half* c, int M, hipStream
 bool try_tile256(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, int cus,
                  hipError_t* err);
 
-// gemm_block.hip: middle M (17 to a few hundred rows), blocks of W and x as square as one round of
-// workgroups allows, hooked calls included; false (nothing launched) when another kernel is ahead.
+// gemm_block.hip: middle M (17 to some hundred rows, at long K from 3 on), blocks of W and x as square as few rounds
+// of workgroups allow, hooked calls included; false (nothing launched) when another kernel is ahead.
 bool try_block(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out,
                hipError_t* err);
+// Its block for operands aligned to 16 bytes: 10 x tiles of W + row tiles of x; 0: not its shape.
+int block_shape(const WView& v, int M);
 
 // gemm_decode_resident.hip: M <= 64 with the activations fetched once per workgroup
 // (several 16-row tiles each).  Same order of additions as the K-split decode
