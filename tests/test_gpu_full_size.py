@@ -97,7 +97,8 @@ def test_c3_mxfp4_outliers_n14336():
                                       (13824, True, (32,))])
 def test_long_k_two_tiles_per_workgroup(K, sym, Ms):
     """Long K on a grid of more 16-row tiles than compute units (N = 4128: 258) with more than 16
-    activation rows: two tiles share a workgroup's activations.  Hook bytes on the device, sampled
+    activation rows: a round of blocks (two tiles that share a resident workgroup's activations are in
+    test_gpu_gemm.py::test_long_k_tiles_that_share_their_activations).  Hook bytes on the device, sampled
     outputs against the oracle, hooked against unhooked within the cross gate."""
     c = w4amd.capi()
     N, gs = 4128, 128

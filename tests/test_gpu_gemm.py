@@ -334,11 +334,94 @@ def test_unhooked_kernels_with_one_signed_and_offset_activations(shape):
             cross_gate(ch, cu, ref, name)
 
 
+def _past_the_blocks(call, view, x, M, N):
+    """Unhooked output of the decode kernels for shapes that aligned calls take to blocks: c is only 8-byte aligned."""
+    out = halves(M * N + 8, 0x7E00)
+    call(view, ptr(to_dev(x)), ptr(out) + 8, M, 0, 0)
+    got = bits(out)
+    assert (got[:4] == 0x7E00).all() and (got[M * N + 4:] == 0x7E00).all()
+    return got[4:M * N + 4]
+
+
+@pytest.mark.parametrize("fmt", ["w4", "w4z", "mx"])
+@pytest.mark.parametrize("K", [1152, 3072, 3968, 5120, 5248, 6144, 7168, 8192, 9216, 10240, 11008, 12288, 13312, 14336, 15360, 16384])
+def test_long_k_kernel_at_every_depth(K, fmt):
+    """The long-K kernel's instantiations, 2 to 16 chunks a wave (K = 1152 and 9216: the last waves own fewer), 3 to 64 rows."""
+    c = w4amd.capi()
+    N = 48
+    w = orc.normal_weights(N * K, 0x10F0 + K) * 0.02 + (0.01 if fmt == "w4z" else 0.0)
+    p = orc.quantize_mx(w, N, K) if fmt == "mx" else orc.quantize(w, N, K, 64, fmt == "w4")
+    dp, call = (DevPackedMx(p), c.gemm_mma_mx) if fmt == "mx" else (DevPacked(p), c.gemm_mma)
+    w_ref = orc.dequant_all_mx(p) if fmt == "mx" else orc.dequant_all(p)
+    x = orc.normal_activations(64 * K, 0x10F1 + K)
+    ref = orc.gemm_oracle(x, 64, K, w_ref, N).reshape(64, N)
+    for M in (3, 7, 11, 16, 24, 40, 52, 64):
+        if (K, fmt, M) == (16384, "w4z", 24):
+            continue  # a test of captured calls is the first to ask for this one's LDS
+        got = _past_the_blocks(call, dp.view, x[:M * K], M, N)
+        assert orc.rel_l2(got.view(np.float16), ref[:M].ravel()) <= 5e-4, M
+
+
+@pytest.mark.parametrize("K,sym,Ms", [(8192, True, (13, 24, 64)), (8192, False, (32, 64)), (11008, False, (24,)),
+                                      (13824, True, (32,)), (8192, None, (24, 64))])
+def test_long_k_tiles_that_share_their_activations(K, sym, Ms):
+    """The resident kernel at long K on a grid of more 16-row tiles than compute units (None: MXFP4): two tiles a
+    workgroup.  Aligned calls have it from N = 16400 on, where blocks are no single round."""
+    c = w4amd.capi()
+    N = 4128
+    fmt = 2 if sym is None else 0 if sym else 1
+    assert c.gemm_plan_for(fmt, 32, 16400, 8192, 128) == 2
+    w = orc.normal_weights(N * K, 0x110C + K) * 0.02 + (0.01 if fmt == 1 else 0.0)
+    p = orc.quantize_mx(w, N, K) if sym is None else orc.quantize(w, N, K, 128, sym)
+    dp, call = (DevPackedMx(p), c.gemm_mma_mx) if sym is None else (DevPacked(p), c.gemm_mma)
+    w_ref = (orc.dequant_all_mx(p) if sym is None else orc.dequant_all(p)).reshape(N, K)
+    ns = np.unique(np.random.default_rng(K).choice(N, size=96))
+    for M in Ms:
+        x = orc.normal_activations(M * K, 0x110D + M)
+        got = _past_the_blocks(call, dp.view, x, M, N).reshape(M, N)
+        rows = np.array([0, M // 3, M - 1])
+        ref = orc.gemm_oracle(np.ascontiguousarray(x.reshape(M, K)[rows]), 3, K, np.ascontiguousarray(w_ref[ns]), len(ns))
+        assert orc.rel_l2(np.ascontiguousarray(got[rows][:, ns]).view(np.float16), ref) <= 5e-4, M
+
+
+@pytest.mark.parametrize("sym", [True, False])
+def test_wide_long_k_calls_without_a_round_of_blocks(sym):
+    """Aligned calls that go to the long-K and the resident kernel: more than 1024 tiles of W."""
+    c = w4amd.capi()
+    N, K, gs = 16400, 4224, 64
+    p = orc.quantize(orc.normal_weights(N * K, 0x110E) * 0.02 + (0.0 if sym else 0.01), N, K, gs, sym)
+    dp, w_ref = DevPacked(p), orc.dequant_all(p).reshape(N, K)
+    ns = np.unique(np.concatenate([[0, N - 1], np.random.default_rng(1).choice(N, size=96)]))
+    for M, plan in ((5, 1), (8, 1)):
+        assert c.gemm_plan_for(0 if sym else 1, M, N, K, gs) == plan, M
+        x = orc.normal_activations(M * K, 0x110F + M)
+        out = halves(M * N, 0x7E00)
+        c.gemm_mma(dp.view, ptr(to_dev(x)), ptr(out), M, 0, 0)
+        ref = orc.gemm_oracle(x, M, K, np.ascontiguousarray(w_ref[ns]), len(ns))
+        got = np.ascontiguousarray(bits(out).reshape(M, N)[:, ns])
+        assert orc.rel_l2(got.view(np.float16), ref) <= 5e-4, M
+
+
+@pytest.mark.parametrize("N,K,sym", [(1024, 4096, True), (1024, 4096, False), (512, 11008, True)])
+def test_resident_kernel_with_one_signed_and_offset_activations(N, K, sym):
+    """The bias sums of the resident kernel's gs = 128 form at 24 rows, for activations with a large mean."""
+    c = w4amd.capi()
+    M = 24
+    p = orc.quantize(orc.normal_weights(N * K, 0x0FF5E7) * 0.02, N, K, 128, sym)
+    dp, w_ref = DevPacked(p), orc.dequant_all(p)
+    rng = np.random.default_rng(6)
+    for x64 in (np.abs(rng.standard_normal(M * K)), 30 + rng.standard_normal(M * K),
+                1000 * np.abs(rng.standard_normal(M * K)), np.ones(M * K)):
+        x = np.asarray(x64, np.float16).view(np.uint16)
+        got = _past_the_blocks(c.gemm_mma, dp.view, x, M, N)
+        assert orc.rel_l2(got.view(np.float16), orc.gemm_oracle(x, M, K, w_ref, N)) <= 5e-4
+
+
 @pytest.mark.parametrize("fmt", ["w4", "w4z", "mx"])
 @pytest.mark.parametrize("K", [14336, 10368, 8192, 5120, 3072])
 def test_long_k_rows_that_do_not_fill_the_last_tile(K, fmt):
-    """Long K, 33 to 64 activation rows: three row tiles, and four with half of the last one's rows
-    fetched.  A row's bytes do not depend on how many others there are; nothing is stored past
+    """Long K, 33 to 64 activation rows (blocks of one tile of W at these sizes; the long-K kernel's row tiles are in
+    test_long_k_kernel_at_every_depth).  A row's bytes do not depend on how many others there are; nothing is stored past
     the last one."""
     c = w4amd.capi()
     N = 48

@@ -16,8 +16,7 @@ from devutil import DevKV, DevPacked, bits, halves, ptr, to_dev
 
 pytestmark = pytest.mark.gpu
 
-# (M, N, K, gs, symmetric): decode shape, decode batch, thin grid of small tiles, long K (two row tiles:
-# the pipelined kernel asks for its 128 KB of LDS on first use, inside the capture)
+# (M, N, K, gs, symmetric): decode shape, decode batch, thin grid of small tiles, long K (a block kernel)
 GEMMS = [(1, 256, 4096, 128, True), (8, 4128, 2048, 64, False), (100, 256, 2048, 128, True),
          (24, 64, 11008, 128, False)]
 
@@ -46,6 +45,28 @@ def test_gemm_replays_equal_eager_calls(i):
         c.gemm(dp.view, ptr(x_d), ptr(out_e), M, 0, 0)
         torch.cuda.synchronize()
         assert np.array_equal(bits(out_g), bits(out_e)), f"replay {rep} differs from the eager call"
+
+
+def test_first_call_of_a_pipelined_kernel_inside_a_capture():
+    """Two row tiles at sixteen chunks a wave: the long-K kernel asks for its 128 KB of LDS on first use, inside the
+    capture.  (c is 8-byte aligned only, so that the call is not a block kernel's.)"""
+    c = w4amd.capi()
+    M, N, K = 24, 64, 16384
+    p = orc.quantize(orc.normal_weights(N * K, 77), N, K, 128, False)
+    dp = DevPacked(p)
+    x_d = to_dev(orc.normal_activations(M * K, 78))
+    out_g, out_e = halves(M * N + 4, 0x7E00), halves(M * N + 4, 0x7E00)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        c.gemm(dp.view, ptr(x_d), ptr(out_g) + 8, M, torch.cuda.current_stream().cuda_stream, 0)
+    for rep in range(3):
+        x_d.copy_(to_dev(orc.normal_activations(M * K, 80 + rep)))
+        out_g.fill_(0x7E00)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        c.gemm(dp.view, ptr(x_d), ptr(out_e) + 8, M, 0, 0)
+        assert np.array_equal(bits(out_g), bits(out_e)), rep
 
 
 # matrix-core flash kernel (D = 128) and the vector flash kernel (D = 96, zero-points)
