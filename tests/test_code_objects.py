@@ -80,3 +80,16 @@ def test_wave64_and_workgroup_sizes(kernels):
         assert k[".wavefront_size"] == 64
         assert k[".max_flat_workgroup_size"] <= 1024
         assert k.get(".group_segment_fixed_size", 0) <= 160 * 1024
+
+
+def test_direct_to_lds_loads_wait_for_m0():
+    """A load to LDS takes its address from M0, which needs one wait state between a scalar write and the load on
+    this architecture: the compiler puts an s_nop between its own, and knows nothing of the ones inside an asm."""
+    csrc = os.path.join(ROOT, "w4a16-dequant-gemm_amd", "csrc")
+    found = 0
+    for name in sorted(os.listdir(csrc)):
+        text = open(os.path.join(csrc, name)).read()
+        for m in re.finditer(r"s_mov_b32 m0, %\d(.{0,20})", text):
+            assert m.group(1).startswith("\\n\\ts_nop 0\\n"), (name, m.group(0))
+            found += 1
+    assert found >= 13

@@ -621,10 +621,10 @@ __global__ __launch_bounds__(FM_WAVES * 64) void flash_mfma_phase1(const FlashAr
     const int upos = lane / P, upiece = lane % P;
     const int odd = (int)((rows0 * G) & 1);  // one group per row: a slab may start in the middle of a dword
     auto dma16 = [](const void* base, uint32_t off, uint32_t lds) {
-      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(off), "s"(base), "s"(lds) : "memory", "m0");
     };
     auto dma4 = [](const void* base, uint32_t off, uint32_t lds) {
-      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(lds) : "memory", "m0");
     };
     const int last16 = (s1 - 1) & ~15;  // the last half tile that has a position below s1
     // row, in the slab, of the half tile that starts at position t (clamped to the last one)

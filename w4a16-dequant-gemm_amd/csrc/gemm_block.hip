@@ -56,8 +56,9 @@ __device__ __forceinline__ void bk_for(F&& f, std::integer_sequence<int, I...>) 
   (f(std::integral_constant<int, I>{}), ...);
 }
 
+// (One wait state between the write of M0 and the load that takes its LDS address from it.)
 __device__ __forceinline__ void bk_dma(uint32_t off, const void* base, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(dst) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(dst) : "memory", "m0");
 }
 
 // FMT: 0 W4 symmetric, 1 W4 with zero-points, 2 MXFP4.  G: groups (W4) or blocks (MXFP4) per row.

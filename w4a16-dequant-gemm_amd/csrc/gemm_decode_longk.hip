@@ -167,7 +167,7 @@ __global__ __launch_bounds__(LK_THREADS) void mfma_decode_longk_kernel(
       const uint32_t off = (uint32_t)min(row, M - 1) * (uint32_t)(K * 2) + (uint32_t)cidx * 256u +
                            (uint32_t)(((lane & 15) ^ r16) * 16);
       const uint32_t dst = region + (uint32_t)((u % NBUF) * SLOT + rq) * 1024u;
-      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                    :
                    : "v"(off), "s"(xb), "s"(dst)
                    : "memory", "m0");

@@ -280,7 +280,7 @@ __global__ __launch_bounds__(DR_THREADS) void mfma_decode_resident_kernel(
                                (uint32_t)((EXACT || cidx < nchunks) ? cidx : nchunks - 1) * 256u +
                                (uint32_t)(((lane & 15) ^ r16) * 16);
           const uint32_t dst = region + (uint32_t)((mt * CP + cc) * 4 + rq) * 1024u;
-          asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+          asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                        :
                        : "v"(off), "s"(xb), "s"(dst)
                        : "memory", "m0");

@@ -416,13 +416,13 @@ __global__ __launch_bounds__(DM_THREADS) void mxn_tile_dma_kernel(
   // wait for all of them before any LDS read) nor moves LDS reads across them; the
   // vmcnt waits below are by hand.  M0 carries the wave-uniform LDS address.
   auto dma16 = [](const void* gbase, uint32_t goff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
                  : "v"(goff), "s"(gbase), "s"(lds_addr)
                  : "memory", "m0");
   };
   auto dma4 = [](const void* gbase, uint32_t goff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                  :
                  : "v"(goff), "s"(gbase), "s"(lds_addr)
                  : "memory", "m0");
@@ -626,13 +626,13 @@ __global__ __launch_bounds__(D4_THREADS) void mxn_tile4_kernel(
   const char* xqb = (const char*)xq;
   const int stages = K >> 8;
   auto dma16 = [](const void* gbase, uint32_t goff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
                  : "v"(goff), "s"(gbase), "s"(lds_addr)
                  : "memory", "m0");
   };
   auto dma4 = [](const void* gbase, uint32_t goff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                  :
                  : "v"(goff), "s"(gbase), "s"(lds_addr)
                  : "memory", "m0");
@@ -885,13 +885,13 @@ __global__ __launch_bounds__(T8_THREADS) void mxn_tile8_kernel(
   const char* xqb = (const char*)xq;
   const int stages = K >> 8;
   auto dma16 = [](const void* gbase, uint32_t goff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
                  : "v"(goff), "s"(gbase), "s"(lds_addr)
                  : "memory", "m0");
   };
   auto dma4 = [](const void* gbase, uint32_t goff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                  :
                  : "v"(goff), "s"(gbase), "s"(lds_addr)
                  : "memory", "m0");
