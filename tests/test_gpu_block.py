@@ -134,7 +134,7 @@ def test_last_group_near_the_largest_half(M, N, K, kind):
     _check(fn, dp.view, w_ref, x, M, N, K, K)
 
 
-@pytest.mark.parametrize("M,N,K,gs,sym", [(9, 4096, 4096, 128, True), (32, 4096, 4096, 128, False), (17, 8192, 8192, 256, True),
+@pytest.mark.parametrize("M,N,K,gs,sym", [(9, 2048, 4096, 128, True), (32, 4096, 4096, 128, False), (17, 8192, 8192, 256, True),
                                           (32, 8192, 8192, 128, False), (24, 528, 4352, 4352, True), (200, 4096, 4224, 128, True),
                                           (333, 4080, 4096, 128, False)])
 def test_whole_chunk_groups_keep_their_scales_out_of_fp16(M, N, K, gs, sym):
@@ -202,9 +202,9 @@ def test_plan_lines():
              (0, 14, 1024, 4096, 128), (2, 3, 128, 4224, 32), (0, 4, 11008, 13824, 64), (0, 3, 11008, 6144, 32),
              (0, 17, 3952, 1920, 128), (0, 42, 2800, 1152, 64), (0, 72, 8192, 1152, 128), (2, 146, 6144, 2304, 32),
              (2, 2857, 288, 11904, 32), (2, 1256, 544, 4608, 32), (0, 984, 8192, 1088, 64), (0, 895, 8192, 5120, 96),
-             (0, 28, 8736, 512, 128), (0, 236, 28672, 1088, 128), (2, 503, 16384, 1088, 32)]
+             (0, 28, 8736, 512, 128), (0, 12, 4096, 4096, 128), (0, 236, 28672, 1088, 128), (2, 503, 16384, 1088, 32)]
     assert [a for a in other if plan(*a) > 9] == []
     blocks = [(2, 50, 4096, 14336, 32), (1, 333, 4096, 4096, 64), (0, 16, 4096, 14336, 128), (0, 128, 4096, 4096, 128),
               (0, 64, 5120, 13824, 128), (0, 448, 3072, 9760, 128), (0, 7, 4096, 13824, 64), (2, 12, 8192, 8192, 32),
-              (0, 667, 13824, 5120, 96), (1, 1140, 5120, 13824, 96), (0, 89, 4096, 1152, 128), (1, 82, 6560, 1664, 32)]
+              (0, 12, 4096, 4096, 64), (0, 667, 13824, 5120, 96), (1, 1140, 5120, 13824, 96), (0, 89, 4096, 1152, 128), (1, 82, 6560, 1664, 32)]
     assert [a for a in blocks if plan(*a) < 10] == []

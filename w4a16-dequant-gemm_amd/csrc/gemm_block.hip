@@ -522,6 +522,9 @@ bool block_ahead(const WView& v, int M, const BkShape& s, long long rounds, bool
     // rounds: N = 11008, K = 6144 15.5 against 14.1 (N = 13824, K = 5120 14.5 against 17.0)
     if (tiles > cus) return s.nt < 4 || M > 4 || !sym || tiles > 3 * cus;
     if (K < 4096) return false;  // M = 11: N = 128, K = 2304 4.4 against 4.0; M = 14: N = 1024, K = 3072 5.1 against 4.6
+    // W4 with whole-chunk groups, whose scales the resident kernel has in registers: N = K = 4096, gs = 128, M = 12 / 16
+    // 6.0 / 6.2 us against 5.6 / 6.0 (gs = 64 5.9 / 6.1 against 5.9 / 6.3)
+    if (K == 4096 && !v.mx && v.gs % 128 == 0 && 2 * tiles > cus) return false;
     return K > BK_LONGEST[v.mx ? 2 : sym ? 0 : 1][(M - 1) / 4][2 * tiles >= cus];
   }
   if (whole && M <= 64 && tiles <= cus && K > 1024 && K != 2048 && K != 4096) {
@@ -566,9 +569,9 @@ int block_plan(const WView& v, int M) {
   if (v.K >= 1 << 24) return -1;  // offsets inside a block have 32 bits
   const int cus = bk_cus();
   if (cus < 8) return -1;
-  // Few rows: one 16-row tile of W a workgroup (N = K = 4096, M = 8 / 12 / 16: 5.2 / 5.3 / 5.4 against
-  // 5.0 / 5.5 / 5.8 us; K = 2048, M = 16 4.2 against 3.9), wider matrices at long K only (N = 11008, K = 4096,
-  // M = 16 9.4 against 7.7 us).  (Ruled out first: calls this short see host time.)
+  // Few rows: one 16-row tile of W a workgroup (N = K = 4096, M = 8 5.2 against 5.0 us; K = 2048, M = 16 4.2 against
+  // 3.9), wider matrices at long K only (N = 11008, K = 4096, M = 16 9.4 against 7.7 us).  (Ruled out first: calls this
+  // short see host time.)
   if (M < 17 && v.K <= 4096 && v.N > 16 * cus) return -1;
   // The direct-to-LDS tile kernel's operands: one round of workgroups only (K = 8192, N = 8192, M = 256: two take 50 us
   // against its 48).
