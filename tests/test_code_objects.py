@@ -89,7 +89,7 @@ def test_direct_to_lds_loads_wait_for_m0():
     found = 0
     for name in sorted(os.listdir(csrc)):
         text = open(os.path.join(csrc, name)).read()
-        for m in re.finditer(r"s_mov_b32 m0, %\d(.{0,20})", text):
+        for m in re.finditer(r"s_\w+ m0, %\d(?:, %\d)?(.{0,20})", text):
             assert m.group(1).startswith("\\n\\ts_nop 0\\n"), (name, m.group(0))
             found += 1
     assert found >= 13

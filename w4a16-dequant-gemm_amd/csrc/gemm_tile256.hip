@@ -117,11 +117,11 @@ __global__ __launch_bounds__(T2_THREADS) void w4_tile256_kernel(
   // The loads are asm so that the compiler neither tracks them (it would wait for all of
   // them before any LDS read) nor moves LDS reads across them; the vmcnt waits below are
   // by hand.  M0 carries the wave-uniform LDS address.
-  auto dma16 = [](const void* gbase, uint32_t goff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+  auto dma16 = [](const void* gbase, uint32_t goff, uint32_t lds_addr, int lds_off) __attribute__((always_inline)) {
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
-                 : "v"(goff), "s"(gbase), "s"(lds_addr)
-                 : "memory", "m0");
+                 : "v"(goff), "s"(gbase), "s"(lds_addr), "i"(lds_off)
+                 : "memory", "m0", "scc");
   };
   auto dma4 = [](const void* gbase, uint32_t goff, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
@@ -138,10 +138,10 @@ __global__ __launch_bounds__(T2_THREADS) void w4_tile256_kernel(
     const uint32_t dd = (uint32_t)(d < stages ? d : stages - 1);
     const uint32_t st = lds0 + buf;
     if (part < WI) {  // the stage's offset goes into the scalar base: no vector arithmetic
-      dma16(wqb + dd * 32u, wo[part], st + (wave + WAVES * part) * 1024);
+      dma16(wqb + dd * 32u, wo[part], st + wave * 1024, WAVES * part * 1024);
     } else if (part < WI + XI) {
       const int i = part - WI;
-      dma16(xb + dd * 128u, xo[i], st + T2_W_BYTES + (wave + WAVES * i) * 1024);
+      dma16(xb + dd * 128u, xo[i], st + wave * 1024, T2_W_BYTES + WAVES * i * 1024);
     } else if (part == WI + XI) {
       // MXFP4: the dword around the stage's two E8M0 bytes; gs = 32: the dword of its two
       // scales; else the dword around its one scale

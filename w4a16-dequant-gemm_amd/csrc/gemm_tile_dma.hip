@@ -160,11 +160,11 @@ __global__ __launch_bounds__(TD_THREADS * KG) void w4_tile_dma_kernel(
   // The loads are asm so that the compiler neither tracks them (it would wait for
   // all of them before any LDS read) nor moves LDS reads across them; the vmcnt
   // waits below are by hand.  M0 carries the wave-uniform LDS address.
-  auto dma16 = [](const void* gbase, uint32_t goff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+  auto dma16 = [](const void* gbase, uint32_t goff, uint32_t lds_addr, int lds_off) __attribute__((always_inline)) {
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
-                 : "v"(goff), "s"(gbase), "s"(lds_addr)
-                 : "memory", "m0");
+                 : "v"(goff), "s"(gbase), "s"(lds_addr), "i"(lds_off)
+                 : "memory", "m0", "scc");
   };
   auto dma4 = [](const void* gbase, uint32_t goff, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
@@ -180,10 +180,10 @@ __global__ __launch_bounds__(TD_THREADS * KG) void w4_tile_dma_kernel(
     const uint32_t dd = (uint32_t)(d < d_end ? d : d_end - 1);  // past the set's end: valid, never used
     const uint32_t st = lds0 + buf;
     if (part < TD_WI) {  // the stage's offset goes into the scalar base: no vector arithmetic
-      dma16(wqb + dd * 64u, wo[part], st + (wave + TD_WAVES * part) * 1024);
+      dma16(wqb + dd * 64u, wo[part], st + wave * 1024, TD_WAVES * part * 1024);
     } else if (part < TD_WI + TD_XI) {
       const int i = part - TD_WI;
-      dma16(xb + dd * 256u, xo[i], st + TD_W_BYTES + (wave + TD_WAVES * i) * 1024);
+      dma16(xb + dd * 256u, xo[i], st + wave * 1024, TD_W_BYTES + TD_WAVES * i * 1024);
     } else {
       // the stage's scales of this wave's row 64 wave + lane: the dword with the one
       // FP16 scale (GSM 0), the dword of its two (GSM 1), the two dwords of its four
