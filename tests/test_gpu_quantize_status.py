@@ -3,6 +3,7 @@ condition that the host reports by throwing (pack.hpp:64-72, mx.hpp:71-76, kvcac
 wherever the element lies -- with one workgroup and with thousands, on several streams at once, and on
 every replay of a captured call."""
 import ctypes
+import threading
 
 import pytest
 import torch
@@ -188,6 +189,35 @@ def test_no_other_call_clears_the_word_again():
         call(k, v, ptr(st) + 8, s2.cuda_stream)
         torch.cuda.synchronize()
         assert st.tolist() == [BAD | RANGE, 0, 0]
+
+
+def test_threads_that_share_streams():
+    """Four threads that enqueue calls on the legacy stream and on one other stream, each call with a word of its own."""
+    stream = torch.cuda.Stream()
+    jobs = []
+    for i in range(4):
+        call, keep = _kv(KINDS[i], 2, 257, 128, 32)
+        k, v = _inputs(2, 257, 128)
+        bad = k.clone()
+        bad.view(-1)[1234 + i] = INF
+        jobs.append((call, keep, k, bad, v))
+    st = torch.full((4, 200), 0x44, dtype=torch.int32, device=DEV)
+    torch.cuda.synchronize()
+
+    def work(i):
+        call, _, k, bad, v = jobs[i]
+        for j in range(200):
+            call(bad if j % 3 == i % 3 else k, v, ptr(st) + 4 * (200 * i + j), stream.cuda_stream if j % 2 else 0)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i, row in enumerate(st.tolist()):
+        for j, x in enumerate(row):
+            assert bool(x & BAD) == (j % 3 == i % 3) and (x & BAD or x == 0), (i, j, x)
 
 
 def test_more_streams_than_slots():
