@@ -4,7 +4,9 @@
 //
 // What bounds these shapes is the path from L2 into a compute unit: it takes 1 KB per 7 - 10 ns
 // whatever lies in it, as long as the 4 (better 8) neighbouring lanes of a load instruction lie in
-// one line; a load in MFMA operand layout (neighbouring lanes in different rows) takes 28 ns.  So
+// one line; a load in MFMA operand layout (neighbouring lanes in different rows) takes 28 ns.  (A block
+// takes 15 ns a KB with its arithmetic: MXFP4, N = 4096, M = 50 2.0 us for each further unit of 256 k of the eight
+// waves, 128 KB, whether the codes come from memory or from a cache.)  So
 //   * the block is as square as the operands' sizes ask for: per k a workgroup moves 8 NT bytes of codes
 //     and 32 MT bytes of activations, N = 4096, M = 64: 64 B with 64 x 16 blocks against 136 with one
 //     16-row tile of W per workgroup and all of x;
@@ -478,7 +480,8 @@ hipError_t block_go(const WView& v, const w4_half* x, w4_half* c, int M, hipStre
 }
 
 // Blocks and what a wave needs for 128 k of one, in units of 10 ns, W4 and MXFP4 (N = 4096, K = 14336 with
-// as many rows as make one round of workgroups, and N = 5120, K = 13824; a call takes 3.5 us more).
+// as many rows as make one round of workgroups, and N = 5120, K = 13824; a call takes 3.5 us more).  Groups of whole
+// chunks cost 0.97 to 1.03 of it.
 struct BkShape {
   int nt, mt, cost_w4, cost_mx;
 };

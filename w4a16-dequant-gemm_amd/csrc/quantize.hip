@@ -353,8 +353,8 @@ __device__ __forceinline__ void load8(const _Float16* p, float v[8]) {
 // of a group combine their extrema with lane exchanges and every lane derives
 // the group's scale itself -- no LDS round trip, fully coalesced 16-byte loads.
 // Bound by vector instructions, not by memory: 8 slabs x 4096 x 128 FP16 keys and values (21.5 MB)
-// took 10.1 us a call with some 220 of them a thread and take 7.3 with 97 (6.7 are the two launches
-// of a call at S = 16); E4M3 bytes 12.4 -> 8.4.
+// took 10.1 us a call with some 220 of them a thread and 7.3 with 97 (E4M3 bytes 12.4 -> 8.4) while a launch of its
+// own cleared the status word, and take 5.3 (6.5) now (3.5 at S = 16, which is the launch).
 // ZPACK: zero-point words are assembled through LDS (G and the groups per workgroup both
 // multiples of 8, or whole rows per workgroup: cache rows); otherwise nibbles are OR-ed in
 // atomically, into words that a launch per side has cleared before (8 x 4096 x 128 with gs = 32:
@@ -628,8 +628,8 @@ __device__ __forceinline__ uint32_t pack_e2m1(const float* u) {
 // E2M1 codes, or (F8: the MXFP8 activation format, no host counterpart in the
 // reference; same block rule with 448 in place of 6) eight E4M3 bytes.  FP16 sources
 // were bound by vector instructions (seven compares and selects a code, the exponent in FP64):
-// 2048 x 4096 took 12.7 us a call into MXFP4 and 12.0 into MXFP8, and takes 6.4 and 7.0 with the
-// hardware conversions and the exponent from integer arithmetic (the two launches alone: 5.7).
+// 2048 x 4096 took 12.7 us a call into MXFP4 and 12.0 into MXFP8, 6.4 and 7.0 with the hardware conversions and
+// the exponent from integer arithmetic, and takes 5.0 and 5.7 since the status word has no launch of its own (16 rows: 3.3).
 template <typename T, bool FULL, bool F8>
 __global__ __launch_bounds__(QT) void quantize_mx_kernel(const T* __restrict__ src,
                                                          long long rows, int K, int B,
