@@ -228,8 +228,8 @@ int w4_quantize_cache_f8(const w4_kv_f8_view* out, const void* k, const void* v,
 /* Which kernel the matrix-core GEMM runs on the current GPU (no counterpart in the reference): fmt 0 W4
  * symmetric, 1 W4 with zero-points, 2 MXFP4 (gs ignored); no hook, arrays aligned to 16 bytes.  *plan: 10 x the
  * 16-row tiles of W + the row tiles of x of a block (11 .. 46); 1 the long-K decode kernel, 2 the one that keeps
- * the activations, 3 the one for odd group sizes and ragged K; 0 tiles, stream and the others.  Without a
- * GPU no kernel is told apart (0, or 3). */
+ * the activations, 3 the one for odd group sizes and ragged K; 0 tiles, stream and the others.  W4_ERUNTIME
+ * without a GPU. */
 int w4_gemm_plan_for(int fmt, int M, int N, int K, int gs, int* plan);
 
 /* ---- W4A4 on the scaled matrix cores (no counterpart in the reference, whose

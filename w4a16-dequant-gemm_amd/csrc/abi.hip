@@ -571,6 +571,8 @@ int w4_gemm_plan_for(int fmt, int M, int N, int K, int gs, int* plan) {
   v.mx = fmt == 2, v.N = N, v.K = K, v.symmetric = fmt != 1;
   v.gs = fmt == 2 ? 32 : gs;
   v.G = v.B = (K + v.gs - 1) / v.gs;
+  int dev = 0;
+  if (int rc = done("gemm plan", hipGetDevice(&dev))) return rc;  // the kernels' rules ask for its compute units
   *plan = w4k::gemm_plan(v, M);
   return W4_OK;
 }
