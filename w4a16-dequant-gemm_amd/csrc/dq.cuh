@@ -33,6 +33,9 @@ __device__ __forceinline__ h2 splat_bits(uint32_t b16) { return as_h2(b16 * 0x00
 
 __host__ __device__ __forceinline__ int words(int n) { return (n + 7) >> 3; }
 
+// Operand of s_waitcnt that waits for vmcnt(n) alone (gfx9 encoding: vmcnt in [3:0] and [15:14]).
+constexpr int waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
+
 // Group index of each of the four 8-k words of a lane's 32-k slice that starts
 // at k0 (gs: a multiple of 8).  One division (a shift when gs is a power of two:
 // gs_shift >= 0), then compares: 32 k span at most four groups.
@@ -96,6 +99,22 @@ __device__ __forceinline__ void dq_w4(uint32_t w, const W4Group& g, h2 d[4]) {
   d[1] = (a1 * sixteenth - g.zhi) * g.s;     // (64 + n) - (64 + z): exact
   d[2] = (a2 - g.zlo) * g.s;
   d[3] = (a3 * sixteenth - g.zhi) * g.s;
+}
+
+// Eight codes of a packed word -> eight FP16 values in k order, as an MFMA operand.  cneg: packed {-(1024 + z),
+// -(64 + z)}; s2: the group scale in both halves; mask, magic: 0x00F0000F and 0x54006400 held in registers (the
+// three-operand and-or takes no literal).  SCALED: the weights, else the codes minus the zero-point.
+template <bool SCALED = true>
+__device__ __forceinline__ h8 expand_word(uint32_t w, h2 cneg, h2 s2, uint32_t mask, uint32_t magic) {
+  u4 out;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t p = __builtin_amdgcn_perm(0u, w, 0x0c000c00u | (uint32_t)(i << 16) | (uint32_t)i);
+    const uint32_t v = (p & mask) | magic;
+    const h2 d = as_h2(v) + cneg;
+    out[i] = as_u32(SCALED ? d * s2 : d);
+  }
+  return __builtin_bit_cast(h8, out);
 }
 
 // ---- MXFP4: E2M1 codes with an E8M0 block scale ----------------------------

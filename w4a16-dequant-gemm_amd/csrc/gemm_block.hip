@@ -34,22 +34,7 @@ constexpr int BK_WAVES = 8, BK_THREADS = 64 * BK_WAVES;
 constexpr int BK_UNIT = 256;  // k of a unit: one 128-byte line of a row of codes, two of a row of x
 constexpr int BK_XS = 2;      // pieces in a wave's ring of x
 constexpr int bk_wave_bytes(int NT, int XS) { return NT * 2048 + XS * 4096; }
-constexpr int bk_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
 extern __shared__ __attribute__((aligned(16))) uint8_t bk_lds[];
-
-// SCALED: times the group's scale (s2), else the codes minus the zero-point.
-template <bool SCALED>
-__device__ __forceinline__ h8 bk_expand(uint32_t w, h2 cneg, h2 s2, uint32_t mask, uint32_t magic) {
-  u4 out;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t p = __builtin_amdgcn_perm(0u, w, 0x0c000c00u | (uint32_t)(i << 16) | (uint32_t)i);
-    const uint32_t v = (p & mask) | magic;
-    const h2 d = as_h2(v) + cneg;
-    out[i] = as_u32(SCALED ? d * s2 : d);
-  }
-  return __builtin_bit_cast(h8, out);
-}
 
 // f(integral_constant<int, 0>), f(integral_constant<int, 1>), ...: a loop whose index is
 // a constant expression inside the body (wait counts are instruction immediates)
@@ -182,9 +167,9 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
     request_codes(wave);
 #pragma unroll
     for (int p = 0; p < XS; ++p) request_x(wave, p, p);
-    __builtin_amdgcn_s_waitcnt(bk_vm(2 * NT + 4 * XS));
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * NT + 4 * XS));
   } else {
-    __builtin_amdgcn_s_waitcnt(bk_vm(0));
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
   }
   asm volatile("s_barrier" ::: "memory");  // the parameters are there
 
@@ -270,7 +255,7 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
           dq_mx(w[t][j], sf, n4);
           A[t][j] = __builtin_bit_cast(h8, u4{as_u32(n4[0]), as_u32(n4[1]), as_u32(n4[2]), as_u32(n4[3])});
         } else {
-          A[t][j] = bk_expand<!LATE>(w[t][j], cneg, s2, mask, magic);
+          A[t][j] = expand_word<!LATE>(w[t][j], cneg, s2, mask, magic);
         }
       }
     }
@@ -342,7 +327,7 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
     // 19.7 -> 17.9 us; with larger blocks the second set of registers costs more than it gives).
     h8 xv[2][4];
     if (nu > 0) {
-      __builtin_amdgcn_s_waitcnt(bk_vm(4 * (XS - 1)));
+      __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 * (XS - 1)));
       landed();
       read_codes(0, cw[0]), read_codes(1, cw[1]);
       read_x(0, xv[0]);
@@ -368,8 +353,8 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
         // requests younger than the next piece: the ring's others and, early in a unit, the next unit's codes
         if (p + 1 < NP || more) {
           constexpr int left = NP - 2 - p < 0 ? 0 : NP - 2 - p < XS - 1 ? NP - 2 - p : XS - 1;
-          if (more) __builtin_amdgcn_s_waitcnt(bk_vm(4 * (XS - 1) + (p < XS - 1 ? 2 * NT : 0)));
-          else __builtin_amdgcn_s_waitcnt(bk_vm(4 * left));
+          if (more) __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 * (XS - 1) + (p < XS - 1 ? 2 * NT : 0)));
+          else __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 * left));
           landed();
           if (MT > 1 && p == NP - 1) read_codes(0, cw[0]), read_codes(1, cw[1]);
           read_x(slot, xv[(p + 1) & 1]);
@@ -390,8 +375,8 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
         constexpr int p = decltype(pc)::value, ch = p / MT, mt = p % MT;
         // requests younger than the ones needed: the ring's other pieces, and next unit's codes
         constexpr int R = XS - 1, left = NP - 1 - p < R ? NP - 1 - p : R;
-        if (more) __builtin_amdgcn_s_waitcnt(bk_vm(4 * R + (p > PC && p < PC + XS ? 2 * NT : 0)));
-        else __builtin_amdgcn_s_waitcnt(bk_vm(4 * left));
+        if (more) __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 * R + (p > PC && p < PC + XS ? 2 * NT : 0)));
+        else __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 * left));
         landed();
         if (PC && mt == 0) read_codes(ch, cw[0]);
         if (!PC && p == 0) read_codes(0, cw[0]), read_codes(1, cw[PC ? 0 : 1]);
@@ -488,18 +473,6 @@ struct BkShape {
 constexpr BkShape BK_SHAPES[] = {{1, 1, 50, 45},   {2, 1, 83, 56},   {2, 2, 106, 89},  {4, 1, 136, 80},  {2, 4, 171, 155},
                                  {4, 2, 175, 125}, {3, 4, 195, 173}, {4, 4, 260, 215}, {4, 5, 290, 250}, {4, 6, 330, 290}};
 
-// Compute units of the current device (per-device cache); 0 on error.
-int bk_cus() {
-  static std::atomic<int> cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  if (dev >= 0 && dev < 64 && cached[dev]) return cached[dev];
-  int n = 0;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  if (dev >= 0 && dev < 64) cached[dev] = n;
-  return n;
-}
-
 // Few rows (M < 17) and at most one tile of W a compute unit, K in whole chunks: the longest K that stays with the long-K
 // kernel, which fetches only the quads of x that exist and has no parameters to wait for.  [symmetric W4, with
 // zero-points, MXFP4][M up to 4, 8, 12, 16][tiles for half of the compute units, or more].  M = 3: N = 128, K = 5120 5.5 us
@@ -570,7 +543,7 @@ int block_plan(const WView& v, int M) {
   if (M < 3 || M > 8192 || (M < 9 && v.K <= 4096) || (M < 17 && v.K <= 2048)) return -1;
   if (v.K % 32 || v.N % 16 || (!v.mx && v.gs % 32)) return -1;
   if (v.K >= 1 << 24) return -1;  // offsets inside a block have 32 bits
-  const int cus = bk_cus();
+  const int cus = device_cus();
   if (cus < 8) return -1;
   // Few rows: one 16-row tile of W a workgroup (N = K = 4096, M = 8 5.2 against 5.0 us; K = 2048, M = 16 4.2 against
   // 3.9), wider matrices at long K only (N = 11008, K = 4096, M = 16 9.4 against 7.7 us).  (Ruled out first: calls this

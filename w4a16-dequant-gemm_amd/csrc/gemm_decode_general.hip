@@ -33,22 +33,7 @@ namespace {
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
 constexpr int DG_WAVES = 8, DG_THREADS = 64 * DG_WAVES;
-constexpr int dg_waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
 extern __shared__ __attribute__((aligned(16))) uint8_t dg_lds[];
-
-// Eight codes of a packed word -> eight FP16 weights in k order (as in the
-// resident-activation kernel): cneg = packed {-(1024 + z), -(64 + z)}, s2 = the scale
-// in both halves, mask / magic = 0x00F0000F / 0x54006400 held in registers.
-__device__ __forceinline__ h8 dg_expand_word(uint32_t w, h2 cneg, h2 s2, uint32_t mask, uint32_t magic) {
-  u4 out;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t p = __builtin_amdgcn_perm(0u, w, 0x0c000c00u | (uint32_t)(i << 16) | (uint32_t)i);
-    const uint32_t v = (p & mask) | magic;
-    out[i] = as_u32((as_h2(v) + cneg) * s2);
-  }
-  return __builtin_bit_cast(h8, out);
-}
 
 // ASYM: zero-points.  CH = ceil(ceil(K / 128) / 8) chunks per wave.  T tiles of 16 rows
 // per workgroup (tile blockIdx.x + gridDim.x t), MT tiles of 16 activation rows
@@ -212,7 +197,7 @@ __global__ __launch_bounds__(DG_THREADS) void mfma_decode_general_kernel(
   // At most the codes of tile 1 may still be outstanding (CH vector loads; a wave that
   // issued word-by-word loads instead waits for more than it must): phase 0 of x, the
   // codes of tile 0 and the parameter loads have landed.
-  __builtin_amdgcn_s_waitcnt(dg_waitcnt_vm(T > 1 ? CH : 0));
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(T > 1 ? CH : 0));
   const int PB = SB + ZB;  // parameter block of one tile, behind the x regions
   uint8_t* params = dg_lds + DG_WAVES * XBYTES;
 #pragma unroll
@@ -237,7 +222,7 @@ __global__ __launch_bounds__(DG_THREADS) void mfma_decode_general_kernel(
 
 #pragma unroll
   for (int ph = 0; ph < PH; ++ph) {
-    if (ph > 0) __builtin_amdgcn_s_waitcnt(dg_waitcnt_vm(0));  // later phases are the youngest requests
+    if (ph > 0) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // later phases are the youngest requests
     // B operands: MFMA j of chunk i contracts k = lane_k(i) + 8 j .. + 7 = piece 4 b + j
     u4 xv[MT][CP][4];
     {
@@ -286,9 +271,9 @@ __global__ __launch_bounds__(DG_THREADS) void mfma_decode_general_kernel(
         __builtin_amdgcn_sched_barrier(0);
         if (t + 1 < T) load_tile(t + 1);
         __builtin_amdgcn_sched_barrier(0);
-        if (t == 1) __builtin_amdgcn_s_waitcnt(dg_waitcnt_vm(NX1 + (T > 2 ? CH : 0)));
-        else if (t + 1 < T) __builtin_amdgcn_s_waitcnt(dg_waitcnt_vm(CH));
-        else __builtin_amdgcn_s_waitcnt(dg_waitcnt_vm(0));
+        if (t == 1) __builtin_amdgcn_s_waitcnt(waitcnt_vm(NX1 + (T > 2 ? CH : 0)));
+        else if (t + 1 < T) __builtin_amdgcn_s_waitcnt(waitcnt_vm(CH));
+        else __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
       }
 #pragma unroll
       for (int cc = 0; cc < CP; ++cc) {
@@ -318,7 +303,7 @@ __global__ __launch_bounds__(DG_THREADS) void mfma_decode_general_kernel(
             cneg = first[i][j - 1] ? cn[0] : cn[1];
             s2 = first[i][j - 1] ? sp[0] : sp[1];
           }
-          const h8 a = dg_expand_word(qw[t][i][j], cneg, s2, mask, magic);
+          const h8 a = expand_word(qw[t][i][j], cneg, s2, mask, magic);
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt)
             acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(h8, xv[mt][cc][j]),
@@ -390,19 +375,6 @@ int max_lds_bytes() {
   return n;
 }
 
-int cu_count() {
-  static std::atomic<int> cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  if (dev >= 0 && dev < 64) {
-    if (const int have = cached[dev].load(std::memory_order_relaxed)) return have;
-  }
-  int n = 0;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  if (dev >= 0 && dev < 64) cached[dev].store(n, std::memory_order_relaxed);
-  return n;
-}
-
 // Whether, and how, the kernel takes these arguments: W4 only, whole 16-row tiles,
 // whole packed words, 1024 < K <= 5120 (two to five chunks per wave), M <= 64, aligned
 // activations / outputs / parameter arrays, and LDS for the activations of a
@@ -417,7 +389,7 @@ bool general_plan(const WView& v, const w4_half* x, const w4_half* c, int M, Gen
   const int pb = 32 * v.G + (v.symmetric ? 0 : 64 * ((v.G + 7) / 8));
   const int ps = (2 * v.G + DG_THREADS - 1) / DG_THREADS;
   if (ps > 3 || (!v.symmetric && 4 * ((v.G + 7) / 8) > DG_THREADS)) return false;
-  const int lds_max = max_lds_bytes(), cus = cu_count();
+  const int lds_max = max_lds_bytes(), cus = device_cus();
   if (lds_max < 1 || cus < 1) return false;
   // tiles per workgroup: enough that one workgroup per compute unit covers N, at most
   // four; with one activation row tile the x regions may shrink to two chunks per

@@ -62,19 +62,7 @@ constexpr int lk_nbuf(int MT, int NQ) {
 constexpr int lk_quads(int MT, int NQ, int mt) { return mt < MT - 1 ? 4 : NQ; }
 constexpr int lk_slot(int MT, int NQ) { return MT > 1 ? 4 : NQ; }  // KB of a ring slot
 constexpr int lk_lau(int MT, int NQ) { return lk_nbuf(MT, NQ) / MT / 2 > 2 ? lk_nbuf(MT, NQ) / MT / 2 : 2; }
-constexpr int lk_waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
 extern __shared__ __attribute__((aligned(16))) uint8_t lk_lds[];
-
-__device__ __forceinline__ h8 lk_expand_word(uint32_t w, h2 cneg, h2 s2, uint32_t mask, uint32_t magic) {
-  u4 out;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t p = __builtin_amdgcn_perm(0u, w, 0x0c000c00u | (uint32_t)(i << 16) | (uint32_t)i);
-    const uint32_t v = (p & mask) | magic;
-    out[i] = as_u32((as_h2(v) + cneg) * s2);
-  }
-  return __builtin_bit_cast(h8, out);
-}
 
 // The issue order of a wave, replayed at compile time.  allowed[u]: how many vector
 // memory requests may still be outstanding when unit u of the activations (chunk
@@ -261,7 +249,7 @@ __global__ __launch_bounds__(LK_THREADS) void mfma_decode_longk_kernel(
   u4 xv[MT][4];  // B operands: MFMA j contracts k = 128 chunk + 32 b + 8 j .. + 7 = piece 4 b + j
   lk_for([&](auto uc) {
     constexpr int u = decltype(uc)::value, i = u / MT, mt = u % MT;
-    __builtin_amdgcn_s_waitcnt(lk_waitcnt_vm(SCH.allowed[u]));
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(SCH.allowed[u]));
     if (mt == 0) {
       // the registers of this chunk's codes are defined from here on
       asm volatile("" : "+v"(qw[i]), "+v"(sc[i]));
@@ -308,7 +296,7 @@ __global__ __launch_bounds__(LK_THREADS) void mfma_decode_longk_kernel(
         dq_mx(qw[i][j], sf, n4);
         a = __builtin_bit_cast(h8, u4{as_u32(n4[0]), as_u32(n4[1]), as_u32(n4[2]), as_u32(n4[3])});
       } else {
-        a = lk_expand_word(qw[i][j], cneg, s2, mask, magic);
+        a = expand_word(qw[i][j], cneg, s2, mask, magic);
       }
 #pragma unroll
       for (int m2 = 0; m2 < MT; ++m2)
@@ -349,18 +337,6 @@ int longk_chunks(int K) {
   if (K % 128) return 0;
   const int per_wave = (K / 128 + LK_WAVES - 1) / LK_WAVES;
   return (per_wave >= 2 && per_wave <= 16) ? per_wave : 0;
-}
-
-// Compute units of the current device (per-device cache); 0 on error.
-int lk_cus() {
-  static std::atomic<int> cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  if (dev >= 0 && dev < 64 && cached[dev]) return cached[dev];
-  int n = 0;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  if (dev >= 0 && dev < 64) cached[dev] = n;
-  return n;
 }
 
 template <int FMT, int CH, int MT, int NQ>
@@ -432,14 +408,14 @@ bool decode_longk_applies(const WView& v, const w4_half* x, const w4_half* c, in
   // K up to 5120 on grids of more than one tile per compute unit, W4: from M = 9 the kernel
   // that shares a workgroup's activations between several tiles is ahead (N = 16384,
   // K = 5120, M = 16 / 32 / 64: 17.7 / 20.0 / 35.8 us against 21.3 / 31.3 / 42.0; M = 8: 17.2 against 17.0)
-  if (longk_chunks(v.K) == 5 && !v.mx && M > 8 && v.N / 16 > lk_cus()) return false;
+  if (longk_chunks(v.K) == 5 && !v.mx && M > 8 && v.N / 16 > device_cus()) return false;
   if (longk_chunks(v.K) < 5) {
     // Shorter K: only where the kernels that share x between the tiles of a workgroup
     // would have one tile per workgroup too (N / 16 <= compute units).  At K = 2048 and
     // 4096, the resident kernel's own, this one is ahead while few quads of x are
     // fetched and most compute units have a tile (N = 4096, K = 4096, M = 5 / 8: 5.5 ->
     // 4.8 / 5.0 us; M = 16: 5.6 -> 5.9; N = 2048, M = 8: 5.35 -> 5.66).
-    const int tiles = v.N / 16, cus = lk_cus();
+    const int tiles = v.N / 16, cus = device_cus();
     if (cus < 1 || tiles > cus) return false;
     if ((v.K == 2048 || v.K == 4096) && (M > 8 || 2 * tiles <= cus)) return false;
   }

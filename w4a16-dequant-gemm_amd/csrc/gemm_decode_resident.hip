@@ -31,22 +31,7 @@ namespace {
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
 constexpr int DR_WAVES = 8, DR_THREADS = 64 * DR_WAVES;
-constexpr int waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
 extern __shared__ __attribute__((aligned(16))) uint8_t dr_lds[];
-
-// Eight codes of a packed word -> eight FP16 weights in k order.  cneg: packed
-// {-(1024 + z), -(64 + z)}; s2: the group scale in both halves; mask, magic:
-// 0x00F0000F and 0x54006400 in registers.
-__device__ __forceinline__ h8 expand_word(uint32_t w, h2 cneg, h2 s2, uint32_t mask, uint32_t magic) {
-  u4 out;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t p = __builtin_amdgcn_perm(0u, w, 0x0c000c00u | (uint32_t)(i << 16) | (uint32_t)i);
-    const uint32_t v = (p & mask) | magic;
-    out[i] = as_u32((as_h2(v) + cneg) * s2);
-  }
-  return __builtin_bit_cast(h8, out);
-}
 
 // FMT: 0 W4 symmetric, 1 W4 with zero-points, 2 MXFP4.  K = 1024 CH.  POW2: gs is a
 // power of two (shift gs_shift); GSV: 1, 2, 3 for gs = 128, 64, 32 with scale arrays
@@ -515,8 +500,6 @@ int resident_chunks(int K) {
   return (per_wave == 8 || per_wave == 11 || per_wave == 14) ? per_wave : 0;
 }
 
-int device_cus();
-
 template <int FMT, int CH, bool POW2, int GSV, int T, int MT, int CPV>
 hipError_t launch_t_impl(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, int sh,
                          int tiles, unsigned grid) {
@@ -657,18 +640,6 @@ hipError_t launch_fmt(const WView& v, const w4_half* x, w4_half* c, int M, hipSt
   }
 #undef W4_LONG
 #undef W4_GO
-}
-
-// Compute units of the current device (per-device cache); 0 on error.
-int device_cus() {
-  static std::atomic<int> cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  if (dev >= 0 && dev < 64 && cached[dev]) return cached[dev];
-  int n = 0;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  if (dev >= 0 && dev < 64) cached[dev] = n;
-  return n;
 }
 
 // A K this kernel is built for, whole 16-row tiles, a lane's 32-k slice inside one

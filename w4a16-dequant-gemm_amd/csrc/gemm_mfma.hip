@@ -15,6 +15,8 @@
 // up to 64 activation rows; its 4 waves split K chunk-wise and combine through
 // LDS in a fixed order, so results are deterministic and every CU streams W
 // even when N/16 is only a few hundred.
+#include <atomic>
+
 #include "dq.cuh"
 #include "kernels.h"
 
@@ -941,6 +943,17 @@ static hipError_t launch_fmt(const WView& v, const w4_half* x, w4_half* c, int M
   if (M <= 16) return launch_tiles<MX, 1>(v, x, c, M, s, w_out);
   if (M <= 32) return launch_tiles<MX, 2>(v, x, c, M, s, w_out);
   return launch_tiles<MX, 4>(v, x, c, M, s, w_out);
+}
+
+int device_cus() {
+  static std::atomic<int> cached[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  if (dev >= 0 && dev < 64 && cached[dev]) return cached[dev];
+  int n = 0;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+  if (dev >= 0 && dev < 64) cached[dev] = n;
+  return n;
 }
 
 int gemm_plan(const WView& v, int M) {

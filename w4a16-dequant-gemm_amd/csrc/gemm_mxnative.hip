@@ -353,9 +353,6 @@ __device__ __forceinline__ f16v mfma_fp4_fp8_32(u4 a, uint32_t sa, u4 b0, u4 b1,
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
 
-// s_waitcnt vmcnt(N) alone (gfx9 encoding: vmcnt in [3:0] and [15:14])
-constexpr int waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
-
 extern __shared__ __attribute__((aligned(16))) uint8_t dm_lds[];
 
 template <bool XF8>

@@ -40,9 +40,6 @@ constexpr int T2_C_BYTES = 4 * 256 * T2_C_PITCH;
 constexpr int T2_LDS = T2_STAGES * T2_STAGE > T2_C_BYTES ? T2_STAGES * T2_STAGE : T2_C_BYTES;
 static_assert(T2_LDS <= 160 * 1024, "stage buffers and the output staging fit LDS");
 
-// s_waitcnt vmcnt(N) alone (gfx9 encoding: vmcnt in [3:0] and [15:14])
-constexpr int t2_waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
-
 extern __shared__ __attribute__((aligned(16))) uint8_t t2_lds[];
 
 // Position of 16-byte piece p of X row R in a stage buffer.  A load instruction writes
@@ -274,7 +271,7 @@ __global__ __launch_bounds__(T2_THREADS) void w4_tile256_kernel(
   for (int part = 0; part < LOADS; ++part) request_part(1, b1, part);
 #pragma unroll
   for (int part = 0; part < CH; ++part) request_part(2, b2, part);
-  __builtin_amdgcn_s_waitcnt(t2_waitcnt_vm(LOADS + CH));  // stage 0 has landed
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(LOADS + CH));  // stage 0 has landed
   __syncthreads();
   read_x(xv[0], b0, 0, 0, MJ);
   read_w(b0);
@@ -310,7 +307,7 @@ __global__ __launch_bounds__(T2_THREADS) void w4_tile256_kernel(
     // Step 3.  Every LDS read of stage d has been issued (the X operands of this step during
     // step 2, the words at the stage's start): once all waves are here its buffer can take
     // stage d + 3, and stage d + 1 has landed for everyone (outstanding: all of stage d + 2).
-    __builtin_amdgcn_s_waitcnt(t2_waitcnt_vm(LOADS));
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(LOADS));
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -349,7 +346,7 @@ __global__ __launch_bounds__(T2_THREADS) void w4_tile256_kernel(
     b1 = b2;
     b2 = first;
   }
-  __builtin_amdgcn_s_waitcnt(t2_waitcnt_vm(0));  // nothing may still be writing LDS at exit
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // nothing may still be writing LDS at exit
 
   // A lane holds, of each 32 x 32 tile, n = 8 q + 4 h + e for m = tile row r.  The tiles go
   // through LDS (free by now) so that every store instruction writes eight whole 128-byte

@@ -41,9 +41,6 @@ constexpr int td_tile(int tm, int tn) { return tn * 64 + tm * 256; }
 constexpr int td_stage(int tm, int tn) { return td_tile(tm, tn) + 3 * tn * 4; }
 constexpr int td_lds_bytes(int tm, int tn) { return TD_STAGES * td_stage(tm, tn); }
 
-// s_waitcnt vmcnt(N) alone (gfx9 encoding: vmcnt in [3:0] and [15:14])
-constexpr int waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
-
 extern __shared__ __attribute__((aligned(16))) uint8_t td_lds[];
 
 // Position of 16-byte piece p of row R.  A load instruction writes lane l's 16
@@ -56,21 +53,6 @@ __device__ __forceinline__ int w_at(int R, int p) {
 }
 __device__ __forceinline__ int x_at(int R, int p) {
   return (R >> 2) * 1024 + ((R & 3) * 16 + (p ^ (R & 15))) * 16;
-}
-
-// Eight codes of a packed word -> eight FP16 weights in k order (as an MFMA operand).
-// cneg: packed {-(1024 + z), -(64 + z)}; s2: the group scale in both halves.
-// mask, magic: 0x00F0000F and 0x54006400 held in registers (the three-operand
-// and-or takes no literal).
-__device__ __forceinline__ h8 expand_word(uint32_t w, h2 cneg, h2 s2, uint32_t mask, uint32_t magic) {
-  u4 out;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t p = __builtin_amdgcn_perm(0u, w, 0x0c000c00u | (uint32_t)(i << 16) | (uint32_t)i);
-    const uint32_t v = (p & mask) | magic;
-    out[i] = as_u32((as_h2(v) + cneg) * s2);
-  }
-  return __builtin_bit_cast(h8, out);
 }
 
 // One wave per SIMD, so the three pipes have to overlap inside a wave: a stage is

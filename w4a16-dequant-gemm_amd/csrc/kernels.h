@@ -27,6 +27,9 @@ inline WView view_of(const w4_packed_mx_view& p) {
   return WView{1, p.N, p.K, 32, p.B, 1, p.B, p.q, p.scales, nullptr};
 }
 
+// Compute units of the current device (kept per device); 0 on error.
+int device_cus();
+
 // dequant.hip
 hipError_t launch_dequant(const WView& v, w4_half* w, hipStream_t s);
 hipError_t launch_dequant_f8(const uint8_t* q, const w4_half* sc, w4_half* w,
