@@ -228,7 +228,8 @@ int w4_quantize_cache_f8(const w4_kv_f8_view* out, const void* k, const void* v,
 /* Which kernel the matrix-core GEMM runs on the current GPU (no counterpart in the reference): fmt 0 W4
  * symmetric, 1 W4 with zero-points, 2 MXFP4 (gs ignored); no hook, arrays aligned to 16 bytes.  *plan: 10 x the
  * 16-row tiles of W + the row tiles of x of a block (11 .. 46); 1 the long-K decode kernel, 2 the one that keeps
- * the activations, 3 the one for odd group sizes and ragged K; 0 tiles, stream and the others.  W4_ERUNTIME
+ * the activations, 3 the one for odd group sizes and ragged K, 4 - 7 tiles of 32 x 128, 64 x 128, 128 x 128 and 128 x
+ * 256 (rows of x, of W) for any group size and K; 0 other tiles, stream and the others.  W4_ERUNTIME
  * without a GPU. */
 int w4_gemm_plan_for(int fmt, int M, int N, int K, int gs, int* plan);
 

@@ -1,0 +1,114 @@
+"""Group sizes, K and N that do not come in whole chunks and tiles (mma.cuh:63-230, the reference's kernel, takes
+any gs % 8 == 0 and zero-pads the edges): blocks and tiles at the edges where they can go wrong -- rows that end inside a
+16-byte piece, a slice of 32 k, a chunk or a stage, groups that begin anywhere in a slice, scale arrays that end
+inside a dword, matrices that end inside a tile of rows.
+
+Outputs are held to 5e-4 of the FP64 oracle on sampled rows and columns (FP16 weights and outputs, FP32 sums: 2.1e-4 is
+what these shapes measure; the reference's gate is 1e-3, tests/test_gpu.cu:184-193); hooked bytes are the oracle's."""
+import numpy as np
+import pytest
+import torch
+
+import orc
+import w4amd
+from devutil import DevPacked, DevPackedMx, bits, halves, ptr, to_dev
+
+pytestmark = pytest.mark.gpu
+TOL = 5e-4
+
+
+def _check(fmt, M, N, K, gs, scale=None):
+    c = w4amd.capi()
+    seed = M + N + K + gs + fmt
+    x = orc.normal_activations(M * K, seed)
+    if fmt == 2:
+        p = orc.quantize_mx(orc.outlier_weights(N, K, seed), N, K)
+        dp, fn, w_ref = DevPackedMx(p), c.gemm_mma_mx, orc.dequant_all_mx(p)
+    else:
+        p = orc.quantize(orc.normal_weights(N * K, seed) * 0.02 + 0.01 * fmt, N, K, gs, fmt == 0)
+        dp, fn, w_ref = DevPacked(p), c.gemm_mma, orc.dequant_all(p)
+    x_d = to_dev(x)
+    rng = np.random.default_rng(seed)
+    ms = np.unique(np.concatenate([[0, M - 1], rng.choice(M, size=min(M, 20), replace=False)]))
+    ns = np.unique(np.concatenate([np.arange(min(N, 40)), np.arange(max(0, N - 40), N), rng.choice(N, size=min(N, 80), replace=False)]))
+    ref = orc.gemm_oracle(np.ascontiguousarray(x.reshape(M, K)[ms]), len(ms), K,
+                          np.ascontiguousarray(w_ref.reshape(N, K)[ns]), len(ns))
+    for hook in (False, True):
+        out, w = halves(M * N + 64, 0x7E00), halves(N * K + 64, 0x7E00)
+        fn(dp.view, ptr(x_d), ptr(out), M, 0, ptr(w) if hook else 0)
+        got = bits(out)
+        assert (got[M * N:] == 0x7E00).all(), "nothing is written behind the result"
+        got = np.ascontiguousarray(got[: M * N].reshape(M, N)[ms][:, ns]).view(np.float16)
+        assert orc.rel_l2(got, ref) <= TOL, hook
+        if hook:
+            assert torch.equal(w[: N * K], to_dev(w_ref)) and bool((w[N * K:] == 0x7E00).all())
+    return c.gemm_plan_for(fmt, M, N, K, gs)
+
+
+# (plan, fmt, M, N, K, gs): tiles of 32 x 128 (4) to 128 x 256 (7) in every compiled form; K ends inside a chunk and, 264,
+# inside a piece; gs = 40 .. 136 begin in any word; N * G odd (MXFP4: N * B % 4): the last scale is part of a dword
+TILES = [(4, 0, 1100, 257, 2080, 24), (4, 0, 2049, 257, 264, 8), (4, 0, 2049, 129, 1056, 72), (4, 0, 520, 257, 264, 40),
+         (4, 1, 2049, 129, 2080, 24), (4, 1, 900, 777, 264, 24), (4, 1, 1100, 257, 1056, 40), (4, 1, 130, 3001, 264, 40),
+         (4, 2, 2049, 129, 1056, 32), (4, 2, 520, 257, 264, 32), (5, 0, 1300, 777, 2080, 24), (5, 0, 1300, 777, 264, 16),
+         (5, 0, 1300, 777, 1056, 104), (5, 0, 900, 1034, 264, 48), (5, 1, 520, 2051, 2080, 24), (5, 1, 1300, 777, 264, 8),
+         (5, 1, 1300, 777, 1056, 96), (5, 1, 1300, 777, 264, 40), (5, 2, 900, 1034, 1056, 32), (5, 2, 900, 1034, 264, 32),
+         (6, 0, 1100, 2051, 2080, 24), (6, 0, 1100, 2051, 264, 8), (6, 0, 1100, 2051, 1056, 104), (6, 0, 700, 3001, 264, 40),
+         (6, 1, 900, 3001, 2080, 24), (6, 1, 1100, 2051, 264, 8), (6, 1, 700, 3001, 1056, 40), (6, 1, 700, 3001, 264, 96),
+         (6, 2, 900, 2310, 1056, 32), (6, 2, 900, 2310, 264, 32), (7, 0, 1300, 3001, 1056, 1056), (7, 0, 1300, 3001, 264, 40),
+         (7, 1, 2049, 2051, 1152, 40), (7, 1, 1300, 3001, 264, 128), (7, 2, 1700, 2310, 1056, 32), (7, 2, 1300, 3001, 264, 32)]
+BLOCKS = [(0, 5, 130, 4104, 8), (1, 9, 33, 3336, 24), (1, 17, 1034, 2056, 48), (0, 20, 15, 264, 40), (1, 33, 281, 1000, 16), (0, 50, 513, 5176, 72),
+          (1, 64, 3, 1032, 1032), (1, 40, 2063, 4104, 8), (0, 100, 129, 2080, 128), (1, 130, 40, 1384, 48), (2, 17, 281, 1000, 32), (2, 50, 7, 3336, 32),
+          (2, 130, 1001, 2072, 32), (1, 100, 2064, 1152, 48), (0, 333, 4080, 4096, 48), (1, 64, 3000, 2048, 96), (0, 120, 1477, 2304, 128),
+          (1, 48, 1477, 4096, 32)]
+
+
+@pytest.mark.parametrize("plan,fmt,M,N,K,gs", TILES)
+def test_tiles_of_any_group(plan, fmt, M, N, K, gs):
+    assert _check(fmt, M, N, K, gs) == plan
+
+
+@pytest.mark.parametrize("fmt,M,N,K,gs", BLOCKS)
+def test_blocks_of_any_group(fmt, M, N, K, gs):
+    assert _check(fmt, M, N, K, gs) >= 10
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 1302, 1160), (50, 282, 2088), (1300, 2050, 1048)])
+@pytest.mark.parametrize("gs", [8, 48, 0])
+def test_ends_of_rows_bring_no_infinity(M, N, K, gs):
+    """The codes that stand in for a row's end are other groups', here with scales that overflow FP16, and the activations
+    that the last stage shares with the one before it are infinite in one row: results are infinite where the oracle's
+    are, NaN nowhere else."""
+    mx = gs == 0
+    rng = np.random.default_rng(M + K + gs)
+    G = (K + 31) // 32 if mx else (K + gs - 1) // gs
+    codes = rng.integers(0, 16, (N, K))
+    codes[:, (G - 1) * (gs or 32):] = 2 if mx else 9  # 1.0
+    words = (codes.reshape(N, K // 8, 8).astype(np.uint64) << (4 * np.arange(8, dtype=np.uint64))).sum(-1).astype(np.uint32)
+    c = w4amd.capi()
+    x = orc.normal_activations(M * K, 3).view(np.float16).reshape(M, K).copy()
+    x[2, K - 100] = np.inf  # in the stage before the last as well
+    if mx:
+        p = orc.quantize_mx(np.ones(N * K), N, K)
+        s = np.full((N, G), 127 - 6, np.uint8)
+        s[:, -1] = 127 + 14
+        dp, fn = (lambda: DevPackedMx(p)), c.gemm_mma_mx
+    else:
+        p = orc.quantize(np.ones(N * K), N, K, gs, True)
+        s = np.full((N, G), 0.01, np.float16)
+        s[:, -1] = 60000
+        s = s.view(np.uint16)
+        dp, fn = (lambda: DevPacked(p)), c.gemm_mma
+    p.q[:], p.scales[:] = words.ravel(), s.ravel()
+    x[:, (G - 1) * (gs or 32):] *= np.float16(2.0 ** -12)
+    w = (orc.dequant_all_mx(p) if mx else orc.dequant_all(p)).view(np.float16).reshape(N, K).astype(np.float64)
+    d, out = dp(), halves(M * N)
+    fn(d.view, ptr(to_dev(x.view(np.uint16).ravel())), ptr(out), M)
+    got = bits(out).view(np.float16).reshape(M, N).astype(np.float64)
+    rows = np.array([0, 1, 3, M - 1])
+    with np.errstate(invalid="ignore"):
+        ref = x[rows].astype(np.float64) @ w.T
+        bad = x[2].astype(np.float64)[None] @ w.T
+    assert np.isfinite(ref).any() and np.isfinite(got[rows]).sum() >= np.isfinite(ref).sum() * 0.99
+    ok = np.isfinite(ref) & np.isfinite(got[rows])
+    assert np.linalg.norm((got[rows] - ref)[ok]) <= 1e-3 * np.linalg.norm(ref[ok])
+    assert np.array_equal(np.isnan(got[2]), np.isnan(bad[0])) and np.array_equal(np.isinf(got[2]), np.isinf(bad[0]))

@@ -11,9 +11,9 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "lib", "libw4amd.so")
 BENCH_LIB = os.path.join(PKG, "lib", "libw4bench.so")
-SOURCES = ["abi.hip", "dequant.hip", "gemm_simt.hip", "gemm_mfma.hip", "flash.hip", "flash_mfma.hip", "quantize.hip", "gemm_mxnative.hip", "gemm_tile_dma.hip", "gemm_tile256.hip", "gemm_decode_resident.hip", "gemm_decode_general.hip", "gemm_decode_longk.hip", "gemm_block.hip",
+SOURCES = ["abi.hip", "dequant.hip", "gemm_simt.hip", "gemm_mfma.hip", "flash.hip", "flash_mfma.hip", "quantize.hip", "gemm_mxnative.hip", "gemm_tile_dma.hip", "gemm_tile_any.hip", "gemm_tile256.hip", "gemm_decode_resident.hip", "gemm_decode_general.hip", "gemm_decode_longk.hip", "gemm_block.hip",
            "baseline.hip"]
-HEADERS = ["dq.cuh", "kernels.h", "simt_rows4.cuh", "bench_kernels.hip", os.path.join("..", "..", "include", "w4_abi.h")]
+HEADERS = ["dq.cuh", "kernels.h", "simt_rows4.cuh", "tile_dma.cuh", "bench_kernels.hip", os.path.join("..", "..", "include", "w4_abi.h")]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     # packed-FP32 VALU forms stay off for every kernel in this library
@@ -30,7 +30,10 @@ FLAGS = [
 # vector-ALU multiplies between matrix instructions: with the accumulators in
 # the AGPR half of the register file the compiler copies all 36 of them across
 # every loop edge, so keep its MFMA results in ordinary VGPRs.
-EXTRA_FLAGS = {"flash_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# The tile kernels for any group unroll eight steps that are longer than the
+# threshold allows (the LDS addresses in their loads are immediates).
+EXTRA_FLAGS = {"flash_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+               "gemm_tile_any.hip": ["-mllvm", "-pragma-unroll-threshold=100000"]}
 
 
 def _stale():

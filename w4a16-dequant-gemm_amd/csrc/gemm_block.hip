@@ -48,19 +48,30 @@ __device__ __forceinline__ void bk_dma(uint32_t off, const void* base, uint32_t 
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(dst) : "memory", "m0");
 }
 
+__device__ __forceinline__ void bk_dma4(uint32_t off, const void* base, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(dst) : "memory", "m0");
+}
+
 // FMT: 0 W4 symmetric, 1 W4 with zero-points, 2 MXFP4.  G: groups (W4) or blocks (MXFP4) per row.
-// gs_shift: log2(gs) if gs is a power of two, else -1.  mgroups: blocks along M.  XS: pieces of x (16 rows x 128 k, 4 KB) in a
+// group_mul: ceil(2^31 / (gs / 8)): the group of word w is (2 w group_mul) >> 32.  mgroups: blocks along M.  XS: pieces of x (16 rows x 128 k, 4 KB) in a
 // wave's ring; three measured no better than two.  LATE (W4, gs a multiple of 128: a chunk of 128 k is in one
 // group): the operands are the codes minus the zero-point, exact in FP16, and the scale is applied to a
 // chunk's FP32 sums, as the resident kernel does in the shapes that this one took over from it
 // (rounding q s to FP16 first: 2.7e-4 from the product in FP64 instead of 2.1e-4, K = 4096, M = 16).
-template <int FMT, int NT, int MT, int XS, bool AHEAD, bool LATE>
+// GM (W4 with groups that a lane's 32 k of a chunk do not all belong to one of): 1 groups of 32 or more k, at most two
+// of which meet in such a slice, 2 smaller ones, at most four.  A slice's runs of scales and zero-points come as
+// whole dwords and are moved to the bottom of their registers, from which a word picks its own by a
+// selector of bytes and a shift.  RAG: K is no multiple of 32 (rows of codes are 4-byte aligned only) or N none of 16: codes
+// come dword by dword.
+template <int FMT, int NT, int MT, int XS, bool AHEAD, bool LATE, int GM, bool RAG>
 __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
     const uint32_t* __restrict__ q, const void* __restrict__ scales, const uint32_t* __restrict__ zeros,
     const w4_half* __restrict__ x, w4_half* __restrict__ c, const int N, const int K, const int M,
-    const int gs_shift, const int G, const int gs, const int mgroups, w4_half* __restrict__ w_out) {
+    const uint32_t group_mul, const int G, const int gs, const int mgroups, w4_half* __restrict__ w_out) {
   constexpr bool MX = FMT == 2;
   static_assert(!(MX && LATE), "an MXFP4 chunk has four scales");
+  static_assert(GM == 0 || (!MX && !LATE), "scales of a chunk or of MXFP4 blocks need no selector");
+  constexpr int CL = RAG ? 8 * NT : 2 * NT;  // load instructions of a unit's codes
   constexpr int WB = bk_wave_bytes(NT, XS), ROWS = 16 * NT, NP = 2 * MT;
   // Step of a unit at which its codes have been read back and the next unit's are requested: with
   // many row tiles one chunk's codes are read at a time (registers).
@@ -81,16 +92,31 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
 
   // ---- group parameters of the block's rows: one contiguous run each, 1 KB a load ----
   const int live = min(ROWS, N - n0);
+  [[maybe_unused]] uint8_t* rest_s = nullptr;  // RAG: bytes of the matrix's last rows that are no whole 16, and their places
+  [[maybe_unused]] uint8_t* rest_z = nullptr;
+  [[maybe_unused]] uint8_t byte_s = 0, byte_z = 0;
   const int pb = live * G * (MX ? 1 : 2), wg = words(G), zb = live * wg * 4;
   const int zoff = (ROWS * G * (MX ? 1 : 2) + 1023) & ~1023;
   {
     const char* ps = (const char*)scales + (size_t)n0 * G * (MX ? 1 : 2);
-    for (int o = wave * 1024; o < pb; o += BK_WAVES * 1024)
-      bk_dma((uint32_t)min(o + lane * 16, pb - 16), ps, lds0 + BK_WAVES * WB + o);
+    const int pw = RAG ? pb & ~15 : pb, zw16 = RAG ? zb & ~15 : zb;  // (16 rows have whole pieces of 16 bytes)
+    for (int o = wave * 1024; o < pw; o += BK_WAVES * 1024)
+      bk_dma((uint32_t)min(o + lane * 16, pw - 16), ps, lds0 + BK_WAVES * WB + o);
+    const char* pz = FMT == 1 ? (const char*)zeros + (size_t)n0 * wg * 4 : nullptr;
+    if constexpr (RAG) {
+      // (written by the wave whose load ends there, once it has landed: its lanes past the end write behind it)
+      if (lane < (pb & 15) && wave == (max(pw - 1, 0) >> 10) % BK_WAVES) {
+        rest_s = params + pw + lane;
+        byte_s = (uint8_t)ps[pw + lane];
+      }
+      if (FMT == 1 && lane < (zb & 15) && wave == (max(zw16 - 1, 0) >> 10) % BK_WAVES) {
+        rest_z = params + zoff + zw16 + lane;
+        byte_z = (uint8_t)pz[zw16 + lane];
+      }
+    }
     if (FMT == 1) {
-      const char* pz = (const char*)zeros + (size_t)n0 * wg * 4;
-      for (int o = wave * 1024; o < zb; o += BK_WAVES * 1024)
-        bk_dma((uint32_t)min(o + lane * 16, zb - 16), pz, lds0 + BK_WAVES * WB + zoff + o);
+      for (int o = wave * 1024; o < zw16; o += BK_WAVES * 1024)
+        bk_dma((uint32_t)min(o + lane * 16, zw16 - 16), pz, lds0 + BK_WAVES * WB + zoff + o);
     }
   }
 
@@ -110,6 +136,32 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
   const char* const qb = (const char*)q + (size_t)n0 * wrow;
   auto request_codes = [&](int U) BK_INLINE {
     const bool tail = (U + 1) * BK_UNIT > K;
+    if constexpr (RAG) {  // two rows a load, a dword a lane, to the places that the 16-byte loads give them
+      int lr = lane;
+      asm volatile("" : "+v"(lr) : : "memory");  // (offsets ahead of the loop would take registers)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int row = 2 * e + (lr >> 5);
+        const uint32_t in = (uint32_t)((((lr & 31) >> 2) ^ e) * 16 + (lr & 3) * 4);
+        uint32_t o = in;
+        if (tail) {
+          if ((uint32_t)U * 128 + in >= wrow) o = 0;
+          asm volatile("" : "+v"(o) : : "memory");
+        }
+        const uint32_t own = o + (uint32_t)row * wrow;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const int first = 16 * t < live ? 16 * t : 0;
+          uint32_t ot = own;
+          if (first + 16 > live) {  // rows past N repeat the last one
+            ot = o + (uint32_t)min(row, live - 1 - first) * wrow;
+            asm volatile("" : "+v"(ot) : : "memory");
+          }
+          bk_dma4(ot, qb + (size_t)first * wrow + (size_t)U * 128, region + t * 2048u + e * 256u);
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const char* base = qb + (16 * t < live ? (size_t)(16 * t) * wrow : 0) + (size_t)U * 128;
@@ -167,9 +219,14 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
     request_codes(wave);
 #pragma unroll
     for (int p = 0; p < XS; ++p) request_x(wave, p, p);
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * NT + 4 * XS));
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(CL + 4 * XS));
   } else {
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+  }
+  if constexpr (RAG) {
+    if (rest_s) *rest_s = byte_s;
+    if (rest_z) *rest_z = byte_z;
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
   }
   asm volatile("s_barrier" ::: "memory");  // the parameters are there
 
@@ -184,9 +241,14 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
   u4 cw[PC ? 1 : 2][NT];
   h8 A[NT][4];
   // group parameters of a lane's 32 k of a chunk, and their group; LATE: scales of the rows of its four sums
-  typedef std::conditional_t<LATE, h4, uint32_t> scale_t;
+  struct runs_t {  // GM: dwords that hold the slice's scales
+    uint32_t d[GM == 2 ? 3 : 2];
+  };
+  typedef std::conditional_t<LATE, h4, std::conditional_t<(GM > 0), runs_t, uint32_t>> scale_t;
+  typedef std::conditional_t<(GM > 0), u2, uint32_t> zero_t;
   scale_t sc[NT];
-  uint32_t zw[NT];
+  zero_t zw[NT];
+  [[maybe_unused]] const int gsw = gs >> 3;
   [[maybe_unused]] h4 late[NT];  // the scales of the chunk that is multiplied
   int g = 0, slot = 0;  // slot: of the piece that is multiplied
   const bool hook = w_out && m0 == 0;
@@ -202,8 +264,20 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
       v[j] = *(const h8*)(mine + NT * 2048 + at * 4096 + (r >> 2) * 1024 + ((r & 3) * 16 + ((4 * b + j) ^ r)) * 16);
   };
   auto read_params = [&](int chunk) BK_INLINE {
-    const int kc = min(chunk * 128 + (LATE ? 0 : 32 * b), K - 32);
-    g = MX ? (kc >> 5) : gs_shift >= 0 ? (kc >> gs_shift) : kc / gs;
+    const int kc = min(chunk * 128 + (LATE ? 0 : 32 * b), RAG ? K - 8 : K - 32);
+    g = MX ? (kc >> 5) : (int)__umulhi((uint32_t)kc >> 2, group_mul);
+    if constexpr (GM > 0) {
+      const uint8_t* ps = params + ((r * G + g) >> 1) * 4;
+      const uint8_t* pz = params + zoff + (r * wg + (g >> 3)) * 4;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+#pragma unroll
+        for (int e = 0; e < (GM == 2 ? 3 : 2); ++e) sc[t].d[e] = *(const uint32_t*)(ps + t * 32 * G + e * 4);
+        if (FMT == 1) zw[t] = u2{*(const uint32_t*)(pz + t * 64 * wg), *(const uint32_t*)(pz + t * 64 * wg + 4)};
+      }
+      return;
+    }
+    if constexpr (GM == 0) {
     const uint8_t* ps = params + ((LATE ? 4 * b : r) * G + g) * (MX ? 1 : 2);
     const uint8_t* pz = params + zoff + (r * wg + (g >> 3)) * 4;
 #pragma unroll
@@ -226,6 +300,7 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
       }
       asm volatile("" ::: "memory");
     }
+    }
   };
   auto request_next = [&](auto pc, int U, bool more) BK_INLINE {  // into the places that are free at step p of unit U
     constexpr int p = decltype(pc)::value;
@@ -235,7 +310,37 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
     slot = slot + 1 < XS ? slot + 1 : 0;
   };
   // the codes in w, with the parameters given, become the weights of a chunk; k: the lane's first
-  auto expand = [&](const u4* w, const scale_t* scale, const uint32_t* zword, int group, int k) BK_INLINE {
+  auto expand = [&](const u4* w, const scale_t* scale, const zero_t* zword, int group, int k) BK_INLINE {
+    if constexpr (GM > 0) {
+      const int rem = (int)((uint32_t)min(k, RAG ? K - 8 : K - 32) >> 3) - group * gsw;
+      uint32_t sel[4], zsh[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        sel[j] = 0x01000100u, zsh[j] = 0u;
+        if (j > 0) sel[j] = rem + j >= gsw ? 0x03020302u : sel[j], zsh[j] = rem + j >= gsw ? 4u : zsh[j];
+        if (GM == 2 && j > 1) sel[j] = rem + j >= 2 * gsw ? 0x05040504u : sel[j], zsh[j] = rem + j >= 2 * gsw ? 8u : zsh[j];
+        if (GM == 2 && j > 2) sel[j] = rem + j >= 3 * gsw ? 0x07060706u : sel[j], zsh[j] = rem + j >= 3 * gsw ? 12u : zsh[j];
+      }
+      if ((k & ~127) + 128 > K) {  // words past the end of the row: zeros, whatever scale they would have
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sel[j] = k + 8 * j >= K ? 0x0c0c0c0cu : sel[j];
+        asm volatile("" ::: "memory");
+      }
+      const uint32_t odd = ((uint32_t)(r * G + group) & 1u) * 16u;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const uint32_t lo = __builtin_amdgcn_alignbit(scale[t].d[1], scale[t].d[0], odd);
+        uint32_t hi = lo, zr = 0;
+        if constexpr (GM == 2) hi = __builtin_amdgcn_alignbit(scale[t].d[2], scale[t].d[1], odd);
+        if constexpr (FMT == 1) zr = __builtin_amdgcn_alignbit(zword[t][1], zword[t][0], 4 * (group & 7));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t z = FMT == 1 ? (zr >> zsh[j]) & 0xFu : 8u;
+          const h2 cneg = as_h2(0xD400E400u + z * 0x00100001u), s2 = as_h2(__builtin_amdgcn_perm(hi, lo, sel[j]));
+          A[t][j] = expand_word(w[t][j], cneg, s2, mask, magic);
+        }
+      }
+    } else {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       h2 cneg, s2 = h2{0, 0};
@@ -259,16 +364,29 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
         }
       }
     }
+    }
+    if constexpr (RAG && MX) {  // (a scale may overflow the codes of a slice that the row ends in)
+      if ((k & ~127) + 128 > K) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (k + 8 * j >= K) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) A[t][j] = __builtin_bit_cast(h8, u4{0u, 0u, 0u, 0u});
+          }
+        asm volatile("" ::: "memory");
+      }
+    }
     if (hook) {  // these registers are the weights (LATE: times the scale of the lane's row)
       int row = r;
       asm volatile("" : "+v"(row) : : "memory");  // (addresses ahead of the loop would take registers in every call)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
-        if (16 * t < live && k < K) {
+        if (16 * t + (RAG ? row : 0) < live && k < K) {
           const _Float16 own = LATE ? *(const _Float16*)(params + ((t * 16 + row) * G + group) * 2) : (_Float16)1.f;
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            *(h8*)(w_out + (size_t)(n0 + 16 * t + row) * K + k + 8 * j) = LATE ? A[t][j] * own : A[t][j];
+            if (!RAG || k + 8 * j < K)
+              *(h8*)(w_out + (size_t)(n0 + 16 * t + row) * K + k + 8 * j) = LATE ? A[t][j] * own : A[t][j];
         }
     }
   };
@@ -287,7 +405,11 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
   };
   auto multiply = [&](auto mtc, int chunk, h8* v) BK_INLINE {
     if (chunk * 128 + 128 > K) {  // the row ends inside this chunk: activations past it are zero
-      if (chunk * 128 + 32 * b >= K) {
+      if constexpr (RAG) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (chunk * 128 + 32 * b + 8 * j >= K) v[j] = __builtin_bit_cast(h8, u4{0u, 0u, 0u, 0u});
+      } else if (chunk * 128 + 32 * b >= K) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] = __builtin_bit_cast(h8, u4{0u, 0u, 0u, 0u});
       }
@@ -341,7 +463,7 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
         landed();
         request_next(pc, U, more);
         scale_t scale[NT];
-        uint32_t zword[NT];
+        zero_t zword[NT];
         const int group = g;
         if (mt == 0) {
 #pragma unroll
@@ -353,7 +475,7 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
         // requests younger than the next piece: the ring's others and, early in a unit, the next unit's codes
         if (p + 1 < NP || more) {
           constexpr int left = NP - 2 - p < 0 ? 0 : NP - 2 - p < XS - 1 ? NP - 2 - p : XS - 1;
-          if (more) __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 * (XS - 1) + (p < XS - 1 ? 2 * NT : 0)));
+          if (more) __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 * (XS - 1) + (p < XS - 1 ? CL : 0)));
           else __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 * left));
           landed();
           if (MT > 1 && p == NP - 1) read_codes(0, cw[0]), read_codes(1, cw[1]);
@@ -375,7 +497,7 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
         constexpr int p = decltype(pc)::value, ch = p / MT, mt = p % MT;
         // requests younger than the ones needed: the ring's other pieces, and next unit's codes
         constexpr int R = XS - 1, left = NP - 1 - p < R ? NP - 1 - p : R;
-        if (more) __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 * R + (p > PC && p < PC + XS ? 2 * NT : 0)));
+        if (more) __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 * R + (p > PC && p < PC + XS ? CL : 0)));
         else __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 * left));
         landed();
         if (PC && mt == 0) read_codes(ch, cw[0]);
@@ -420,21 +542,34 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
       }
       const h8 hv = h8{(_Float16)s0[0], (_Float16)s0[1], (_Float16)s0[2], (_Float16)s0[3],
                        (_Float16)s1[0], (_Float16)s1[1], (_Float16)s1[2], (_Float16)s1[3]};
-      *(h8*)(c + (size_t)m * N + n) = hv;
+      w4_half* const dst = c + (size_t)m * N + n;
+      if (RAG && (N & 7)) {
+        const int left = N - n;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const _Float16 h = hv[j];  // (a bit cast of a vector's element takes the first)
+          if (j < left) dst[j] = __builtin_bit_cast(uint16_t, h);
+        }
+      } else {
+        *(h8*)dst = hv;
+      }
     }
   }
 }
+
+bool bk_ragged(const WView& v) { return v.K % 32 || v.N % 16; }
 
 // Bytes of LDS of a workgroup with NT tiles of W.
 int bk_lds_bytes(const WView& v, int NT) {
   const int G = v.mx ? v.B : v.G;
   const long long p = 16LL * NT * G * (v.mx ? 1 : 2), z = v.mx || v.symmetric ? 0 : 64LL * NT * words(G);
-  const long long bytes = BK_WAVES * bk_wave_bytes(NT, BK_XS) + ((p + 1023) & ~1023LL) + ((z + 1023) & ~1023LL);
+  const int slack = !v.mx && (v.gs % 32 || bk_ragged(v)) ? 16 : 0;  // GM: the last dword of a run may lie behind the parameters
+  const long long bytes = BK_WAVES * bk_wave_bytes(NT, BK_XS) + ((p + 1023) & ~1023LL) + ((z + 1023) & ~1023LL) + slack;
   return bytes > (1 << 20) ? 1 << 20 : (int)bytes;
 }
 constexpr int BK_MAX_LDS = 160 * 1024;
 
-template <int FMT, int NT, int MT, bool LATE>
+template <int FMT, int NT, int MT, bool LATE, int GM, bool RAG>
 hipError_t block_go_as(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out) {
   constexpr int XS = BK_XS;
   constexpr bool AHEAD = NT <= 2;
@@ -443,35 +578,77 @@ hipError_t block_go_as(const WView& v, const w4_half* x, w4_half* c, int M, hipS
   int dev = 0;
   if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
   if (dev < 0 || dev >= 64 || !granted[dev]) {
-    const hipError_t e = hipFuncSetAttribute((const void*)mfma_block_kernel<FMT, NT, MT, XS, AHEAD, LATE>,
+    const hipError_t e = hipFuncSetAttribute((const void*)mfma_block_kernel<FMT, NT, MT, XS, AHEAD, LATE, GM, RAG>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, BK_MAX_LDS);
     if (e != hipSuccess) return e;
     if (dev >= 0 && dev < 64) granted[dev] = true;
   }
-  const bool pow2 = !v.mx && (v.gs & (v.gs - 1)) == 0;
   const int mg = (M + 16 * MT - 1) / (16 * MT), ng = (v.N + 16 * NT - 1) / (16 * NT);
-  mfma_block_kernel<FMT, NT, MT, XS, AHEAD, LATE><<<dim3((unsigned)(8 * ((ng + 7) / 8) * mg)), BK_THREADS, lds_bytes, s>>>(
-      v.q, v.scales, v.zeros, x, c, v.N, v.K, M, pow2 ? __builtin_ctz((unsigned)v.gs) : -1,
-      v.mx ? v.B : v.G, v.gs, mg, w_out);
+  const uint32_t mul = v.mx ? 0u : (uint32_t)(((1ULL << 31) + v.gs / 8 - 1) / (v.gs / 8));
+  mfma_block_kernel<FMT, NT, MT, XS, AHEAD, LATE, GM, RAG><<<dim3((unsigned)(8 * ((ng + 7) / 8) * mg)), BK_THREADS, lds_bytes, s>>>(
+      v.q, v.scales, v.zeros, x, c, v.N, v.K, M, mul, v.mx ? v.B : v.G, v.gs, mg, w_out);
   return hipGetLastError();
+}
+
+// Forms that are compiled for blocks of NT x MT.  Rows of words that are only 4-byte aligned take four times the load
+// instructions, small groups take LDS for their parameters: neither has blocks of more than two tiles of W.
+constexpr bool bk_has(int fmt, int NT, int MT, int gm, bool rag) {
+  (void)MT;
+  return fmt == 2 || gm == 0 || NT <= 2 || (gm == 1 && !rag);
 }
 
 template <int FMT, int NT, int MT>
 hipError_t block_go(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out) {
-  if constexpr (FMT != 2) {
-    if (v.gs % 128 == 0) return block_go_as<FMT, NT, MT, true>(v, x, c, M, s, w_out);
+  const bool rag = bk_ragged(v);
+  if constexpr (FMT == 2) {
+    return rag ? block_go_as<2, NT, MT, false, 0, true>(v, x, c, M, s, w_out) : block_go_as<2, NT, MT, false, 0, false>(v, x, c, M, s, w_out);
+  } else {
+    const int gm = v.gs < 32 ? 2 : rag || v.gs % 32 ? 1 : 0;
+    if (gm == 0)
+      return v.gs % 128 == 0 ? block_go_as<FMT, NT, MT, true, 0, false>(v, x, c, M, s, w_out)
+                             : block_go_as<FMT, NT, MT, false, 0, false>(v, x, c, M, s, w_out);
+    if constexpr (bk_has(FMT, NT, MT, 1, false))
+      if (gm == 1 && !rag) return block_go_as<FMT, NT, MT, false, 1, false>(v, x, c, M, s, w_out);
+    if constexpr (bk_has(FMT, NT, MT, 1, true))
+      if (gm == 1 && rag) return block_go_as<FMT, NT, MT, false, 1, true>(v, x, c, M, s, w_out);
+    if constexpr (bk_has(FMT, NT, MT, 2, false))
+      if (gm == 2 && !rag) return block_go_as<FMT, NT, MT, false, 2, false>(v, x, c, M, s, w_out);
+    if constexpr (bk_has(FMT, NT, MT, 2, true))
+      if (gm == 2 && rag) return block_go_as<FMT, NT, MT, false, 2, true>(v, x, c, M, s, w_out);
+    return hipErrorInvalidValue;
   }
-  return block_go_as<FMT, NT, MT, false>(v, x, c, M, s, w_out);
 }
 
 // Blocks and what a wave needs for 128 k of one, in units of 10 ns, W4 and MXFP4 (N = 4096, K = 14336 with
 // as many rows as make one round of workgroups, and N = 5120, K = 13824; a call takes 3.5 us more).  Groups of whole
 // chunks cost 0.97 to 1.03 of it.
+// start, round, per_n: the time of a call is start + rounds of workgroups x (round + per_n x units of the first wave), per_n
+// for symmetric W4, W4 with zero-points (groups as GM = 1) and MXFP4 (as RAG); fitted to 6657 shapes of 3 to 4000 rows
+// that are not whole chunks and groups, K = 256 to 14336, to within 8 to 18 % (r.m.s.).
 struct BkShape {
-  int nt, mt, cost_w4, cost_mx;
+  int nt, mt, cost_w4, cost_mx, start, round, per_n[3];
 };
-constexpr BkShape BK_SHAPES[] = {{1, 1, 50, 45},   {2, 1, 83, 56},   {2, 2, 106, 89},  {4, 1, 136, 80},  {2, 4, 171, 155},
-                                 {4, 2, 175, 125}, {3, 4, 195, 173}, {4, 4, 260, 215}, {4, 5, 290, 250}, {4, 6, 330, 290}};
+constexpr BkShape BK_SHAPES[] = {
+    {1, 1, 50, 45, 170, 130, {118, 133, 99}},      {2, 1, 83, 56, 140, 150, {188, 211, 139}},
+    {2, 2, 106, 89, 85, 210, {228, 247, 200}},     {4, 1, 136, 80, 110, 150, {334, 382, 223}},
+    {2, 4, 171, 155, 5, 300, {320, 335, 314}},     {4, 2, 175, 125, 70, 240, {390, 443, 303}},
+    {3, 4, 195, 173, -20, 370, {397, 426, 378}},   {4, 4, 260, 215, -45, 370, {505, 543, 458}},
+    {4, 5, 290, 250, -100, 450, {570, 617, 550}},  {4, 6, 330, 290, -110, 490, {624, 668, 634}}};
+constexpr int BK_COUNT = sizeof BK_SHAPES / sizeof BK_SHAPES[0];
+
+long long bk_rounds(const WView& v, int M, const BkShape& s, int cus) {
+  const long long ng = (v.N + 16 * s.nt - 1) / (16 * s.nt), mg = (M + 16 * s.mt - 1) / (16 * s.mt);
+  return ((ng + 7) / 8 * mg + cus / 8 - 1) / (cus / 8);
+}
+
+// Small groups take 1.15 of it (four selectors, more parameters), codes by the dword 1.06.
+int bk_time(const WView& v, int M, const BkShape& s, int cus) {
+  const int n = ((v.K + BK_UNIT - 1) / BK_UNIT + BK_WAVES - 1) / BK_WAVES;
+  long long per = s.per_n[v.mx ? 2 : v.symmetric ? 0 : 1];
+  if (!v.mx) per = per * (v.gs < 32 ? 115 : 100) / 100 * (bk_ragged(v) ? 106 : 100) / 100;
+  const long long t = s.start + bk_rounds(v, M, s, cus) * (s.round + per * n);
+  return t > 1 << 30 ? 1 << 30 : (int)t;
+}
 
 // Few rows (M < 17) and at most one tile of W a compute unit, K in whole chunks: the longest K that stays with the long-K
 // kernel, which fetches only the quads of x that exist and has no parameters to wait for.  [symmetric W4, with
@@ -542,7 +719,7 @@ bool block_ahead(const WView& v, int M, const BkShape& s, long long rounds, bool
 int block_plan(const WView& v, int M) {
   if (M < 3 || M > 8192 || (M < 9 && v.K <= 4096) || (M < 17 && v.K <= 2048)) return -1;
   if (v.K % 32 || v.N % 16 || (!v.mx && v.gs % 32)) return -1;
-  if (v.K >= 1 << 24) return -1;  // offsets inside a block have 32 bits
+  if (v.K >= 1 << 24 || !any_group_fits(v)) return -1;  // offsets inside a block have 32 bits
   const int cus = device_cus();
   if (cus < 8) return -1;
   // Few rows: one 16-row tile of W a workgroup (N = K = 4096, M = 8 5.2 against 5.0 us; K = 2048, M = 16 4.2 against
@@ -554,11 +731,10 @@ int block_plan(const WView& v, int M) {
   const bool dma = v.K % 128 == 0 && (v.mx || v.gs == 32 || v.gs == 64 || v.gs % 128 == 0);
   int best = -1;
   long long least = 0, best_rounds = 0;
-  for (int i = 0; i < (int)(sizeof BK_SHAPES / sizeof BK_SHAPES[0]); ++i) {
+  for (int i = 0; i < BK_COUNT; ++i) {
     const BkShape& s = BK_SHAPES[i];
     if (bk_lds_bytes(v, s.nt) > BK_MAX_LDS) continue;
-    const long long ng = (v.N + 16 * s.nt - 1) / (16 * s.nt), mg = (M + 16 * s.mt - 1) / (16 * s.mt);
-    const long long per_xcd = (ng + 7) / 8 * mg, rounds = (per_xcd + cus / 8 - 1) / (cus / 8);
+    const long long rounds = bk_rounds(v, M, s, cus);
     if (rounds > (dma || M < 17 ? 1 : 8)) continue;
     const long long cost = rounds * (v.mx ? s.cost_mx : s.cost_w4);
     if (best < 0 || cost < least) best = i, least = cost, best_rounds = rounds;
@@ -593,15 +769,35 @@ hipError_t block_fmt(int shape, const WView& v, const w4_half* x, w4_half* c, in
 
 }  // namespace
 
-int block_shape(const WView& v, int M) {
+int block_plan_time(const WView& v, int M, int* time) {
   const int i = block_plan(v, M);
+  if (i >= 0) *time = bk_time(v, M, BK_SHAPES[i], device_cus());
+  return i;
+}
+
+int block_any_time(const WView& v, int M, int cus, int* time) {
+  if (v.K % 8 || v.K < 32 || v.K >= 1 << 24 || M > 8192 || !any_group_fits(v)) return -1;
+  const int gm = v.mx ? 0 : v.gs < 32 ? 2 : 1;
+  int best = -1;
+  for (int i = 0; i < BK_COUNT; ++i) {
+    const BkShape& s = BK_SHAPES[i];
+    if (!bk_has(v.mx ? 2 : 0, s.nt, s.mt, gm, bk_ragged(v)) || bk_lds_bytes(v, s.nt) > BK_MAX_LDS) continue;
+    const int t = bk_time(v, M, s, cus);
+    if (best < 0 || t < *time) best = i, *time = t;
+  }
+  return best;
+}
+
+int block_shape(const WView& v, int M) {
+  const AnyPlan any = any_plan(v, M);
+  const int i = any.kind == 1 ? any.shape : block_plan(v, M);
   return i < 0 ? 0 : 10 * BK_SHAPES[i].nt + BK_SHAPES[i].mt;
 }
 
-bool try_block(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out, hipError_t* err) {
+bool try_block(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out, int shape, hipError_t* err) {
   if (((uintptr_t)v.q | (uintptr_t)v.scales | (uintptr_t)v.zeros | (uintptr_t)x | (uintptr_t)c | (uintptr_t)w_out) & 15)
     return false;
-  const int shape = block_plan(v, M);
+  if (shape < 0) shape = block_plan(v, M);
   if (shape < 0) return false;
   if (v.mx) *err = block_fmt<2>(shape, v, x, c, M, s, w_out);
   else if (v.symmetric) *err = block_fmt<0>(shape, v, x, c, M, s, w_out);

@@ -904,7 +904,9 @@ template <int MX>
 static hipError_t launch_fmt(const WView& v, const w4_half* x, w4_half* c, int M,
                              hipStream_t s, w4_half* w_out) {
   hipError_t terr = hipSuccess;
-  if (try_block(v, x, c, M, s, w_out, &terr)) return terr;
+  const AnyPlan any = any_plan(v, M);
+  if (any.kind == 2 && w_out == nullptr && try_tile_any(v, x, c, M, s, any.shape, &terr)) return terr;
+  if (try_block(v, x, c, M, s, w_out, any.kind == 1 ? any.shape : -1, &terr)) return terr;
   // Shapes of the kernel that fetches the activations once per workgroup (M <= 256):
   // hooked calls take the K-split kernel, which adds in the same order.
   const bool wvec = (v.K % 32 == 0) && (((uintptr_t)v.q) & 15) == 0;
@@ -957,6 +959,8 @@ int device_cus() {
 }
 
 int gemm_plan(const WView& v, int M) {
+  const AnyPlan any = any_plan(v, M);
+  if (any.kind == 2) return any.shape == 4 ? 4 : any.shape == 2 ? 5 : any.shape == 3 ? 6 : 7;
   if (const int shape = block_shape(v, M)) return shape;
   if (v.K % 32 == 0 && decode_longk_applies(v, nullptr, nullptr, M)) return 1;
   if (v.K % 32 == 0 && decode_resident_applies(v, nullptr, nullptr, M)) return 2;

@@ -1,0 +1,129 @@
+// The large-M W4A16 / MXFP4 GEMM of tile_dma.cuh for weights whose groups do not tile a 128-k stage: any
+// group size and any K that are multiples of 8 (mma.cuh:63-230, the reference's kernel, takes them all).
+#include "tile_dma.cuh"
+
+namespace w4k {
+namespace {
+
+// shape: 0 = 128 x 256 (rows of X x rows of W), 2 = 64 x 128, 3 = 128 x 128, 4 = 32 x 128
+template <int FMT, int GSM, int KT>
+hipError_t any_go(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, int tn, int tm, int shape,
+                  uint32_t mul) {
+  if (shape == 4) return launch<FMT, GSM, false, 32, 128, 2, KT>(v, x, c, nullptr, M, s, tn, tm, 0, mul);
+  if constexpr (GSM == 4) {
+    if (shape == 2) return launch<FMT, GSM, false, 64, 128, 1, KT>(v, x, c, nullptr, M, s, tn, tm, 0, mul);
+  } else {
+    if (shape == 2) return launch<FMT, GSM, false, 64, 128, 2, KT>(v, x, c, nullptr, M, s, tn, tm, 0, mul);
+    if (shape == 0) return launch<FMT, GSM, false, 128, 256, 1, KT>(v, x, c, nullptr, M, s, tn, tm, 0, mul);
+  }
+  return launch<FMT, GSM, false, 128, 128, 1, KT>(v, x, c, nullptr, M, s, tn, tm, 0, mul);
+}
+
+// Time of a call in units of 10 ns: start + rounds of workgroups x (round + per_n x n), n in stages of 128 k. Fitted to
+// 6657 shapes of 3 to 4000 rows, K = 256 to 14336, to within 4 to 10 % (r.m.s.); per_n: [symmetric W4, with
+// zero-points, MXFP4], small: the same for groups of less than 32.
+struct AnyShape {
+  int shape, tm, tn, start, round, per_n[3], small_round, small_n[2];
+};
+constexpr AnyShape ANY_SHAPES[] = {{4, 32, 128, 130, 285, {57, 66, 43}, 290, {71, 88}},
+                                   {2, 64, 128, 50, 430, {70, 74, 55}, 300, {98, 117}},
+                                   {3, 128, 128, -70, 490, {105, 115, 90}, 510, {115, 133}},
+                                   {0, 128, 256, -270, 850, {170, 186, 148}, 0, {0, 0}}};
+
+// Whether the tile kernels for any group take the operands, their alignment apart.
+bool any_applies(const WView& v, int M) {
+  if (v.K < 128 || v.K % 8 || v.K >= 1 << 24) return false;
+  if ((long long)v.N * v.K / 2 >= (1LL << 32) || (long long)M * v.K * 2 >= (1LL << 32)) return false;
+  if ((long long)((v.N + 127) / 128) * ((M + 31) / 32) > 0x7FFFFFFFLL) return false;
+  if (v.mx) return true;  // (a row has four blocks: one dword of scales is there)
+  return (long long)v.N * v.G >= 2 && (long long)v.N * v.G < (1LL << 31) && any_group_fits(v);
+}
+
+// The fastest tile and its time; -1: none.
+int any_shape(const WView& v, int M, int cus, int* time) {
+  const bool rag = v.K % 32 != 0, small = !v.mx && v.gs < 32;
+  const int stages = (v.K + 127) / 128, f = v.mx ? 2 : v.symmetric ? 0 : 1;
+  int best = -1;
+  long long least = 0;
+  for (const AnyShape& s : ANY_SHAPES) {
+    if (small && s.shape == 0) continue;  // (its parameters would not fit LDS)
+    const long long tiles = (long long)((v.N + s.tn - 1) / s.tn) * ((M + s.tm - 1) / s.tm), rounds = (tiles + cus - 1) / cus;
+    // (dword loads of codes: a tenth more)
+    const long long per = (long long)(small ? s.small_n[f] : s.per_n[f]) * stages * (rag ? 11 : 10) / 10;
+    const long long t = s.start + rounds * ((small ? s.small_round : s.round) + per);
+    if (best < 0 || t < least) best = s.shape, least = t;
+  }
+  *time = least > 1 << 30 ? 1 << 30 : (int)least;
+  return best;
+}
+
+// Time of the kernel that has the call otherwise, in the same units; of the stream kernel and the register-staged tiles
+// up to K = 1024 (from there on they took 1.3 to 5 times the others' time).
+int other_time(const WView& v, int M, int cus) {
+  const int stages = (v.K + 127) / 128, cpw = (stages + 7) / 8;
+  const long long tiles = (v.N + 15) / 16;
+  if (decode_general_applies(v, nullptr, nullptr, M)) {
+    const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4, per = (v.gs < 32 ? 9 : 0) + (v.symmetric ? 64 : 74);
+    return (int)(400 + (tiles + cus - 1) / cus * (cpw * (per + 19 * mt) - 30));
+  }
+  if (M <= 8 || (M <= 16 && v.N < 8192)) {  // (its times spread by a third: less a tenth)
+    if (v.K < 1024) return 0;
+    const long long share = tiles > cus ? tiles * 64 / cus : 64;  // tiles a compute unit, in 64ths
+    return (int)((v.K < 3072 ? 240 + share * (10 + 109 * cpw) / 64 : 80 + share * (175 * cpw - 70) / 64) * 9 / 10);
+  }
+  if (v.K >= 1024) return 1 << 30;
+  if (v.K % 64 == 0 && M >= 96) {
+    const long long rounds = ((long long)((v.N + 127) / 128) * ((M + 255) / 256) + cus - 1) / cus;
+    return (int)(rounds * (950 + 113 * (v.K / 64)) - 300);
+  }
+  const int rows = M <= 32 ? 32 : 64;
+  const long long wgs = (long long)((v.N + 63) / 64) * ((M + rows - 1) / rows), share = 2 * wgs > cus ? wgs * 64 / cus : 32;
+  return (int)(M <= 32 ? 440 + share * 50 * stages / 64 : 275 + 38 * stages + share * (127 + 110 * stages) / 64);
+}
+
+}  // namespace
+
+bool any_group_fits(const WView& v) { return v.mx || (long long)(v.K / 8) * (v.gs / 8) < (1LL << 31); }
+
+AnyPlan any_plan(const WView& v, int M) {
+  const AnyPlan none{0, -1};
+  const int cus = device_cus();
+  // (shorter rows: no more than a launch for the kernels that have them)
+  if (M < 5 || v.K % 8 || v.K < (M < 17 ? 1024 : 256) || cus < 8) return none;
+  const bool dma = v.K % 128 == 0 && (v.mx || v.gs == 32 || v.gs == 64 || v.gs % 128 == 0);
+  const bool whole = v.N % 16 == 0 && v.K % 32 == 0 && (v.mx || v.gs % 32 == 0);
+  // shapes of the kernels for whole tiles, chunks and groups
+  if (whole && (M < 17 || (v.K % 128 == 0 && M <= 64))) return none;
+  // the direct-to-LDS tiles take any N (but no fewer than eight tiles, and no scales that end inside a dword)
+  if (dma && M >= 65 && (long long)((v.N + 255) / 256) * ((M + 127) / 128) >= 8 &&
+      (v.mx || v.gs < 128 || (long long)v.N * v.G % 2 == 0)) return none;
+  int tile = -1, tile_time = 1 << 30, block_shape = -1, block_t = 1 << 30;
+  if (any_applies(v, M)) tile = any_shape(v, M, cus, &tile_time);
+  if (whole) {
+    // blocks as block_plan() has them; tiles where these are ahead by a quarter (the error of the times on both sides)
+    block_shape = block_plan_time(v, M, &block_t);
+    if (block_shape < 0) return tile_time < other_time(v, M, cus) ? AnyPlan{2, tile} : none;
+    return 5 * tile_time < 4 * block_t ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
+  }
+  block_shape = block_any_time(v, M, cus, &block_t);
+  const int other = other_time(v, M, cus);
+  if (tile_time >= other && block_t >= other) return none;
+  return tile_time < block_t ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
+}
+
+bool try_tile_any(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, int shape, hipError_t* err) {
+  const bool rag = v.K % 32 != 0;
+  if (((uintptr_t)x & 15) || ((uintptr_t)v.q & (rag ? 3 : 15)) || ((uintptr_t)v.scales & 3)) return false;
+  if (!v.mx && !v.symmetric && ((uintptr_t)v.zeros & 3)) return false;
+  const int TN = shape == 0 ? 256 : 128, TM = shape == 2 ? 64 : shape == 4 ? 32 : 128;
+  const int tn = (v.N + TN - 1) / TN, tm = (M + TM - 1) / TM;
+  const uint32_t mul = v.mx ? 0u : (uint32_t)(((1ULL << 31) + v.gs / 8 - 1) / (v.gs / 8));
+#define W4_GO(F, G) (rag ? any_go<F, G, 2>(v, x, c, M, s, tn, tm, shape, mul) : any_go<F, G, 1>(v, x, c, M, s, tn, tm, shape, mul))
+  if (v.mx) *err = W4_GO(2, 3);
+  else if (v.symmetric) *err = v.gs >= 32 ? W4_GO(0, 3) : W4_GO(0, 4);
+  else *err = v.gs >= 32 ? W4_GO(1, 3) : W4_GO(1, 4);
+#undef W4_GO
+  return true;
+}
+
+}  // namespace w4k

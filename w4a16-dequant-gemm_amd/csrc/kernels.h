@@ -58,9 +58,27 @@ bool try_tile256(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_
 // gemm_block.hip: middle M (17 to some hundred rows, at long K from 3 on), blocks of W and x as square as few rounds
 // of workgroups allow, hooked calls included; false (nothing launched) when another kernel is ahead.
 bool try_block(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out,
-               hipError_t* err);
+               int shape, hipError_t* err);
+// shape: the block that any_plan() names, or -1: block_plan()'s own.
 // Its block for operands aligned to 16 bytes: 10 x tiles of W + row tiles of x; 0: not its shape.
 int block_shape(const WView& v, int M);
+
+// Time of its best block in units of 10 ns, and which; -1: none.  block_plan_time: for shapes of whole tiles, chunks and
+// groups, where another kernel may be ahead as well; block_any_time: for every other.
+int block_plan_time(const WView& v, int M, int* time);
+int block_any_time(const WView& v, int M, int cus, int* time);
+
+// gemm_tile_any.hip: the kernel of gemm_tile_dma.hip for any group size and any K that are multiples of 8, and the
+// plan for calls whose sizes the kernels for whole tiles, chunks and groups do not take: kind 1 a block
+// (shape: its index), 2 a tile, 0 another kernel.
+struct AnyPlan {
+  int kind, shape;
+};
+AnyPlan any_plan(const WView& v, int M);
+// Whether a reciprocal gives the group of every word (see launch() in tile_dma.cuh).
+bool any_group_fits(const WView& v);
+// Launches the planned tile (no hook); false (nothing launched) when the arrays are not aligned for it.
+bool try_tile_any(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, int shape, hipError_t* err);
 
 // gemm_decode_resident.hip: M <= 64 with the activations fetched once per workgroup
 // (several 16-row tiles each).  Same order of additions as the K-split decode
