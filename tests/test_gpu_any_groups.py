@@ -112,3 +112,17 @@ def test_ends_of_rows_bring_no_infinity(M, N, K, gs):
     ok = np.isfinite(ref) & np.isfinite(got[rows])
     assert np.linalg.norm((got[rows] - ref)[ok]) <= 1e-3 * np.linalg.norm(ref[ok])
     assert np.array_equal(np.isnan(got[2]), np.isnan(bad[0])) and np.array_equal(np.isinf(got[2]), np.isinf(bad[0]))
+
+
+@pytest.mark.parametrize("M,N,K", [(136, 1639, 1152), (500, 2050, 384), (129, 2048, 128), (1100, 1024, 1024), (70, 2306, 1280)])
+def test_thin_grids_of_32_groups_with_zero_points(M, N, K):
+    """gs = 32 with zero-points on the two smallest tiles (one stage, an odd number of them, ragged rows): the hooked kernel
+    splits its sum over K at the same stage, so both calls return the same bytes."""
+    c = w4amd.capi()
+    assert _check(1, M, N, K, 32) == 0
+    p = orc.quantize(orc.normal_weights(N * K, 7) * 0.02 + 0.01, N, K, 32, False)
+    dp, x_d = DevPacked(p), to_dev(orc.normal_activations(M * K, 8))
+    plain, hooked, w = halves(M * N), halves(M * N), halves(N * K)
+    c.gemm_mma(dp.view, ptr(x_d), ptr(plain), M)
+    c.gemm_mma(dp.view, ptr(x_d), ptr(hooked), M, 0, ptr(w))
+    assert torch.equal(plain, hooked)

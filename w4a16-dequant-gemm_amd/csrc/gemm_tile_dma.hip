@@ -59,18 +59,23 @@ bool try_tile_dma(const WView& v, const w4_half* x, w4_half* c, int M, hipStream
   const long long m128 = (M + 127) / 128, m64 = (M + 63) / 64, m32 = (M + 31) / 32;
   // the shape an unhooked call takes; the hooked kernel has 128 x 256 tiles only, but follows
   // the unhooked call's split of the sum over K (below)
+  // Groups of 32 with zero-points have three dwords of parameters a row and stage, which 128 rows of W a workgroup cannot
+  // fetch here: the two smallest tiles are those of the kernels for any group (N = 1639, K = 6784, M = 136
+  // 61.3 -> 40.2 us; N = K = 4096, M = 512 37.7 -> 32.3; N = K = 5120, M = 300 46.2 -> 35.7).
+  const bool planes3 = gsm == 2 && !v.mx && !v.symmetric;
   int shape = 0;
   {
-    const bool planes3 = gsm == 2 && !v.mx && !v.symmetric;  // needs 256 rows of W per workgroup
-    if (!planes3 && n128 * m32 <= 256) shape = 4;
-    else if (!planes3 && n128 * m64 <= 256) shape = 2;
+    if (n128 * m32 <= 256) shape = 4;
+    else if (n128 * m64 <= 256) shape = 2;
     else if (!planes3 && n128 * m128 <= 256) shape = 3;
     else if (n256 * m64 <= 256) shape = 1;
   }
   // The two smallest tiles run with two sets of waves, each on one half of K (their stages
   // are a serial chain; see the kernel): the sum over K is then (first half) + (second half).
   const int stages = v.K / 128;
-  const int sets = (shape == 2 || shape == 4) && stages >= 8 ? 2 : 1;
+  const bool any = planes3 && (shape == 2 || shape == 4);
+  const int any_tile = shape;
+  const int sets = (shape == 2 || shape == 4) && (stages >= 8 || any) ? 2 : 1;
   const int split_at = sets == 2 ? (stages + 1) / 2 : v.K;
   if (w_out) shape = 0;
   const long long tiles_n = (shape == 2 || shape == 3 || shape == 4) ? n128 : n256;
@@ -84,6 +89,7 @@ bool try_tile_dma(const WView& v, const w4_half* x, w4_half* c, int M, hipStream
   if (w_out && ((uintptr_t)w_out & 15)) return false;
   // grids of more than one round: 256 x 256 tiles where they halve the rounds
   if (!w_out && try_tile256(v, x, c, M, s, 256, err)) return true;
+  if (any && !w_out) return try_tile_any(v, x, c, M, s, any_tile, err);
   const int tn = (int)tiles_n, tm = (int)tiles_m;
   if (v.mx) *err = launch_hook<2, 2>(v, x, c, w_out, M, s, tn, tm, shape, sets, split_at);
   else if (v.symmetric) *err = launch_gsm<0>(gsm, v, x, c, w_out, M, s, tn, tm, shape, sets, split_at);
