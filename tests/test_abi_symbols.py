@@ -234,3 +234,29 @@ def test_noalloc_entry_contracts_without_a_device():
     # 512 splits x 64 query heads x 130 floats = 17 MB of partials
     with pytest.raises(ValueError, match="exceed the built-in scratch"):
         c.attention_w4_flash_noalloc(c.kv_view(1, 1 << 19, 128, 32, 4, 1, one, one, 0, one, one, 0), one, one, group=64)
+
+
+def test_native_calls_take_and_refuse_what_ctypes_does():
+    """The callables behind the Python entry points: positional, keyword and missing arguments, None and wrong types, each
+    against the ctypes function that stands behind (validation fails in every call: nothing reaches a device)."""
+    capi = w4amd.capi()
+    lib = capi.load()
+    assert all(hasattr(getattr(capi, n), "__wrapped__") for n in capi._NATIVE)
+    v, kv = capi.packed_view(2, 32, 7, 4, 1, 1, 1), capi.kv_f8_view(1, 1, 128, 7, 1, 1, 1, 1, 1)
+    calls = [("gemm", (v, 1, 1, 1), {}), ("gemm", (v, 1, 1), {"M": 1, "stream": None}), ("gemm", (v, 1, 1), {}),
+             ("gemm", (v, 1, 1, 1), {"M": 2}), ("gemm", (v, 1, 1, 1), {"other": 2}), ("gemm", (v, 1, 1, 1, 0, 0, 0), {}),
+             ("gemm", (3, 1, 1, 1), {}), ("gemm", (kv, 1, 1, 1), {}), ("gemm", (v, 2.0, 1, 1), {}), ("gemm", (v, None, 1, 1), {}),
+             ("gemm", (), {}), ("gemm", (v, 1, 1, "1"), {}), ("attention_f8_flash", (kv, 1, 1), {"scale_mode": 1, "group": 3}),
+             ("quantize_cache_f8", (kv, 1, 1, 1), {"src_f16": True}), ("quantize_cache_f8", (kv, 1, 1), {"status": None}),
+             ("attention_fp16_flash", (1, 1, 1, 1, 0, 1, 128), {"group": 0})]
+    for name, args, options in calls:
+        said = []
+        for f in (getattr(capi, name), getattr(capi, name).__wrapped__):
+            with pytest.raises(Exception) as e:
+                f(*args, **options)
+            said.append((e.type, str(e.value)))
+        assert said[0] == said[1], (name, args, options)
+    # arguments in the C functions' order: a validator that names what it found
+    with pytest.raises(ValueError, match="group"):
+        capi.attention_w4_flash(capi.kv_view(1, 64, 128, 32, 4, 1, 16, 16, 0, 16, 16, 0), 16, 16, group=-1)
+    assert lib.w4_last_error()

@@ -6,11 +6,13 @@
 import os
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "lib", "libw4amd.so")
 BENCH_LIB = os.path.join(PKG, "lib", "libw4bench.so")
+CALLS = os.path.join(PKG, "lib", "w4calls.so")  # the Python entry points' native calls (csrc/pycalls.cpp)
 SOURCES = ["abi.hip", "dequant.hip", "gemm_simt.hip", "gemm_mfma.hip", "flash.hip", "flash_mfma.hip", "quantize.hip", "gemm_mxnative.hip", "gemm_tile_dma.hip", "gemm_tile_any.hip", "gemm_tile256.hip", "gemm_decode_resident.hip", "gemm_decode_general.hip", "gemm_decode_longk.hip", "gemm_block.hip",
            "baseline.hip"]
 HEADERS = ["dq.cuh", "kernels.h", "simt_rows4.cuh", "tile_dma.cuh", "bench_kernels.hip", os.path.join("..", "..", "include", "w4_abi.h")]
@@ -37,10 +39,10 @@ EXTRA_FLAGS = {"flash_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 
 
 def _stale():
-    if not os.path.exists(LIB):
+    if not os.path.exists(LIB) or not os.path.exists(CALLS):
         return True
     t = os.path.getmtime(LIB)
-    deps = [os.path.join(CSRC, f) for f in SOURCES + HEADERS] + [os.path.abspath(__file__)]
+    deps = [os.path.join(CSRC, f) for f in SOURCES + HEADERS + ["pycalls.cpp"]] + [os.path.abspath(__file__)]
     return any(os.path.getmtime(d) > t for d in deps)
 
 
@@ -69,6 +71,10 @@ def build(force=False, verbose=True):
             print(err, file=sys.stderr)
     subprocess.check_call(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs,
                            "-lhipblaslt"])
+    calls_src = os.path.join(CSRC, "pycalls.cpp")
+    if force or not os.path.exists(CALLS) or os.path.getmtime(CALLS) < max(hdr_t, os.path.getmtime(calls_src)):
+        subprocess.check_call(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
+                               "-I" + sysconfig.get_paths()["include"], calls_src, "-o", CALLS])
     # bandwidth yardsticks used only by bench.py
     bench_src = os.path.join(CSRC, "bench_kernels.hip")
     if (force or not os.path.exists(BENCH_LIB)

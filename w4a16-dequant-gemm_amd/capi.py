@@ -1,8 +1,14 @@
 """ctypes view of libw4amd.so.  Arguments are raw device addresses (ints, e.g.
 ``tensor.data_ptr()``); 0 stands for a null pointer.  Errors map like the C++
 wrappers: W4_EINVAL -> ValueError (std::invalid_argument), W4_ERUNTIME ->
-RuntimeError.  There is no fallback: a missing library raises at load()."""
+RuntimeError.  There is no fallback: a missing library raises at load().
+
+From load() on the entry points of _NATIVE are callables of lib/w4calls.so, which convert
+the usual arguments themselves; the functions below stay behind them for the rest."""
 import ctypes as C
+import importlib.machinery
+import importlib.util
+import inspect
 import os
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
@@ -91,8 +97,62 @@ def load():
         for name, (args, res) in SIGNATURES.items():
             fn = getattr(L, name)
             fn.argtypes, fn.restype = args, res
+        _bind(L)
         _lib = L
     return _lib
+
+
+# Python entry point -> its C function, and the Python parameters in the C function's order (None: its own)
+_NATIVE = {
+    "dequant": ("w4_dequant", None),
+    "gemm_fused": ("w4_gemm_fused", None),
+    "gemm_mma": ("w4_gemm_mma", None),
+    "gemm": ("w4_gemm", None),
+    "dequant_mx": ("w4_dequant_mx", None),
+    "gemm_fused_mx": ("w4_gemm_fused_mx", None),
+    "gemm_mma_mx": ("w4_gemm_mma_mx", None),
+    "gemm_mx": ("w4_gemm_mx", None),
+    "attention_w4_flash": ("w4_attention_w4_flash_gqa", "view group q out stream k_out v_out"),
+    "attention_w4_flash_noalloc": ("w4_attention_w4_flash_gqa_noalloc", "view group q out stream k_out v_out"),
+    "attention_fp16_flash": ("w4_attention_fp16_flash_gqa", "q k16 v16 out H group S D stream"),
+    "attention_f8_flash": ("w4_attention_f8_flash_gqa", "view group scale_mode q out stream k_out v_out"),
+    "attention_w4_flash_paged": ("w4_attention_w4_flash_paged", None),
+    "attention_w4_flash_paged_batched": ("w4_attention_w4_flash_paged_batched", None),
+    "quantize": ("w4_quantize", None),
+    "quantize_mx": ("w4_quantize_mx", None),
+    "quantize_mx_f16": ("w4_quantize_mx_f16", None),
+    "quantize_mx8_f16": ("w4_quantize_mx8_f16", None),
+    "quantize_cache": ("w4_quantize_cache", "view k v src_f16 status stream"),
+    "quantize_cache_f8": ("w4_quantize_cache_f8", "view k v src_f16 status stream"),
+    "gemm_mx_w4a4": ("w4_gemm_mx_w4a4", None),
+    "gemm_mx_w4a8": ("w4_gemm_mx_w4a8", None),
+}
+
+
+def _bind(lib):
+    """Puts native callables in the place of the functions that _NATIVE names."""
+    path = os.path.join(_PKG, "lib", "w4calls.so")
+    loader = importlib.machinery.ExtensionFileLoader("w4calls", path)
+    native = importlib.util.module_from_spec(importlib.util.spec_from_file_location("w4calls", path, loader=loader))
+    loader.exec_module(native)
+    here = globals()
+
+    def address(name):
+        return C.cast(getattr(lib, name), vp).value
+
+    for name, (symbol, order) in _NATIVE.items():
+        params = inspect.signature(here[name]).parameters
+        names = tuple(params)
+        slots = names if order is None else tuple(order.split())
+        kinds = SIGNATURES[symbol][0]
+        if sorted(slots) != sorted(names) or len(kinds) != len(names):
+            raise RuntimeError(f"{name} and {symbol} take different arguments")
+        views = tuple(getattr(kinds[slots.index(n)], "_type_", None) if issubclass(kinds[slots.index(n)], C._Pointer)
+                      else None for n in names)
+        defaults = tuple(0 if p.default is p.empty else int(p.default) for p in params.values())
+        required = sum(p.default is p.empty for p in params.values())
+        here[name] = native.make(address(symbol), address("w4_last_error"), here[name], names, views, defaults,
+                                 tuple(slots.index(n) for n in names), required)
 
 
 def check(rc):
