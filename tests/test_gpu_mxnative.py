@@ -448,3 +448,31 @@ def test_activation_quantizers_nan_and_infinity(fmt, K):
     assert np.array_equal(got[~cols], base[~cols])
     if fmt == "mx8":
         assert (got[3, 40] & 0x7F) == 0x7E and (got[5, K - 1] & 0x7F) == 0x7E
+
+
+@pytest.mark.parametrize("x8", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 48, 128), (16, 64, 1152), (9, 33, 5504), (17, 40, 2176), (32, 520, 1408), (33, 80, 4224), (48, 12304, 384),
+                                   (40, 8208, 640), (64, 100, 1920), (64, 8208, 896), (5, 4100, 256), (70, 64, 11008)])
+def test_skinny_kernel_with_whole_groups_of_blocks(M, N, K, x8):
+    """K a multiple of 128 and not of 512 (one to three of the last super-step's four groups exist; K = 128: waves without
+    one) for one to four tiles of X and one to three of W.  The codes and scales that stand in for a missing group are
+    the last group's, where the activations are the largest: nothing of them may reach the product twice."""
+    c = w4amd.capi()
+    rng = np.random.default_rng(M + K)
+    wq = orc.quantize_mx(orc.outlier_weights(N, K, M + N), N, K)
+    xf = orc.normal_activations(M * K, M + 1).view(np.float16).astype(np.float64).reshape(M, K)
+    xf[:, K - 128:] = rng.choice([-6.0, 6.0], (M, 128))
+    xq = (orc.quantize_mx8 if x8 else orc.quantize_mx)(xf.ravel(), M, K)
+    x_d, s_d, dw, out = to_dev(xq.q), to_dev(xq.scales), DevPackedMx(wq), halves(M * N + 16, 0x7E00)
+    if x8:
+        c.gemm_mx_w4a8(dw.view, c.act_mx8_view(M, K, K // 32, ptr(x_d), ptr(s_d)), ptr(out))
+        xd = orc.dequant_mx8(xq)
+    else:
+        c.gemm_mx_w4a4(dw.view, c.packed_mx_view(M, K, K // 32, ptr(x_d), ptr(s_d)), ptr(out))
+        xd = orc.dequant_all_mx(xq).view(np.float16).astype(np.float64)
+    got = bits(out)
+    assert (got[M * N:] == 0x7E00).all()
+    ns = np.unique(np.concatenate([np.arange(min(N, 20)), np.arange(max(0, N - 20), N), rng.choice(N, size=min(N, 150))]))
+    wd = np.ascontiguousarray(orc.dequant_all_mx(wq).view(np.float16).astype(np.float64).reshape(N, K)[ns])
+    ref = np.asarray(xd, np.float64).reshape(M, K) @ wd.T
+    assert orc.rel_l2(np.ascontiguousarray(got[: M * N].reshape(M, N)[:, ns]).view(np.float16), ref.ravel()) <= TOL

@@ -60,15 +60,24 @@ __device__ __forceinline__ f4 mfma_fp4_fp8(u4 a, uint32_t sa, u4 b0, u4 b1, uint
 // A lane's share of one 512-k super-step of a packed row: block 4j + g of the
 // super-step for j = 0..3 (g = lane / 16), so that load j of the four lane
 // groups covers one contiguous 64-byte piece of every row, and MFMA j contracts
-// 128 consecutive k.  sc[j] carries the block's scale in byte 0.  FULL: every
-// block exists and rows are 16-byte aligned.  Otherwise words past the row read
-// as zero codes, codes past K are masked off, and missing blocks take the
-// neutral scale byte 127.
-template <bool FULL>
+// 128 consecutive k.  sc[j] carries the block's scale in byte 0.  MX_FULL: every
+// block exists and rows are 16-byte aligned.  MX_GROUPS (K a multiple of 128): a group of four
+// blocks exists or it does not, the same for the whole wave; rows are 16-byte, their scales 4-byte aligned.  MX_ANY:
+// words past the row read as zero codes, codes past K are masked off.  Missing blocks are zero
+// codes and take the neutral scale byte 127.
+enum { MX_ANY = 0, MX_FULL = 1, MX_GROUPS = 2 };
+template <int FORM>
 __device__ __forceinline__ void load_blocks(const uint32_t* __restrict__ qrow,
                                             const uint8_t* __restrict__ srow, int ss, int g,
                                             int B, int wk, int K, u4 q[4], uint32_t sc[4]) {
-  if (FULL) {
+  if (FORM == MX_GROUPS) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int there = min(ss * 4 + j, (B >> 2) - 1);  // (a missing group's place: the last one)
+      q[j] = *(const u4*)(qrow + (size_t)(there * 4 + g) * 4);
+      sc[j] = *(const uint32_t*)(srow + there * 4);
+    }
+  } else if (FORM == MX_FULL) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) q[j] = *(const u4*)(qrow + (size_t)(ss * 16 + 4 * j + g) * 4);
     const u4 s16 = *(const u4*)(srow + ss * 16);
@@ -96,11 +105,20 @@ __device__ __forceinline__ void load_blocks(const uint32_t* __restrict__ qrow,
 // first four registers and k 64+16g..64+16g+15 in the other four, while its scale
 // register still carries the scale of 32-block g of those 128 k.  The four lane
 // groups of either load cover 64 contiguous bytes of every row.
-template <bool FULL>
+template <int FORM>
 __device__ __forceinline__ void load_blocks8(const uint8_t* __restrict__ qrow,
                                              const uint8_t* __restrict__ srow, int ss, int g,
                                              int B, int K, u4 q[4][2], uint32_t sc[4]) {
-  if (FULL) {
+  if (FORM == MX_GROUPS) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int there = min(ss * 4 + j, (B >> 2) - 1);
+      const uint8_t* p = qrow + (size_t)there * 128 + 16 * g;
+      q[j][0] = *(const u4*)p;
+      q[j][1] = *(const u4*)(p + 64);
+      sc[j] = *(const uint32_t*)(srow + there * 4);
+    }
+  } else if (FORM == MX_FULL) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const uint8_t* p = qrow + (size_t)ss * 512 + 128 * j + 16 * g;
@@ -128,7 +146,7 @@ __device__ __forceinline__ void load_blocks8(const uint8_t* __restrict__ qrow,
 // tiles, so X crosses L2 -> CU once per workgroup.  Partial sums meet in LDS
 // and are added in wave order.
 // XF8: X holds E4M3 bytes (K per row) instead of packed E2M1 codes.
-template <int MT, int NT, bool FULL, bool XF8>
+template <int MT, int NT, int FORM, bool XF8>
 __global__ __launch_bounds__(NV_WAVES * 64) void mxn_decode_kernel(
     const uint32_t* __restrict__ wq, const uint8_t* __restrict__ ws,
     const uint32_t* __restrict__ xq, const uint8_t* __restrict__ xs, w4_half* __restrict__ c,
@@ -166,20 +184,44 @@ __global__ __launch_bounds__(NV_WAVES * 64) void mxn_decode_kernel(
     uint32_t sb[MT][4], sa[NT][4];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
-      load_blocks<FULL>(wrow[nt], wsrow[nt], ss, g, B, wk, K, a[nt], sa[nt]);
+      load_blocks<FORM>(wrow[nt], wsrow[nt], ss, g, B, wk, K, a[nt], sa[nt]);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       if constexpr (XF8) {
-        load_blocks8<FULL>((const uint8_t*)xrow[mt], xsrow[mt], ss, g, B, K, b[mt], sb[mt]);
+        load_blocks8<FORM>((const uint8_t*)xrow[mt], xsrow[mt], ss, g, B, K, b[mt], sb[mt]);
       } else {
         u4 q[4];
-        load_blocks<FULL>(xrow[mt], xsrow[mt], ss, g, B, wk, K, q, sb[mt]);
+        load_blocks<FORM>(xrow[mt], xsrow[mt], ss, g, B, wk, K, q, sb[mt]);
 #pragma unroll
         for (int j = 0; j < 4; ++j) b[mt][j][0] = q[j];
       }
     }
     // every load of the super-step is in flight before the first product waits
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (FORM == MX_GROUPS) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) sa[nt][j] >>= 8 * g;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) sb[mt][j] >>= 8 * g;
+      }
+      if (ss * 16 + 16 > B) {  // the row's last super-step
+#pragma unroll
+        for (int j = 1; j < 4; ++j)
+          if (ss * 16 + 4 * j >= B) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) a[nt][j] = u4{0u, 0u, 0u, 0u}, sa[nt][j] = 127u;
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+              for (int e = 0; e < (XF8 ? 2 : 1); ++e) b[mt][j][e] = u4{0u, 0u, 0u, 0u};
+              sb[mt][j] = 127u;
+            }
+          }
+        asm volatile("" ::: "memory");  // (a branch: as selects it would cost every super-step)
+      }
+    }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -223,25 +265,30 @@ __global__ __launch_bounds__(NV_WAVES * 64) void mxn_decode_kernel(
   }
 }
 
-// FULL_ONLY: the caller has checked K % 512 == 0 and the guarded form of this shape is
+// FULL_ONLY: the caller has checked K % 128 == 0 and the guarded form of this shape is
 // not compiled (it does not fit the register file); unaligned operands then take two
 // row tiles.
 template <int MT, int NT, bool XF8, bool FULL_ONLY = false>
 hipError_t launch_decode_nt(const w4_packed_mx_view& w, const void* xq, const uint8_t* xs, int M,
                             w4_half* c, hipStream_t s) {
   const int N = w.N, K = w.K;
-  const bool full = K % 512 == 0 && ((uintptr_t)w.q & 15) == 0 && ((uintptr_t)xq & 15) == 0 &&
-                    ((uintptr_t)w.scales & 15) == 0 && ((uintptr_t)xs & 15) == 0;
+  const bool rows = K % 128 == 0 && ((uintptr_t)w.q & 15) == 0 && ((uintptr_t)xq & 15) == 0;
+  const bool full = rows && K % 512 == 0 && ((uintptr_t)w.scales & 15) == 0 && ((uintptr_t)xs & 15) == 0;
   const dim3 grid((unsigned)((N + 16 * NT - 1) / (16 * NT)),
                   (unsigned)((M + 16 * MT - 1) / (16 * MT)));
   const dim3 block(NV_WAVES * 64);
   if (full) {
-    mxn_decode_kernel<MT, NT, true, XF8><<<grid, block, 0, s>>>(
+    mxn_decode_kernel<MT, NT, MX_FULL, XF8><<<grid, block, 0, s>>>(
+        w.q, w.scales, (const uint32_t*)xq, xs, c, N, K, w.B, M);
+  } else if (rows && (((uintptr_t)w.scales | (uintptr_t)xs) & 3) == 0) {
+    // K = 11008, N = 4096, guarded loads -> these: 4-bit X, M = 1 14.0 -> 6.8 us, 16 23.0 -> 8.7; 8-bit X 14.3 -> 7.5, M = 32
+    // 24.0 -> 17.2 (K = 14336: 6.6, 9.2; 7.1, 18.5); K = 5504, N = 2048, 4-bit X, M = 64 27.3 -> 8.6
+    mxn_decode_kernel<MT, NT, MX_GROUPS, XF8><<<grid, block, 0, s>>>(
         w.q, w.scales, (const uint32_t*)xq, xs, c, N, K, w.B, M);
   } else if constexpr (FULL_ONLY) {
     return launch_decode_nt<MT, 2, XF8>(w, xq, xs, M, c, s);
   } else {
-    mxn_decode_kernel<MT, NT, false, XF8><<<grid, block, 0, s>>>(
+    mxn_decode_kernel<MT, NT, MX_ANY, XF8><<<grid, block, 0, s>>>(
         w.q, w.scales, (const uint32_t*)xq, xs, c, N, K, w.B, M);
   }
   return hipGetLastError();
@@ -264,7 +311,7 @@ hipError_t launch_decode(const w4_packed_mx_view& w, const void* xq, const uint8
   if constexpr (MT < 4) {
     if (nt >= 3) {
       constexpr bool fits_ragged = !(XF8 && MT == 3);
-      const bool full = w.K % 512 == 0;
+      const bool full = w.K % 128 == 0;
       if (fits_ragged || full) return launch_decode_nt<MT, 3, XF8, !fits_ragged>(w, xq, xs, M, c, s);
     }
   }
@@ -1128,12 +1175,11 @@ bool tile_operands_ok(const w4_packed_mx_view& w, const void* xq, const uint8_t*
 // M = 97 - 128 up to 64; 8-bit X up to 32 1.1 - 1.3; 4-bit X at N = 4096, K = 14336 0.83 - 0.86 and 1.25 - 1.27 (K = 4096
 // 0.83 - 0.87 and 1.11 - 1.15, which stays with the tiles).  At K <= 2048 up to 64 with either (N = 2048, 4-bit X: 4.5
 // against 5.0).
-// Where K is no multiple of 512 the skinny kernel's guarded loads cost it 2 to 3 times as much and it keeps 32 rows
-// (16 with 4-bit X; N = 4096, K = 11008, M = 17: 20.1 against 21.9 and 24.0 -> 21.0; M = 33 26.1 -> 20.0)
-// and short K with 8-bit X (N = 1000, K = 1280, M = 64: 4.5 against 4.7).
+// Where K is a multiple of 256 and not of 512 the skinny kernel, as fast as elsewhere up to 16 rows (4-bit X; 32 with
+// 8-bit X), keeps those, and short K with 8-bit X (N = 1000, K = 1280, M = 64: 4.5 against 4.7).
 template <bool XF8>
 int fewest_tile_workgroups(int M, int K) {
-  if (K % 512) return M > (XF8 ? 32 : 16) ? 0 : M <= 4 ? 160 : 100;
+  if (K % 512 && M > (XF8 ? 32 : 16)) return 0;
   if (XF8) return M <= 4 ? 160 : M <= 8 && K > 4096 ? 121 : 100;
   if (M <= 12) return M <= 2 ? 200 : M <= 4 ? 171 : M <= 8 ? 140 : 121;
   return M <= 16 && K > 4096 ? 121 : M > 32 && M <= 48 && K > 6144 ? 140 : 100;
