@@ -141,3 +141,23 @@ def test_short_caches_overlap_on_two_streams():
     for i in range(2):
         for n in range(20):
             assert np.array_equal(bits(outs[i][n]), want[i]), (i, n)
+
+
+@pytest.mark.parametrize("H,S,D,group,splits", [(1, 2000, 64, 5, 16), (1, 8666, 64, 3, 68), (1, 33108, 64, 2, 130), (3, 2000, 128, 5, 16),
+                                                (1, 8666, 128, 3, 68), (1, 16443, 128, 2, 129), (1, 64000, 128, 2, 250)])
+def test_second_launch_that_merges(H, S, D, group, splits):
+    """The kernel that merges what the last workgroup does not: fewer splits than waves times rows, one load a row and wave
+    and more than that, one to four maxima a lane."""
+    c = w4amd.capi()
+    plan = c.flash_plan_for(F16, H, group, S, D, 32, 0)
+    assert (plan[0], plan[2]) == (splits, 0), plan
+    k, v = (orc.normal_activations(H * S * D, 91 + i) for i in range(2))
+    q = orc.normal_activations(H * group * D, 93)
+    k_d, v_d, q_d, out = to_dev(k), to_dev(v), to_dev(q), halves(H * group * D + 16, 0x7E00)
+    runs = []
+    for _ in range(2):
+        c.attention_fp16_flash(ptr(q_d), ptr(k_d), ptr(v_d), ptr(out), H, S, D, group=group)
+        runs.append(bits(out).copy())
+    assert np.array_equal(*runs) and (runs[0][H * group * D:] == 0x7E00).all()
+    ref = orc.attention_f16(q, k, v, H, group, S, D)
+    assert orc.rel_l2(runs[0][: H * group * D].view(np.float16), ref) <= TOL
