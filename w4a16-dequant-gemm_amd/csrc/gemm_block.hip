@@ -641,12 +641,14 @@ long long bk_rounds(const WView& v, int M, const BkShape& s, int cus) {
   return ((ng + 7) / 8 * mg + cus / 8 - 1) / (cus / 8);
 }
 
-// Small groups take 1.15 of it (four selectors, more parameters), codes by the dword 1.06.
+// Small groups take 1.15 of it (four selectors) and 0.03 us for every KB of a block's parameters, which are copied
+// first (N = 11008, K = 4096, gs = 8, M = 16, 32 x 16 blocks 15.7 us, the decode kernel 14.0), codes by the dword 1.06.
 int bk_time(const WView& v, int M, const BkShape& s, int cus) {
   const int n = ((v.K + BK_UNIT - 1) / BK_UNIT + BK_WAVES - 1) / BK_WAVES;
   long long per = s.per_n[v.mx ? 2 : v.symmetric ? 0 : 1];
   if (!v.mx) per = per * (v.gs < 32 ? 115 : 100) / 100 * (bk_ragged(v) ? 106 : 100) / 100;
-  const long long t = s.start + bk_rounds(v, M, s, cus) * (s.round + per * n);
+  const long long copy = v.mx || v.gs >= 32 ? 0 : 16LL * s.nt * (2 * v.G + (v.symmetric ? 0 : 4 * words(v.G))) * 3 / 1024;
+  const long long t = s.start + bk_rounds(v, M, s, cus) * (s.round + copy + per * n);
   return t > 1 << 30 ? 1 << 30 : (int)t;
 }
 

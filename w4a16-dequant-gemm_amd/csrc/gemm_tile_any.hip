@@ -66,10 +66,10 @@ int other_time(const WView& v, int M, int cus) {
     const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4, per = (v.gs < 32 ? 9 : 0) + (v.symmetric ? 64 : 74);
     return (int)(400 + (tiles + cus - 1) / cus * (cpw * (per + 19 * mt) - 30));
   }
-  if (M <= 8 || (M <= 16 && v.N < 8192)) {  // (its times spread by a third: less a tenth)
-    if (v.K < 1024) return 0;
+  if (M <= 8 || (M <= 16 && v.N < 8192)) {  // (its times spread by a third: less a tenth; small groups take half as much again)
     const long long share = tiles > cus ? tiles * 64 / cus : 64;  // tiles a compute unit, in 64ths
-    return (int)((v.K < 3072 ? 240 + share * (10 + 109 * cpw) / 64 : 80 + share * (175 * cpw - 70) / 64) * 9 / 10);
+    const long long t = v.K < 3072 ? 240 + share * (10 + 109 * cpw) / 64 : 80 + share * (175 * cpw - 70) / 64;
+    return (int)(t * (!v.mx && v.gs < 32 && v.K >= 3072 ? 135 : 90) / 100);
   }
   if (v.K >= 1024) return 1 << 30;
   if (v.K % 64 == 0 && M >= 96) {
@@ -88,8 +88,11 @@ bool any_group_fits(const WView& v) { return v.mx || (long long)(v.K / 8) * (v.g
 AnyPlan any_plan(const WView& v, int M) {
   const AnyPlan none{0, -1};
   const int cus = device_cus();
-  // (shorter rows: no more than a launch for the kernels that have them)
-  if (M < 5 || v.K % 8 || v.K < (M < 17 ? 1024 : 256) || cus < 8) return none;
+  if (M < 5 || v.K % 8 || cus < 8) return none;
+  // Shorter rows are no more than a launch for the kernels that have them.  Up to 16 rows on few tiles: N < 2048, K = 1281 to
+  // 3072 0.83 to 1.0 times as fast, up to 4096 1.05 to 1.13; N = 2048 to 4096, K up to 2048 0.9 to 1.03.
+  const int tiles = (v.N + 15) / 16;
+  if (v.K < (M >= 17 ? 256 : 2 * tiles < cus ? 3073 : tiles <= cus ? 2049 : 1152)) return none;
   const bool dma = v.K % 128 == 0 && (v.mx || v.gs == 32 || v.gs == 64 || v.gs % 128 == 0);
   const bool whole = v.N % 16 == 0 && v.K % 32 == 0 && (v.mx || v.gs % 32 == 0);
   // shapes of the kernels for whole tiles, chunks and groups
