@@ -59,7 +59,10 @@ TILES = [(4, 0, 1100, 257, 2080, 24), (4, 0, 2049, 257, 264, 8), (4, 0, 2049, 12
 BLOCKS = [(0, 5, 130, 4104, 8), (1, 9, 33, 3336, 24), (1, 17, 1034, 2056, 48), (0, 20, 15, 264, 40), (1, 33, 281, 1000, 16), (0, 50, 513, 5176, 72),
           (1, 64, 3, 1032, 1032), (1, 40, 2063, 4104, 8), (0, 100, 129, 2080, 128), (1, 130, 40, 1384, 48), (2, 17, 281, 1000, 32), (2, 50, 7, 3336, 32),
           (2, 130, 1001, 2072, 32), (1, 100, 2064, 1152, 48), (0, 333, 4080, 4096, 48), (1, 64, 3000, 2048, 96), (0, 120, 1477, 2304, 128),
-          (1, 48, 1477, 4096, 32)]
+          (1, 48, 1477, 4096, 32),
+          # parameters that LDS holds a window of units at a time: three of one tile of W, two and three of two; the
+          # last window shorter, waves without a unit in it
+          (0, 17, 515, 20480, 8), (1, 70, 2050, 11024, 8), (0, 100, 2064, 12304, 8), (1, 33, 1034, 20496, 16)]
 
 
 @pytest.mark.parametrize("plan,fmt,M,N,K,gs", TILES)

@@ -62,12 +62,15 @@ __device__ __forceinline__ void bk_dma4(uint32_t off, const void* base, uint32_t
 // of which meet in such a slice, 2 smaller ones, at most four.  A slice's runs of scales and zero-points come as
 // whole dwords and are moved to the bottom of their registers, from which a word picks its own by a
 // selector of bytes and a shift.  RAG: K is no multiple of 32 (rows of codes are 4-byte aligned only) or N none of 16: codes
-// come dword by dword.
+// come dword by dword.  window (GM = 2): at long K the parameters of small groups are more than LDS holds (gs = 8, K = 11008: 3.4 KB
+// a row), and the block has those of this many units of every wave at a time, copied while all waves wait (K = 11008, gs = 8,
+// N = 4096, M = 99: 32 x 64 blocks 34 us; 16 x 16 ones, whose parameters fit, and 32 x 128 tiles 79).
 template <int FMT, int NT, int MT, int XS, bool AHEAD, bool LATE, int GM, bool RAG>
 __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
     const uint32_t* __restrict__ q, const void* __restrict__ scales, const uint32_t* __restrict__ zeros,
     const w4_half* __restrict__ x, w4_half* __restrict__ c, const int N, const int K, const int M,
-    const uint32_t group_mul, const int G, const int gs, const int mgroups, w4_half* __restrict__ w_out) {
+    const uint32_t group_mul, const int G, const int gs, const int mgroups, w4_half* __restrict__ w_out,
+    const int window) {
   constexpr bool MX = FMT == 2;
   static_assert(!(MX && LATE), "an MXFP4 chunk has four scales");
   static_assert(GM == 0 || (!MX && !LATE), "scales of a chunk or of MXFP4 blocks need no selector");
@@ -96,8 +99,30 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
   [[maybe_unused]] uint8_t* rest_z = nullptr;
   [[maybe_unused]] uint8_t byte_s = 0, byte_z = 0;
   const int pb = live * G * (MX ? 1 : 2), wg = words(G), zb = live * wg * 4;
-  const int zoff = (ROWS * G * (MX ? 1 : 2) + 1023) & ~1023;
-  {
+  const int units_most = (units + BK_WAVES - 1) / BK_WAVES;  // of a wave
+  const bool windows = GM == 2 && window < units_most;
+  const int GP = windows ? window * (BK_WAVES * BK_UNIT) / gs : G;  // groups of a row that LDS has
+  const int wgp = windows ? GP >> 3 : wg;
+  const int zoff = (ROWS * GP * (MX ? 1 : 2) + 1023) & ~1023;
+  // the parameters of window j, a dword a lane: scales of a row in whole loads, zero-points of all rows as one run
+  auto copy_window = [&](int j) BK_INLINE {
+    const int left = min(GP, G - j * GP);
+    for (int row = wave; row < ROWS; row += BK_WAVES) {
+      const char* ps = (const char*)scales + ((size_t)(n0 + min(row, live - 1)) * G + (size_t)j * GP) * 2;
+      for (int o = 0; o < GP * 2; o += 256)
+        bk_dma4((uint32_t)min(o + lane * 4, left * 2 - 4), ps, lds0 + BK_WAVES * WB + row * GP * 2 + o);
+    }
+    if constexpr (FMT == 1) {
+      const char* pz = (const char*)zeros + ((size_t)n0 * wg + (size_t)j * wgp) * 4;
+      for (int o = wave * 64; o < ROWS * wgp; o += BK_WAVES * 64) {
+        const int row = (o + lane) / wgp, col = (o + lane) - row * wgp;
+        bk_dma4((uint32_t)(min(row, live - 1) * wg + min(col, words(left) - 1)) * 4, pz, lds0 + BK_WAVES * WB + zoff + o * 4);
+      }
+    }
+  };
+  if (windows) {
+    copy_window(0);
+  } else {
     const char* ps = (const char*)scales + (size_t)n0 * G * (MX ? 1 : 2);
     const int pw = RAG ? pb & ~15 : pb, zw16 = RAG ? zb & ~15 : zb;  // (16 rows have whole pieces of 16 bytes)
     for (int o = wave * 1024; o < pw; o += BK_WAVES * 1024)
@@ -251,6 +276,7 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
   [[maybe_unused]] const int gsw = gs >> 3;
   [[maybe_unused]] h4 late[NT];  // the scales of the chunk that is multiplied
   int g = 0, slot = 0;  // slot: of the piece that is multiplied
+  [[maybe_unused]] int g_first = 0, done = 0;  // the window's first group; units that the wave has begun
   const bool hook = w_out && m0 == 0;
 
   auto read_codes = [&](int h, u4* w) BK_INLINE {
@@ -267,13 +293,14 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
     const int kc = min(chunk * 128 + (LATE ? 0 : 32 * b), RAG ? K - 8 : K - 32);
     g = MX ? (kc >> 5) : (int)__umulhi((uint32_t)kc >> 2, group_mul);
     if constexpr (GM > 0) {
-      const uint8_t* ps = params + ((r * G + g) >> 1) * 4;
-      const uint8_t* pz = params + zoff + (r * wg + (g >> 3)) * 4;
+      const int gw = GM == 2 ? g - g_first : g, pitch = GM == 2 ? GP : G, zpitch = GM == 2 ? wgp : wg;
+      const uint8_t* ps = params + ((r * pitch + gw) >> 1) * 4;
+      const uint8_t* pz = params + zoff + (r * zpitch + (gw >> 3)) * 4;
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
 #pragma unroll
-        for (int e = 0; e < (GM == 2 ? 3 : 2); ++e) sc[t].d[e] = *(const uint32_t*)(ps + t * 32 * G + e * 4);
-        if (FMT == 1) zw[t] = u2{*(const uint32_t*)(pz + t * 64 * wg), *(const uint32_t*)(pz + t * 64 * wg + 4)};
+        for (int e = 0; e < (GM == 2 ? 3 : 2); ++e) sc[t].d[e] = *(const uint32_t*)(ps + t * 32 * pitch + e * 4);
+        if (FMT == 1) zw[t] = u2{*(const uint32_t*)(pz + t * 64 * zpitch), *(const uint32_t*)(pz + t * 64 * zpitch + 4)};
       }
       return;
     }
@@ -444,6 +471,17 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
     __builtin_amdgcn_sched_barrier(0);
   };
 
+  // between a wave's units: where the next one begins another window, every wave is done with this one
+  [[maybe_unused]] auto next_window = [&]() BK_INLINE {
+    ++done;
+    if (windows && done % window == 0 && done < units_most) {
+      asm volatile("s_barrier" ::: "memory");
+      copy_window(done / window);
+      g_first += GP;
+      asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+  };
+
   if constexpr (AHEAD) {
     // A piece is read back while the one before it is multiplied (few row tiles: N = 4096, K = 14336, M = 64
     // 19.7 -> 17.9 us; with larger blocks the second set of registers costs more than it gives).
@@ -481,7 +519,10 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
           if (MT > 1 && p == NP - 1) read_codes(0, cw[0]), read_codes(1, cw[1]);
           read_x(slot, xv[(p + 1) & 1]);
           if (p == MT - 1) read_params(2 * U + 1);
-          if (p == NP - 1) read_params(2 * (U + BK_WAVES));
+          if (p == NP - 1) {
+            if constexpr (GM == 2) next_window();
+            read_params(2 * (U + BK_WAVES));
+          }
         }
         __builtin_amdgcn_sched_barrier(0);
         if (mt == 0) expand(cw[ch], scale, zword, group, U * BK_UNIT + ch * 128 + 32 * b);
@@ -490,6 +531,7 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
         __builtin_amdgcn_sched_barrier(0);
       }, std::make_integer_sequence<int, NP>{});
     }
+    if constexpr (GM == 2) next_window();  // (a wave without a unit in the last window meets the others there)
   } else {
     for (int U = wave; U < units; U += BK_WAVES) {
       const bool more = U + BK_WAVES < units;
@@ -559,21 +601,34 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
 
 bool bk_ragged(const WView& v) { return v.K % 32 || v.N % 16; }
 
-// Bytes of LDS of a workgroup with NT tiles of W.
-int bk_lds_bytes(const WView& v, int NT) {
-  const int G = v.mx ? v.B : v.G;
+// Bytes of LDS of a workgroup with NT tiles of W, of whose rows it has the parameters of G groups.
+int bk_lds_bytes(const WView& v, int NT, int G) {
   const long long p = 16LL * NT * G * (v.mx ? 1 : 2), z = v.mx || v.symmetric ? 0 : 64LL * NT * words(G);
   const int slack = !v.mx && (v.gs % 32 || bk_ragged(v)) ? 16 : 0;  // GM: the last dword of a run may lie behind the parameters
   const long long bytes = BK_WAVES * bk_wave_bytes(NT, BK_XS) + ((p + 1023) & ~1023LL) + ((z + 1023) & ~1023LL) + slack;
   return bytes > (1 << 20) ? 1 << 20 : (int)bytes;
 }
+int bk_lds_bytes(const WView& v, int NT) { return bk_lds_bytes(v, NT, v.mx ? v.B : v.G); }
 constexpr int BK_MAX_LDS = 160 * 1024;
+
+// Units of a wave whose parameters LDS holds at a time: all (BK_WHOLE), or as many as fit, where a unit is whole groups
+// and rows are whole dwords; 0: not even one's.
+constexpr int BK_WHOLE = 1 << 20;
+int bk_window(const WView& v, int NT) {
+  if (bk_lds_bytes(v, NT) <= BK_MAX_LDS) return BK_WHOLE;
+  if (v.mx || v.gs >= 32 || 32 % v.gs || v.G % 2) return 0;
+  int w = ((v.K + BK_UNIT - 1) / BK_UNIT + BK_WAVES - 1) / BK_WAVES;
+  while (w > 0 && bk_lds_bytes(v, NT, w * (BK_WAVES * BK_UNIT / v.gs)) > BK_MAX_LDS) --w;
+  return w;
+}
 
 template <int FMT, int NT, int MT, bool LATE, int GM, bool RAG>
 hipError_t block_go_as(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out) {
   constexpr int XS = BK_XS;
   constexpr bool AHEAD = NT <= 2;
-  const int lds_bytes = bk_lds_bytes(v, NT);
+  const int window = GM == 2 ? bk_window(v, NT) : BK_WHOLE;
+  if (window < 1) return hipErrorInvalidValue;
+  const int lds_bytes = window == BK_WHOLE ? bk_lds_bytes(v, NT) : bk_lds_bytes(v, NT, window * (BK_WAVES * BK_UNIT / v.gs));
   static std::atomic<bool> granted[64] = {};  // more than 64 KB of LDS has to be granted per device, once
   int dev = 0;
   if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
@@ -586,7 +641,7 @@ hipError_t block_go_as(const WView& v, const w4_half* x, w4_half* c, int M, hipS
   const int mg = (M + 16 * MT - 1) / (16 * MT), ng = (v.N + 16 * NT - 1) / (16 * NT);
   const uint32_t mul = v.mx ? 0u : (uint32_t)(((1ULL << 31) + v.gs / 8 - 1) / (v.gs / 8));
   mfma_block_kernel<FMT, NT, MT, XS, AHEAD, LATE, GM, RAG><<<dim3((unsigned)(8 * ((ng + 7) / 8) * mg)), BK_THREADS, lds_bytes, s>>>(
-      v.q, v.scales, v.zeros, x, c, v.N, v.K, M, mul, v.mx ? v.B : v.G, v.gs, mg, w_out);
+      v.q, v.scales, v.zeros, x, c, v.N, v.K, M, mul, v.mx ? v.B : v.G, v.gs, mg, w_out, window);
   return hipGetLastError();
 }
 
@@ -648,7 +703,8 @@ int bk_time(const WView& v, int M, const BkShape& s, int cus) {
   long long per = s.per_n[v.mx ? 2 : v.symmetric ? 0 : 1];
   if (!v.mx) per = per * (v.gs < 32 ? 115 : 100) / 100 * (bk_ragged(v) ? 106 : 100) / 100;
   const long long copy = v.mx || v.gs >= 32 ? 0 : 16LL * s.nt * (2 * v.G + (v.symmetric ? 0 : 4 * words(v.G))) * 3 / 1024;
-  const long long t = s.start + bk_rounds(v, M, s, cus) * (s.round + copy + per * n);
+  const int window = copy ? bk_window(v, s.nt) : BK_WHOLE, more = window > 0 && window < n ? (n - 1) / window : 0;
+  const long long t = s.start + bk_rounds(v, M, s, cus) * (s.round + copy + per * n + 150 * more);  // (another window: 1.5 us)
   return t > 1 << 30 ? 1 << 30 : (int)t;
 }
 
@@ -778,12 +834,14 @@ int block_plan_time(const WView& v, int M, int* time) {
 }
 
 int block_any_time(const WView& v, int M, int cus, int* time) {
-  if (v.K % 8 || v.K < 32 || v.K >= 1 << 24 || M > 8192 || !any_group_fits(v)) return -1;
+  // (more rows of x than L2 holds, which every block of W reads again, are the tiles': N = 276, K = 11104, M = 3020 143 us
+  // in 32 x 64 blocks)
+  if (v.K % 8 || v.K < 32 || v.K >= 1 << 24 || M > 1536 || !any_group_fits(v)) return -1;
   const int gm = v.mx ? 0 : v.gs < 32 ? 2 : 1;
   int best = -1;
   for (int i = 0; i < BK_COUNT; ++i) {
     const BkShape& s = BK_SHAPES[i];
-    if (!bk_has(v.mx ? 2 : 0, s.nt, s.mt, gm, bk_ragged(v)) || bk_lds_bytes(v, s.nt) > BK_MAX_LDS) continue;
+    if (!bk_has(v.mx ? 2 : 0, s.nt, s.mt, gm, bk_ragged(v)) || bk_window(v, s.nt) < 1) continue;
     const int t = bk_time(v, M, s, cus);
     if (best < 0 || t < *time) best = i, *time = t;
   }
