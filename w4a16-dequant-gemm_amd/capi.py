@@ -308,7 +308,8 @@ def gemm_mx_w4a8(w_view, x_view, c, stream=0):
 
 
 def gemm_plan_for(fmt, M, N, K, gs=32):
-    """10 x tiles of W + row tiles of a block / 1 long-K / 2 resident / 3 general decode kernel / 0 others"""
+    """10 x tiles of W + row tiles of a block / 4 .. 7 tiles for any group size, K and N / 1 long-K / 2 resident /
+    3 general decode kernel / 0 others"""
     plan = C.c_int()
     check(load().w4_gemm_plan_for(fmt, M, N, K, gs, C.byref(plan)))
     return plan.value
