@@ -62,7 +62,9 @@ BLOCKS = [(0, 5, 130, 4104, 8), (1, 9, 33, 3336, 24), (1, 17, 1034, 2056, 48), (
           (1, 48, 1477, 4096, 32),
           # parameters that LDS holds a window of units at a time: three of one tile of W, two and three of two; the
           # last window shorter, waves without a unit in it
-          (0, 17, 515, 20480, 8), (1, 70, 2050, 11024, 8), (0, 100, 2064, 12304, 8), (1, 33, 1034, 20496, 16)]
+          (0, 17, 515, 20480, 8), (1, 70, 2050, 11024, 8), (0, 100, 2064, 12304, 8), (1, 33, 1034, 20496, 16),
+          # the general decode kernel would take three rounds, its LDS holds one tile's parameters
+          (1, 61, 11008, 4096, 8)]
 
 
 @pytest.mark.parametrize("plan,fmt,M,N,K,gs", TILES)

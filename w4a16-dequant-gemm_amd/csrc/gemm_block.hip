@@ -305,28 +305,28 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
       return;
     }
     if constexpr (GM == 0) {
-    const uint8_t* ps = params + ((LATE ? 4 * b : r) * G + g) * (MX ? 1 : 2);
-    const uint8_t* pz = params + zoff + (r * wg + (g >> 3)) * 4;
+      const uint8_t* ps = params + ((LATE ? 4 * b : r) * G + g) * (MX ? 1 : 2);
+      const uint8_t* pz = params + zoff + (r * wg + (g >> 3)) * 4;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      if constexpr (LATE) {
-        const _Float16* p = (const _Float16*)ps + t * 16 * G;
-        sc[t] = h4{p[0], p[G], p[2 * G], p[3 * G]};
-      } else {
-        sc[t] = MX ? ps[t * 16 * G] : *(const uint16_t*)(ps + t * 32 * G);
+      for (int t = 0; t < NT; ++t) {
+        if constexpr (LATE) {
+          const _Float16* p = (const _Float16*)ps + t * 16 * G;
+          sc[t] = h4{p[0], p[G], p[2 * G], p[3 * G]};
+        } else {
+          sc[t] = MX ? ps[t * 16 * G] : *(const uint16_t*)(ps + t * 32 * G);
+        }
+        if (FMT == 1) zw[t] = *(const uint32_t*)(pz + t * 64 * wg);
       }
-      if (FMT == 1) zw[t] = *(const uint32_t*)(pz + t * 64 * wg);
-    }
-    // Lanes past the end of the row hold codes of another group than g's: with its scale they can overflow FP16,
-    // and infinity times the zeroed activations is NaN.  A scale of 0 (MXFP4: 2^-127) makes them zeros.
-    // (LATE: the codes are finite, the scale of a chunk that is past the end as a whole may not be.)
-    if (chunk * 128 + 128 > K) {
-      if (chunk * 128 + (LATE ? 0 : 32 * b) >= K) {
+      // Lanes past the end of the row hold codes of another group than g's: with its scale they can overflow FP16,
+      // and infinity times the zeroed activations is NaN.  A scale of 0 (MXFP4: 2^-127) makes them zeros.
+      // (LATE: the codes are finite, the scale of a chunk that is past the end as a whole may not be.)
+      if (chunk * 128 + 128 > K) {
+        if (chunk * 128 + (LATE ? 0 : 32 * b) >= K) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t) sc[t] = scale_t{};
+          for (int t = 0; t < NT; ++t) sc[t] = scale_t{};
+        }
+        asm volatile("" ::: "memory");
       }
-      asm volatile("" ::: "memory");
-    }
     }
   };
   auto request_next = [&](auto pc, int U, bool more) BK_INLINE {  // into the places that are free at step p of unit U
@@ -369,28 +369,28 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
       }
     } else {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      h2 cneg, s2 = h2{0, 0};
-      float sf = 0.f;
-      if constexpr (MX) {
-        sf = mx_scale(scale[t]);
-      } else {
-        const uint32_t z = FMT == 1 ? ((zword[t] >> (4 * (group & 7))) & 0xFu) : 8u;
-        cneg = as_h2(0xD400E400u | (z << 20) | z);
-        if constexpr (LATE) late[t] = scale[t];
-        else s2 = splat_bits(scale[t]);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (MX) {
-          h2 n4[4];
-          dq_mx(w[t][j], sf, n4);
-          A[t][j] = __builtin_bit_cast(h8, u4{as_u32(n4[0]), as_u32(n4[1]), as_u32(n4[2]), as_u32(n4[3])});
+      for (int t = 0; t < NT; ++t) {
+        h2 cneg, s2 = h2{0, 0};
+        float sf = 0.f;
+        if constexpr (MX) {
+          sf = mx_scale(scale[t]);
         } else {
-          A[t][j] = expand_word<!LATE>(w[t][j], cneg, s2, mask, magic);
+          const uint32_t z = FMT == 1 ? ((zword[t] >> (4 * (group & 7))) & 0xFu) : 8u;
+          cneg = as_h2(0xD400E400u | (z << 20) | z);
+          if constexpr (LATE) late[t] = scale[t];
+          else s2 = splat_bits(scale[t]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (MX) {
+            h2 n4[4];
+            dq_mx(w[t][j], sf, n4);
+            A[t][j] = __builtin_bit_cast(h8, u4{as_u32(n4[0]), as_u32(n4[1]), as_u32(n4[2]), as_u32(n4[3])});
+          } else {
+            A[t][j] = expand_word<!LATE>(w[t][j], cneg, s2, mask, magic);
+          }
         }
       }
-    }
     }
     if constexpr (RAG && MX) {  // (a scale may overflow the codes of a slice that the row ends in)
       if ((k & ~127) + 128 > K) {

@@ -511,6 +511,11 @@ bool decode_general_applies(const WView& v, const w4_half* x, const w4_half* c, 
   return general_plan(v, x, c, M, &pl);
 }
 
+int decode_general_tiles(const WView& v, int M) {
+  GeneralPlan pl;
+  return general_plan(v, nullptr, nullptr, M, &pl) ? pl.t : 0;
+}
+
 // Precondition: decode_general_applies(v, x, c, M); no hook.
 hipError_t launch_decode_general(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s) {
   GeneralPlan pl;

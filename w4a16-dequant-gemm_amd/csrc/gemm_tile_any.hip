@@ -81,6 +81,17 @@ int other_time(const WView& v, int M, int cus) {
   return (int)(M <= 32 ? 440 + share * 50 * stages / 64 : 275 + 38 * stages + share * (127 + 110 * stages) / 64);
 }
 
+// What the general decode kernel takes on top of that: next to the activations of 33 to 64 rows LDS has room for the
+// parameters of one or two tiles of small groups, so that there are further rounds of workgroups, each of which fetches the
+// activations again: 3.5 us with one tile, 0.9 with two (one tile: 1.17 to 1.44 of the time above, 0.96 to 1.04 of the sum).
+int general_rounds(const WView& v, int M, int cus) {
+  if (v.mx || v.gs >= 32 || M <= 32) return 0;
+  const int held = decode_general_tiles(v, M);
+  if (!held) return 0;
+  const long long tiles = (v.N + 15) / 16, rounds = ((tiles + held - 1) / held + cus - 1) / cus;
+  return (int)((rounds - 1) * (held == 1 ? 350 : 90));
+}
+
 }  // namespace
 
 bool any_group_fits(const WView& v) { return v.mx || (long long)(v.K / 8) * (v.gs / 8) < (1LL << 31); }
@@ -110,8 +121,12 @@ AnyPlan any_plan(const WView& v, int M) {
   }
   block_shape = block_any_time(v, M, cus, &block_t);
   const int other = other_time(v, M, cus);
-  if (tile_time >= other && block_t >= other) return none;
-  return tile_time < block_t ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
+  // (tiles are asked to beat that kernel's time without its further rounds: 33 to 64 rows of small groups take them 0.95 to
+  // 1.4 times that kernel's time, and blocks 0.65 to 0.9; N = 11008, gs = 8, M = 64: K = 4096 29.2 -> 24.5 us)
+  const bool tiles_ahead = tile_time < other;
+  const bool blocks_ahead = block_t < other + general_rounds(v, M, cus);
+  if (!tiles_ahead && !blocks_ahead) return none;
+  return tiles_ahead && (!blocks_ahead || tile_time < block_t) ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
 }
 
 bool try_tile_any(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, int shape, hipError_t* err) {

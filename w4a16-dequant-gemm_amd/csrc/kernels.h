@@ -55,8 +55,9 @@ bool try_tile_dma(const WView& v, const w4_half* x, w4_half* c, int M, hipStream
 bool try_tile256(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, int cus,
                  hipError_t* err);
 
-// gemm_block.hip: middle M (17 to some hundred rows, at long K from 3 on), blocks of W and x as square as few rounds
-// of workgroups allow, hooked calls included; false (nothing launched) when another kernel is ahead.
+// gemm_block.hip: middle M (17 to some hundred rows, at long K from 3 on; from 5 for sizes that are not whole), blocks
+// of W and x as square as few rounds of workgroups allow, hooked calls included; false (nothing launched) when another
+// kernel is ahead.
 bool try_block(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out,
                int shape, hipError_t* err);
 // shape: the block that any_plan() names, or -1: block_plan()'s own.
@@ -102,6 +103,8 @@ hipError_t launch_decode_longk(const WView& v, const w4_half* x, w4_half* c, int
 // with 1024 < K <= 5120, group parameters through LDS; same order of additions as the
 // K-split decode kernels of gemm_mfma.hip.
 bool decode_general_applies(const WView& v, const w4_half* x, const w4_half* c, int M);
+// Tiles of W per workgroup of that kernel; 0: not its arguments.
+int decode_general_tiles(const WView& v, int M);
 hipError_t launch_decode_general(const WView& v, const w4_half* x, w4_half* c, int M,
                                  hipStream_t s);
 
