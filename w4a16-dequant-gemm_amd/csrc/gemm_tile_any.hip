@@ -123,7 +123,10 @@ AnyPlan any_plan(const WView& v, int M) {
   const int other = other_time(v, M, cus);
   // (tiles are asked to beat that kernel's time without its further rounds: 33 to 64 rows of small groups take them 0.95 to
   // 1.4 times that kernel's time, and blocks 0.65 to 0.9; N = 11008, gs = 8, M = 64: K = 4096 29.2 -> 24.5 us)
-  const bool tiles_ahead = tile_time < other;
+  // Up to five rounds of its tiles they have to be ahead by a quarter: M = 41, N = 11504, K = 2176, gs = 8 13.1 us there and 18.3
+  // on tiles, M = 54, N = 13936, K = 2752 18.1 and 21.6; past them M = 40, N = 28672, K = 4096 55 and 42.
+  const bool close = !v.mx && v.gs < 32 && M > 32 && tiles <= 5 * cus && decode_general_applies(v, nullptr, nullptr, M);
+  const bool tiles_ahead = close ? 4LL * tile_time < 3LL * other : tile_time < other;
   const bool blocks_ahead = block_t < other + general_rounds(v, M, cus);
   if (!tiles_ahead && !blocks_ahead) return none;
   return tiles_ahead && (!blocks_ahead || tile_time < block_t) ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
