@@ -161,3 +161,43 @@ def test_second_launch_that_merges(H, S, D, group, splits):
     assert np.array_equal(*runs) and (runs[0][H * group * D:] == 0x7E00).all()
     ref = orc.attention_f16(q, k, v, H, group, S, D)
     assert orc.rel_l2(runs[0][: H * group * D].view(np.float16), ref) <= TOL
+
+
+# D = 64: a wave of that kernel takes two splits at a time.  (cache, positions, query heads, page, splits): odd numbers of
+# splits whose last one is held by a lane of the upper half (33 .. 63, 97 .. 127) or of the lower (65 .. 95, 129)
+@pytest.mark.parametrize("kind,S,group,page,splits", [(F16, 4111, 4, 0, 33), (F16, 7954, 3, 0, 63), (F16, 8198, 2, 0, 65), (F16, 12346, 2, 0, 97),
+                                                      (F16, 32293, 2, 0, 127), (F16, 32781, 2, 0, 129), (W4, 4111, 8, 0, 33), (W4, 14359, 4, 0, 57),
+                                                      (W4, 4111, 8, 16, 33), (W4, 24607, 2, 0, 65), (F8, 10760, 3, 0, 43), (F8, 24607, 2, 0, 97)])
+def test_second_launch_takes_an_odd_last_split(kind, S, group, page, splits):
+    """The values of the last split are thirty times the others', so that its share of 1 / splits is a good part of the result."""
+    c = w4amd.capi()
+    D = 64
+    plan = c.flash_plan_for(kind, 1, group, S, D, 32, page)
+    assert (plan[0], plan[2]) == (splits, 0), plan
+    k, v = orc.normal_weights(S * D, 95), orc.normal_weights(S * D, 96)
+    v.reshape(S, D)[(splits - 1) * plan[1]:] *= 30
+    q, out = orc.normal_activations(group * D, 97), halves(group * D + 16, 0x7E00)
+    q_d = to_dev(q)
+    if kind == F8:
+        cache = orc.quantize_cache_f8(k, v, 1, S, D, 32)
+        kd, vd = orc.dequant_cache_f8(cache, False), orc.dequant_cache_f8(cache, True)
+        dk = DevKVF8(cache)
+        c.attention_f8_flash(dk.view, ptr(q_d), ptr(out), group=group)
+    else:
+        cache = orc.quantize_cache(k, v, 1, S, D, 32, True)
+        kd, vd = orc.dequant_cache(cache, False), orc.dequant_cache(cache, True)
+        if kind == F16:
+            k_d, v_d = to_dev(kd), to_dev(vd)
+            c.attention_fp16_flash(ptr(q_d), ptr(k_d), ptr(v_d), ptr(out), 1, S, D, group=group)
+        elif page:
+            npages = (S + page - 1) // page
+            bt = np.random.default_rng(S).permutation(npages).astype(np.int32)
+            keep, view = _paged_pool(cache, page, bt)
+            bt_d = to_dev(bt)
+            c.attention_w4_flash_paged_batched(view, ptr(bt_d), 1, npages, page, npages, group, ptr(q_d), ptr(out))
+        else:
+            dk = DevKV(cache)
+            c.attention_w4_flash(dk.view, ptr(q_d), ptr(out), group=group)
+    got = bits(out)
+    assert (got[group * D:] == 0x7E00).all()
+    assert orc.rel_l2(got[: group * D].view(np.float16), orc.attention_f16(q, kd, vd, 1, group, S, D)) <= TOL

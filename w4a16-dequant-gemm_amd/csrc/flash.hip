@@ -410,7 +410,7 @@ __global__ __launch_bounds__(P2W_WAVES * 64) void flash_phase2_wide(const float*
       const int t = split_of(i0 + i);  // (a wave's rows lie within one set of 64 splits)
       const int k = (RPL * (wave + P2W_WAVES * (i0 + i))) >> 6;
       const float own = k == 0 ? wt[0] : k == 1 ? wt[1] : k == 2 ? wt[2] : wt[3];
-      const float e = t < T ? __shfl(own, t & 63, 64) : 0.0f;
+      const float e = __shfl(own, t & 63, 64);  // (every lane takes part; 0 past the last split)
       sum0 += e * col[i].x;
       sum1 += e * col[i].y;
     }
