@@ -201,3 +201,21 @@ def test_second_launch_takes_an_odd_last_split(kind, S, group, page, splits):
     got = bits(out)
     assert (got[group * D:] == 0x7E00).all()
     assert orc.rel_l2(got[: group * D].view(np.float16), orc.attention_f16(q, kd, vd, 1, group, S, D)) <= TOL
+
+
+@pytest.mark.parametrize("S,D,group,splits", [(4200, 64, 5, 33), (4096, 64, 5, 32), (16443, 128, 2, 129), (8666, 128, 3, 68)])
+def test_second_launch_keeps_infinities(S, D, group, splits):
+    """Infinite values in the last split and in the first: their columns are infinite in the result, NaN comes from NaN alone."""
+    c = w4amd.capi()
+    plan = c.flash_plan_for(F16, 1, group, S, D, 32, 0)
+    assert (plan[0], plan[2]) == (splits, 0), plan
+    k, v, q = (orc.normal_activations(n * D, 98 + i) for i, n in enumerate((S, S, group)))
+    k, q = ((a.view(np.float16) * np.float16(0.1)).view(np.uint16) for a in (k, q))
+    rows = v.view(np.float16).reshape(S, D)
+    rows[S - 2, 3], rows[7, 6], rows[S - 3, 9] = np.inf, -np.inf, np.nan
+    k_d, v_d, q_d, out = to_dev(k), to_dev(v), to_dev(q), halves(group * D)
+    c.attention_fp16_flash(ptr(q_d), ptr(k_d), ptr(v_d), ptr(out), 1, S, D, group=group)
+    got = bits(out).view(np.float16).reshape(group, D)
+    assert (got[:, 3] == np.inf).all() and (got[:, 6] == -np.inf).all() and np.isnan(got[:, 9]).all()
+    others = np.delete(np.arange(D), [3, 6, 9])
+    assert np.isfinite(got[:, others]).all()

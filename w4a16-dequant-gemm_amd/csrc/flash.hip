@@ -411,8 +411,9 @@ __global__ __launch_bounds__(P2W_WAVES * 64) void flash_phase2_wide(const float*
       const int k = (RPL * (wave + P2W_WAVES * (i0 + i))) >> 6;
       const float own = k == 0 ? wt[0] : k == 1 ? wt[1] : k == 2 ? wt[2] : wt[3];
       const float e = __shfl(own, t & 63, 64);  // (every lane takes part; 0 past the last split)
-      sum0 += e * col[i].x;
-      sum1 += e * col[i].y;
+      // (past the last split stands its own row again, which may hold infinities: 0 times them would be NaN)
+      sum0 += e * (t < T ? col[i].x : 0.0f);
+      sum1 += e * (t < T ? col[i].y : 0.0f);
     }
   }
   sums[wave][lane] = float2{sum0, sum1};
