@@ -131,3 +131,25 @@ def test_thin_grids_of_32_groups_with_zero_points(M, N, K):
     c.gemm_mma(dp.view, ptr(x_d), ptr(plain), M)
     c.gemm_mma(dp.view, ptr(x_d), ptr(hooked), M, 0, ptr(w))
     assert torch.equal(plain, hooked)
+
+
+@pytest.mark.parametrize("M,N,K,gs,sym", [(1134, 736, 576, 128, False), (222, 9776, 576, 256, True), (180, 11648, 1504, 128, True),
+                                          (128, 2064, 1504, 128, True), (559, 5728, 1056, 128, False)])
+def test_groups_of_whole_chunks_keep_their_scales_in_fp32(M, N, K, gs, sym):
+    """Groups of whole chunks, K no multiple of one: the scale belongs to FP32 sums and no weight is rounded.  Distance from the
+    FP64 product of codes and scales: an output rounded to FP16 alone is 2^-10 / sqrt(12) sqrt(E m^-2) = 2.1e-4 off (m: significands
+    spread over their logarithm), rounded weights add 1.7e-4 to it in squares (2.7e-4)."""
+    c = w4amd.capi()
+    p = orc.quantize(orc.normal_weights(N * K, M) * 0.02 + (0 if sym else 0.01), N, K, gs, sym)
+    dp, x, out = DevPacked(p), orc.normal_activations(M * K, N), halves(M * N)
+    assert c.gemm_plan_for(0 if sym else 1, M, N, K, gs) >= 10
+    c.gemm_mma(dp.view, ptr(to_dev(x)), ptr(out), M)
+    ns = np.random.default_rng(K).choice(N, 256, replace=False)
+    code = (p.q.reshape(N, K // 8)[ns][:, :, None] >> (4 * np.arange(8, dtype=np.uint32))) & 15
+    group = np.arange(K) // gs
+    zero = np.full((256, K), 8.0)
+    if not sym:
+        zero = ((p.zeros.reshape(N, -1)[ns][:, group // 8] >> (4 * (group % 8)).astype(np.uint32)) & 15).astype(np.float64)
+    w = (code.reshape(256, K) - zero) * p.scales.view(np.float16).reshape(N, -1)[ns][:, group].astype(np.float64)
+    ref = x.view(np.float16).reshape(M, K).astype(np.float64) @ w.T
+    assert orc.rel_l2(np.ascontiguousarray(bits(out).reshape(M, N)[:, ns]).view(np.float16), ref) <= 2.4e-4

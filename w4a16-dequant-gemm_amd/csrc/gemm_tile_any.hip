@@ -116,6 +116,9 @@ AnyPlan any_plan(const WView& v, int M) {
   if (whole) {
     // blocks as block_plan() has them; tiles where these are ahead by a quarter (the error of the times on both sides)
     block_shape = block_plan_time(v, M, &block_t);
+    // (W4 groups of whole chunks: blocks scale a chunk's FP32 sums, tiles round every weight; 2.1e-4 and 2.7e-4 from the
+    // product in FP64)
+    if (block_shape >= 0 && !v.mx && v.gs % 128 == 0) return AnyPlan{1, block_shape};
     if (block_shape < 0) return tile_time < other_time(v, M, cus) ? AnyPlan{2, tile} : none;
     return 5 * tile_time < 4 * block_t ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
   }
