@@ -33,15 +33,18 @@ def _check(fmt, M, N, K, gs, scale=None):
     ns = np.unique(np.concatenate([np.arange(min(N, 40)), np.arange(max(0, N - 40), N), rng.choice(N, size=min(N, 80), replace=False)]))
     ref = orc.gemm_oracle(np.ascontiguousarray(x.reshape(M, K)[ms]), len(ms), K,
                           np.ascontiguousarray(w_ref.reshape(N, K)[ns]), len(ns))
+    seen = []
     for hook in (False, True):
         out, w = halves(M * N + 64, 0x7E00), halves(N * K + 64, 0x7E00)
         fn(dp.view, ptr(x_d), ptr(out), M, 0, ptr(w) if hook else 0)
         got = bits(out)
         assert (got[M * N:] == 0x7E00).all(), "nothing is written behind the result"
+        seen.append(got)
         got = np.ascontiguousarray(got[: M * N].reshape(M, N)[ms][:, ns]).view(np.float16)
         assert orc.rel_l2(got, ref) <= TOL, hook
         if hook:
             assert torch.equal(w[: N * K], to_dev(w_ref)) and bool((w[N * K:] == 0x7E00).all())
+    assert np.array_equal(*seen), "the hook changes no byte of the result"
     return c.gemm_plan_for(fmt, M, N, K, gs)
 
 

@@ -5,12 +5,21 @@
 namespace w4k {
 namespace {
 
-// shape: 0 = 128 x 256 (rows of X x rows of W), 2 = 64 x 128, 3 = 128 x 128, 4 = 32 x 128
+// Whether a tile has two sets of waves, each on one half of K.
+constexpr bool any_two_sets(int gsm, int shape) { return shape == 4 || (shape == 2 && gsm != 4); }
+
+// shape: 0 = 128 x 256 (rows of X x rows of W), 2 = 64 x 128, 3 = 128 x 128, 4 = 32 x 128.  Hooked calls have the third
+// only and split their sum over K where the unhooked call's tile does: both return the same bytes.
 template <int FMT, int GSM, int KT>
-hipError_t any_go(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, int tn, int tm, int shape,
+hipError_t any_go(const WView& v, const w4_half* x, w4_half* c, w4_half* w_out, int M, hipStream_t s, int tn, int tm, int shape,
                   uint32_t mul) {
+  if (w_out) {
+    const int split_at = any_two_sets(GSM, shape) ? ((v.K + 127) / 128 + 1) / 2 : v.K;
+    return launch<FMT, GSM, true, 128, 128, 1, KT>(v, x, c, w_out, M, s, (v.N + 127) / 128, (M + 127) / 128, split_at, mul);
+  }
   if (shape == 4) return launch<FMT, GSM, false, 32, 128, 2, KT>(v, x, c, nullptr, M, s, tn, tm, 0, mul);
   if constexpr (GSM == 4) {
+    static_assert(!any_two_sets(4, 2) && any_two_sets(3, 2), "one set for small groups");
     if (shape == 2) return launch<FMT, GSM, false, 64, 128, 1, KT>(v, x, c, nullptr, M, s, tn, tm, 0, mul);
   } else {
     if (shape == 2) return launch<FMT, GSM, false, 64, 128, 2, KT>(v, x, c, nullptr, M, s, tn, tm, 0, mul);
@@ -135,14 +144,15 @@ AnyPlan any_plan(const WView& v, int M) {
   return tiles_ahead && (!blocks_ahead || tile_time < block_t) ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
 }
 
-bool try_tile_any(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, int shape, hipError_t* err) {
+bool try_tile_any(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out, int shape,
+                  hipError_t* err) {
   const bool rag = v.K % 32 != 0;
   if (((uintptr_t)x & 15) || ((uintptr_t)v.q & (rag ? 3 : 15)) || ((uintptr_t)v.scales & 3)) return false;
-  if (!v.mx && !v.symmetric && ((uintptr_t)v.zeros & 3)) return false;
+  if ((!v.mx && !v.symmetric && ((uintptr_t)v.zeros & 3)) || ((uintptr_t)w_out & 15)) return false;
   const int TN = shape == 0 ? 256 : 128, TM = shape == 2 ? 64 : shape == 4 ? 32 : 128;
   const int tn = (v.N + TN - 1) / TN, tm = (M + TM - 1) / TM;
   const uint32_t mul = v.mx ? 0u : (uint32_t)(((1ULL << 31) + v.gs / 8 - 1) / (v.gs / 8));
-#define W4_GO(F, G) (rag ? any_go<F, G, 2>(v, x, c, M, s, tn, tm, shape, mul) : any_go<F, G, 1>(v, x, c, M, s, tn, tm, shape, mul))
+#define W4_GO(F, G) (rag ? any_go<F, G, 2>(v, x, c, w_out, M, s, tn, tm, shape, mul) : any_go<F, G, 1>(v, x, c, w_out, M, s, tn, tm, shape, mul))
   if (v.mx) *err = W4_GO(2, 3);
   else if (v.symmetric) *err = v.gs >= 32 ? W4_GO(0, 3) : W4_GO(0, 4);
   else *err = v.gs >= 32 ? W4_GO(1, 3) : W4_GO(1, 4);

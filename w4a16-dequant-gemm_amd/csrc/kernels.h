@@ -78,8 +78,9 @@ struct AnyPlan {
 AnyPlan any_plan(const WView& v, int M);
 // Whether a reciprocal gives the group of every word (see launch() in tile_dma.cuh).
 bool any_group_fits(const WView& v);
-// Launches the planned tile (no hook); false (nothing launched) when the arrays are not aligned for it.
-bool try_tile_any(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, int shape, hipError_t* err);
+// Launches the planned tile; false (nothing launched) when the arrays are not aligned for it.
+bool try_tile_any(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out, int shape,
+                  hipError_t* err);
 
 // gemm_decode_resident.hip: M <= 64 with the activations fetched once per workgroup
 // (several 16-row tiles each).  Same order of additions as the K-split decode

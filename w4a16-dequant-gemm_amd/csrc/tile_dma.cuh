@@ -107,7 +107,7 @@ __global__ __launch_bounds__(TD_THREADS * KG) void w4_tile_dma_kernel(
     int split_at, uint32_t group_mul) {
   constexpr bool ASYM = FMT == 1, MX = FMT == 2;
   constexpr bool ANY = KT > 0;
-  static_assert(!ANY || (!HOOK && GSM >= 3), "no hooked kernel for any group");
+  static_assert(!ANY || GSM >= 3, "the kernels for any group take parameters as runs");
   constexpr int NSC = (!MX && GSM == 2) ? 2 : 1;           // scale dwords per row and stage
   // ANY: a load instruction takes one dword of 64 rows.  The twelve of a row of small groups would hold up the thinnest
   // tile, whose stage is short: there neighbouring lanes take neighbouring dwords of a row (RUNS: N = 11008, K =
@@ -442,8 +442,10 @@ __global__ __launch_bounds__(TD_THREADS * KG) void w4_tile_dma_kernel(
     __syncthreads();
   };
   auto hook_store = [&](const u4* src, int d, int u, int i) {
-    if (HOOK && hook && d < stages && n0 + wrow[i] < N)
-      *(u4*)(w_out + (size_t)(n0 + wrow[i]) * K + d * 128 + (u >> 2) * 64 + h * 32 + (u & 3) * 8) = src[i];
+    if (HOOK && hook && d < stages && n0 + wrow[i] < N) {
+      if (ANY && (u & 3) < dup[u >> 2]) return;  // (the stage before has stored it)
+      *(u4*)(w_out + (size_t)(n0 + wrow[i]) * K + (ANY ? first_k(d) : d * 128u) + (u >> 2) * 64 + h * 32 + (u & 3) * 8) = src[i];
+    }
   };
   auto expand = [&](u4* dst, int d, int u) {
 #pragma unroll
