@@ -248,7 +248,11 @@ def test_native_calls_take_and_refuse_what_ctypes_does():
              ("gemm", (3, 1, 1, 1), {}), ("gemm", (kv, 1, 1, 1), {}), ("gemm", (v, 2.0, 1, 1), {}), ("gemm", (v, None, 1, 1), {}),
              ("gemm", (), {}), ("gemm", (v, 1, 1, "1"), {}), ("attention_f8_flash", (kv, 1, 1), {"scale_mode": 1, "group": 3}),
              ("quantize_cache_f8", (kv, 1, 1, 1), {"src_f16": True}), ("quantize_cache_f8", (kv, 1, 1), {"status": None}),
-             ("attention_fp16_flash", (1, 1, 1, 1, 0, 1, 128), {"group": 0})]
+             ("attention_fp16_flash", (1, 1, 1, 1, 0, 1, 128), {"group": 0}),
+             # None stands for a null address only
+             ("gemm", (v, 1, 1, None), {}), ("gemm_mma", (v, 1, 1), {"M": None}), ("attention_f8_flash", (kv, 1, 1), {"scale_mode": None}),
+             ("attention_f8_flash", (kv, 1, 1), {"group": None}), ("quantize_cache_f8", (kv, 1, 1, 1), {"src_f16": None}),
+             ("attention_fp16_flash", (1, 1, 1, 1, None, 1, 128), {}), ("attention_fp16_flash", (1, 1, 1, 1, 1, 1, 128, None, None), {})]
     for name, args, options in calls:
         said = []
         for f in (getattr(capi, name), getattr(capi, name).__wrapped__):

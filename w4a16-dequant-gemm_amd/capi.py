@@ -149,9 +149,10 @@ def _bind(lib):
             raise RuntimeError(f"{name} and {symbol} take different arguments")
         views = tuple(getattr(kinds[slots.index(n)], "_type_", None) if issubclass(kinds[slots.index(n)], C._Pointer)
                       else None for n in names)
+        addresses = tuple(kinds[slots.index(n)] is vp for n in names)
         defaults = tuple(0 if p.default is p.empty else int(p.default) for p in params.values())
         required = sum(p.default is p.empty for p in params.values())
-        here[name] = native.make(address(symbol), address("w4_last_error"), here[name], names, views, defaults,
+        here[name] = native.make(address(symbol), address("w4_last_error"), here[name], names, views, addresses, defaults,
                                  tuple(slots.index(n) for n in names), required)
 
 

@@ -5,8 +5,9 @@
 // same function 2.55; through these callables 2.66 (1 x 4096 x 4096 back to back 3.95 -> 3.45, a batched paged
 // attention call's host side 4.5 -> 2.9, a cache quantizer's 3.9 -> 2.6).
 //
-// Arguments of the usual types are converted here: a view of exactly the expected type, an int or None.  Anything
-// else (another type, a missing or unknown argument) goes to the ctypes function that stands behind the callable.
+// Arguments of the usual types are converted here: a view of exactly the expected type, an int, and None for an
+// address.  Anything else (another type, None for a number, a missing or unknown argument) goes to the ctypes function that
+// stands behind the callable.
 // Errors are raised as check() in capi.py raises them.  The interpreter lock is given up around the C function,
 // as ctypes does.
 #define PY_SSIZE_T_CLEAN
@@ -28,6 +29,7 @@ struct Call {
   PyObject* slow;             // the same function through ctypes
   PyObject* names[MAX_ARGS];  // interned
   PyObject* views[MAX_ARGS];  // the type of a view argument, or null: an integer or an address
+  bool addresses[MAX_ARGS];   // whether it is an address
   long defaults[MAX_ARGS];
   int slots[MAX_ARGS];        // place of the parameter among the C function's
   int count, required;
@@ -63,7 +65,7 @@ PyObject* call_vector(PyObject* self, PyObject* const* args, size_t nargsf, PyOb
       out = (long)PyLong_AsUnsignedLongLongMask(v);
       usual = !(out == -1 && PyErr_Occurred());
     } else {
-      usual = v == Py_None;
+      usual = v == Py_None && c->addresses[i];
       out = 0;
     }
     a[c->slots[i]] = out;
@@ -118,17 +120,18 @@ PyType_Slot call_slots[] = {{Py_tp_dealloc, (void*)call_dealloc},
 PyType_Spec call_spec = {"w4calls.Call", sizeof(Call), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL, call_slots};
 PyTypeObject* call_type = nullptr;
 
-// make(function, last_error, slow, names, views, defaults, slots, required): addresses, the ctypes function, and a
-// tuple for each property of the parameters
+// make(function, last_error, slow, names, views, addresses, defaults, slots, required): addresses, the ctypes function,
+// and a tuple for each property of the parameters
 PyObject* make(PyObject*, PyObject* args) {
   unsigned long long fn, last_error;
-  PyObject *slow, *names, *views, *defaults, *slots;
+  PyObject *slow, *names, *views, *addresses, *defaults, *slots;
   int required;
-  if (!PyArg_ParseTuple(args, "KKOO!O!O!O!i", &fn, &last_error, &slow, &PyTuple_Type, &names, &PyTuple_Type, &views,
-                        &PyTuple_Type, &defaults, &PyTuple_Type, &slots, &required))
+  if (!PyArg_ParseTuple(args, "KKOO!O!O!O!O!i", &fn, &last_error, &slow, &PyTuple_Type, &names, &PyTuple_Type, &views,
+                        &PyTuple_Type, &addresses, &PyTuple_Type, &defaults, &PyTuple_Type, &slots, &required))
     return nullptr;
   const Py_ssize_t n = PyTuple_GET_SIZE(names);
-  if (n > MAX_ARGS || PyTuple_GET_SIZE(views) != n || PyTuple_GET_SIZE(defaults) != n || PyTuple_GET_SIZE(slots) != n) {
+  if (n > MAX_ARGS || PyTuple_GET_SIZE(views) != n || PyTuple_GET_SIZE(addresses) != n || PyTuple_GET_SIZE(defaults) != n ||
+      PyTuple_GET_SIZE(slots) != n) {
     PyErr_SetString(PyExc_ValueError, "w4calls: the parameters' properties do not match");
     return nullptr;
   }
@@ -151,6 +154,7 @@ PyObject* make(PyObject*, PyObject* args) {
       Py_INCREF(view);
       c->views[i] = view;
     }
+    c->addresses[i] = PyTuple_GET_ITEM(addresses, i) == Py_True;
     c->defaults[i] = PyLong_AsLong(PyTuple_GET_ITEM(defaults, i));
     c->slots[i] = (int)PyLong_AsLong(PyTuple_GET_ITEM(slots, i));
     if (!PyErr_Occurred() && (c->slots[i] < 0 || c->slots[i] >= MAX_ARGS)) PyErr_SetString(PyExc_ValueError, "w4calls: bad slot");
