@@ -3,6 +3,9 @@ include/w4_abi.h declares (no compute calls here)."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
+import sysconfig
 
 import pytest
 
@@ -264,3 +267,15 @@ def test_native_calls_take_and_refuse_what_ctypes_does():
     with pytest.raises(ValueError, match="group"):
         capi.attention_w4_flash(capi.kv_view(1, 64, 128, 32, 4, 1, 16, 16, 0, 16, 16, 0), 16, 16, group=-1)
     assert lib.w4_last_error()
+
+
+def test_entry_points_without_the_native_callables():
+    """No extension for this Python: every entry point is its ctypes call; and one built for another Python is not loaded."""
+    capi = w4amd.capi()
+    assert capi.CALLS_PATH.endswith(sysconfig.get_config_var("EXT_SUFFIX")) and os.path.exists(capi.CALLS_PATH)
+    code = ("import w4amd; c = w4amd.capi(); c.CALLS_PATH += '.absent'; lib = c.load()\n"
+            "assert not any(hasattr(getattr(c, n), '__wrapped__') for n in c._NATIVE)\n"
+            "try: c.gemm(c.packed_view(2, 32, 7, 4, 1, 1, 1), 1, 1, 1)\n"
+            "except ValueError as e: print('refused:', e)\n")
+    run = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.abspath(__file__)), capture_output=True, text=True)
+    assert run.returncode == 0 and run.stdout.startswith("refused:"), run.stderr

@@ -12,7 +12,10 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "lib", "libw4amd.so")
 BENCH_LIB = os.path.join(PKG, "lib", "libw4bench.so")
-CALLS = os.path.join(PKG, "lib", "w4calls.so")  # the Python entry points' native calls (csrc/pycalls.cpp)
+# the Python entry points' native calls (csrc/pycalls.cpp), for this Python; without its headers they are ctypes calls
+CALLS = os.path.join(PKG, "lib", "w4calls" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
+CALLS_SRC = os.path.join(CSRC, "pycalls.cpp")
+PY_INCLUDE = sysconfig.get_paths()["include"]
 SOURCES = ["abi.hip", "dequant.hip", "gemm_simt.hip", "gemm_mfma.hip", "flash.hip", "flash_mfma.hip", "quantize.hip", "gemm_mxnative.hip", "gemm_tile_dma.hip", "gemm_tile_any.hip", "gemm_tile256.hip", "gemm_decode_resident.hip", "gemm_decode_general.hip", "gemm_decode_longk.hip", "gemm_block.hip",
            "baseline.hip"]
 HEADERS = ["dq.cuh", "kernels.h", "simt_rows4.cuh", "tile_dma.cuh", "bench_kernels.hip", os.path.join("..", "..", "include", "w4_abi.h")]
@@ -38,18 +41,32 @@ EXTRA_FLAGS = {"flash_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                "gemm_tile_any.hip": ["-mllvm", "-pragma-unroll-threshold=100000"]}
 
 
+def _calls_stale():
+    if not os.path.exists(os.path.join(PY_INCLUDE, "Python.h")):
+        return False
+    return not os.path.exists(CALLS) or any(os.path.getmtime(d) > os.path.getmtime(CALLS)
+                                            for d in (CALLS_SRC, os.path.abspath(__file__)))
+
+
 def _stale():
-    if not os.path.exists(LIB) or not os.path.exists(CALLS):
+    if not os.path.exists(LIB):
         return True
     t = os.path.getmtime(LIB)
-    deps = [os.path.join(CSRC, f) for f in SOURCES + HEADERS + ["pycalls.cpp"]] + [os.path.abspath(__file__)]
+    deps = [os.path.join(CSRC, f) for f in SOURCES + HEADERS] + [os.path.abspath(__file__)]
     return any(os.path.getmtime(d) > t for d in deps)
 
 
+def _build_calls(force):
+    if _calls_stale() or (force and os.path.exists(os.path.join(PY_INCLUDE, "Python.h"))):
+        subprocess.check_call(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-I" + PY_INCLUDE, CALLS_SRC,
+                               "-o", CALLS])
+
+
 def build(force=False, verbose=True):
+    os.makedirs(os.path.dirname(LIB), exist_ok=True)
+    _build_calls(force)
     if not force and not _stale():
         return LIB
-    os.makedirs(os.path.dirname(LIB), exist_ok=True)
     objs, procs = [], []
     os.makedirs(os.path.join(PKG, "lib", "obj"), exist_ok=True)
     hdr_t = max(os.path.getmtime(os.path.join(CSRC, h)) for h in HEADERS if not h.endswith(".hip"))
@@ -71,10 +88,6 @@ def build(force=False, verbose=True):
             print(err, file=sys.stderr)
     subprocess.check_call(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs,
                            "-lhipblaslt"])
-    calls_src = os.path.join(CSRC, "pycalls.cpp")
-    if force or not os.path.exists(CALLS) or os.path.getmtime(CALLS) < max(hdr_t, os.path.getmtime(calls_src)):
-        subprocess.check_call(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
-                               "-I" + sysconfig.get_paths()["include"], calls_src, "-o", CALLS])
     # bandwidth yardsticks used only by bench.py
     bench_src = os.path.join(CSRC, "bench_kernels.hip")
     if (force or not os.path.exists(BENCH_LIB)

@@ -3,17 +3,21 @@
 wrappers: W4_EINVAL -> ValueError (std::invalid_argument), W4_ERUNTIME ->
 RuntimeError.  There is no fallback: a missing library raises at load().
 
-From load() on the entry points of _NATIVE are callables of lib/w4calls.so, which convert
-the usual arguments themselves; the functions below stay behind them for the rest."""
+From load() on the entry points of _NATIVE are callables of the extension at CALLS_PATH, which
+convert the usual arguments themselves; the functions below stay behind them for the rest, and
+serve all calls where the extension has not been built for this Python."""
 import ctypes as C
 import importlib.machinery
 import importlib.util
 import inspect
 import os
+import sysconfig
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 # W4AMD_LIB points at another build of the same library (kernel tuning builds)
 LIB_PATH = os.environ.get("W4AMD_LIB") or os.path.join(_PKG, "lib", "libw4amd.so")
+# (named for this Python's ABI: another Python does not find it)
+CALLS_PATH = os.path.join(_PKG, "lib", "w4calls" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 
 W4_OK, W4_EINVAL, W4_ERUNTIME = 0, 1, 2
 
@@ -130,10 +134,11 @@ _NATIVE = {
 
 
 def _bind(lib):
-    """Puts native callables in the place of the functions that _NATIVE names."""
-    path = os.path.join(_PKG, "lib", "w4calls.so")
-    loader = importlib.machinery.ExtensionFileLoader("w4calls", path)
-    native = importlib.util.module_from_spec(importlib.util.spec_from_file_location("w4calls", path, loader=loader))
+    """Puts native callables in the place of the functions that _NATIVE names, if they are built."""
+    if not os.path.exists(CALLS_PATH):
+        return
+    loader = importlib.machinery.ExtensionFileLoader("w4calls", CALLS_PATH)
+    native = importlib.util.module_from_spec(importlib.util.spec_from_file_location("w4calls", CALLS_PATH, loader=loader))
     loader.exec_module(native)
     here = globals()
 
