@@ -1,7 +1,10 @@
 """The shipped library loads without a GPU and exports exactly the C ABI that
 include/w4_abi.h declares (no compute calls here)."""
+import copy
 import ctypes
+import inspect
 import os
+import pickle
 import re
 import subprocess
 import sys
@@ -279,3 +282,13 @@ def test_entry_points_without_the_native_callables():
             "except ValueError as e: print('refused:', e)\n")
     run = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.abspath(__file__)), capture_output=True, text=True)
     assert run.returncode == 0 and run.stdout.startswith("refused:"), run.stderr
+
+
+def test_native_callables_are_named_copied_and_pickled_as_functions_are():
+    capi = w4amd.capi()
+    capi.load()
+    for n in capi._NATIVE:
+        f, behind = getattr(capi, n), getattr(capi, n).__wrapped__
+        assert (f.__name__, f.__qualname__, f.__module__, f.__doc__) == (n, n, behind.__module__, behind.__doc__)
+        assert inspect.signature(f) == inspect.signature(behind)
+        assert pickle.loads(pickle.dumps(f)) is f and copy.deepcopy(f) is f

@@ -98,24 +98,29 @@ void call_dealloc(PyObject* self) {
   Py_DECREF(t);
 }
 
-PyObject* call_doc(PyObject* self, void*) { return PyObject_GetAttrString(((Call*)self)->slow, "__doc__"); }
-PyObject* call_name(PyObject* self, void*) { return PyObject_GetAttrString(((Call*)self)->slow, "__name__"); }
+// What a function says of itself, from the one behind; pickled, as functions are, by its name in its module.
+PyObject* call_attribute(PyObject* self, void* name) { return PyObject_GetAttrString(((Call*)self)->slow, (const char*)name); }
+PyObject* call_reduce(PyObject* self, PyObject*) { return PyObject_GetAttrString(((Call*)self)->slow, "__qualname__"); }
 PyObject* call_slow(PyObject* self, void*) {
   PyObject* const s = ((Call*)self)->slow;
   Py_INCREF(s);
   return s;
 }
-PyGetSetDef call_getset[] = {{"__doc__", call_doc, nullptr, nullptr, nullptr},
-                             {"__name__", call_name, nullptr, nullptr, nullptr},
+PyGetSetDef call_getset[] = {{"__doc__", call_attribute, nullptr, nullptr, (void*)"__doc__"},
+                             {"__name__", call_attribute, nullptr, nullptr, (void*)"__name__"},
+                             {"__qualname__", call_attribute, nullptr, nullptr, (void*)"__qualname__"},
+                             {"__module__", call_attribute, nullptr, nullptr, (void*)"__module__"},
                              {"__wrapped__", call_slow, nullptr, nullptr, nullptr},
                              {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyMemberDef call_members[] = {{"__vectorcalloffset__", T_PYSSIZET, offsetof(Call, call), 1, nullptr},
                               {nullptr, 0, 0, 0, nullptr}};
+PyMethodDef call_methods[] = {{"__reduce__", call_reduce, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 
 PyType_Slot call_slots[] = {{Py_tp_dealloc, (void*)call_dealloc},
                             {Py_tp_call, (void*)PyVectorcall_Call},
                             {Py_tp_getset, (void*)call_getset},
                             {Py_tp_members, (void*)call_members},
+                            {Py_tp_methods, (void*)call_methods},
                             {0, nullptr}};
 PyType_Spec call_spec = {"w4calls.Call", sizeof(Call), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL, call_slots};
 PyTypeObject* call_type = nullptr;
