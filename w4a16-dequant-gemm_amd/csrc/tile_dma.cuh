@@ -42,8 +42,8 @@ constexpr int TD_STAGES = 3;
 constexpr int td_tile(int tm, int tn) { return tn * 64 + tm * 256; }
 constexpr int td_stage(int tm, int tn, int planes = 3) { return td_tile(tm, tn) + planes * tn * 4; }
 constexpr int td_lds_bytes(int tm, int tn, int planes = 3) { return TD_STAGES * td_stage(tm, tn, planes); }
-// (KT > 0: a slice's run is read as whole dwords, of which the last may lie behind the last row's)
-constexpr int td_any_slack(int kt) { return kt ? 512 : 0; }
+// (KT > 0: a slice's run is read as whole dwords, of which the last may be one more than a stage has: a dword a row further)
+constexpr int td_any_slack(int tn, int kt) { return kt ? tn * 4 : 0; }
 // Parameter dwords per W row and stage of the kernels for any group (KT > 0): scales, then zero-points.
 // 128 k that start at a multiple of 8 touch five groups of 32 or more k (gsm 3), sixteen of 8 (gsm 4) or five
 // MXFP4 blocks, whose run starts at any half (MXFP4: byte) of the first dword.
@@ -117,6 +117,7 @@ __global__ __launch_bounds__(TD_THREADS * KG) void w4_tile_dma_kernel(
   constexpr bool RUNS = GSM == 4 && TM == 32;
   constexpr int SROW = RUNS ? PS * 4 : 4, SDW = RUNS ? 4 : TN * 4;  // bytes between rows, and between the dwords of one
   constexpr int ZROW = RUNS ? PZ * 4 : 4, ZDW = RUNS ? 4 : TN * 4;
+  static_assert(!ANY || (SDW <= td_any_slack(TN, KT) && ZDW <= td_any_slack(TN, KT)), "what a slice reads ends inside LDS");
   constexpr int PSN = TN * PS / 64, PZN = TN * PZ / 64, PSI = (PSN + 3) / 4, PZI = (PZN + 3) / 4;
   constexpr int TD_TM = TM, MJ = TM / 32;                  // 32-row tiles of X per wave
   constexpr int TD_TN = TN, NI = TN / 128;                 // 32-row tiles of W per wave
@@ -752,7 +753,7 @@ __global__ __launch_bounds__(TD_THREADS * KG) void w4_tile_dma_kernel(
 template <int FMT, int GSM, bool HOOK, int TM, int TN, int KG = 1, int KT = 0>
 hipError_t launch(const WView& v, const w4_half* x, w4_half* c, w4_half* w_out, int M,
                   hipStream_t s, int tiles_n, int tiles_m, int split_at, uint32_t group_mul = 0) {
-  constexpr int TD_LDS = KG * td_lds_bytes(TM, TN, td_planes(FMT, GSM, KT)) + td_any_slack(KT);
+  constexpr int TD_LDS = KG * td_lds_bytes(TM, TN, td_planes(FMT, GSM, KT)) + td_any_slack(TN, KT);
   static_assert(TD_LDS <= 160 * 1024, "the stage buffers of every set of waves fit LDS");
   // more than 64 KB of LDS has to be granted per device, once
   static std::atomic<bool> granted[64] = {};
