@@ -156,3 +156,22 @@ def test_groups_of_whole_chunks_keep_their_scales_in_fp32(M, N, K, gs, sym):
     w = (code.reshape(256, K) - zero) * p.scales.view(np.float16).reshape(N, -1)[ns][:, group].astype(np.float64)
     ref = x.view(np.float16).reshape(M, K).astype(np.float64) @ w.T
     assert orc.rel_l2(np.ascontiguousarray(bits(out).reshape(M, N)[:, ns]).view(np.float16), ref) <= 2.4e-4
+
+
+def test_blocks_along_more_rows_of_w_than_one_grid_dimension_has():
+    """N = 17 million: more blocks of W (eight a row of the grid) than 65535, the grid's second dimension; columns around its end."""
+    c = w4amd.capi()
+    M, N, K = 17, 17_000_007, 1032
+    assert c.gemm_plan_for(0, M, N, K, K) in (11, 21, 22, 24) and N > 65535 * 8 * 32
+    q = torch.empty(N, K // 8, dtype=torch.int32, device="cuda")
+    q.random_(-2 ** 31, 2 ** 31 - 1, generator=torch.Generator(device="cuda").manual_seed(5))
+    s = (torch.rand(N, 1, device="cuda") * 0.01 + 0.01).half()
+    x, out = torch.randn(M, K, device="cuda").half(), torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    c.gemm_mma(c.packed_view(N, K, K, 1, True, ptr(q), ptr(s)), ptr(x), ptr(out), M)
+    for n in (0, 65535 * 8 * 16, 65535 * 8 * 32, N):
+        ns = slice(max(0, n - 200), min(N, n + 200))
+        code = (q[ns][:, :, None] >> (4 * torch.arange(8, device="cuda"))) & 15
+        w = ((code.reshape(-1, K) - 8) * s[ns].float()).half().double()
+        ref = (x.double() @ w.T).cpu().numpy()
+        assert orc.rel_l2(out[:, ns].contiguous().cpu().numpy(), ref) <= TOL, n
+    assert not bool(torch.isnan(out).any())

@@ -33,6 +33,7 @@ typedef __attribute__((address_space(3))) void* lds_ptr;
 constexpr int BK_WAVES = 8, BK_THREADS = 64 * BK_WAVES;
 constexpr int BK_UNIT = 256;  // k of a unit: one 128-byte line of a row of codes, two of a row of x
 constexpr int BK_XS = 2;      // pieces in a wave's ring of x
+constexpr uint32_t BK_GRID_Y = 65535;
 constexpr int bk_wave_bytes(int NT, int XS) { return NT * 2048 + XS * 4096; }
 extern __shared__ __attribute__((aligned(16))) uint8_t bk_lds[];
 
@@ -53,7 +54,7 @@ __device__ __forceinline__ void bk_dma4(uint32_t off, const void* base, uint32_t
 }
 
 // FMT: 0 W4 symmetric, 1 W4 with zero-points, 2 MXFP4.  G: groups (W4) or blocks (MXFP4) per row.
-// group_mul: ceil(2^31 / (gs / 8)): the group of word w is (2 w group_mul) >> 32.  mgroups: blocks along M.  XS: pieces of x (16 rows x 128 k, 4 KB) in a
+// group_mul: ceil(2^31 / (gs / 8)): the group of word w is (2 w group_mul) >> 32.  XS: pieces of x (16 rows x 128 k, 4 KB) in a
 // wave's ring; three measured no better than two.  LATE (W4, gs a multiple of 128: a chunk of 128 k is in one
 // group): the operands are the codes minus the zero-point, exact in FP16, and the scale is applied to a
 // chunk's FP32 sums, as the resident kernel does in the shapes that this one took over from it
@@ -68,9 +69,8 @@ __device__ __forceinline__ void bk_dma4(uint32_t off, const void* base, uint32_t
 template <int FMT, int NT, int MT, int XS, bool AHEAD, bool LATE, int GM, bool RAG>
 __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
     const uint32_t* __restrict__ q, const void* __restrict__ scales, const uint32_t* __restrict__ zeros,
-    const w4_half* __restrict__ x, w4_half* __restrict__ c, const int N, const int K, const int M,
-    const uint32_t group_mul, const int G, const int gs, const int mgroups, w4_half* __restrict__ w_out,
-    const int window) {
+    const w4_half* __restrict__ x, w4_half* __restrict__ c, const int N, const int K, const int M, const int G,
+    const int gs, const uint32_t group_mul, const int window, w4_half* __restrict__ w_out) {
   constexpr bool MX = FMT == 2;
   static_assert(!(MX && LATE), "an MXFP4 chunk has four scales");
   static_assert(GM == 0 || (!MX && !LATE), "scales of a chunk or of MXFP4 blocks need no selector");
@@ -83,9 +83,12 @@ __global__ __launch_bounds__(BK_THREADS) void mfma_block_kernel(
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, b = lane >> 4;
-  const int local = (int)(blockIdx.x >> 3);
-  const int n0 = ((int)(blockIdx.x & 7) + 8 * (local / mgroups)) * ROWS, m0 = (local % mgroups) * (16 * MT);
-  if (n0 >= N) return;
+  // x: XCD + 8 x block along M, y (and z, from 65535 on): eight blocks along N.  (As one number, whose division by a count
+  // in memory came before the first request, a call took 0.2 us longer.  The arguments up to G are in registers when a wave
+  // starts.)
+  const uint32_t first_n = ((blockIdx.x & 7) + 8 * (blockIdx.y + BK_GRID_Y * blockIdx.z)) * ROWS;
+  if (first_n >= (uint32_t)N) return;
+  const int n0 = (int)first_n, m0 = (int)(blockIdx.x >> 3) * (16 * MT);
   const int units = (K + BK_UNIT - 1) / BK_UNIT;
   const uint32_t wrow = (uint32_t)(K >> 1), xrow = (uint32_t)(K * 2);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)bk_lds;
@@ -638,10 +641,11 @@ hipError_t block_go_as(const WView& v, const w4_half* x, w4_half* c, int M, hipS
     if (e != hipSuccess) return e;
     if (dev >= 0 && dev < 64) granted[dev] = true;
   }
-  const int mg = (M + 16 * MT - 1) / (16 * MT), ng = (v.N + 16 * NT - 1) / (16 * NT);
+  const uint32_t mg = (M + 16 * MT - 1) / (16 * MT), ng8 = ((uint32_t)v.N + 128 * NT - 1) / (128 * NT);
+  const dim3 grid(8 * mg, ng8 < BK_GRID_Y ? ng8 : BK_GRID_Y, (ng8 + BK_GRID_Y - 1) / BK_GRID_Y);
   const uint32_t mul = v.mx ? 0u : (uint32_t)(((1ULL << 31) + v.gs / 8 - 1) / (v.gs / 8));
-  mfma_block_kernel<FMT, NT, MT, XS, AHEAD, LATE, GM, RAG><<<dim3((unsigned)(8 * ((ng + 7) / 8) * mg)), BK_THREADS, lds_bytes, s>>>(
-      v.q, v.scales, v.zeros, x, c, v.N, v.K, M, mul, v.mx ? v.B : v.G, v.gs, mg, w_out, window);
+  mfma_block_kernel<FMT, NT, MT, XS, AHEAD, LATE, GM, RAG><<<grid, BK_THREADS, lds_bytes, s>>>(
+      v.q, v.scales, v.zeros, x, c, v.N, v.K, M, v.mx ? v.B : v.G, v.gs, mul, window, w_out);
   return hipGetLastError();
 }
 
