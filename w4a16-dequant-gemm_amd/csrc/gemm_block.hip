@@ -651,8 +651,7 @@ hipError_t block_go_as(const WView& v, const w4_half* x, w4_half* c, int M, hipS
 
 // Forms that are compiled for blocks of NT x MT.  Rows of words that are only 4-byte aligned take four times the load
 // instructions, small groups take LDS for their parameters: neither has blocks of more than two tiles of W.
-constexpr bool bk_has(int fmt, int NT, int MT, int gm, bool rag) {
-  (void)MT;
+constexpr bool bk_has(int fmt, int NT, int gm, bool rag) {
   return fmt == 2 || gm == 0 || NT <= 2 || (gm == 1 && !rag);
 }
 
@@ -666,13 +665,13 @@ hipError_t block_go(const WView& v, const w4_half* x, w4_half* c, int M, hipStre
     if (gm == 0)
       return v.gs % 128 == 0 ? block_go_as<FMT, NT, MT, true, 0, false>(v, x, c, M, s, w_out)
                              : block_go_as<FMT, NT, MT, false, 0, false>(v, x, c, M, s, w_out);
-    if constexpr (bk_has(FMT, NT, MT, 1, false))
+    if constexpr (bk_has(FMT, NT, 1, false))
       if (gm == 1 && !rag) return block_go_as<FMT, NT, MT, false, 1, false>(v, x, c, M, s, w_out);
-    if constexpr (bk_has(FMT, NT, MT, 1, true))
+    if constexpr (bk_has(FMT, NT, 1, true))
       if (gm == 1 && rag) return block_go_as<FMT, NT, MT, false, 1, true>(v, x, c, M, s, w_out);
-    if constexpr (bk_has(FMT, NT, MT, 2, false))
+    if constexpr (bk_has(FMT, NT, 2, false))
       if (gm == 2 && !rag) return block_go_as<FMT, NT, MT, false, 2, false>(v, x, c, M, s, w_out);
-    if constexpr (bk_has(FMT, NT, MT, 2, true))
+    if constexpr (bk_has(FMT, NT, 2, true))
       if (gm == 2 && rag) return block_go_as<FMT, NT, MT, false, 2, true>(v, x, c, M, s, w_out);
     return hipErrorInvalidValue;
   }
@@ -845,7 +844,7 @@ int block_any_time(const WView& v, int M, int cus, int* time) {
   int best = -1;
   for (int i = 0; i < BK_COUNT; ++i) {
     const BkShape& s = BK_SHAPES[i];
-    if (!bk_has(v.mx ? 2 : 0, s.nt, s.mt, gm, bk_ragged(v)) || bk_window(v, s.nt) < 1) continue;
+    if (!bk_has(v.mx ? 2 : 0, s.nt, gm, bk_ragged(v)) || bk_window(v, s.nt) < 1) continue;
     const int t = bk_time(v, M, s, cus);
     if (best < 0 || t < *time) best = i, *time = t;
   }
