@@ -48,13 +48,13 @@ def _check(fmt, M, N, K, gs, scale=None):
     return c.gemm_plan_for(fmt, M, N, K, gs)
 
 
-# (plan, fmt, M, N, K, gs): tiles of 32 x 128 (4) to 128 x 256 (7) in every compiled form; K ends inside a chunk and, 264,
-# inside a piece; gs = 40 .. 136 begin in any word; N * G odd (MXFP4: N * B % 4): the last scale is part of a dword
-TILES = [(4, 0, 1100, 257, 2080, 24), (4, 0, 2049, 257, 264, 8), (4, 0, 2049, 129, 1056, 72), (4, 0, 520, 257, 264, 40),
-         (4, 1, 2049, 129, 2080, 24), (4, 1, 900, 777, 264, 24), (4, 1, 1100, 257, 1056, 40), (4, 1, 130, 3001, 264, 40),
-         (4, 2, 2049, 129, 1056, 32), (4, 2, 520, 257, 264, 32), (5, 0, 1300, 777, 2080, 24), (5, 0, 1300, 777, 264, 16),
+# (plan, fmt, M, N, K, gs): tiles of 32 x 128 (4) to 128 x 256 (7) in every compiled form; K ends inside a chunk and, 264, 520 and
+# 1032, inside a piece; gs = 40 .. 136 begin in any word; N * G odd (MXFP4: N * B % 4): the last scale is part of a dword
+TILES = [(4, 0, 1100, 257, 2080, 24), (4, 0, 2049, 257, 1032, 8), (4, 0, 2049, 129, 1056, 72), (4, 0, 520, 257, 264, 40),
+         (4, 1, 2049, 129, 2080, 24), (4, 1, 2049, 257, 1032, 24), (4, 1, 1100, 257, 1056, 40), (4, 1, 900, 777, 520, 40),
+         (4, 2, 2049, 129, 1056, 32), (4, 2, 2049, 257, 1032, 32), (5, 0, 1300, 777, 2080, 24), (5, 0, 1300, 777, 264, 16),
          (5, 0, 1300, 777, 1056, 104), (5, 0, 900, 1034, 264, 48), (5, 1, 520, 2051, 2080, 24), (5, 1, 1300, 777, 264, 8),
-         (5, 1, 1300, 777, 1056, 96), (5, 1, 1300, 777, 264, 40), (5, 2, 900, 1034, 1056, 32), (5, 2, 900, 1034, 264, 32),
+         (5, 1, 1300, 777, 1056, 96), (5, 1, 1300, 777, 264, 40), (5, 2, 1700, 1034, 1056, 32), (5, 2, 1700, 1034, 1032, 32),
          (6, 0, 1100, 2051, 2080, 24), (6, 0, 1100, 2051, 264, 8), (6, 0, 1100, 2051, 1056, 104), (6, 0, 700, 3001, 264, 40),
          (6, 1, 900, 3001, 2080, 24), (6, 1, 1100, 2051, 264, 8), (6, 1, 700, 3001, 1056, 40), (6, 1, 700, 3001, 264, 96),
          (6, 2, 900, 2310, 1056, 32), (6, 2, 900, 2310, 264, 32), (7, 0, 1300, 3001, 1056, 1056), (7, 0, 1300, 3001, 264, 40),
@@ -175,3 +175,18 @@ def test_blocks_along_more_rows_of_w_than_one_grid_dimension_has():
         ref = (x.double() @ w.T).cpu().numpy()
         assert orc.rel_l2(out[:, ns].contiguous().cpu().numpy(), ref) <= TOL, n
     assert not bool(torch.isnan(out).any())
+
+
+# Calls that the kernels before are ahead in, and calls beside them in which blocks or tiles are (us then and now): the times of both
+# sides depend on whole 16-byte pieces of codes, on steps that the stream kernel's ring rounds up, on outputs stored one by one
+PLAN = [((1, 3991, 1551, 2048, 16), False), ((1, 3991, 1551, 2056, 16), True),    # 52 and 72
+        ((0, 5, 15272, 1408, 128), False), ((0, 5, 15272, 4104, 128), True),      # 6.6 and 9.5
+        ((1, 2964, 304, 352, 64), False), ((1, 2964, 304, 1056, 64), True),       # 5.7 and 8.4
+        ((2, 30, 16320, 352, 32), False), ((2, 30, 16320, 1056, 32), True),       # 4.5 and 6.1
+        ((1, 9, 8778, 1792, 1792), False), ((1, 9, 8778, 4096, 4096), True),      # 7.8 and 9.8
+        ((1, 3052, 2271, 256, 96), False), ((1, 3052, 2272, 264, 96), True)]      # 20.6 and 25.1
+
+
+@pytest.mark.parametrize("call,ahead", PLAN)
+def test_blocks_and_tiles_are_planned_where_they_are_ahead(call, ahead):
+    assert (w4amd.capi().gemm_plan_for(*call) >= 4) == ahead

@@ -28,16 +28,17 @@ hipError_t any_go(const WView& v, const w4_half* x, w4_half* c, w4_half* w_out, 
   return launch<FMT, GSM, false, 128, 128, 1, KT>(v, x, c, nullptr, M, s, tn, tm, 0, mul);
 }
 
-// Time of a call in units of 10 ns: start + rounds of workgroups x (round + per_n x n), n in stages of 128 k. Fitted to
-// 6657 shapes of 3 to 4000 rows, K = 256 to 14336, to within 4 to 10 % (r.m.s.); per_n: [symmetric W4, with
-// zero-points, MXFP4], small: the same for groups of less than 32.
+// Time of a call in units of 10 ns: start + rounds of workgroups x (round + per_n x n) + rounds, a begun one in part, x store, n in
+// stages of 128 k. Fitted to 6657 shapes of 3 to 4000 rows, K = 256 to 14336, to within 4 to 10 % (r.m.s.); per_n: [symmetric
+// W4, with zero-points, MXFP4], small: the same for groups of less than 32; store: what the outputs take, N a multiple of 4
+// or not (halves one by one: M = 3052, N = 2271, K = 256 25.1 us).
 struct AnyShape {
-  int shape, tm, tn, start, round, per_n[3], small_round, small_n[2];
+  int shape, tm, tn, start, round, per_n[3], small_round, small_n[2], store[2];
 };
-constexpr AnyShape ANY_SHAPES[] = {{4, 32, 128, 130, 285, {57, 66, 43}, 290, {71, 88}},
-                                   {2, 64, 128, 50, 430, {70, 74, 55}, 300, {98, 117}},
-                                   {3, 128, 128, -70, 490, {105, 115, 90}, 510, {115, 133}},
-                                   {0, 128, 256, -270, 850, {170, 186, 148}, 0, {0, 0}}};
+constexpr AnyShape ANY_SHAPES[] = {{4, 32, 128, 130, 285, {57, 66, 43}, 290, {71, 88}, {10, 200}},
+                                   {2, 64, 128, 50, 430, {70, 74, 55}, 300, {98, 117}, {110, 430}},
+                                   {3, 128, 128, -70, 490, {105, 115, 90}, 510, {115, 133}, {160, 770}},
+                                   {0, 128, 256, -270, 850, {170, 186, 148}, 0, {0, 0}, {230, 1500}}};
 
 // Whether the tile kernels for any group take the operands, their alignment apart.
 bool any_applies(const WView& v, int M) {
@@ -59,35 +60,77 @@ int any_shape(const WView& v, int M, int cus, int* time) {
     const long long tiles = (long long)((v.N + s.tn - 1) / s.tn) * ((M + s.tm - 1) / s.tm), rounds = (tiles + cus - 1) / cus;
     // (dword loads of codes: a tenth more)
     const long long per = (long long)(small ? s.small_n[f] : s.per_n[f]) * stages * (rag ? 11 : 10) / 10;
-    const long long t = s.start + rounds * ((small ? s.small_round : s.round) + per);
+    const long long t = s.start + rounds * ((small ? s.small_round : s.round) + per) + tiles * s.store[v.N % 4 != 0] / cus;
     if (best < 0 || t < least) best = s.shape, least = t;
   }
   *time = least > 1 << 30 ? 1 << 30 : (int)least;
   return best;
 }
 
-// Time of the kernel that has the call otherwise, in the same units; of the stream kernel and the register-staged tiles
-// up to K = 1024 (from there on they took 1.3 to 5 times the others' time).
+// Time of the kernel that has the call otherwise, in the same units: start + per_n x n + share x (share_0 + share_n x n).  n: steps of a
+// wave (K-split kernel: chunks of 128 k; stream kernel: chunks, or pairs of them up to 32 rows, as many as its ring
+// takes at a time), share: rounds of workgroups after the first (stream kernel: workgroups a compute unit has).  Rows of codes
+// that are whole 16-byte pieces are loaded so and take 0.25 to 0.7 of the others' time.  Fitted to 14000 shapes of 5 to 4000
+// rows, K = 64 to 14336, to within 6 to 13 % in whole pieces and 9 to 18 % otherwise (r.m.s.).
+struct OtherShape {
+  int start, per_n, share_0, share_n;
+};
+// [whole pieces][MXFP4, groups of whole slices of 32 k, other groups]
+constexpr OtherShape OTHER_KSPLIT[2][3] = {{{210, 149, -304, 330}, {204, 158, -290, 312}, {171, 196, -348, 390}},
+                                           {{298, 64, -106, 110}, {300, 73, -110, 114}, {223, 144, -164, 180}}};
+// up to 32 rows: eight waves that share K by four (fewer than 128 workgroups of 64 rows of W) or by two
+constexpr OtherShape OTHER_STREAM_BY4[2][3] = {{{180, 316, -24, 200}, {135, 379, 81, 133}, {202, 450, 5, 222}},
+                                               {{224, 196, 86, 18}, {237, 207, 8, 62}, {191, 388, 103, 6}}};
+constexpr OtherShape OTHER_STREAM_BY2[2][3] = {{{100, 375, 150, 20}, {146, 415, 25, 14}, {193, 518, -21, 19}},
+                                               {{261, 134, 3, 23}, {257, 129, -36, 66}, {150, 380, 80, -20}}};
+constexpr OtherShape OTHER_STREAM64[2][3] = {{{213, 76, -18, 239}, {251, 76, 0, 260}, {218, 115, -38, 306}},
+                                             {{251, 44, 27, 150}, {273, 46, 29, 168}, {230, 96, 4, 221}}};
+// The register-staged tiles of 256 x 128: start + (n + share x begun round) x k + further rounds x (round + round_n x k), k in
+// steps of 64; 1, 2 or 4 steps in flight (fitted to 3200 shapes, to within 7 to 13 %).
+constexpr int OTHER_TILE[3][5] = {{470, 124, 65, 510, 175}, {480, 101, 65, 600, 135}, {560, 84, 50, 650, 107}};
+
 int other_time(const WView& v, int M, int cus) {
-  const int stages = (v.K + 127) / 128, cpw = (stages + 7) / 8;
+  const int chunks = (v.K + 127) / 128, cpw = (chunks + 7) / 8;
   const long long tiles = (v.N + 15) / 16;
   if (decode_general_applies(v, nullptr, nullptr, M)) {
     const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4, per = (v.gs < 32 ? 9 : 0) + (v.symmetric ? 64 : 74);
     return (int)(400 + (tiles + cus - 1) / cus * (cpw * (per + 19 * mt) - 30));
   }
-  if (M <= 8 || (M <= 16 && v.N < 8192)) {  // (its times spread by a third: less a tenth; small groups take half as much again)
-    const long long share = tiles > cus ? tiles * 64 / cus : 64;  // tiles a compute unit, in 64ths
-    const long long t = v.K < 3072 ? 240 + share * (10 + 109 * cpw) / 64 : 80 + share * (175 * cpw - 70) / 64;
-    return (int)(t * (!v.mx && v.gs < 32 && v.K >= 3072 ? 135 : 90) / 100);
+  const bool pieces = v.K % 32 == 0, halves = v.N % 4 != 0;  // (halves: outputs are stored one by one)
+  long long t;
+  if (M >= 96 && v.K % 64 == 0) {
+    const int k = v.K / 64, *const c = OTHER_TILE[(!v.mx && v.gs % 16) || k % 2 ? 0 : k % 4 ? 1 : 2];
+    const long long wgs = (long long)((v.N + 127) / 128) * ((M + 255) / 256), more = (wgs + cus - 1) / cus - 1;
+    const long long part = wgs < cus ? wgs * 64 / cus : 64;  // of the first round, in 64ths
+    t = c[0] + (c[1] * 64 + c[2] * part) * k / 64 + more * (c[3] + c[4] * k);
+    if (halves) t += 430 + 500 * part / 64 + 700 * more;
+  } else {
+    const int form = v.mx ? 0 : v.gs % 32 == 0 ? 1 : 2;
+    const OtherShape* c = &OTHER_STREAM64[pieces][form];
+    int n = cpw;
+    long long share, whole = 64;  // in 64ths
+    if (M <= 8 || (M <= 16 && v.N < 8192)) {
+      c = &OTHER_KSPLIT[pieces][form];
+      share = 64 * ((tiles + cus - 1) / cus - 1);
+    } else {
+      long long wgs = (long long)((v.N + 63) / 64) * ((M + 63) / 64);
+      if (M <= 32) {
+        const bool by4 = wgs < 128;
+        c = by4 ? &OTHER_STREAM_BY4[pieces][form] : &OTHER_STREAM_BY2[pieces][form];
+        n = ((chunks + 1) / 2 + (by4 ? 3 : 1)) / (by4 ? 4 : 2);
+        if (n >= 2) n = (n + 1) / 2 * 2;
+        if (by4) wgs = (v.N + 31) / 32;
+      } else {
+        n = (chunks + 1) / 2;
+        if (n >= 4) n = (n + 3) / 4 * 4;
+      }
+      share = 2 * wgs > cus ? wgs * 64 / cus : 32;
+      // (up to 32 rows the shapes end at N = 16384, a workgroup a compute unit: on from there all but the start grows)
+      if (M <= 32 && share > 64) whole = share;
+    }
+    t = c->start + whole * c->per_n * n / 64 + share * (c->share_0 + c->share_n * n + (halves && M > 32 ? 110 : 0)) / 64;
   }
-  if (v.K >= 1024) return 1 << 30;
-  if (v.K % 64 == 0 && M >= 96) {
-    const long long rounds = ((long long)((v.N + 127) / 128) * ((M + 255) / 256) + cus - 1) / cus;
-    return (int)(rounds * (950 + 113 * (v.K / 64)) - 300);
-  }
-  const int rows = M <= 32 ? 32 : 64;
-  const long long wgs = (long long)((v.N + 63) / 64) * ((M + rows - 1) / rows), share = 2 * wgs > cus ? wgs * 64 / cus : 32;
-  return (int)(M <= 32 ? 440 + share * 50 * stages / 64 : 275 + 38 * stages + share * (127 + 110 * stages) / 64);
+  return t > 1 << 30 ? 1 << 30 : (int)t;
 }
 
 // What the general decode kernel takes on top of that: next to the activations of 33 to 64 rows LDS has room for the
@@ -107,8 +150,9 @@ bool any_group_fits(const WView& v) { return v.mx || (long long)(v.K / 8) * (v.g
 
 AnyPlan any_plan(const WView& v, int M) {
   const AnyPlan none{0, -1};
+  if (M < 5 || v.K % 8) return none;
   const int cus = device_cus();
-  if (M < 5 || v.K % 8 || cus < 8) return none;
+  if (cus < 8) return none;
   // Shorter rows are no more than a launch for the kernels that have them.  Up to 16 rows on few tiles: N < 2048, K = 1281 to
   // 3072 0.83 to 1.0 times as fast, up to 4096 1.05 to 1.13; N = 2048 to 4096, K up to 2048 0.9 to 1.03.
   const int tiles = (v.N + 15) / 16;
@@ -123,13 +167,17 @@ AnyPlan any_plan(const WView& v, int M) {
   int tile = -1, tile_time = 1 << 30, block_shape = -1, block_t = 1 << 30;
   if (any_applies(v, M)) tile = any_shape(v, M, cus, &tile_time);
   if (whole) {
-    // blocks as block_plan() has them; tiles where these are ahead by a quarter (the error of the times on both sides)
+    // blocks as block_plan() has them; tiles where these take less than three quarters of the time (the error of the times on
+    // both sides: M = 157, N = 9904, K = 12768, gs = 32 with zero-points at 0.79 92 us in blocks and 105 on tiles)
     block_shape = block_plan_time(v, M, &block_t);
     // (W4 groups of whole chunks: blocks scale a chunk's FP32 sums, tiles round every weight; 2.1e-4 and 2.7e-4 from the
     // product in FP64)
     if (block_shape >= 0 && !v.mx && v.gs % 128 == 0) return AnyPlan{1, block_shape};
-    if (block_shape < 0) return tile_time < other_time(v, M, cus) ? AnyPlan{2, tile} : none;
-    return 5 * tile_time < 4 * block_t ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
+    if (block_shape < 0) {
+      if (decode_resident_applies(v, nullptr, nullptr, M)) return none;
+      return 8LL * tile_time < 7LL * other_time(v, M, cus) ? AnyPlan{2, tile} : none;
+    }
+    return 4LL * tile_time < 3LL * block_t ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
   }
   block_shape = block_any_time(v, M, cus, &block_t);
   const int other = other_time(v, M, cus);
@@ -138,10 +186,13 @@ AnyPlan any_plan(const WView& v, int M) {
   // Up to five rounds of its tiles they have to be ahead by a quarter: M = 41, N = 11504, K = 2176, gs = 8 13.1 us there and 18.3
   // on tiles, M = 54, N = 13936, K = 2752 18.1 and 21.6; past them M = 40, N = 28672, K = 4096 55 and 42.
   const bool close = !v.mx && v.gs < 32 && M > 32 && tiles <= 5 * cus && decode_general_applies(v, nullptr, nullptr, M);
-  const bool tiles_ahead = close ? 4LL * tile_time < 3LL * other : tile_time < other;
-  const bool blocks_ahead = block_t < other + general_rounds(v, M, cus);
+  // Otherwise blocks and tiles have to be ahead by an eighth, about the error of the times (44570 random shapes, 13147 of which
+  // blocks or tiles took over: without it 578 lost more than 5 %, with it 74; it gives up 0.5 % of the gain).
+  const bool tiles_ahead = close ? 4LL * tile_time < 3LL * other : 8LL * tile_time < 7LL * other;
+  const bool blocks_ahead = 8LL * block_t < 7LL * ((long long)other + general_rounds(v, M, cus));
   if (!tiles_ahead && !blocks_ahead) return none;
-  return tiles_ahead && (!blocks_ahead || tile_time < block_t) ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
+  // (blocks take about a tenth more than their time above where it is the least of all)
+  return tiles_ahead && (!blocks_ahead || 10LL * tile_time < 11LL * block_t) ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
 }
 
 bool try_tile_any(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out, int shape,
