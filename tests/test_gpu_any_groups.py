@@ -184,7 +184,9 @@ PLAN = [((1, 3991, 1551, 2048, 16), False), ((1, 3991, 1551, 2056, 16), True),  
         ((1, 2964, 304, 352, 64), False), ((1, 2964, 304, 1056, 64), True),       # 5.7 and 8.4
         ((2, 30, 16320, 352, 32), False), ((2, 30, 16320, 1056, 32), True),       # 4.5 and 6.1
         ((1, 9, 8778, 1792, 1792), False), ((1, 9, 8778, 4096, 4096), True),      # 7.8 and 9.8
-        ((1, 3052, 2271, 256, 96), False), ((1, 3052, 2272, 264, 96), True)]      # 20.6 and 25.1
+        ((1, 3052, 2271, 256, 96), False), ((1, 3052, 2272, 264, 96), True),      # 20.6 and 25.1
+        # gs = 32 with zero-points, blocks against its two smallest tiles (plan 0): 6.0 and 7.1, 7.4 and 8.0
+        ((1, 68, 5712, 384, 32), False), ((1, 68, 2736, 384, 32), True), ((1, 66, 6464, 640, 32), False), ((1, 66, 4704, 640, 32), True)]
 
 
 @pytest.mark.parametrize("call,ahead", PLAN)

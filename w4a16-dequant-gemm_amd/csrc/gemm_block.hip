@@ -753,8 +753,13 @@ bool block_ahead(const WView& v, int M, const BkShape& s, long long rounds, bool
     // one for the others: K = 2304, N = 6144, M = 146 12.4 against 9.9.
     // N = 288, K = 11904, M = 2857 84.6 against 57.4; N = 544, K = 4608 (18 units), M = 1256 21.1 against 18.5
     if (M > 1536 || (M > 1024 && v.N >= 256 && 32 * ((units + 7) / 8) > 5 * units)) return false;
-    // gs = 32 with zero-points has tiles of 256 rows of W only there: N = 6560, K = 1664, M = 82 10.7 against 18.3
-    if (!v.mx && !sym && v.gs == 32) return units > 1 || area <= 2;
+    // gs = 32 with zero-points has two smallest tiles of its own there, which are behind from four units on (M = 95, N = 14416,
+    // K = 3072 16.3 against 25.6); shorter K: M = 68, N = 5712, K = 384 7.1 against 6.0, N = 4784, M = 118 7.1 and 6.1, K = 640,
+    // N = 6464, M = 66 8.0 and 7.4 (2700 calls: blocks of up to 8 tiles of 16 x 16 at two units and 12 at three are ahead)
+    if (!v.mx && !sym && v.gs == 32) {
+      constexpr int largest32[5] = {0, 2, 8, 12, 20};
+      return units > 4 || area <= largest32[units];
+    }
     constexpr int largest[14] = {0, 2, 2, 4, 8, 8, 12, 12, 24, 12, 20, 20, 20, 20};
     return units > 13 || area <= largest[units];
   }
