@@ -116,8 +116,11 @@ def test_ends_of_rows_bring_no_infinity(M, N, K, gs):
     with np.errstate(invalid="ignore"):
         ref = x[rows].astype(np.float64) @ w.T
         bad = x[2].astype(np.float64)[None] @ w.T
-    assert np.isfinite(ref).any() and np.isfinite(got[rows]).sum() >= np.isfinite(ref).sum() * 0.99
-    ok = np.isfinite(ref) & np.isfinite(got[rows])
+    # an output is finite where the oracle's stays below the largest half by more than 2^-10 of the sum of magnitudes (FP32 sums
+    # of K < 2^13 products are off by less than 2^-11 of it)
+    sure = np.abs(ref) < 65504 - 2.0 ** -10 * (np.abs(x[rows].astype(np.float64)) @ np.abs(w.T))
+    assert sure.mean() > 0.9 and not np.isnan(got[rows]).any() and np.isfinite(got[rows][sure]).all()
+    ok = np.isfinite(got[rows]) & (np.abs(ref) < 65504)
     assert np.linalg.norm((got[rows] - ref)[ok]) <= 1e-3 * np.linalg.norm(ref[ok])
     assert np.array_equal(np.isnan(got[2]), np.isnan(bad[0])) and np.array_equal(np.isinf(got[2]), np.isinf(bad[0]))
 
