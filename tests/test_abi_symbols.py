@@ -156,6 +156,8 @@ def test_mx_plan():
     eight_waves = [(0, 33, 14336, 4096), (1, 8, 14336, 4096), (1, 64, 14336, 4096), (0, 17, 4096, 11008),
                    (0, 1, 28672, 4096), (1, 192, 14336, 4096), (0, 101, 4096, 4096)]
     assert [a for a in eight_waves if plan(*a) not in (1, 2, 3, 4)] == []
+    # K a multiple of 256 and not of 512
+    assert [plan(0, M, 20480, 2816) for M in (2, 3, 4, 5)] == [0, 1, 1, 1] and plan(0, 5, 13000, 2816) == plan(1, 7, 13000, 7424) == 0
     assert plan(0, 2048, 4096, 4096) == plan(1, 2048, 4096, 4096) == 8
     for bad in [(0, 0, 8, 64), (0, 8, 0, 64), (1, 8, 8, 0)]:
         with pytest.raises(ValueError):

@@ -1175,13 +1175,15 @@ bool tile_operands_ok(const w4_packed_mx_view& w, const void* xq, const uint8_t*
 // M = 97 - 128 up to 64; 8-bit X up to 32 1.1 - 1.3; 4-bit X at N = 4096, K = 14336 0.83 - 0.86 and 1.25 - 1.27 (K = 4096
 // 0.83 - 0.87 and 1.11 - 1.15, which stays with the tiles).  At K <= 2048 up to 64 with either (N = 2048, 4-bit X: 4.5
 // against 5.0).
-// Where K is a multiple of 256 and not of 512 the skinny kernel, as fast as elsewhere up to 16 rows (4-bit X; 32 with
-// 8-bit X), keeps those, and short K with 8-bit X (N = 1000, K = 1280, M = 64: 4.5 against 4.7).
+// Where K is a multiple of 256 and not of 512 the same lines hold up to 16 rows (4-bit X; 32 with 8-bit X: from there on tiles;
+// tile / skinny, K = 1280 to 12032, cache and memory: M = 5 - 8, 100 - 125 workgroups 0.97 and 1.28, M = 9 - 12 0.92 and 1.23,
+// M <= 2, 160 - 172 0.93 and 1.14; 8-bit X, M = 5 - 8 0.85 and 1.18), but for M = 3, 4 with 4-bit X, 160: 0.84 and 1.05.  The
+// skinny kernel keeps short K with 8-bit X (N = 1000, K = 1280, M = 64: 4.5 against 4.7).
 template <bool XF8>
 int fewest_tile_workgroups(int M, int K) {
   if (K % 512 && M > (XF8 ? 32 : 16)) return 0;
   if (XF8) return M <= 4 ? 160 : M <= 8 && K > 4096 ? 121 : 100;
-  if (M <= 12) return M <= 2 ? 200 : M <= 4 ? 171 : M <= 8 ? 140 : 121;
+  if (M <= 12) return M <= 2 ? 200 : M <= 4 ? (K % 512 ? 160 : 171) : M <= 8 ? 140 : 121;
   return M <= 16 && K > 4096 ? 121 : M > 32 && M <= 48 && K > 6144 ? 140 : 100;
 }
 
