@@ -858,7 +858,7 @@ int block_any_time(const WView& v, int M, int cus, int* time) {
 
 int block_shape(const WView& v, int M) {
   const AnyPlan any = any_plan(v, M);
-  const int i = any.kind == 1 ? any.shape : block_plan(v, M);
+  const int i = any.kind == 1 ? any.shape : any.kind == 3 ? -1 : block_plan(v, M);
   return i < 0 ? 0 : 10 * BK_SHAPES[i].nt + BK_SHAPES[i].mt;
 }
 

@@ -906,7 +906,7 @@ static hipError_t launch_fmt(const WView& v, const w4_half* x, w4_half* c, int M
   hipError_t terr = hipSuccess;
   const AnyPlan any = any_plan(v, M);
   if (any.kind == 2 && try_tile_any(v, x, c, M, s, w_out, any.shape, &terr)) return terr;
-  if (try_block(v, x, c, M, s, w_out, any.kind == 1 ? any.shape : -1, &terr)) return terr;
+  if (any.kind != 3 && try_block(v, x, c, M, s, w_out, any.kind == 1 ? any.shape : -1, &terr)) return terr;
   // Shapes of the kernel that fetches the activations once per workgroup (M <= 256):
   // hooked calls take the K-split kernel, which adds in the same order.
   const bool wvec = (v.K % 32 == 0) && (((uintptr_t)v.q) & 15) == 0;

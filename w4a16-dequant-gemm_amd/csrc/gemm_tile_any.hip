@@ -174,8 +174,8 @@ AnyPlan any_plan(const WView& v, int M) {
     // product in FP64)
     if (block_shape >= 0 && !v.mx && v.gs % 128 == 0) return AnyPlan{1, block_shape};
     if (block_shape < 0) {
-      if (decode_resident_applies(v, nullptr, nullptr, M)) return none;
-      return 8LL * tile_time < 7LL * other_time(v, M, cus) ? AnyPlan{2, tile} : none;
+      if (decode_resident_applies(v, nullptr, nullptr, M)) return AnyPlan{3, -1};
+      return 8LL * tile_time < 7LL * other_time(v, M, cus) ? AnyPlan{2, tile} : AnyPlan{3, -1};
     }
     return 4LL * tile_time < 3LL * block_t ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
   }

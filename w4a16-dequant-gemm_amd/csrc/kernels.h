@@ -71,7 +71,7 @@ int block_any_time(const WView& v, int M, int cus, int* time);
 
 // gemm_tile_any.hip: the kernel of gemm_tile_dma.hip for any group size and any K that are multiples of 8, and the
 // plan for calls whose sizes the kernels for whole tiles, chunks and groups do not take: kind 1 a block
-// (shape: its index), 2 a tile, 0 another kernel.
+// (shape: its index), 2 a tile, 0 another kernel, 3 another kernel and no block (block_plan() has been asked).
 struct AnyPlan {
   int kind, shape;
 };
