@@ -1,5 +1,7 @@
 // The large-M W4A16 / MXFP4 GEMM of tile_dma.cuh for weights whose groups do not tile a 128-k stage: any
 // group size and any K that are multiples of 8 (mma.cuh:63-230, the reference's kernel, takes them all).
+#include <algorithm>
+
 #include "tile_dma.cuh"
 
 namespace w4k {
@@ -28,17 +30,17 @@ hipError_t any_go(const WView& v, const w4_half* x, w4_half* c, w4_half* w_out, 
   return launch<FMT, GSM, false, 128, 128, 1, KT>(v, x, c, nullptr, M, s, tn, tm, 0, mul);
 }
 
-// Time of a call in units of 10 ns: start + rounds of workgroups x (round + per_n x n) + rounds, a begun one in part, x store, n in
-// stages of 128 k. Fitted to 6657 shapes of 3 to 4000 rows, K = 256 to 14336, to within 4 to 10 % (r.m.s.); per_n: [symmetric
-// W4, with zero-points, MXFP4], small: the same for groups of less than 32; store: what the outputs take, N a multiple of 4
-// or not (halves one by one: M = 3052, N = 2271, K = 256 25.1 us).
+// Time of a call in units of 10 ns: start + rounds of workgroups x (round + per_n x n) + store, n in stages of 128 k. Fitted to 6657
+// shapes of 3 to 4000 rows, K = 256 to 14336, to within 4 to 10 % (r.m.s.); per_n: [symmetric W4, with zero-points,
+// MXFP4], small: the same for groups of less than 32; store: what the outputs take, [N a multiple of 4 or not: halves one by one][the first
+// round, or the part that is begun; a further one] (M = 3052, N = 2271, K = 256 25.1 us), fitted to 4600 shapes.
 struct AnyShape {
-  int shape, tm, tn, start, round, per_n[3], small_round, small_n[2], store[2];
+  int shape, tm, tn, start, round, per_n[3], small_round, small_n[2], store[2][2];
 };
-constexpr AnyShape ANY_SHAPES[] = {{4, 32, 128, 130, 285, {57, 66, 43}, 290, {71, 88}, {10, 200}},
-                                   {2, 64, 128, 50, 430, {70, 74, 55}, 300, {98, 117}, {110, 430}},
-                                   {3, 128, 128, -70, 490, {105, 115, 90}, 510, {115, 133}, {160, 770}},
-                                   {0, 128, 256, -270, 850, {170, 186, 148}, 0, {0, 0}, {230, 1500}}};
+constexpr AnyShape ANY_SHAPES[] = {{4, 32, 128, 130, 285, {57, 66, 43}, 290, {71, 88}, {{60, 0}, {245, 200}}},
+                                   {2, 64, 128, 50, 430, {70, 74, 55}, 300, {98, 117}, {{140, 200}, {505, 500}}},
+                                   {3, 128, 128, -70, 490, {105, 115, 90}, 510, {115, 133}, {{300, -60}, {960, 650}}},
+                                   {0, 128, 256, -270, 850, {170, 186, 148}, 0, {0, 0}, {{560, -160}, {1860, 1090}}}};
 
 // Whether the tile kernels for any group take the operands, their alignment apart.
 bool any_applies(const WView& v, int M) {
@@ -60,7 +62,9 @@ int any_shape(const WView& v, int M, int cus, int* time) {
     const long long tiles = (long long)((v.N + s.tn - 1) / s.tn) * ((M + s.tm - 1) / s.tm), rounds = (tiles + cus - 1) / cus;
     // (dword loads of codes: a tenth more)
     const long long per = (long long)(small ? s.small_n[f] : s.per_n[f]) * stages * (rag ? 11 : 10) / 10;
-    const long long t = s.start + rounds * ((small ? s.small_round : s.round) + per) + tiles * s.store[v.N % 4 != 0] / cus;
+    const int* const store = s.store[v.N % 4 != 0];
+    const long long out = tiles < cus ? tiles * store[0] / cus : store[0] + (tiles - cus) * store[1] / cus;
+    const long long t = s.start + rounds * ((small ? s.small_round : s.round) + per) + out;
     if (best < 0 || t < least) best = s.shape, least = t;
   }
   *time = least > 1 << 30 ? 1 << 30 : (int)least;
@@ -108,10 +112,11 @@ int other_time(const WView& v, int M, int cus) {
     const int form = v.mx ? 0 : v.gs % 32 == 0 ? 1 : 2;
     const OtherShape* c = &OTHER_STREAM64[pieces][form];
     int n = cpw;
-    long long share, whole = 64;  // in 64ths
+    long long share, whole = 64, more_rows = 0;  // share, whole: in 64ths
     if (M <= 8 || (M <= 16 && v.N < 8192)) {
       c = &OTHER_KSPLIT[pieces][form];
       share = 64 * ((tiles + cus - 1) / cus - 1);
+      if (M > 8 && n > 8) more_rows = 100 * (n - 8);
     } else {
       long long wgs = (long long)((v.N + 63) / 64) * ((M + 63) / 64);
       if (M <= 32) {
@@ -128,7 +133,7 @@ int other_time(const WView& v, int M, int cus) {
       // (up to 32 rows the shapes end at N = 16384, a workgroup a compute unit: on from there all but the start grows)
       if (M <= 32 && share > 64) whole = share;
     }
-    t = c->start + whole * c->per_n * n / 64 + share * (c->share_0 + c->share_n * n + (halves && M > 32 ? 110 : 0)) / 64;
+    t = c->start + more_rows + whole * c->per_n * n / 64 + share * (c->share_0 + c->share_n * n + (halves && M > 32 ? 110 : 0)) / 64;
   }
   return t > 1 << 30 ? 1 << 30 : (int)t;
 }
@@ -143,6 +148,11 @@ int general_rounds(const WView& v, int M, int cus) {
   const long long tiles = (v.N + 15) / 16, rounds = ((tiles + held - 1) / held + cus - 1) / cus;
   return (int)((rounds - 1) * (held == 1 ? 350 : 90));
 }
+
+// By how much blocks and tiles have to be ahead of the kernel before, of that kernel's time: an eighth, but no more than 1 us (the
+// general decode kernel: a twelfth), about the error of the times.  Of 12743 random shapes that blocks and tiles took over, 233
+// lost more than 5 % without a lead, 72 do with it, nearly all of them calls of less than 20 us (and 198 that gained as much are given up).
+int any_lead(int other, bool general) { return std::min(other, 800) / (general ? 12 : 8); }
 
 }  // namespace
 
@@ -167,32 +177,33 @@ AnyPlan any_plan(const WView& v, int M) {
   int tile = -1, tile_time = 1 << 30, block_shape = -1, block_t = 1 << 30;
   if (any_applies(v, M)) tile = any_shape(v, M, cus, &tile_time);
   if (whole) {
-    // blocks as block_plan() has them; tiles where these take less than three quarters of the time (the error of the times on
-    // both sides: M = 157, N = 9904, K = 12768, gs = 32 with zero-points at 0.79 92 us in blocks and 105 on tiles)
+    // blocks as block_plan() has them; tiles where these take less than 0.85 of the time (up to there 3 of 380 calls lost: M = 157,
+    // N = 9904, K = 12768, gs = 32 with zero-points 92 us in blocks and 105 on tiles; as many again gained 20 % between 0.75 and 0.85)
     block_shape = block_plan_time(v, M, &block_t);
     // (W4 groups of whole chunks: blocks scale a chunk's FP32 sums, tiles round every weight; 2.1e-4 and 2.7e-4 from the
     // product in FP64)
     if (block_shape >= 0 && !v.mx && v.gs % 128 == 0) return AnyPlan{1, block_shape};
     if (block_shape < 0) {
       if (decode_resident_applies(v, nullptr, nullptr, M)) return AnyPlan{3, -1};
-      return 8LL * tile_time < 7LL * other_time(v, M, cus) ? AnyPlan{2, tile} : AnyPlan{3, -1};
+      const int other = other_time(v, M, cus);
+      return tile_time < other - any_lead(other, false) ? AnyPlan{2, tile} : AnyPlan{3, -1};
     }
-    return 4LL * tile_time < 3LL * block_t ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
+    return 20LL * tile_time < 17LL * block_t ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
   }
   block_shape = block_any_time(v, M, cus, &block_t);
-  const int other = other_time(v, M, cus);
+  const bool general = !v.mx && decode_general_applies(v, nullptr, nullptr, M);
+  const int other = other_time(v, M, cus), rounds = (int)std::min((long long)other + general_rounds(v, M, cus), 1LL << 30);
   // (tiles are asked to beat that kernel's time without its further rounds: 33 to 64 rows of small groups take them 0.95 to
   // 1.4 times that kernel's time, and blocks 0.65 to 0.9; N = 11008, gs = 8, M = 64: K = 4096 29.2 -> 24.5 us)
   // Up to five rounds of its tiles they have to be ahead by a quarter: M = 41, N = 11504, K = 2176, gs = 8 13.1 us there and 18.3
   // on tiles, M = 54, N = 13936, K = 2752 18.1 and 21.6; past them M = 40, N = 28672, K = 4096 55 and 42.
-  const bool close = !v.mx && v.gs < 32 && M > 32 && tiles <= 5 * cus && decode_general_applies(v, nullptr, nullptr, M);
-  // Otherwise blocks and tiles have to be ahead by an eighth, about the error of the times (44570 random shapes, 13147 of which
-  // blocks or tiles took over: without it 578 lost more than 5 %, with it 74; it gives up 0.5 % of the gain).
-  const bool tiles_ahead = close ? 4LL * tile_time < 3LL * other : 8LL * tile_time < 7LL * other;
-  const bool blocks_ahead = 8LL * block_t < 7LL * ((long long)other + general_rounds(v, M, cus));
+  const bool close = general && v.gs < 32 && M > 32 && tiles <= 5 * cus;
+  // Otherwise blocks and tiles have to be ahead by any_lead().
+  const bool tiles_ahead = close ? 4LL * tile_time < 3LL * other : tile_time < other - any_lead(other, general);
+  const bool blocks_ahead = block_t < rounds - any_lead(rounds, general);
   if (!tiles_ahead && !blocks_ahead) return none;
-  // (blocks take about a tenth more than their time above where it is the least of all)
-  return tiles_ahead && (!blocks_ahead || 10LL * tile_time < 11LL * block_t) ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
+  // (50 calls of both: up to 1.05 tiles take 0.91 of the blocks' time, from 1.06 to 1.11 1.02 of it)
+  return tiles_ahead && (!blocks_ahead || 20LL * tile_time < 21LL * block_t) ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
 }
 
 bool try_tile_any(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out, int shape,
