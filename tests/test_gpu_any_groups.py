@@ -120,7 +120,8 @@ def test_ends_of_rows_bring_no_infinity(M, N, K, gs):
     # of K < 2^13 products are off by less than 2^-11 of it)
     sure = np.abs(ref) < 65504 - 2.0 ** -10 * (np.abs(x[rows].astype(np.float64)) @ np.abs(w.T))
     assert sure.mean() > 0.9 and not np.isnan(got[rows]).any() and np.isfinite(got[rows][sure]).all()
-    ok = np.isfinite(got[rows]) & (np.abs(ref) < 65504)
+    assert np.isfinite(ref).any() and np.isfinite(got[rows]).sum() >= np.isfinite(ref).sum() * 0.99
+    ok = np.isfinite(ref) & np.isfinite(got[rows])
     assert np.linalg.norm((got[rows] - ref)[ok]) <= 1e-3 * np.linalg.norm(ref[ok])
     assert np.array_equal(np.isnan(got[2]), np.isnan(bad[0])) and np.array_equal(np.isinf(got[2]), np.isinf(bad[0]))
 
