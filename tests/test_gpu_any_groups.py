@@ -58,7 +58,10 @@ TILES = [(4, 0, 1100, 257, 2080, 24), (4, 0, 2049, 257, 1032, 8), (4, 0, 2049, 1
          (6, 0, 1100, 2051, 2080, 24), (6, 0, 1100, 2051, 264, 8), (6, 0, 1100, 2051, 1056, 104), (6, 0, 700, 3001, 264, 40),
          (6, 1, 900, 3001, 2080, 24), (6, 1, 1100, 2051, 264, 8), (6, 1, 700, 3001, 1056, 40), (6, 1, 700, 3001, 264, 96),
          (6, 2, 900, 2310, 1056, 32), (6, 2, 900, 2310, 264, 32), (7, 0, 1300, 3001, 1056, 1056), (7, 0, 1300, 3001, 264, 40),
-         (7, 1, 2049, 2051, 1152, 40), (7, 1, 1300, 3001, 264, 128), (7, 2, 1700, 2310, 1056, 32), (7, 2, 1300, 3001, 264, 32)]
+         (7, 1, 2049, 2051, 1152, 40), (7, 1, 1300, 3001, 264, 128), (7, 2, 1700, 2310, 1056, 32), (7, 2, 1300, 3001, 264, 32),
+         (4, 1, 130, 3001, 264, 40), (5, 2, 900, 1034, 1056, 32)]
+# calls that tiles are behind in (us on tiles and on the kernels before): 8.1 and 7.5, 9.2 and 8.3, 6.0 and 5.8, 8.2 and 6.8
+TILES_BEHIND = [(0, 2049, 257, 264, 8), (1, 900, 777, 264, 24), (2, 520, 257, 264, 32), (2, 900, 1034, 264, 32)]
 BLOCKS = [(0, 5, 130, 4104, 8), (1, 9, 33, 3336, 24), (1, 17, 1034, 2056, 48), (0, 20, 15, 264, 40), (1, 33, 281, 1000, 16), (0, 50, 513, 5176, 72),
           (1, 64, 3, 1032, 1032), (1, 40, 2063, 4104, 8), (0, 100, 129, 2080, 128), (1, 130, 40, 1384, 48), (2, 17, 281, 1000, 32), (2, 50, 7, 3336, 32),
           (2, 130, 1001, 2072, 32), (1, 100, 2064, 1152, 48), (0, 333, 4080, 4096, 48), (1, 64, 3000, 2048, 96), (0, 120, 1477, 2304, 128),
@@ -73,6 +76,11 @@ BLOCKS = [(0, 5, 130, 4104, 8), (1, 9, 33, 3336, 24), (1, 17, 1034, 2056, 48), (
 @pytest.mark.parametrize("plan,fmt,M,N,K,gs", TILES)
 def test_tiles_of_any_group(plan, fmt, M, N, K, gs):
     assert _check(fmt, M, N, K, gs) == plan
+
+
+@pytest.mark.parametrize("fmt,M,N,K,gs", TILES_BEHIND)
+def test_calls_that_tiles_are_behind_in(fmt, M, N, K, gs):
+    assert _check(fmt, M, N, K, gs) == 0
 
 
 @pytest.mark.parametrize("fmt,M,N,K,gs", BLOCKS)
@@ -189,6 +197,8 @@ PLAN = [((1, 3991, 1551, 2048, 16), False), ((1, 3991, 1551, 2056, 16), True),  
         ((2, 30, 16320, 352, 32), False), ((2, 30, 16320, 1056, 32), True),       # 4.5 and 6.1
         ((1, 9, 8778, 1792, 1792), False), ((1, 9, 8778, 4096, 4096), True),      # 7.8 and 9.8
         ((1, 3052, 2271, 256, 96), False), ((1, 3052, 2272, 264, 96), True),      # 20.6 and 25.1
+        # small groups with zero-points on the stream kernel: 11.1 and 19.9
+        ((1, 53, 9712, 1024, 8), True), ((1, 20, 13824, 1024, 16), True),           # 9.5 and 18.8
         # gs = 32 with zero-points, blocks against its two smallest tiles (plan 0): 6.0 and 7.1, 7.4 and 8.0
         ((1, 68, 5712, 384, 32), False), ((1, 68, 2736, 384, 32), True), ((1, 66, 6464, 640, 32), False), ((1, 66, 4704, 640, 32), True)]
 

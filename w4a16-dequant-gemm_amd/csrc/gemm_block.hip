@@ -680,18 +680,28 @@ hipError_t block_go(const WView& v, const w4_half* x, w4_half* c, int M, hipStre
 // Blocks and what a wave needs for 128 k of one, in units of 10 ns, W4 and MXFP4 (N = 4096, K = 14336 with
 // as many rows as make one round of workgroups, and N = 5120, K = 13824; a call takes 3.5 us more).  Groups of whole
 // chunks cost 0.97 to 1.03 of it.
-// start, round, per_n: the time of a call is start + rounds of workgroups x (round + per_n x units of the first wave), per_n
-// for symmetric W4, W4 with zero-points (groups as GM = 1) and MXFP4 (as RAG); fitted to 6657 shapes of 3 to 4000 rows
-// that are not whole chunks and groups, K = 256 to 14336, to within 8 to 18 % (r.m.s.).
+// The time of a call is start + rounds of workgroups x (round + per_n x units of the first wave + store), per_n for symmetric
+// W4, W4 with zero-points and MXFP4, store where N is no multiple of 8 and halves leave one by one.  any: shapes that are not
+// whole tiles, chunks and groups (MXFP4: as RAG), fitted to 8000 of 5 to 4000 rows, K = 256 to 14336, to within 8 to 10 %
+// (r.m.s.); whole: the others.
+struct BkTime {
+  int start, round, per_n[3], store;
+};
 struct BkShape {
-  int nt, mt, cost_w4, cost_mx, start, round, per_n[3];
+  int nt, mt, cost_w4, cost_mx;
+  BkTime whole, any;
 };
 constexpr BkShape BK_SHAPES[] = {
-    {1, 1, 50, 45, 170, 130, {118, 133, 99}},      {2, 1, 83, 56, 140, 150, {188, 211, 139}},
-    {2, 2, 106, 89, 85, 210, {228, 247, 200}},     {4, 1, 136, 80, 110, 150, {334, 382, 223}},
-    {2, 4, 171, 155, 5, 300, {320, 335, 314}},     {4, 2, 175, 125, 70, 240, {390, 443, 303}},
-    {3, 4, 195, 173, -20, 370, {397, 426, 378}},   {4, 4, 260, 215, -45, 370, {505, 543, 458}},
-    {4, 5, 290, 250, -100, 450, {570, 617, 550}},  {4, 6, 330, 290, -110, 490, {624, 668, 634}}};
+    {1, 1, 50, 45, {170, 130, {118, 133, 99}, 0}, {149, 134, {104, 114, 95}, 20}},
+    {2, 1, 83, 56, {140, 150, {188, 211, 139}, 0}, {118, 184, {162, 182, 139}, 23}},
+    {2, 2, 106, 89, {85, 210, {228, 247, 200}, 0}, {114, 199, {197, 217, 192}, 37}},
+    {4, 1, 136, 80, {110, 150, {334, 382, 223}, 0}, {134, 192, {319, 335, 236}, 24}},
+    {2, 4, 171, 155, {5, 300, {320, 335, 314}, 0}, {79, 254, {283, 302, 373}, 50}},
+    {4, 2, 175, 125, {70, 240, {390, 443, 303}, 0}, {78, 296, {362, 415, 306}, 33}},
+    {3, 4, 195, 173, {-20, 370, {397, 426, 378}, 0}, {-18, 412, {416, 401, 395}, 100}},
+    {4, 4, 260, 215, {-45, 370, {505, 543, 458}, 0}, {-37, 448, {504, 485, 491}, 110}},
+    {4, 5, 290, 250, {-100, 450, {570, 617, 550}, 0}, {-75, 516, {543, 529, 560}, 90}},
+    {4, 6, 330, 290, {-110, 490, {624, 668, 634}, 0}, {-82, 586, {605, 626, 621}, 110}}};
 constexpr int BK_COUNT = sizeof BK_SHAPES / sizeof BK_SHAPES[0];
 
 long long bk_rounds(const WView& v, int M, const BkShape& s, int cus) {
@@ -699,15 +709,19 @@ long long bk_rounds(const WView& v, int M, const BkShape& s, int cus) {
   return ((ng + 7) / 8 * mg + cus / 8 - 1) / (cus / 8);
 }
 
-// Small groups take 1.15 of it (four selectors) and 0.03 us for every KB of a block's parameters, which are copied
-// first (N = 11008, K = 4096, gs = 8, M = 16, 32 x 16 blocks 15.7 us, the decode kernel 14.0), codes by the dword 1.06.
-int bk_time(const WView& v, int M, const BkShape& s, int cus) {
+// Small groups take 0.035 us for every KB of a block's parameters, which are copied first (N = 11008, K = 4096, gs = 8, M = 16,
+// 32 x 16 blocks 15.7 us, the decode kernel 14.0), and 4.5 us for another window of them; codes by the dword and rows past N
+// 1.23 of W4's units.  From three rounds on a call takes 1.08 of the sum (M = 789, N = 2896, K = 11680, gs = 40, twelve rounds
+// of 32 x 64: 137 us, tiles 97).
+int bk_time(const WView& v, int M, const BkShape& s, int cus, bool whole) {
+  const BkTime& b = whole ? s.whole : s.any;
   const int n = ((v.K + BK_UNIT - 1) / BK_UNIT + BK_WAVES - 1) / BK_WAVES;
-  long long per = s.per_n[v.mx ? 2 : v.symmetric ? 0 : 1];
-  if (!v.mx) per = per * (v.gs < 32 ? 115 : 100) / 100 * (bk_ragged(v) ? 106 : 100) / 100;
-  const long long copy = v.mx || v.gs >= 32 ? 0 : 16LL * s.nt * (2 * v.G + (v.symmetric ? 0 : 4 * words(v.G))) * 3 / 1024;
+  const long long per = b.per_n[v.mx ? 2 : v.symmetric ? 0 : 1] * (!v.mx && bk_ragged(v) ? 123 : 100) / 100;
+  const long long copy = v.mx || v.gs >= 32 ? 0 : 16LL * s.nt * (2 * v.G + (v.symmetric ? 0 : 4 * words(v.G))) * 7 / 2048;
   const int window = copy ? bk_window(v, s.nt) : BK_WHOLE, more = window > 0 && window < n ? (n - 1) / window : 0;
-  const long long t = s.start + bk_rounds(v, M, s, cus) * (s.round + copy + per * n + 150 * more);  // (another window: 1.5 us)
+  const long long rounds = bk_rounds(v, M, s, cus);
+  const long long sum = b.start + rounds * (b.round + copy + per * n + 450 * more + (v.N % 8 ? b.store : 0));
+  const long long t = rounds > 2 && !whole ? sum * 108 / 100 : sum;
   return t > 1 << 30 ? 1 << 30 : (int)t;
 }
 
@@ -837,7 +851,7 @@ hipError_t block_fmt(int shape, const WView& v, const w4_half* x, w4_half* c, in
 
 int block_plan_time(const WView& v, int M, int* time) {
   const int i = block_plan(v, M);
-  if (i >= 0) *time = bk_time(v, M, BK_SHAPES[i], device_cus());
+  if (i >= 0) *time = bk_time(v, M, BK_SHAPES[i], device_cus(), true);
   return i;
 }
 
@@ -850,7 +864,7 @@ int block_any_time(const WView& v, int M, int cus, int* time) {
   for (int i = 0; i < BK_COUNT; ++i) {
     const BkShape& s = BK_SHAPES[i];
     if (!bk_has(v.mx ? 2 : 0, s.nt, gm, bk_ragged(v)) || bk_window(v, s.nt) < 1) continue;
-    const int t = bk_time(v, M, s, cus);
+    const int t = bk_time(v, M, s, cus, false);
     if (best < 0 || t < *time) best = i, *time = t;
   }
   return best;

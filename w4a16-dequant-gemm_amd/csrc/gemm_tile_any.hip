@@ -38,7 +38,7 @@ struct AnyShape {
   int shape, tm, tn, start, round, per_n[3], small_round, small_n[2], store[2][2];
 };
 constexpr AnyShape ANY_SHAPES[] = {{4, 32, 128, 130, 285, {57, 66, 43}, 290, {71, 88}, {{60, 0}, {245, 200}}},
-                                   {2, 64, 128, 50, 430, {70, 74, 55}, 300, {98, 117}, {{140, 200}, {505, 500}}},
+                                   {2, 64, 128, 20, 430, {70, 74, 55}, 300, {98, 117}, {{140, 200}, {505, 500}}},
                                    {3, 128, 128, -70, 490, {105, 115, 90}, 510, {115, 133}, {{300, -60}, {960, 650}}},
                                    {0, 128, 256, -270, 850, {170, 186, 148}, 0, {0, 0}, {{560, -160}, {1860, 1090}}}};
 
@@ -116,7 +116,9 @@ int other_time(const WView& v, int M, int cus) {
     if (M <= 8 || (M <= 16 && v.N < 8192)) {
       c = &OTHER_KSPLIT[pieces][form];
       share = 64 * ((tiles + cus - 1) / cus - 1);
+      // (a second half of 16 rows: N = 2874, K = 4096, gs = 32 with zero-points, M = 15 8.4 us, 5.9 without the term)
       if (M > 8 && n > 8) more_rows = 100 * (n - 8);
+      if (M > 8 && n > 2 && pieces) more_rows += 30 * std::min(n, 8);
     } else {
       long long wgs = (long long)((v.N + 63) / 64) * ((M + 63) / 64);
       if (M <= 32) {
@@ -134,6 +136,9 @@ int other_time(const WView& v, int M, int cus) {
       if (M <= 32 && share > 64) whole = share;
     }
     t = c->start + more_rows + whole * c->per_n * n / 64 + share * (c->share_0 + c->share_n * n + (halves && M > 32 ? 110 : 0)) / 64;
+    // (a word's zero-point in small groups: 1.2 to 1.4 of the time in the stream kernels, N = 9712, K = 1024, gs = 8, M = 53 20.0 us,
+    // tiles 11.1)
+    if (pieces && !v.mx && !v.symmetric && v.gs < 32 && c != &OTHER_KSPLIT[pieces][form]) t = t * 5 / 4;
   }
   return t > 1 << 30 ? 1 << 30 : (int)t;
 }
@@ -149,10 +154,10 @@ int general_rounds(const WView& v, int M, int cus) {
   return (int)((rounds - 1) * (held == 1 ? 350 : 90));
 }
 
-// By how much blocks and tiles have to be ahead of the kernel before, of that kernel's time: an eighth, but no more than 1 us (the
-// general decode kernel: a twelfth), about the error of the times.  Of 12743 random shapes that blocks and tiles took over, 233
-// lost more than 5 % without a lead, 72 do with it, nearly all of them calls of less than 20 us (and 198 that gained as much are given up).
-int any_lead(int other, bool general) { return std::min(other, 800) / (general ? 12 : 8); }
+// By how much blocks and tiles have to be ahead of the kernel before: a twelfth of that kernel's time, but no more than 0.67 us,
+// about the error of the times.  Of 6009 random shapes with N, K >= 1024, all three kernels timed, 147 take more than 1.1 of the
+// best one's time with an eighth, 136 with a twelfth and 144 with a sixteenth; 69, 74 and 89 more than 1.05 of the kernel before's.
+int any_lead(int other) { return std::min(other, 800) / 12; }
 
 }  // namespace
 
@@ -186,7 +191,7 @@ AnyPlan any_plan(const WView& v, int M) {
     if (block_shape < 0) {
       if (decode_resident_applies(v, nullptr, nullptr, M)) return AnyPlan{3, -1};
       const int other = other_time(v, M, cus);
-      return tile_time < other - any_lead(other, false) ? AnyPlan{2, tile} : AnyPlan{3, -1};
+      return tile_time < other - any_lead(other) ? AnyPlan{2, tile} : AnyPlan{3, -1};
     }
     return 20LL * tile_time < 17LL * block_t ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
   }
@@ -199,11 +204,11 @@ AnyPlan any_plan(const WView& v, int M) {
   // on tiles, M = 54, N = 13936, K = 2752 18.1 and 21.6; past them M = 40, N = 28672, K = 4096 55 and 42.
   const bool close = general && v.gs < 32 && M > 32 && tiles <= 5 * cus;
   // Otherwise blocks and tiles have to be ahead by any_lead().
-  const bool tiles_ahead = close ? 4LL * tile_time < 3LL * other : tile_time < other - any_lead(other, general);
-  const bool blocks_ahead = block_t < rounds - any_lead(rounds, general);
+  const bool tiles_ahead = close ? 4LL * tile_time < 3LL * other : tile_time < other - any_lead(other);
+  const bool blocks_ahead = block_t < rounds - any_lead(rounds);
   if (!tiles_ahead && !blocks_ahead) return none;
-  // (50 calls of both: up to 1.05 tiles take 0.91 of the blocks' time, from 1.06 to 1.11 1.02 of it)
-  return tiles_ahead && (!blocks_ahead || 20LL * tile_time < 21LL * block_t) ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
+  // (with tiles up to 0.95, 1 and 1.05 of the blocks' time 259, 228 and 229 of 8000 calls take more than 1.1 of the best time)
+  return tiles_ahead && (!blocks_ahead || tile_time < block_t) ? AnyPlan{2, tile} : AnyPlan{1, block_shape};
 }
 
 bool try_tile_any(const WView& v, const w4_half* x, w4_half* c, int M, hipStream_t s, w4_half* w_out, int shape,
